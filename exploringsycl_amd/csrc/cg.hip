@@ -144,12 +144,24 @@ struct FusedWArgs {
   double alpha, beta;
   int apply_u, ring;
   // Pair-per-thread kernel only: the new u goes to u_out (u itself for the
-  // iteration the host asked for, a spare buffer when it runs ahead), and
-  // with dev_beta non-null beta is read from the device (the value the run
-  // ahead formed from the device's own partials).
+  // iteration the host asked for, a spare buffer when it runs ahead).
   double* u_out;
-  const double* dev_beta;
 };
+
+template <bool CONSUME>
+__device__ inline double ra_scalar(const RaScalar& s, double value) {
+  if (!CONSUME) return s.dev ? *s.dev : value;
+  double sum[1];
+  const double rro = s.rro_dev ? *s.rro_dev : s.rro;
+  consume_sums<1>(s.sub, s.nblk, sum);
+  const double q = s.inverse ? sum[0] / rro : rro / sum[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (s.sum_dev) *s.sum_dev = sum[0];
+    s.out[0] = sum[0];
+    s.out[1] = q;
+  }
+  return q;
+}
 
 // Cells of one thread are visited in batches of BATCH: all loads of a batch
 // are issued before any of its arithmetic and stores, so each wave keeps
@@ -351,11 +363,10 @@ __device__ inline void fused_pair_load(const Geo& g, const FusedWArgs& a,
 // the in-lane pair sum of p_new . w (the first level of the reduction tree).
 template <bool APPLY_P>
 __device__ inline double fused_pair_compute(const Geo& g, const FusedWArgs& a,
-                                            const FusedPair& s, int lane) {
+                                            const FusedPair& s, int lane, double beta) {
   const int x = g.x;
   const int xl = g.h, xr = g.x - g.h - 1, yb = g.h, yt = g.y - g.h - 1;
   const double* __restrict__ P = a.p_old;
-  const double beta = a.dev_beta ? *a.dev_beta : a.beta;
   const int i = s.e0;
   // Neighbours across the pair boundary, from the adjacent lanes.
   double pl = from_prev_lane(s.P0.y), pr = from_next_lane(s.P0.x);
@@ -464,27 +475,27 @@ __global__ __launch_bounds__(kBlock) void fused_w2_kernel(Geo g, FusedWArgs a,
     for (int j = 0; j < SB; ++j) fused_pair_load<APPLY_P>(g, a, s[j]);
 #pragma unroll
     for (int j = 0; j < SB; ++j)
-      psum[s0 + j] = fused_pair_compute<APPLY_P>(g, a, s[j], lane);
+      psum[s0 + j] = fused_pair_compute<APPLY_P>(g, a, s[j], lane, a.beta);
   }
   span_reduce_pairs(psum, partials, nspan, span, single_group != 0);
 }
 
 // One pair per thread: a 256-thread block covers 512 cells (8 groups of the
-// reduction tree) and stores their 8-leaf subtree sum in sub[block];
-// span_finish_kernel then combines the 8 blocks of each span.  Small blocks
+// reduction tree) and stores their 8-leaf subtree sum.  Small blocks
 // keep 4x more waves per SIMD in flight than the span-per-block kernel.
-template <bool APPLY_P, int KS>
-__global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs a,
+// With CONSUME beta is formed from the sums of the r-step before it.
+template <bool APPLY_P, int KS, bool CONSUME = false>
+__global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs a, RaScalar sc,
                                                                double* sub, int nblk, int S) {
   int tid;
   const int blk = stacked_block<KS, kBlock>(S, &tid);
-  if (blk >= nblk) return;
   const int lane = threadIdx.x & (kWave - 1);
   FusedPair s;
-  fused_pair_index(g, blk * kPairBlock + 2 * tid, s);
+  fused_pair_index(g, blk < nblk ? blk * kPairBlock + 2 * tid : g.n, s);
   fused_pair_load<APPLY_P>(g, a, s);
-  double v[1] = {fused_pair_compute<APPLY_P>(g, a, s, lane)};
-  wave_subtree_pairs<1>(v, sub, nblk, blk, tid / kWave);
+  const double beta = ra_scalar<CONSUME>(sc, a.beta);
+  const double v[1] = {fused_pair_compute<APPLY_P>(g, a, s, lane, beta)};
+  block_sums_pairs<1, KS>(v, sub, nblk, blk, tid);
 }
 
 // Launches fused_w1_kernel with stack_factor(c) blocks one row apart per
@@ -493,18 +504,17 @@ __global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs
 // iteration from 269.2 to 267.6 us and the mixed-precision w-step from 83.2
 // to 79.0 us (four: 270.6 us).
 template <bool APPLY_P>
-void launch_fused_w1(tea_hip_chunk* c, const FusedWArgs& a) {
+void launch_fused_w1(tea_hip_chunk* c, const FusedWArgs& a, const RaScalar& sc = {}) {
   const int S = stack_rows(c), ks = stack_factor(c);
-  const dim3 grid = stacked_grid(c, ks);
-  if (ks == 1)
-    hipLaunchKernelGGL((fused_w1_kernel<APPLY_P, 1>), grid, dim3(kBlock), 0, c->stream,
-                       c->geo, a, c->sub, c->nblk, S);
-  else if (ks == 2)
-    hipLaunchKernelGGL((fused_w1_kernel<APPLY_P, 2>), grid, dim3(2 * kBlock), 0, c->stream,
-                       c->geo, a, c->sub, c->nblk, S);
-  else
-    hipLaunchKernelGGL((fused_w1_kernel<APPLY_P, 4>), grid, dim3(4 * kBlock), 0, c->stream,
-                       c->geo, a, c->sub, c->nblk, S);
+  const auto kernel =
+      sc.sub ? (ks == 1   ? fused_w1_kernel<APPLY_P, 1, true>
+                : ks == 2 ? fused_w1_kernel<APPLY_P, 2, true>
+                          : fused_w1_kernel<APPLY_P, 4, true>)
+             : (ks == 1   ? fused_w1_kernel<APPLY_P, 1>
+                : ks == 2 ? fused_w1_kernel<APPLY_P, 2>
+                          : fused_w1_kernel<APPLY_P, 4>);
+  hipLaunchKernelGGL(kernel, stacked_grid(c, ks), dim3(ks * kBlock), 0, c->stream, c->geo, a, sc,
+                     c->sub, c->nblk, S);
 }
 
 __global__ __launch_bounds__(kBlock) void fused_r2_kernel(
@@ -538,12 +548,11 @@ __global__ __launch_bounds__(kBlock) void fused_r2_kernel(
 
 // fused_r2's arithmetic with one pair per thread; the block stores its
 // 8-leaf subtree of r.r (see fused_w1_kernel).  The new r goes to r_out (r
-// itself, or a spare buffer when the iteration runs ahead), and with
-// dev_alpha non-null alpha is read from the device.
+// itself, or a spare buffer when the iteration runs ahead).
+template <bool CONSUME>
 __global__ __launch_bounds__(kBlock) void fused_r1_kernel(
-    Geo g, const double* r, double* r_out, const double* __restrict__ w, double alpha,
-    const double* __restrict__ dev_alpha, double* sub, int nblk) {
-  if (dev_alpha) alpha = *dev_alpha;
+    Geo g, const double* r, double* r_out, const double* __restrict__ w, double value,
+    RaScalar sc, double* sub, int nblk) {
   const int blk = blockIdx.x;
   const int e = blk * kPairBlock + 2 * threadIdx.x;
   const int row = e < g.n ? (int)g.dx.div((uint32_t)e) : 0;
@@ -552,11 +561,12 @@ __global__ __launch_bounds__(kBlock) void fused_r1_kernel(
   const bool in1 = e < g.n && interior(g, kk + 1, row);
   const int i = (in0 || in1) ? e : 0;
   const double2 rv = ld2_nt(r, i), wv = ld2_nt(w, i);
+  const double alpha = ra_scalar<CONSUME>(sc, value);
   const double ra = rv.x - alpha * wv.x;
   const double rb = rv.y - alpha * wv.y;
-  double v[1] = {(in0 ? ra * ra : 0.0) + (in1 ? rb * rb : 0.0)};
+  const double v[1] = {(in0 ? ra * ra : 0.0) + (in1 ? rb * rb : 0.0)};
   st2_nt(r_out, e, in0, in1, ra, rb);
-  wave_subtree_pairs<1>(v, sub, nblk, blk);
+  block_sums_pairs<1>(v, sub, nblk, blk, threadIdx.x);
 }
 
 // r -= alpha w and r.r: all 16 cells' loads first, then the updates.
@@ -641,8 +651,8 @@ __global__ __launch_bounds__(kBlock) void norm_pair_kernel(
     Geo g, const double* __restrict__ b, double* sub, int nblk) {
   const PairAt q = pair_at(g, blockIdx.x * kPairBlock + 2 * threadIdx.x);
   const double2 v = ld2_nt(b, q.ic);
-  double s[1] = {(q.in0 ? v.x * v.x : 0.0) + (q.in1 ? v.y * v.y : 0.0)};
-  wave_subtree_pairs<1>(s, sub, nblk, blockIdx.x);
+  const double s[1] = {(q.in0 ? v.x * v.x : 0.0) + (q.in1 ? v.y * v.y : 0.0)};
+  block_sums_pairs<1>(s, sub, nblk, blockIdx.x, threadIdx.x);
 }
 
 struct FinaliseBody {
@@ -699,7 +709,10 @@ int sync_p_alt(tea_hip_chunk* c) {
 // forms the same scalars itself: the last block of each finisher runs the
 // host's final tree passes over the grid's partials and divides
 // (span_finish_kernel's run-ahead tail, core.hip), and the next pass of the
-// iteration is already queued behind it, writing only spare buffers:
+// iteration is already queued behind it, writing only spare buffers (on grids
+// of at most kConsumeBlocks blocks there is no finisher: the next pass itself
+// sums and divides, see RaScalar, and its first block hands the host the
+// values):
 //   after cg_calc_w  (the r-step): r - alpha w into r_alt, and r.r;
 //   after cg_calc_ur (the w-step): u + alpha p into u_alt, p = beta p + r
 //     into p_alt with the U/P halo ring, w = A p into w_alt, p.w; then the
@@ -764,30 +777,52 @@ int ensure_ra(tea_hip_chunk* c) {
   return TEA_HIP_OK;
 }
 
-// The finisher of a run-ahead pass (into the device's partials) with its
-// scalar (into host slot (set, kind)).
-int ra_finish(tea_hip_chunk* c, int set, int kind, double rro, bool from_dev) {
+// The next pass forms the scalar of the pass before it (RaScalar::sub).
+bool ra_consume(const tea_hip_chunk* c) { return c->nblk <= kConsumeBlocks; }
+
+// Arms host slot (set, kind) for the pass just queued, a w-step (kRaW) or
+// an r-step, and sets *sc to where the pass after it takes its scalar: the
+// device's, left there by a finisher launched here, or the pass's block
+// sums.  Either counts as one cg_ra_finish launch in the statistics.
+int ra_finish(tea_hip_chunk* c, int set, int kind, double rro, bool from_dev, RaScalar* sc) {
   if (c->ra_dirty) {
     // A dropped run-ahead may still be queued and write these slots.
     TEA_HIP_TRY(hipStreamSynchronize(c->stream));
     c->ra_dirty = false;
   }
   arm_host_values(ra_host_slot(c, set, kind), 2);
+  *sc = RaScalar{};
+  if (ra_consume(c)) {
+    sc->sub = kind == kRaW ? c->sub : c->sub2;
+    sc->nblk = c->nblk;
+    sc->inverse = kind == kRaW ? 0 : 1;
+    sc->rro = rro;
+    sc->rro_dev = from_dev ? c->ra_dev + 2 : nullptr;
+    sc->sum_dev = kind == kRaW ? nullptr : c->ra_dev + 2;
+    sc->out = ra_dev_slot(c, set, kind);
+    if (c->timing && c->time_kernel[K_CG_RA_FINISH]) c->launches[K_CG_RA_FINISH] += 1;
+    return TEA_HIP_OK;
+  }
+  sc->dev = c->ra_dev + (kind == kRaW ? 0 : 1);
   const RaTail tail{rro, from_dev ? 1 : 0, kind == kRaW ? 0 : 1, c->ra_dev,
                     ra_dev_slot(c, set, kind), c->ra_count};
   return launch_span_finish_ra(c, c->ra_dev + 3, tail);
 }
 
-// The r-step behind a w-step whose p.w the slot set's ratio turns into
-// alpha: r_alt = r - alpha w, r.r, beta.
+// The r-step behind a w-step that was just queued: alpha from its p.w (and
+// rro), r_alt = r - alpha w, r.r; c->ra_next is where the next w-step will
+// take beta from.
 int ra_launch_r(tea_hip_chunk* c, int set, const double* w, double rro, bool from_dev) {
+  RaScalar sc;
+  TEA_RETURN_IF(ra_finish(c, set, kRaW, rro, from_dev, &sc));
   {
     Timed t(c, K_CG_FUSED_R);
-    hipLaunchKernelGGL(fused_r1_kernel, pair_grid(c), dim3(kBlock), 0, c->stream, c->geo,
-                       c->field[TEA_FIELD_R], c->r_alt, w, 0.0, c->ra_dev, c->sub, c->nblk);
+    hipLaunchKernelGGL(sc.sub ? fused_r1_kernel<true> : fused_r1_kernel<false>, pair_grid(c),
+                       dim3(kBlock), 0, c->stream, c->geo, c->field[TEA_FIELD_R], c->r_alt, w,
+                       0.0, sc, sc.sub ? c->sub2 : c->sub, c->nblk);
   }
   TEA_HIP_TRY(hipGetLastError());
-  return ra_finish(c, set, kRaRStep, rro, from_dev);
+  return ra_finish(c, set, kRaRStep, rro, from_dev, &c->ra_next);
 }
 
 // Waits for a slot's sum and scalar.
@@ -931,7 +966,7 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
   FusedWArgs args{f[TEA_FIELD_P], c->p_alt,        f[TEA_FIELD_R],
                   f[TEA_FIELD_U], f[TEA_FIELD_W],  f[TEA_FIELD_KX],
                   f[TEA_FIELD_KY], c->pend_alpha,  c->pend_beta,
-                  c->pend_u ? 1 : 0, c->pend_halo ? 1 : 0, f[TEA_FIELD_U], nullptr};
+                  c->pend_u ? 1 : 0, c->pend_halo ? 1 : 0, f[TEA_FIELD_U]};
   c->pend_u = c->pend_p = c->pend_halo = false;
   int plen = c->nspan;
   if (use_pair_blocks(c, 1)) {
@@ -958,7 +993,6 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
     TEA_HIP_TRY(hipGetLastError());
     if (ahead) {
       const int set = c->ra_set ^ 1;
-      TEA_RETURN_IF(ra_finish(c, set, kRaW, c->ra_rro, false));
       TEA_RETURN_IF(ra_launch_r(c, set, f[TEA_FIELD_W], c->ra_rro, false));
       if (apply_p) swap_ptr(f[TEA_FIELD_P], c->p_alt);
       c->ra = kRaR;
@@ -1010,32 +1044,33 @@ int tea_hip_cg_calc_ur(tea_hip_chunk* c, double alpha, double* rrn) {
     // The r-step in flight used the device's alpha: take it over when the
     // host's is the same.
     if (alpha == c->ra_alpha && !c->pend_u && !c->pend_p && !c->pend_halo && !c->held &&
-        c->pre_halo < 0) {
+        c->pre_halo < 0 && ra_possible(c)) {
       swap_ptr(f[TEA_FIELD_R], c->r_alt);
       c->pend_u = true;
       c->pend_alpha = alpha;
       const int set = c->ra_set;
       c->ra = kRaNone;
-      if (ra_possible(c)) {
-        // Queue the next w-step (its beta from the device) and r-step
-        // before waiting for this r.r.
-        TEA_RETURN_IF(sync_p_alt(c));
-        const int next = set ^ 1;
-        FusedWArgs a{f[TEA_FIELD_P], c->p_alt,  f[TEA_FIELD_R], f[TEA_FIELD_U],
-                     c->w_alt,       f[TEA_FIELD_KX], f[TEA_FIELD_KY], alpha,
-                     0.0,            1,         1,              c->u_alt,
-                     c->ra_dev + 1};
-        {
-          Timed t(c, K_CG_FUSED_W);
-          launch_fused_w1<true>(c, a);
-        }
-        TEA_HIP_TRY(hipGetLastError());
-        TEA_RETURN_IF(ra_finish(c, next, kRaW, 0.0, true));
-        TEA_RETURN_IF(ra_launch_r(c, next, c->w_alt, 0.0, true));
-        c->ra = kRaWR;
-        c->ra_set = next;
-        c->ra_w_alpha = alpha;
+      // Queue the next w-step (its beta from the device) and r-step
+      // before waiting for this r.r.
+      TEA_RETURN_IF(sync_p_alt(c));
+      const int next = set ^ 1;
+      FusedWArgs a{f[TEA_FIELD_P], c->p_alt,  f[TEA_FIELD_R], f[TEA_FIELD_U],
+                   c->w_alt,       f[TEA_FIELD_KX], f[TEA_FIELD_KY], alpha,
+                   0.0,            1,         1,              c->u_alt};
+      // beta's rro is the r.r the host was last given (a consuming pass
+      // overwrites the device's copy).
+      RaScalar sc = c->ra_next;
+      sc.rro = c->ra_rro;
+      sc.rro_dev = nullptr;
+      {
+        Timed t(c, K_CG_FUSED_W);
+        launch_fused_w1<true>(c, a, sc);
       }
+      TEA_HIP_TRY(hipGetLastError());
+      TEA_RETURN_IF(ra_launch_r(c, next, c->w_alt, 0.0, true));
+      c->ra = kRaWR;
+      c->ra_set = next;
+      c->ra_w_alpha = alpha;
       double sum = 0.0, beta = 0.0;
       TEA_RETURN_IF(ra_wait(c, set, kRaRStep, &sum, &beta));
       c->ra_beta = beta;
@@ -1060,9 +1095,9 @@ int tea_hip_cg_calc_ur(tea_hip_chunk* c, double alpha, double* rrn) {
   if (use_pair_blocks(c, 2)) {
     {
       Timed t(c, K_CG_FUSED_R);
-      hipLaunchKernelGGL(fused_r1_kernel, pair_grid(c), dim3(kBlock), 0,
+      hipLaunchKernelGGL(fused_r1_kernel<false>, pair_grid(c), dim3(kBlock), 0,
                          c->stream, c->geo, f[TEA_FIELD_R], f[TEA_FIELD_R], f[TEA_FIELD_W],
-                         alpha, nullptr, c->sub, c->nblk);
+                         alpha, RaScalar{}, c->sub, c->nblk);
     }
     TEA_HIP_TRY(hipGetLastError());
     TEA_RETURN_IF(launch_span_finish(c, 1, &rlen, 0, true));

@@ -183,16 +183,13 @@ static double host_tree_passes(double* v, size_t len) {
   return v[0];
 }
 
-// Level-2 partial of each span from the 32 wave sums of its 8 blocks (zero
-// for blocks past the grid, as the reference pads its level-2 input with
-// zeros), then the next tree pass.  A 512-thread block covers 64 spans, one
-// group of that pass: thread t takes 512-cell block 512 b + t and its four
-// contiguous wave sums (so the loads coalesce), forms (w0 + w1) + (w2 + w3),
-// lanes 8j..8j+7 then combine the span's 8 blocks pairwise (steps s = 8, 16,
-// 32 of the level-2 tree), and wave 0 runs the group's tree over the 64 span
-// partials (zero past nspan).  With a single span there is no further pass
-// and its partial is the sum.
-constexpr int kFinishBlock = kSubPerSpan * kWave;  // 512 threads = 64 spans
+// The next tree pass over the spans from the block sums (zero past the grid,
+// as the reference pads its level-2 input with zeros).  A 512-thread block
+// covers 512 blocks = 64 spans, one group of that pass: wave w runs the tree
+// over 64 block sums (8 spans), then the eight wave sums are combined.  With
+// a single span there is no further pass and its partial is the sum (the
+// other spans' zeros add nothing).
+constexpr int kFinishBlock = kGroupBlocks;  // 512 threads = 64 spans
 
 // The host's final tree passes (host_tree_passes) over len <= 64^2 values
 // in one wave; buf is LDS of 64 doubles.  Lane 0 returns the sum.
@@ -215,38 +212,27 @@ template <int NR, bool TAIL = false>
 __global__ __launch_bounds__(kFinishBlock) void span_finish_kernel(
     const double* __restrict__ sub, int nblk, double* partials, int nspan,
     RaTail tail = RaTail{}) {
-  __shared__ double lds[NR][kWave];
+  __shared__ double lds[kWave];
+  __shared__ double ws[NR][kFinishBlock / kWave];
   const int t = threadIdx.x;
   const int lane = t & (kWave - 1);
-  const int blk = blockIdx.x * kFinishBlock + t;
-  const int span = blk / kSubPerSpan;
   // Every sum's loads first (a round per sum was waited for sum by sum).
-  const bool in = blk < nblk && span < nspan;
-  double w[NR][kWaves];
+  double w[NR];
 #pragma unroll
   for (int q = 0; q < NR; ++q)
-#pragma unroll
-    for (int k = 0; k < kWaves; ++k)
-      w[q][k] = sub[(size_t)q * kWaves * nblk + (in ? kWaves * blk + k : 0)];
+    w[q] = sub[(size_t)q * sub_stride(nblk) + blockIdx.x * kFinishBlock + t];
 #pragma unroll
   for (int q = 0; q < NR; ++q) {
-    if (!in) w[q][0] = w[q][1] = w[q][2] = w[q][3] = 0.0;
-    double v = (w[q][0] + w[q][1]) + (w[q][2] + w[q][3]);
-    v = v + __shfl_xor(v, 1);
-    v = v + __shfl_xor(v, 2);
-    v = v + __shfl_xor(v, 4);
-    if ((t & (kSubPerSpan - 1)) == 0) lds[q][t / kSubPerSpan] = v;
+    const double v = wave_tree_dpp(w[q]);
+    if (lane == 0) ws[q][t / kWave] = v;
   }
   __syncthreads();
   if (t >= kWave) return;
 #pragma unroll
   for (int q = 0; q < NR; ++q) {
-    if (nspan == 1) {
-      if (blockIdx.x == 0 && lane == 0) partials[q * nspan] = lds[q][0];
-      continue;
-    }
-    const double g3 = wave_tree(lds[q][lane]);
-    if (lane == 0) partials[q * nspan + blockIdx.x] = g3;
+    const double v = ((ws[q][0] + ws[q][1]) + (ws[q][2] + ws[q][3])) +
+                     ((ws[q][4] + ws[q][5]) + (ws[q][6] + ws[q][7]));
+    if (lane == 0) partials[(size_t)q * nspan + blockIdx.x] = v;
   }
   if (!TAIL) return;
   // The last block to store its partial (device-scope release before the
@@ -260,7 +246,7 @@ __global__ __launch_bounds__(kFinishBlock) void span_finish_kernel(
   if (prev != gridDim.x - 1) return;
   __threadfence();
   const int len = nspan == 1 ? 1 : (int)gridDim.x;
-  const double sum = wave_tree_passes(partials, len, &lds[0][0]);
+  const double sum = wave_tree_passes(partials, len, lds);
   if (lane != 0) return;
   const double r0 = tail.from_dev ? tail.ra[2] : tail.rro;
   double q;
@@ -450,10 +436,16 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
     set_error("hipMalloc of the second p buffer failed");
     return fail(TEA_HIP_ENOMEM);
   }
-  if (hipMalloc(&c->sub, (size_t)kSubMaxNr * kWaves * c->nblk * sizeof(double)) != hipSuccess) {
+  const size_t sbytes = (size_t)kSubMaxNr * sub_stride(c->nblk) * sizeof(double);
+  if (hipMalloc(&c->sub, 2 * sbytes) != hipSuccess) {
     c->sub = nullptr;
-    set_error("hipMalloc of the subtree sums failed");
+    set_error("hipMalloc of the block sums failed");
     return fail(TEA_HIP_ENOMEM);
+  }
+  c->sub2 = c->sub + sbytes / sizeof(double);
+  if (hipMemsetAsync(c->sub, 0, 2 * sbytes, c->stream) != hipSuccess) {
+    set_error("hipMemsetAsync failed");
+    return fail(TEA_HIP_EHIP);
   }
   const size_t pbytes = 4 * (size_t)c->nspan * sizeof(double);
   if (hipHostMalloc(&c->host_partials, pbytes,

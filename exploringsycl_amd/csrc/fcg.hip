@@ -150,9 +150,8 @@ __global__ __launch_bounds__(kBlock) void fcg_z2_kernel(
   span_reduce_pairs_n<1>(psum, partials, nspan, span, single_group != 0);
 }
 
-// fcg_z2_kernel's arithmetic with one pair per thread; the waves store their
-// z.w sums for span_finish_kernel (see wave_subtree_pairs).  Lane 63 loads
-// the right neighbour's kx with the pair's own loads.
+// fcg_z2_kernel's arithmetic with one pair per thread.  Lane 63 loads the
+// right neighbour's kx with the pair's own loads.
 template <int NL>
 __global__ __launch_bounds__(kBlock) void fcg_z1_kernel(
     Geo g, const float* __restrict__ r, const float* __restrict__ kx,
@@ -206,7 +205,7 @@ __global__ __launch_bounds__(kBlock) void fcg_z1_kernel(
   double v[1] = {(in0 ? (double)za * (double)W.x : 0.0) +
                  (in1 ? (double)zb * (double)W.y : 0.0)};
   if (any) st2(z, e, in0, in1, za, zb);
-  wave_subtree_pairs<1>(v, sub, nblk, blk);
+  block_sums_pairs<1>(v, sub, nblk, blk, threadIdx.x);
 }
 
 // The coarse values of a quad's four cells for one level.  With a
@@ -277,7 +276,7 @@ __global__ __launch_bounds__(kQuadThreads) void fcg_z4_kernel(
   }
   double v[1] = {(prod[0] + prod[1]) + (prod[2] + prod[3])};
   if (any) st4(z, e, in, zv);
-  wave_subtree_quads<1>(v, sub, nblk, blk, threadIdx.x / kWave);
+  block_sums_quads<1>(v, sub, nblk, blk, threadIdx.x);
 }
 
 // The coarse operator T = P^T A P / c^2: for each coarse cell, the face
@@ -1529,7 +1528,7 @@ static int launch_precondition(tea_hip_chunk* c, int use_net, int slot, int* len
   const CoarseTerm t1 = nl > 1 ? term(1) : none;
   const int kid = nl == 0 ? K_FCG_JACOBI : K_FCG_PROLONG;
   if (precondition_quads(c, use_net)) {
-    double* sub = c->sub + (size_t)(sub_q > 0 ? sub_q : 0) * kWaves * c->nblk;
+    double* sub = c->sub + (size_t)(sub_q > 0 ? sub_q : 0) * sub_stride(c->nblk);
     {
       Timed t(c, kid);
       if (nl == 0)

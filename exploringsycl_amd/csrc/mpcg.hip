@@ -350,8 +350,7 @@ __global__ __launch_bounds__(kBlock) void mp_w2_kernel(Geo g, MpArgs a,
 
 template __global__ void mp_w2_kernel<true, 4>(Geo, MpArgs, double*, int, int);
 
-// One pair per thread: the block's 8-leaf subtrees go to sub (see
-// block_subtree_pairs) and span_finish_kernel completes the spans.
+// One pair per thread.
 template <bool DOT2>
 __global__ __launch_bounds__(kBlock) void mp_w1_kernel(Geo g, MpArgs a,
                                                        double* sub, int nblk) {
@@ -362,7 +361,7 @@ __global__ __launch_bounds__(kBlock) void mp_w1_kernel(Geo g, MpArgs a,
   mp_pair_load<DOT2>(g, a, s);
   double ps[DOT2 ? 2 : 1];
   mp_pair_compute<DOT2>(g, a, s, lane, ps);
-  wave_subtree_pairs<DOT2 ? 2 : 1>(ps, sub, nblk, blk);
+  block_sums_pairs<DOT2 ? 2 : 1>(ps, sub, nblk, blk, threadIdx.x);
 }
 
 template __global__ void mp_w1_kernel<true>(Geo, MpArgs, double*, int);
@@ -388,26 +387,24 @@ __device__ inline void ring_store(T* f, int i, int kc, int rc, int x, int xl, in
 // by cell, with 16-byte loads of the FP32 operands and of u.  The
 // neighbours across lanes move on the DPP wave shifts; lane 0 loads p and r
 // at e0 - 1, lane 63 p, r and kx at e0 + 4.  The in-lane dot sums are
-// ((v0 + v1) + (v2 + v3)), tree steps 1 and 2, and the waves store their
-// sums for span_finish_kernel (wave_subtree_quads).  UM selects the u
+// ((v0 + v1) + (v2 + v3)), tree steps 1 and 2 (block_sums_quads).  UM selects the u
 // update: none, u += alpha p_old, or u = ((u + alpha_h p_h) + alpha_h2
 // p_h2) + alpha p_old (two held updates and this step's, each rounded as
 // when made one by one).  A workgroup of KS x 128 threads takes KS blocks
 // one row apart (block c + S t, t = KS j .. KS j + KS - 1, S = x / 512;
-// blocks past the grid return at once), which share their rows above and
+// blocks past the grid touch no cell), which share their rows above and
 // below in the CU's L1.
 template <bool DOT2, int UM, int KS>
 __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs a, double* sub,
                                                                   int nblk, int S) {
   int tid;
   const int blk = stacked_block<KS, kQuadThreads>(S, &tid);
-  if (blk >= nblk) return;
   const int lane = threadIdx.x & (kWave - 1);
   const int x = g.x;
   const int xl = g.h, xr = g.x - g.h - 1, yb = g.h, yt = g.y - g.h - 1;
   const float* __restrict__ P = a.p_old;
   const float* __restrict__ R = a.r;
-  const int e = blk * kQuadBlock + 4 * tid;
+  const int e = blk < nblk ? blk * kQuadBlock + 4 * tid : g.n;
   const int row = e < g.n ? (int)g.dx.div((uint32_t)e) : 0;
   const int kk = e - row * x;
   bool in[4];
@@ -431,7 +428,7 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
   // each 16-byte load and store covers 1 KB of consecutive cells (32 bytes
   // per lane in the quad layout took two instructions over every other
   // 16 bytes).  The p_old values come from the quad lanes by permute.
-  const int ua = blk * kQuadBlock + (tid / kWave) * (4 * kWave) + 2 * lane;
+  const int ua = blk < nblk ? blk * kQuadBlock + (tid / kWave) * (4 * kWave) + 2 * lane : g.n;
   const int ub = ua + 2 * kWave;
   const int rA = ua < g.n ? (int)g.dx.div((uint32_t)ua) : 0;
   const int kA = ua - rA * x;
@@ -576,7 +573,7 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
         if (in[c]) ring_store(a.p_new, e + c, kk + c, row, x, xl, xr, yb, yt, pc[c]);
     }
   }
-  wave_subtree_quads<DOT2 ? 2 : 1>(v, sub, nblk, blk, tid / kWave);
+  block_sums_quads<DOT2 ? 2 : 1, KS>(v, sub, nblk, blk, tid);
 }
 
 
@@ -636,7 +633,7 @@ __global__ __launch_bounds__(kBlock) void mp_r1_kernel(
     v[RW ? 1 : 0] = (in0 ? (double)ra * (double)wv.x : 0.0) +
                     (in1 ? (double)rb * (double)wv.y : 0.0);
   st2(r, e, in0, in1, ra, rb);
-  wave_subtree_pairs<RW ? 2 : 1>(v, sub, nblk, blk);
+  block_sums_pairs<RW ? 2 : 1>(v, sub, nblk, blk, threadIdx.x);
 }
 
 // The same four cells per lane (x a multiple of 4).
@@ -667,13 +664,12 @@ __global__ __launch_bounds__(kQuadThreads) void mp_r4_kernel(
   for (int q = 0; q < (RW ? 2 : 1); ++q)
     v[q] = (prod[q][0] + prod[q][1]) + (prod[q][2] + prod[q][3]);
   if (any) st4(r, e, in, rn);
-  wave_subtree_quads<RW ? 2 : 1>(v, sub, nblk, blk, threadIdx.x / kWave);
+  block_sums_quads<RW ? 2 : 1>(v, sub, nblk, blk, threadIdx.x);
 }
 
 // MpTrueResidualBody's arithmetic (below) with one cell pair per thread (x
 // even): r = u0 - A u in FP64 with the FP64 coefficients, r rounded to FP32
-// into r32, and the three sums (r32.r32, r.r, r32.w) as wave sums for
-// span_finish_kernel.  u's left and right neighbours come from the adjacent
+// into r32, and the three sums (r32.r32, r.r, r32.w) as block sums.  u's left and right neighbours come from the adjacent
 // lanes by DPP; lane 0 loads u at e - 1, lane 63 u and kx at e + 2.
 __global__ __launch_bounds__(kBlock) void mp_residual1_kernel(
     Geo g, const double* __restrict__ u, const double* __restrict__ u0,
@@ -716,7 +712,7 @@ __global__ __launch_bounds__(kBlock) void mp_residual1_kernel(
                  (in0 ? ra * ra : 0.0) + (in1 ? rb * rb : 0.0),
                  (in0 ? (double)fa * (double)W.x : 0.0) + (in1 ? (double)fb * (double)W.y : 0.0)};
   if (any) st2(r32, e, in0, in1, fa, fb);
-  wave_subtree_pairs<3>(v, sub, nblk, blk);
+  block_sums_pairs<3>(v, sub, nblk, blk, threadIdx.x);
 }
 
 namespace {

@@ -262,9 +262,8 @@ __global__ __launch_bounds__(kBlock * KS) void jacobi_pair_kernel(
     const double* __restrict__ ky, double* sub, int nblk, int S) {
   int tid;
   const int blk = stacked_block<KS, kBlock>(S, &tid);
-  if (blk >= nblk) return;
   const int lane = threadIdx.x & (kWave - 1);
-  const PairAt q = pair_at(g, blk * kPairBlock + 2 * tid);
+  const PairAt q = pair_at(g, blk < nblk ? blk * kPairBlock + 2 * tid : g.n);
   const Operand o = load_operand(u_old, q, g.x, lane);
   const Faces f = load_faces(kx, ky, q, g.x, lane);
   const double2 s = ld2_nt(u0, q.ir);
@@ -275,9 +274,9 @@ __global__ __launch_bounds__(kBlock * KS) void jacobi_pair_kernel(
                                         f.kx2, f.ky.y, f.kyt.y)
                           : o.c.y;
   st2_all(u_new, q, n0, n1);
-  double v[1] = {(q.in0 ? fabs(n0 - o.c.x) : 0.0) +
-                 (q.in1 ? fabs(n1 - o.c.y) : 0.0)};
-  wave_subtree_pairs<1>(v, sub, nblk, blk, tid / kWave);
+  const double v[1] = {(q.in0 ? fabs(n0 - o.c.x) : 0.0) +
+                       (q.in1 ? fabs(n1 - o.c.y) : 0.0)};
+  block_sums_pairs<1, KS>(v, sub, nblk, blk, tid);
 }
 
 __global__ __launch_bounds__(kBlock) void cheby_pair_kernel(

@@ -318,8 +318,8 @@ __device__ inline void st2_nt(float* p, int i, bool in0, bool in1, float v0,
 // 64 level-1 partials (sycl_shared.hpp:59-64: a[2s*l] += a[2s*l + s] for
 // s = 1, 2, 4, ...) sums aligned runs of 8 leaves before it combines them, so
 // a block's 8-leaf subtree is an exact intermediate of that tree: blocks
-// store it in sub[q * nblk + block], and span_finish_kernel combines the 8
-// subtrees of each span into its level-2 partial.
+// store it in sub[q * sub_stride + block], and span_finish_kernel (or, for
+// small grids, the next pass itself: consume_sums) combines them.
 //
 // These kernels keep the launch order of blocks (no xcd_span renumbering):
 // the hardware deals consecutive blocks round-robin to the 8 XCDs, so the
@@ -331,32 +331,50 @@ constexpr int kPairBlock = 2 * kBlock;              // 512 cells
 constexpr int kSubPerSpan = kSpan / kPairBlock;     // 8
 constexpr int kSubMaxNr = 3;                        // dot products per launch
 
-// From each lane's in-lane pair sum (tree step 1): steps 2..32 within each
-// 32-lane half (one group each), then the wave's two groups; lane 0 stores
-// that sum, g(2w) + g(2w+1), in sub[q * 4 * nblk + 4 * blk + w].  The
-// block's four wave sums are combined by span_finish_kernel (tree steps 2
-// and 4 of the 8-leaf subtree), so the streaming kernels need no LDS and no
-// barrier.
-template <int NR>
-__device__ inline void wave_subtree_pairs(double (&v)[NR], double* sub,
-                                          int nblk, int blk, int wv = -1) {
-  const int lane = threadIdx.x & (kWave - 1);
-  if (wv < 0) wv = threadIdx.x / kWave;
+// Length of one dot product's block sums: the blocks rounded up to whole
+// groups of 512 (64 spans), the cells past the grid's blocks zero for good.
+constexpr int kGroupBlocks = kSubPerSpan * kWave;   // 512
+__host__ __device__ inline int sub_stride(int nblk) {
+  return (nblk + kGroupBlocks - 1) / kGroupBlocks * kGroupBlocks;
+}
+
+// wave_tree with the steps within 16 lanes on the DPP path (after each, every
+// lane of an aligned block holds the block's sum; the mirrors pair whole
+// blocks of equal lanes); the sum in every lane.
+__device__ inline double wave_tree_dpp(double t) {
+  t = t + dpp<0xB1>(t);
+  t = t + dpp<0x4E>(t);
+  t = t + dpp<0x141>(t);
+  t = t + dpp<0x140>(t);
+  return (lane_value(t, 0) + lane_value(t, 16)) + (lane_value(t, 32) + lane_value(t, 48));
+}
+
+// Stores the sum of each of a workgroup's KS blocks of NW waves from the
+// lanes' values v (the in-lane sums: tree step 1 for pairs, 1 and 2 for
+// quads).  tid is the thread in its block; blk may lie past the grid.  Every
+// wave of the workgroup calls it.
+template <int NR, int NW, int KS>
+__device__ inline void store_block_sums(const double (&v)[NR], double* sub, int nblk, int blk,
+                                        int tid) {
+  static_assert(NW == 2 || NW == 4, "waves per block");
+  __shared__ double ws[KS][NR][NW];
+  const int slot = KS == 1 ? 0 : (int)threadIdx.x / (NW * kWave);
+  const int wv = tid / kWave;
 #pragma unroll
   for (int q = 0; q < NR; ++q) {
-    // Tree steps 2, 4, 8 and 16 on the DPP path: after each, every lane of
-    // an aligned block holds the block's sum (the mirrors pair whole blocks
-    // of equal lanes).  Then the four 16-lane sums: (r0 + r1) and (r2 + r3)
-    // are the wave's two groups.
-    double t = v[q];
-    t = t + dpp<0xB1>(t);
-    t = t + dpp<0x4E>(t);
-    t = t + dpp<0x141>(t);
-    t = t + dpp<0x140>(t);
-    const double g0 = lane_value(t, 0) + lane_value(t, 16);
-    const double g1 = lane_value(t, 32) + lane_value(t, 48);
-    if (lane == 0) sub[(size_t)q * kWaves * nblk + kWaves * blk + wv] = g0 + g1;
+    const double t = wave_tree_dpp(v[q]);
+    if ((threadIdx.x & (kWave - 1)) == 0) ws[slot][q][wv] = t;
   }
+  __syncthreads();
+  if (tid >= NR || blk >= nblk) return;
+  double s = ws[slot][tid][0] + ws[slot][tid][1];
+  if (NW == 4) s = s + (ws[slot][tid][NW - 2] + ws[slot][tid][NW - 1]);
+  sub[(size_t)tid * sub_stride(nblk) + blk] = s;
+}
+template <int NR, int KS = 1>
+__device__ inline void block_sums_pairs(const double (&v)[NR], double* sub, int nblk, int blk,
+                                        int tid) {
+  store_block_sums<NR, kWaves, KS>(v, sub, nblk, blk, tid);
 }
 
 // ---- four cells per lane ---------------------------------------------------
@@ -368,12 +386,9 @@ __device__ inline void wave_subtree_pairs(double (&v)[NR], double* sub,
 // at x = 4100 lie 8 blocks back and ahead: on the same XCD, whose L2 has
 // them (with 1024-cell blocks they lie 4 blocks away, on another XCD: the
 // prolongation, which reads ky one row up, took 12-22% longer at 4096^2).  The in-lane sum ((v0 + v1) +
-// (v2 + v3)) is tree steps 1 and 2; the four DPP steps of wave_subtree_pairs
-// then finish a 64-cell group in each 16-lane row, so wave w (of 2) holds
-// four groups, g0..g3, and stores the sums pair waves 2w and 2w + 1 would:
-// g0 + g1 and g2 + g3, in sub[q * 4 * nblk + 4 * block + 2 * w] and the slot
-// after it.  span_finish_kernel completes the spans from there, bit for bit
-// as for the pair kernels.
+// (v2 + v3)) is tree steps 1 and 2; the four DPP steps of wave_tree_dpp
+// then finish a 64-cell group in each 16-lane row, and (g0 + g1) + (g2 + g3)
+// is the sum pair waves 2w and 2w + 1 combine to: the same tree, bit for bit.
 
 constexpr int kQuadThreads = kPairBlock / 4;  // 128
 constexpr int kQuadBlock = kPairBlock;        // 512 cells
@@ -430,24 +445,46 @@ __device__ inline void st4_nt(float* p, int i, const bool (&in)[4], const float 
   }
 }
 
+template <int NR, int KS = 1>
+__device__ inline void block_sums_quads(const double (&v)[NR], double* sub, int nblk, int blk,
+                                        int tid) {
+  store_block_sums<NR, kQuadThreads / kWave, KS>(v, sub, nblk, blk, tid);
+}
+
+// The sums a pass before this one left in sub, formed by every block of this
+// pass for itself (the first 256 threads load, every thread gets the sums):
+// with up to 2048 blocks (4 groups) the reference's remaining passes are one
+// pairwise tree over the zero-padded block sums.  It saves the finisher's
+// launch (3.4-4.2 us) between two dependent passes: an FP64 CG iteration at
+// 512^2 takes 17.9 us with it and 22.7 us with finishers.  (Counting the
+// blocks done and letting the last one finish the sum inside its own kernel
+// took 26 us: the count of 512 blocks on 8 XCDs is a serial chain of about
+// 18 ns each.)  Beyond 2048 blocks, more than the chip holds at once, each
+// further round of blocks would repeat the sum, and the finisher stays.
+constexpr int kConsumeBlocks = 4 * kGroupBlocks;
 template <int NR>
-__device__ inline void wave_subtree_quads(double (&v)[NR], double* sub, int nblk, int blk,
-                                          int wv) {
-  const int lane = threadIdx.x & (kWave - 1);
+__device__ inline void consume_sums(const double* __restrict__ sub, int nblk,
+                                    double (&sum)[NR]) {
+  __shared__ double gs[NR][4];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int stride = sub_stride(nblk);
+  if (wv < 4) {
+    const int i0 = kGroupBlocks * wv + kSubPerSpan * lane;
 #pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    double t = v[q];
-    t = t + dpp<0xB1>(t);
-    t = t + dpp<0x4E>(t);
-    t = t + dpp<0x141>(t);
-    t = t + dpp<0x140>(t);
-    const double g01 = lane_value(t, 0) + lane_value(t, 16);
-    const double g23 = lane_value(t, 32) + lane_value(t, 48);
-    if (lane == 0) {
-      double* d = sub + (size_t)q * kWaves * nblk + kWaves * blk + 2 * wv;
-      *reinterpret_cast<dvec2*>(d) = dvec2{g01, g23};
+    for (int q = 0; q < NR; ++q) {
+      double t = 0.0;
+      if (i0 < stride) {
+        const double* p = sub + (size_t)q * stride + i0;
+        const double2 a = ld2(p, 0), b = ld2(p, 2), c = ld2(p, 4), d = ld2(p, 6);
+        t = ((a.x + a.y) + (b.x + b.y)) + ((c.x + c.y) + (d.x + d.y));
+      }
+      t = wave_tree_dpp(t);
+      if (lane == 0) gs[q][wv] = t;
     }
   }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NR; ++q) sum[q] = (gs[q][0] + gs[q][1]) + (gs[q][2] + gs[q][3]);
 }
 
 // The cell pair (e, e + 1) of a pair-per-thread lane, e = 512 b + 2 m for
@@ -606,6 +643,22 @@ __global__ void mp_w1_kernel(Geo g, MpArgs a, double* sub, int nblk);
 template <bool DOT2, int UM, int KS>
 __global__ void mp_w4_kernel(Geo g, MpArgs a, double* sub, int nblk, int S);
 
+// Where a pass of the iteration takes its scalar from: the host's value
+// (dev null), the device's (dev: a finisher of the run-ahead left it there),
+// or, with CONSUME, the block sums sub of the pass before it, which every
+// block reduces for itself; the first block then leaves the scalar and the
+// sum for the next pass and the host.  alpha = rro / sum (r-step), beta =
+// sum / rro (w-step); rro is *rro_dev where that is set, else the value.
+struct RaScalar {
+  const double* dev = nullptr;
+  const double* sub = nullptr;
+  int nblk = 0, inverse = 0;
+  double rro = 0.0;
+  const double* rro_dev = nullptr;
+  double* sum_dev = nullptr;  // set by the w-step: r.r, the next alpha's rro
+  double* out = nullptr;      // host slot {sum, scalar}
+};
+
 }  // namespace tea
 
 struct tea_nn;
@@ -731,9 +784,12 @@ struct tea_hip_chunk {
   // coherent host memory; kernels write through the device view.
   double* partials = nullptr;       // device view
   double* host_partials = nullptr;  // host view of the same memory
-  // Wave sums of the pair-per-thread kernels: kSubMaxNr x 4 x nblk, device.
+  // Block sums of the pair-per-thread kernels, kSubMaxNr x sub_stride(nblk),
+  // device.  sub2: a second set (the same allocation), for a pass that reads
+  // the sums of the pass before it while its own blocks write theirs.
   int nblk = 0;                     // 512-cell blocks covering x*y
   double* sub = nullptr;
+  double* sub2 = nullptr;
   int pair_blocks = 3;              // pair-per-thread kernels: bit 0 fused_w,
                                     // bit 1 fused_r
 
@@ -828,6 +884,8 @@ struct tea_hip_chunk {
   double* r_alt = nullptr;    // spare r, u and w (x*y each)
   double* u_alt = nullptr;
   double* w_alt = nullptr;
+  tea::RaScalar ra_next;      // where the w-step after the r-step in flight
+                              // takes its beta from
   double* ra_dev = nullptr;   // device: [0] alpha, [1] beta, [2] r.r, then the
                               // finisher's partials and its blocks-done count
   unsigned* ra_count = nullptr;
@@ -889,7 +947,7 @@ int resolve_ready(tea_hip_chunk* c);
 // partials; results go to out[0..nr).
 int finish_reduction(tea_hip_chunk* c, int nr, double* out);
 
-// Combines the 8 subtree sums of each span in c->sub (nr dot products) into
+// Combines the 8 block sums of each span in c->sub (nr dot products) into
 // the span's level-2 partials and runs the next tree pass over them, leaving
 // *len partials per dot product in c->partials.
 // The partials go to arrays slot .. slot + nr - 1 of c->partials.  With
