@@ -284,9 +284,9 @@ __global__ __launch_bounds__(kBlock) void fused_w_kernel(Geo g, FusedWArgs a,
 
 // ---- two cells per lane --------------------------------------------------
 //
-// When x is even every cell pair (2m, 2m+1) lies in one row and starts on a
-// 16-byte boundary, so p, r, u, kx, ky and the rows above and below are read
-// with one 16-byte load per pair, and the left/right neighbours come from
+// Every cell pair (2m, 2m+1) starts on a 16-byte boundary, so p, r, u, kx and
+// ky are read with one 16-byte load per pair (the rows above and below too,
+// at 8-byte alignment when x is odd), and the left/right neighbours come from
 // the adjacent lanes (lane l-1 holds 2m-1, lane l+1 holds 2m+2); only lanes
 // 0 and 63 load theirs.  A wave covers 128 consecutive cells = two groups
 // of the reduction tree (lanes 0-31 and 32-63); a 256-thread block covers a
@@ -324,30 +324,29 @@ __device__ inline void fused_pair_index(const Geo& g, int e, FusedPair& s) {
 
 // The pair's own p, r and kx are also the left/right neighbours the adjacent
 // lanes take by shuffle, so they are read whenever the pair is in range; the
-// rows above and below only for interior pairs.  x + 2 is an even index whose
-// +-x rows are in range.
+// rows above and below only for interior pairs.
 template <bool APPLY_P>
 __device__ inline void fused_pair_load(const Geo& g, const FusedWArgs& a,
                                        FusedPair& s) {
   const int x = g.x;
   const double* __restrict__ P = a.p_old;
   const double* __restrict__ R = a.r;
-  const int ic = s.e0 < g.n ? s.e0 : x + 2;
-  const int ir = s.any ? s.e0 : x + 2;
+  const int ic = s.e0 < g.n ? s.e0 : safe_pair(x);
+  const int ir = s.any ? s.e0 : safe_pair(x);
   s.P0 = ld2(P, ic);
-  s.Pt = ld2(P, ir + x);
-  s.Pb = ld2(P, ir - x);
+  s.Pt = ld2u(P, ir + x);
+  s.Pb = ld2u(P, ir - x);
   if (APPLY_P) {
     s.R0 = ld2(R, ic);
-    s.Rt = ld2(R, ir + x);
-    s.Rb = ld2(R, ir - x);
+    s.Rt = ld2u(R, ir + x);
+    s.Rb = ld2u(R, ir - x);
   }
   s.KX = ld2(a.kx, ic);
   s.KY = ld2(a.ky, ir);
-  s.KYt = ld2(a.ky, ir + x);
+  s.KYt = ld2u(a.ky, ir + x);
   if (a.apply_u) s.U = ld2_nt(a.u, ir);
   // Issued with the pair's own loads so the wave waits once; ir - 1 and
-  // ir + 2 are in range (ir is an interior pair's index or x + 2).
+  // ir + 2 are in range (ir is an interior pair's index or the safe one).
   // Lanes 0 and 63 share each load instruction, at their own addresses
   // (lane 0's kx value is not used).
   const int lane = threadIdx.x & (kWave - 1);
@@ -427,30 +426,25 @@ __device__ inline double fused_pair_compute(const Geo& g, const FusedWArgs& a,
     st2_nt(a.u_out, i, s.in0, s.in1, ua, ub);
   }
   if (APPLY_P) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb);
-  // Halo ring of boundary-adjacent cells (rare; per cell).
+  // Halo ring of boundary-adjacent cells (rare; per cell).  With the halo
+  // refresh folded in it takes the new values; without, p (and u, where it
+  // goes to another buffer) keeps its old ring.
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const bool inc = c == 0 ? s.in0 : s.in1;
     const int ic = i + c, kc = ka + c;
-    const bool L = kc == xl, Rg = kc == xr, B = row == yb, T = row == yt;
-    if (!inc || !(L | Rg | B | T)) continue;
-    const double pv = c == 0 ? ca : cb;
-    const double uv = c == 0 ? ua : ub;
-    int ring[8];
-    int nr = 0;
-    if (L) ring[nr++] = ic - 1;
-    if (Rg) ring[nr++] = ic + 1;
-    if (B) ring[nr++] = ic - x;
-    if (T) ring[nr++] = ic + x;
-    if (L && B) ring[nr++] = ic - 1 - x;
-    if (Rg && B) ring[nr++] = ic + 1 - x;
-    if (L && T) ring[nr++] = ic - 1 + x;
-    if (Rg && T) ring[nr++] = ic + 1 + x;
-    for (int q = 0; q < nr; ++q) {
-      if (a.apply_u && (a.ring || a.u_out != a.u))
-        a.u_out[ring[q]] = a.ring ? uv : a.u[ring[q]];
-      if (APPLY_P) a.p_new[ring[q]] = a.ring ? pv : P[ring[q]];
+    if (!(c == 0 ? s.in0 : s.in1) || !(kc == xl || kc == xr || row == yb || row == yt)) continue;
+    if (a.ring) {
+      if (a.apply_u) ring_store(a.u_out, ic, kc, row, x, xl, xr, yb, yt, c == 0 ? ua : ub);
+      if (APPLY_P) ring_store(a.p_new, ic, kc, row, x, xl, xr, yb, yt, c == 0 ? ca : cb);
+      continue;
     }
+    for (int dj = row == yb ? -1 : 0; dj <= (row == yt ? 1 : 0); ++dj)
+      for (int dk = kc == xl ? -1 : 0; dk <= (kc == xr ? 1 : 0); ++dk) {
+        if (dj == 0 && dk == 0) continue;
+        const int q = ic + dj * x + dk;
+        if (a.apply_u && a.u_out != a.u) a.u_out[q] = a.u[q];
+        if (APPLY_P) a.p_new[q] = P[q];
+      }
   }
   return psum;
 }
@@ -645,8 +639,7 @@ struct NormBody {
   }
 };
 
-// The 2-norm over cell pairs, one pair per lane (even rows, more than one
-// group): 8 bytes per cell, the sum tree's first level in-lane.
+// The 2-norm over cell pairs, one pair per lane (more than one group): 8 bytes per cell, the sum tree's first level in-lane.
 __global__ __launch_bounds__(kBlock) void norm_pair_kernel(
     Geo g, const double* __restrict__ b, double* sub, int nblk) {
   const PairAt q = pair_at(g, blockIdx.x * kPairBlock + 2 * threadIdx.x);
@@ -734,7 +727,7 @@ int ra_len(const tea_hip_chunk* c) {
 }
 
 bool ra_possible(const tea_hip_chunk* c) {
-  return c->ra_enabled && c->fused && c->poll && c->pairs && c->ra_rro_known &&
+  return c->ra_enabled && c->fused && c->poll && c->pairs && c->geo.x % 2 == 0 && c->ra_rro_known &&
          c->ra_fail < 3 && use_pair_blocks(c, 1) && use_pair_blocks(c, 2) &&
          ra_len(c) <= kWave * kWave;
 }
@@ -749,7 +742,7 @@ double* ra_dev_slot(tea_hip_chunk* c, int set, int kind) {
 
 int ensure_ra(tea_hip_chunk* c) {
   if (c->ra_host) return TEA_HIP_OK;
-  const size_t bytes = (size_t)c->geo.n * sizeof(double);
+  const size_t bytes = pair_bytes(c->geo.n, sizeof(double));
   for (double** b : {&c->r_alt, &c->u_alt, &c->w_alt}) {
     if (hipMalloc(b, bytes) != hipSuccess) {
       *b = nullptr;

@@ -373,7 +373,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   c->ngroup = (int)((n + kWave - 1) / kWave);
   c->nspan = (int)((n + kSpan - 1) / kSpan);
   if (const char* b = getenv("TEA_HIP_BATCH")) c->batch = atoi(b);
-  c->pairs = (x % 2 == 0) && y >= 3;
+  c->pairs = y >= 3;
   if (const char* pv = getenv("TEA_HIP_PAIRS")) c->pairs = c->pairs && atoi(pv) != 0;
   c->quads = c->pairs && x % 4 == 0;
   if (const char* qv = getenv("TEA_HIP_QUADS")) c->quads = c->quads && atoi(qv) != 0;
@@ -420,7 +420,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   c->field_len[TEA_FIELD_COMMS_BUFFER] = std::max(X, Y) * (size_t)halo_depth;
 
   for (int f = 0; f < TEA_NUM_FIELDS; ++f) {
-    const size_t bytes = c->field_len[f] * sizeof(double);
+    const size_t bytes = pair_bytes((long)c->field_len[f], sizeof(double));
     if (hipMalloc(&c->field[f], bytes) != hipSuccess) {
       c->field[f] = nullptr;
       set_error("hipMalloc of a field failed");
@@ -431,7 +431,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
       return fail(TEA_HIP_EHIP);
     }
   }
-  if (hipMalloc(&c->p_alt, xy * sizeof(double)) != hipSuccess) {
+  if (hipMalloc(&c->p_alt, pair_bytes(n, sizeof(double))) != hipSuccess) {
     c->p_alt = nullptr;
     set_error("hipMalloc of the second p buffer failed");
     return fail(TEA_HIP_ENOMEM);

@@ -102,7 +102,7 @@ struct ProlongBody {
   }
 };
 
-// The same, two cells per lane (x even): z = r / diag (+ the NL coarse
+// The same, two cells per lane: z = r / diag (+ the NL coarse
 // terms) and z.w, the arithmetic of JacobiBody / ProlongBody cell by cell.
 template <int NL>
 __global__ __launch_bounds__(kBlock) void fcg_z2_kernel(
@@ -123,10 +123,10 @@ __global__ __launch_bounds__(kBlock) void fcg_z2_kernel(
     const bool in0 = e < g.n && interior(g, kk, row);
     const bool in1 = e < g.n && interior(g, kk + 1, row);
     const bool any = in0 || in1;
-    const int ic = e < g.n ? e : x + 2;
-    const int ir = any ? e : x + 2;
+    const int ic = e < g.n ? e : safe_pair(x);
+    const int ir = any ? e : safe_pair(x);
     const float2 R = ld2(r, ir), KX = ld2(kx, ic), KY = ld2(ky, ir),
-                 KYt = ld2(ky, ir + x), W = ld2(w, ir);
+                 KYt = ld2u(ky, ir + x), W = ld2(w, ir);
     float kxr = __shfl_down(KX.x, 1);
     if (lane == kWave - 1 && any) kxr = kx[e + 2];
     const double da = (1.0 + ((double)KX.y + (double)KX.x)) + ((double)KYt.x + (double)KY.x);
@@ -166,10 +166,10 @@ __global__ __launch_bounds__(kBlock) void fcg_z1_kernel(
   const bool in0 = e < g.n && interior(g, kk, row);
   const bool in1 = e < g.n && interior(g, kk + 1, row);
   const bool any = in0 || in1;
-  const int ic = e < g.n ? e : x + 2;
-  const int ir = any ? e : x + 2;
+  const int ic = e < g.n ? e : safe_pair(x);
+  const int ir = any ? e : safe_pair(x);
   const float2 R = ld2(r, ir), KX = ld2(kx, ic), KY = ld2(ky, ir),
-               KYt = ld2(ky, ir + x), W = ld2(w, ir);
+               KYt = ld2u(ky, ir + x), W = ld2(w, ir);
   float kxn = 0.0f;
   if (lane == kWave - 1) kxn = kx[ir + 2];
   // The coarse values of both cells, issued with the pair's own loads (index
@@ -1347,12 +1347,13 @@ __global__ __launch_bounds__(kGammaThreads) void joint_gamma_kernel(
 
 int ensure_fcg_buffers(tea_hip_chunk* c) {
   if (c->fcg_z) return TEA_HIP_OK;
-  if (hipMalloc(&c->fcg_z, (size_t)c->geo.n * sizeof(float)) != hipSuccess) {
+  const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
+  if (hipMalloc(&c->fcg_z, bytes) != hipSuccess) {
     c->fcg_z = nullptr;
     set_error("hipMalloc of the FCG z buffer failed");
     return TEA_HIP_ENOMEM;
   }
-  TEA_HIP_TRY(hipMemsetAsync(c->fcg_z, 0, (size_t)c->geo.n * sizeof(float), c->stream));
+  TEA_HIP_TRY(hipMemsetAsync(c->fcg_z, 0, bytes, c->stream));
   return TEA_HIP_OK;
 }
 

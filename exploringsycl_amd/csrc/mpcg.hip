@@ -160,7 +160,7 @@ __global__ __launch_bounds__(kBlock) void mp_r_kernel(
   span_reduce<RW ? 2 : 1>(prod, partials, nspan, span, single_group != 0);
 }
 
-// Two cells per lane (x even): the arithmetic of mp_w_kernel cell by cell,
+// Two cells per lane: the arithmetic of mp_w_kernel cell by cell,
 // with 8-byte loads of the FP32 operands and 16-byte loads of u.  One pair's
 // indices, loads and arithmetic, shared by the span-per-block and
 // pair-per-thread kernels.
@@ -186,28 +186,27 @@ __device__ inline void mp_pair_index(const Geo& g, int e, MpPair& s) {
 
 // A pair's own p, r and kx are also its neighbours' left/right operands (by
 // shuffle), so they are read whenever the pair is in range; the rows above
-// and below only for interior pairs.  x + 2 is an even index whose +-x rows
-// are in range.  The wave-edge neighbours are issued with the rest, at
+// and below only for interior pairs.  The wave-edge neighbours are issued with the rest, at
 // ir - 1 and ir + 2, which are in range too.
 template <bool DOT2>
 __device__ inline void mp_pair_load(const Geo& g, const MpArgs& a, MpPair& s) {
   const int x = g.x;
   const float* __restrict__ P = a.p_old;
   const float* __restrict__ R = a.r;
-  const int ic = s.e0 < g.n ? s.e0 : x + 2;
-  const int ir = s.any ? s.e0 : x + 2;
+  const int ic = s.e0 < g.n ? s.e0 : safe_pair(x);
+  const int ir = s.any ? s.e0 : safe_pair(x);
   // Every load is issued unconditionally, r's and u's also where the step
   // does not use them (the first iteration only): loads under a branch were
   // each waited for inside it, before the next ones were issued.
   s.P0 = ld2(P, ic);
-  s.Pt = ld2(P, ir + x);
-  s.Pb = ld2(P, ir - x);
+  s.Pt = ld2u(P, ir + x);
+  s.Pb = ld2u(P, ir - x);
   s.R0 = ld2(R, ic);
-  s.Rt = ld2(R, ir + x);
-  s.Rb = ld2(R, ir - x);
+  s.Rt = ld2u(R, ir + x);
+  s.Rb = ld2u(R, ir - x);
   s.KX = ld2(a.kx, ic);
   s.KY = ld2(a.ky, ir);
-  s.KYt = ld2(a.ky, ir + x);
+  s.KYt = ld2u(a.ky, ir + x);
   s.U = ld2_nt(a.u, ir);
   if (DOT2) s.RD = ld2(a.rdot, ir);
   // Lanes 0 and 63 share each load instruction, at their own addresses
@@ -296,26 +295,9 @@ __device__ inline void mp_pair_compute(const Geo& g, const MpArgs& a,
   // Halo ring of boundary-adjacent cells (rare; per cell).
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    const bool inc = c == 0 ? s.in0 : s.in1;
-    const int ic = i + c, kc = ka + c;
-    const bool L = kc == xl, Rg = kc == xr, B = row == yb, T = row == yt;
-    if (!inc || !(L | Rg | B | T)) continue;
-    const float pv = c == 0 ? ca : cb;
-    const double uv = c == 0 ? ua : ub;
-    int ring[8];
-    int nr = 0;
-    if (L) ring[nr++] = ic - 1;
-    if (Rg) ring[nr++] = ic + 1;
-    if (B) ring[nr++] = ic - x;
-    if (T) ring[nr++] = ic + x;
-    if (L && B) ring[nr++] = ic - 1 - x;
-    if (Rg && B) ring[nr++] = ic + 1 - x;
-    if (L && T) ring[nr++] = ic - 1 + x;
-    if (Rg && T) ring[nr++] = ic + 1 + x;
-    for (int q = 0; q < nr; ++q) {
-      if (a.apply_u) a.u[ring[q]] = uv;
-      if (a.apply_p) a.p_new[ring[q]] = pv;
-    }
+    if (!(c == 0 ? s.in0 : s.in1)) continue;
+    if (a.apply_u) ring_store(a.u, i + c, ka + c, row, x, xl, xr, yb, yt, c == 0 ? ua : ub);
+    if (a.apply_p) ring_store(a.p_new, i + c, ka + c, row, x, xl, xr, yb, yt, c == 0 ? ca : cb);
   }
 }
 
@@ -365,23 +347,6 @@ __global__ __launch_bounds__(kBlock) void mp_w1_kernel(Geo g, MpArgs a,
 }
 
 template __global__ void mp_w1_kernel<true>(Geo, MpArgs, double*, int);
-
-// The reflection of an interior cell's new value v onto the depth-1 halo
-// ring where the cell borders it (kc, rc its column and row).
-template <class T>
-__device__ inline void ring_store(T* f, int i, int kc, int rc, int x, int xl, int xr, int yb,
-                                  int yt, T v) {
-  const bool L = kc == xl, Rg = kc == xr, B = rc == yb, Tp = rc == yt;
-  if (!(L | Rg | B | Tp)) return;
-  if (L) f[i - 1] = v;
-  if (Rg) f[i + 1] = v;
-  if (B) f[i - x] = v;
-  if (Tp) f[i + x] = v;
-  if (L && B) f[i - 1 - x] = v;
-  if (Rg && B) f[i + 1 - x] = v;
-  if (L && Tp) f[i - 1 + x] = v;
-  if (Rg && Tp) f[i + 1 + x] = v;
-}
 
 // Four cells per lane (x a multiple of 4): the arithmetic of mp_w_kernel cell
 // by cell, with 16-byte loads of the FP32 operands and of u.  The
@@ -667,8 +632,7 @@ __global__ __launch_bounds__(kQuadThreads) void mp_r4_kernel(
   block_sums_quads<RW ? 2 : 1>(v, sub, nblk, blk, threadIdx.x);
 }
 
-// MpTrueResidualBody's arithmetic (below) with one cell pair per thread (x
-// even): r = u0 - A u in FP64 with the FP64 coefficients, r rounded to FP32
+// MpTrueResidualBody's arithmetic (below) with one cell pair per thread: r = u0 - A u in FP64 with the FP64 coefficients, r rounded to FP32
 // into r32, and the three sums (r32.r32, r.r, r32.w) as block sums.  u's left and right neighbours come from the adjacent
 // lanes by DPP; lane 0 loads u at e - 1, lane 63 u and kx at e + 2.
 __global__ __launch_bounds__(kBlock) void mp_residual1_kernel(
@@ -684,10 +648,10 @@ __global__ __launch_bounds__(kBlock) void mp_residual1_kernel(
   const bool in0 = e < g.n && interior(g, kk, row);
   const bool in1 = e < g.n && interior(g, kk + 1, row);
   const bool any = in0 || in1;
-  const int ic = e < g.n ? e : x + 2;
-  const int ir = any ? e : x + 2;
-  const double2 U = ld2(u, ic), Ut = ld2(u, ir + x), Ub = ld2(u, ir - x);
-  const double2 KX = ld2(kx, ic), KY = ld2(ky, ir), KYt = ld2(ky, ir + x);
+  const int ic = e < g.n ? e : safe_pair(x);
+  const int ir = any ? e : safe_pair(x);
+  const double2 U = ld2(u, ic), Ut = ld2u(u, ir + x), Ub = ld2u(u, ir - x);
+  const double2 KX = ld2(kx, ic), KY = ld2(ky, ir), KYt = ld2u(ky, ir + x);
   const double2 B = ld2_nt(u0, ir);
   const float2 W = ld2(w, ir);
   double UN = 0.0, KXN = 0.0;
@@ -798,7 +762,7 @@ struct MpTrueResidualBody {
 
 int ensure_mp_buffers(tea_hip_chunk* c) {
   if (c->mp_r) return TEA_HIP_OK;
-  const size_t bytes = (size_t)c->geo.n * sizeof(float);
+  const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
   float** bufs[] = {&c->mp_p[0], &c->mp_p[1], &c->mp_p[2], &c->mp_r, &c->mp_w, &c->mp_kx,
                     &c->mp_ky};
   for (float** b : bufs) {

@@ -19,8 +19,8 @@
 //              against 80.
 // A double-buffered field's cells outside the interior are copied into the
 // new buffer in the same pass, so every field holds exactly what the
-// reference's in-place kernels leave.  Mode 0 (tea_hip_set_fused) and odd
-// row lengths run one launch per reference kernel instead.  Every FP64
+// reference's in-place kernels leave.  Mode 0 (tea_hip_set_fused) runs one
+// launch per reference kernel instead.  Every FP64
 // expression keeps the reference's operand order; the library is compiled
 // with -ffp-contract=off.
 
@@ -192,14 +192,13 @@ struct PpcgCalcSDBody {  // ppcg.cpp:69-94
 
 // ---- one pair per lane --------------------------------------------------------
 //
-// Lane m of block b holds cells e = 512 b + 2m and e + 1 (x is even, so the
-// pair never straddles a row).  The stencil operand's left and right
+// Lane m of block b holds cells e = 512 b + 2m and e + 1.  The stencil operand's left and right
 // neighbours come from the adjacent lanes; lanes 0 and 63 load theirs.
 
 // A stencil operand at a pair: the pair itself, the rows above and below,
 // and the cells left of e and right of e + 1.  Must be called by every lane
 // of the wave (it shuffles).  Lane 0's and lane 63's extra loads are at
-// ir - 1 and ir + 2, in range for an interior pair and for x + 2.
+// ir - 1 and ir + 2, in range for an interior pair and for the safe index.
 struct Operand {
   double2 c, t, b;
   double l, r;
@@ -209,8 +208,8 @@ __device__ inline Operand load_operand(const double* __restrict__ a,
                                        const PairAt& q, int x, int lane) {
   Operand o;
   o.c = ld2(a, q.ic);
-  o.t = ld2(a, q.ir + x);
-  o.b = ld2(a, q.ir - x);
+  o.t = ld2u(a, q.ir + x);
+  o.b = ld2u(a, q.ir - x);
   double edge = 0.0;
   if (lane == 0 || lane == kWave - 1) edge = a[lane == 0 ? q.ir - 1 : q.ir + 2];
   o.l = __shfl_up(o.c.y, 1);
@@ -233,7 +232,7 @@ __device__ inline Faces load_faces(const double* __restrict__ kx,
   Faces f;
   f.kx = ld2(kx, q.ic);
   f.ky = ld2(ky, q.ir);
-  f.kyt = ld2(ky, q.ir + x);
+  f.kyt = ld2u(ky, q.ir + x);
   double edge = 0.0;
   if (lane == kWave - 1) edge = kx[q.ir + 2];
   f.kx2 = __shfl_down(f.kx.x, 1);
@@ -249,7 +248,8 @@ __device__ inline double op5_hi(const Operand& o, const Faces& f) {
   return op5(o.c.y, o.c.x, o.r, o.b.y, o.t.y, f.kx.y, f.kx2, f.ky.y, f.kyt.y);
 }
 
-// Stores both cells of a valid pair with one 16-byte streaming store.
+// Stores both cells of a valid pair with one 16-byte streaming store (the
+// buffers hold room for the last pair of an odd number of cells).
 __device__ inline void st2_all(double* p, const PairAt& q, double v0,
                                double v1) {
   if (q.valid) st2_nt(p, q.e, true, true, v0, v1);
@@ -334,7 +334,7 @@ int launch_each_cell(tea_hip_chunk* c, int kid, const Body& body) {
 // The fused Chebyshev and PPCG passes need the x*y spare buffer.
 int ensure_spare(tea_hip_chunk* c) {
   if (c->spare) return TEA_HIP_OK;
-  if (hipMalloc(&c->spare, (size_t)c->geo.n * sizeof(double)) != hipSuccess) {
+  if (hipMalloc(&c->spare, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
     c->spare = nullptr;
     set_error("hipMalloc of the spare field buffer failed");
     return TEA_HIP_ENOMEM;
@@ -342,7 +342,7 @@ int ensure_spare(tea_hip_chunk* c) {
   return TEA_HIP_OK;
 }
 
-// Fused passes run on even row lengths in the default mode.
+// Fused passes run in the default mode.
 bool fused_pairs(const tea_hip_chunk* c) { return c->fused && c->pairs; }
 
 // ---- two PPCG inner steps in one pass ---------------------------------------
@@ -808,7 +808,7 @@ __global__ __launch_bounds__(kTSBlock) void cheby_two_step_kernel(
 // The second spare buffer, allocated on first use.
 int ensure_spare2(tea_hip_chunk* c) {
   if (c->spare2) return TEA_HIP_OK;
-  if (hipMalloc(&c->spare2, (size_t)c->geo.n * sizeof(double)) != hipSuccess) {
+  if (hipMalloc(&c->spare2, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
     c->spare2 = nullptr;
     set_error("hipMalloc of the second spare field buffer failed");
     return TEA_HIP_ENOMEM;
@@ -816,8 +816,7 @@ int ensure_spare2(tea_hip_chunk* c) {
   return TEA_HIP_OK;
 }
 
-// One Chebyshev step: the single pass (even rows) or one launch per
-// reference kernel.
+// One Chebyshev step: the single pass or one launch per reference kernel.
 int cheby_step(tea_hip_chunk* c, double alpha, double beta) {
   double** f = c->field;
   const Geo g = c->geo;
@@ -868,8 +867,7 @@ int cheby_two_steps(tea_hip_chunk* c, double a0, double b0, double a1,
   return TEA_HIP_OK;
 }
 
-// One inner step: the single pass (even rows) or one launch per reference
-// kernel; the new sd goes to the second buffer in the single pass.
+// One inner step: the single pass or one launch per reference kernel; the new sd goes to the second buffer in the single pass.
 int ppcg_step(tea_hip_chunk* c, double alpha, double beta) {
   double** f = c->field;
   const Geo g = c->geo;

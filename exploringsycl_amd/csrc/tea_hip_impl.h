@@ -199,10 +199,16 @@ __device__ inline void span_reduce(double (&v)[NR][kItems], double* partials,
 // ---- two cells per lane ---------------------------------------------------
 //
 // Kernels over cell pairs (2m, 2m+1), m = lane index within a 512-cell slot:
-// with x even every pair starts on an aligned boundary, so each operand is
+// every pair starts on an aligned boundary, so each operand is
 // one 8-byte (FP32) or 16-byte (FP64) load, and the left/right neighbours
 // come from the adjacent lanes (lane l-1 holds 2m-1, lane l+1 holds 2m+2);
-// only lanes 0 and 63 load theirs.  A wave covers 128 consecutive cells =
+// only lanes 0 and 63 load theirs.  With x even a pair lies in one row and
+// the pairs above and below are aligned too.  With x odd every other row's
+// pairs are shifted by one cell: the rows above and below are read with
+// loads that need only element alignment (ld2u), and a pair may hold the last
+// cell of a row and the first of the next, neither of which is interior.
+// The last pair of an odd number of cells has no second cell; x*y buffers
+// hold room for it (pair_bytes).  A wave covers 128 consecutive cells =
 // two groups of the reduction tree (lanes 0-31 and 32-63); a 256-thread
 // block covers a 4096-cell span in 8 slots of 512 cells.  The first tree
 // level is the in-lane pair sum, then the butterfly runs over each 32-lane
@@ -217,6 +223,27 @@ __device__ inline double2 ld2(const double* p, int i) {
 __device__ inline float2 ld2(const float* p, int i) {
   return *reinterpret_cast<const float2*>(p + i);
 }
+
+// The same at an index that may be odd (global loads need only 4-byte
+// alignment): on an even index the instruction is ld2's.
+__device__ inline double2 ld2u(const double* p, int i) {
+  typedef double vec2 __attribute__((ext_vector_type(2), aligned(8)));
+  const vec2 v = *reinterpret_cast<const vec2*>(p + i);
+  return double2{v.x, v.y};
+}
+
+__device__ inline float2 ld2u(const float* p, int i) {
+  typedef float vec2 __attribute__((ext_vector_type(2), aligned(4)));
+  const vec2 v = *reinterpret_cast<const vec2*>(p + i);
+  return float2{v.x, v.y};
+}
+
+// An even index whose pair, the pairs one row up and down and the cells
+// next to it are in range (y >= 3).
+__device__ inline int safe_pair(int x) { return (x + 2) & ~1; }
+
+// Bytes of an x*y buffer that pair kernels use.
+inline size_t pair_bytes(long n, size_t elem) { return (size_t)((n + 1) & ~1L) * elem; }
 
 // Stores a cell pair with one vector store, or the interior member alone.
 template <class T>
@@ -488,13 +515,13 @@ __device__ inline void consume_sums(const double* __restrict__ sub, int nblk,
 }
 
 // The cell pair (e, e + 1) of a pair-per-thread lane, e = 512 b + 2 m for
-// lane m of block b (x even: a pair never straddles a row).
+// lane m of block b.
 struct PairAt {
   int e;          // first cell
   bool valid;     // e < x*y
   bool in0, in1;  // interior cells
-  int ic;         // e if valid, else a safe even index (x + 2)
-  int ir;         // e if either cell is interior, else x + 2
+  int ic;         // e if valid, else a safe even index (safe_pair)
+  int ir;         // e if either cell is interior, else the safe index
 };
 
 __device__ inline PairAt pair_at(const Geo& g, int e) {
@@ -505,9 +532,26 @@ __device__ inline PairAt pair_at(const Geo& g, int e) {
   const int kk = e - row * g.x;
   q.in0 = q.valid && interior(g, kk, row);
   q.in1 = q.valid && interior(g, kk + 1, row);
-  q.ic = q.valid ? e : g.x + 2;
-  q.ir = (q.in0 || q.in1) ? e : g.x + 2;
+  q.ic = q.valid ? e : safe_pair(g.x);
+  q.ir = (q.in0 || q.in1) ? e : safe_pair(g.x);
   return q;
+}
+
+// The reflection of an interior cell's new value v onto the depth-1 halo
+// ring where the cell borders it (kc, rc its column and row).
+template <class T>
+__device__ inline void ring_store(T* f, int i, int kc, int rc, int x, int xl, int xr, int yb,
+                                  int yt, T v) {
+  const bool L = kc == xl, Rg = kc == xr, B = rc == yb, Tp = rc == yt;
+  if (!(L | Rg | B | Tp)) return;
+  if (L) f[i - 1] = v;
+  if (Rg) f[i + 1] = v;
+  if (B) f[i - x] = v;
+  if (Tp) f[i + x] = v;
+  if (L && B) f[i - 1 - x] = v;
+  if (Rg && B) f[i + 1 - x] = v;
+  if (L && Tp) f[i - 1 + x] = v;
+  if (Rg && Tp) f[i + 1 + x] = v;
 }
 
 // One block per span: each thread evaluates `body` on its 16 cells (only
@@ -818,7 +862,7 @@ struct tea_hip_chunk {
   // Deferred CG work (fused mode).
   int fused = 1;
   int batch = 0;   // load batch of the fused stencil kernel (0: default)
-  bool pairs = false;  // two-cells-per-lane kernels (x even)
+  bool pairs = false;  // two-cells-per-lane kernels
   bool quads = false;  // four-cells-per-lane mixed-precision kernels (x % 4 == 0)
   bool pend_u = false, pend_p = false, pend_halo = false;
   double pend_alpha = 0.0, pend_beta = 0.0;
@@ -988,7 +1032,7 @@ int wait_host_values(tea_hip_chunk* c, const double* host, int count);
 // The same with a length per array.
 int finish_reduction_lens(tea_hip_chunk* c, int nr, const int* lens, double* out);
 
-// The pair-per-thread kernels apply: x even (pairs) and more than one group
+// The pair-per-thread kernels apply: pairs and more than one group
 // (the reference then runs its level-2 pass; for a single group it stops at
 // level 1, which the span-per-block kernels reproduce).
 inline bool use_pair_blocks(const tea_hip_chunk* c, int kernel_bit) {
