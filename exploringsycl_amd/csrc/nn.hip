@@ -19,6 +19,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -70,16 +71,17 @@ constexpr int nsteps() {
 }
 
 // MODE 0: out = relu(D + bias).  MODE 1: out = D * (mask > 0).
-// Grid (H, B), 256 threads; each wave walks 32-pixel tiles of row y, so the
-// weights it holds in registers serve several tiles.
+// One 32-pixel tile per wave and round, the tiles of all rows and samples
+// numbered in one sequence, so that every wave of a block has work at any
+// width (a block per row left three of four waves idle at width 32: 8.8 us
+// per hidden layer at 64 x 32 x 32); the weights a wave holds in registers
+// serve its further tiles.
 template <int CIN, int MODE>
 __global__ __launch_bounds__(256) void conv_mfma_kernel(
     const bf16* __restrict__ in, const bf16* __restrict__ wt,
     const float* __restrict__ bias, const bf16* __restrict__ mask,
     bf16* __restrict__ out, int H, int W, int B) {
   constexpr int NS = nsteps<CIN>();
-  (void)B;
-  const int y = blockIdx.x, b = blockIdx.y;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int hf = lane >> 5, col = lane & 31;
   const int Wp = W + 2;
@@ -99,9 +101,13 @@ __global__ __launch_bounds__(256) void conv_mfma_kernel(
 #pragma unroll
     for (int v = 0; v < 16; ++v) bco[v] = bias[8 * (v >> 2) + 4 * hf + (v & 3)];
   }
-  const bf16* inb = in + (size_t)b * plane * CIN;
-  for (int tile = wv; tile < W / 32; tile += 4) {
-    const int xo = tile * 32 + col;
+  const int per_row = W / 32;
+  const int tiles = B * H * per_row;
+  // Contiguous tiles per XCD (xcd_span): neighbouring rows share its L2.
+  for (int tile = xcd_span(blockIdx.x, gridDim.x) * 4 + wv; tile < tiles; tile += 4 * gridDim.x) {
+    const int row = tile / per_row, b = row / H, y = row - b * H;
+    const bf16* inb = in + (size_t)b * plane * CIN;
+    const int xo = (tile - row * per_row) * 32 + col;
     bf16x8 Bv[NS];
 #pragma unroll
     for (int t = 0; t < NS; ++t) {
@@ -425,8 +431,19 @@ __global__ __launch_bounds__(320) void out_layer_wgrad_kernel(
     if (t == kW6) {
       for (int x = 0; x < W; ++x) acc += d[x];
     } else {
+      // 32 pixels' loads before any is used (W is a multiple of 32).
       const bf16* a = a5 + ((size_t)b * plane + (size_t)(y + 1 + dy) * Wp + 1 + dx) * kC + ci;
-      for (int x = 0; x < W; ++x) acc += d[x] * (float)a[(size_t)x * kC];
+      for (int x = 0; x < W; x += 32) {
+        bf16 v[32];
+        float e[32];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+          v[k] = a[(size_t)(x + k) * kC];
+          e[k] = d[x + k];
+        }
+#pragma unroll
+        for (int k = 0; k < 32; ++k) acc += e[k] * (float)v[k];
+      }
     }
   }
   partial[(size_t)blockIdx.x * (kW6 + 1) + t] = acc;
@@ -439,7 +456,7 @@ __global__ __launch_bounds__(320) void out_layer_wgrad_kernel(
 // rows; the delta row and the three input rows it needs are staged in LDS,
 // then each wave accumulates its share of the 32-wide n blocks over all
 // pixels with MFMA steps of 16 pixels (A: lane co, 8 pixels; B: lane n,
-// the same 8 pixels).  Per-block partials are summed by wgrad_reduce.
+// the same 8 pixels).  Per-block partials are summed by reduce_grad_kernel.
 template <int CIN>
 __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
     const bf16* __restrict__ delta, const bf16* __restrict__ in,
@@ -459,22 +476,44 @@ __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
   float dbias = 0.0f;
   const int r0 = blockIdx.x * rows_per;
   const int r1 = min(r0 + rows_per, B * H);
-  for (int row = r0; row < r1; ++row) {
+  // delta[b][y+1][1..W][*] and in[b][y..y+2][0..W+1][*] of one row, in 16-byte
+  // chunks: row r + 1's are loaded into registers while row r is computed
+  // from LDS (waiting for each row's loads in turn took 17.6 us per hidden
+  // layer at 64 x 32 x 32; 13.0 us now).
+  constexpr int kD = (kMaxW * kC / 8 + 255) / 256;
+  constexpr int kA = (3 * (kMaxW + 2) * CIN / 8 + 255) / 256;
+  const int nd = W * kC / 8, na = 3 * Wp * CIN / 8;
+  bf16x8 vd[kD], va[kA];
+  auto load_row = [&](int row) {
     const int b = row / H, y = row % H;
-    __syncthreads();
-    // Stage delta[b][y+1][1..W][*] and in[b][y..y+2][0..W+1][*].
-    for (int i = threadIdx.x; i < W * kC / 8; i += 256) {
-      const int x = i / (kC / 8), c8 = (i % (kC / 8)) * 8;
-      *reinterpret_cast<bf16x8*>(sd + x * kC + c8) = *reinterpret_cast<const bf16x8*>(
-          delta + ((size_t)b * plane + (size_t)(y + 1) * Wp + x + 1) * kC + c8);
+    const bf16* d = delta + ((size_t)b * plane + (size_t)(y + 1) * Wp + 1) * kC;
+    const bf16* a = in + ((size_t)b * plane + (size_t)y * Wp) * CIN;
+#pragma unroll
+    for (int k = 0; k < kD; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      if (i < nd) vd[k] = *reinterpret_cast<const bf16x8*>(d + 8 * i);
     }
-    for (int i = threadIdx.x; i < 3 * Wp * CIN / 8; i += 256) {
-      const int rr = i / (Wp * CIN / 8), rem = i % (Wp * CIN / 8);
-      const int x = rem / (CIN / 8), c8 = (rem % (CIN / 8)) * 8;
-      *reinterpret_cast<bf16x8*>(sa + (rr * Wp + x) * CIN + c8) =
-          *reinterpret_cast<const bf16x8*>(in + ((size_t)b * plane + (size_t)(y + rr) * Wp + x) * CIN + c8);
+#pragma unroll
+    for (int k = 0; k < kA; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      if (i < na) va[k] = *reinterpret_cast<const bf16x8*>(a + 8 * i);
+    }
+  };
+  if (r0 < r1) load_row(r0);
+  for (int row = r0; row < r1; ++row) {
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kD; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      if (i < nd) *reinterpret_cast<bf16x8*>(sd + 8 * i) = vd[k];
+    }
+#pragma unroll
+    for (int k = 0; k < kA; ++k) {
+      const int i = threadIdx.x + 256 * k;
+      if (i < na) *reinterpret_cast<bf16x8*>(sa + 8 * i) = va[k];
     }
     __syncthreads();
+    if (row + 1 < r1) load_row(row + 1);
     for (int x0 = 0; x0 < W; x0 += 16) {
       bf16x8 a;
 #pragma unroll
@@ -523,42 +562,35 @@ __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
   }
 }
 
-// Sums nblk partial rows of `len` floats into `out` (fixed order).
-__global__ __launch_bounds__(256) void partial_sum_kernel(
-    const float* __restrict__ partial, int nblk, int len, float* __restrict__ out) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
+// Sums a layer's nblk partial rows ([co][tap][ci_pad] then db) in block order
+// into the master-layout gradient ([co][ci][ky][kx], then b).  One column per
+// thread; kReduceBatch rows are loaded before any is added, or each load's
+// latency would be waited for in turn (a plain loop took 60 us for 256 rows
+// of 9248 columns, 9.5 MB; this takes 5 us on average over the layers).
+constexpr int kReduceBatch = 64;
+__global__ __launch_bounds__(64) void reduce_grad_kernel(
+    const float* __restrict__ partial, int nblk, int cin_pad, int cin, int cout,
+    float* __restrict__ gw, float* __restrict__ gb) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  const int nw = cout * kTaps * cin_pad, len = nw + cout;
   if (i >= len) return;
   float s = 0.0f;
-  for (int b = 0; b < nblk; ++b) s += partial[(size_t)b * len + i];
-  out[i] = s;
-}
-
-// Scatters a layer's summed wgrad ([co][tap][ci_pad] then db) into the
-// master-layout gradient ([co][ci][ky][kx], then b).
-__global__ __launch_bounds__(256) void scatter_grad_kernel(
-    const float* __restrict__ sums, int cin_pad, int cin, int cout,
-    float* __restrict__ gw, float* __restrict__ gb) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  const int nw = cout * kTaps * cin_pad;
-  if (i < nw) {
-    const int co = i / (kTaps * cin_pad), rem = i % (kTaps * cin_pad);
-    const int tap = rem / cin_pad, ci = rem % cin_pad;
-    if (ci < cin) gw[(co * cin + ci) * kTaps + tap] = sums[i];
-  } else if (i < nw + cout) {
-    gb[i - nw] = sums[i];
+  int b = 0;
+  for (; b + kReduceBatch <= nblk; b += kReduceBatch) {
+    float v[kReduceBatch];
+#pragma unroll
+    for (int k = 0; k < kReduceBatch; ++k) v[k] = partial[(size_t)(b + k) * len + i];
+#pragma unroll
+    for (int k = 0; k < kReduceBatch; ++k) s += v[k];
   }
-}
-
-// Output layer: partial sums are [tap][ci] then db6.
-__global__ __launch_bounds__(320) void scatter_grad6_kernel(
-    const float* __restrict__ sums, float* __restrict__ gw, float* __restrict__ gb) {
-  const int t = threadIdx.x;
-  if (t < kW6) {
-    const int tap = t / kC, ci = t % kC;
-    gw[ci * kTaps + tap] = sums[t];
-  } else if (t == kW6) {
-    gb[0] = sums[t];
+  for (; b < nblk; ++b) s += partial[(size_t)b * len + i];
+  if (i >= nw) {
+    gb[i - nw] = s;
+    return;
   }
+  const int co = i / (kTaps * cin_pad), rem = i % (kTaps * cin_pad);
+  const int tap = rem / cin_pad, ci = rem % cin_pad;
+  if (ci < cin) gw[(co * cin + ci) * kTaps + tap] = s;
 }
 
 // ---- parameters ------------------------------------------------------------
@@ -652,7 +684,8 @@ struct tea_nn {
   bf16* act[5] = {};         // a1..a5 [B][H+2][W+2][32]
   bf16* del[5] = {};         // delta1..delta5
   float *out = nullptr, *target = nullptr, *dout = nullptr;
-  float *partial = nullptr, *sums = nullptr, *loss_part = nullptr;
+  float *partial = nullptr, *loss_part = nullptr;
+  size_t loss_len = 0;       // floats loss_part holds
   size_t partial_len = 0;
   int wg_blocks = 0;
   // device-resident training set
@@ -684,7 +717,12 @@ int pack_params(tea_nn* n) {
   return TEA_HIP_OK;
 }
 
-dim3 rows_grid(const tea_nn* n, int batch) { return dim3(n->H, batch); }
+// conv_mfma_kernel's grid: a tile per wave, at most 2048 blocks (the chip
+// holds about that many at once).
+dim3 conv_grid(const tea_nn* n, int batch) {
+  const long tiles = (long)batch * n->H * (n->W / 32);
+  return dim3((unsigned)std::min(2048L, (tiles + 3) / 4));
+}
 unsigned flat_blocks(long count) { return (unsigned)((count + 255) / 256); }
 
 // Forward pass over `batch` samples whose packed input is in n->in0, on
@@ -729,10 +767,10 @@ int forward_on(tea_nn* n, int batch, hipStream_t st, bool with_output = true,
                          n->wfh + (size_t)(l - 1) * kWh, n->bias + l * kC, n->act[l], H, W);
   } else {
     if (first == 0)
-      hipLaunchKernelGGL((conv_mfma_kernel<kC0, 0>), rows_grid(n, batch), dim3(256), 0,
+      hipLaunchKernelGGL((conv_mfma_kernel<kC0, 0>), conv_grid(n, batch), dim3(256), 0,
                          st, n->in0, n->wf1, n->bias, nullptr, n->act[0], H, W, batch);
     for (int l = first > 1 ? first : 1; l < 5; ++l)
-      hipLaunchKernelGGL((conv_mfma_kernel<kC, 0>), rows_grid(n, batch), dim3(256), 0,
+      hipLaunchKernelGGL((conv_mfma_kernel<kC, 0>), conv_grid(n, batch), dim3(256), 0,
                          st, n->act[l - 1], n->wfh + (size_t)(l - 1) * kWh,
                          n->bias + l * kC, nullptr, n->act[l], H, W, batch);
   }
@@ -757,24 +795,44 @@ int wgrad_layer(tea_nn* n, int batch, int layer, const bf16* delta, const bf16* 
   else
     hipLaunchKernelGGL((wgrad_mfma_kernel<kC>), dim3(nblk), dim3(256), 0, n->stream,
                        delta, in, n->partial, batch, n->H, n->W, rows_per);
-  hipLaunchKernelGGL(partial_sum_kernel, dim3((len + 255) / 256), dim3(256), 0, n->stream,
-                     n->partial, nblk, len, n->sums);
-  const int cin = layer == 0 ? kIn : kC;
-  hipLaunchKernelGGL(scatter_grad_kernel, dim3((len + 255) / 256), dim3(256), 0,
-                     n->stream, n->sums, cin_pad, cin, kC, n->grad + w_offset(layer),
-                     n->grad + b_offset(layer));
+  hipLaunchKernelGGL(reduce_grad_kernel, dim3((len + 63) / 64), dim3(64), 0, n->stream,
+                     n->partial, nblk, cin_pad, layer == 0 ? kIn : kC, kC,
+                     n->grad + w_offset(layer), n->grad + b_offset(layer));
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
 }
 
-// Loss and gradients for `batch` samples (input packed, targets in place).
-int loss_and_grad(tea_nn* n, int batch, float* loss) {
+// Blocks of mse_kernel, each leaving one partial of a batch's squared error.
+unsigned loss_blocks(const tea_nn* n, int batch) {
+  return flat_blocks((long)batch * n->H * n->W);
+}
+
+// The losses of `batches` batches from their partials, one batch after the
+// other in n->loss_part (waits for the stream).
+int read_losses(tea_nn* n, int batch, int batches, float* loss) {
+  const size_t nb = loss_blocks(n, batch);
+  const long cnt = (long)batch * n->H * n->W;
+  std::vector<float> lp(nb * batches);
+  TEA_HIP_TRY(hipMemcpyAsync(lp.data(), n->loss_part, lp.size() * sizeof(float),
+                             hipMemcpyDeviceToHost, n->stream));
+  TEA_HIP_TRY(hipStreamSynchronize(n->stream));
+  for (int k = 0; k < batches; ++k) {
+    double s = 0.0;
+    for (size_t i = 0; i < nb; ++i) s += lp[k * nb + i];
+    loss[k] = (float)(s / (double)cnt);
+  }
+  return TEA_HIP_OK;
+}
+
+// Queues the loss partials (batch k's in n->loss_part) and gradients for
+// `batch` samples (input packed, targets in place).
+int loss_and_grad(tea_nn* n, int batch, int k = 0) {
   const int H = n->H, W = n->W;
   TEA_RETURN_IF(forward(n, batch));
   const long cnt = (long)batch * H * W;
-  const unsigned nb = flat_blocks(cnt);
+  const unsigned nb = loss_blocks(n, batch);
   hipLaunchKernelGGL(mse_kernel, dim3(nb), dim3(256), 0, n->stream, n->out, n->target,
-                     n->dout, n->loss_part, cnt);
+                     n->dout, n->loss_part + (size_t)k * nb, cnt);
   // Output layer.
   hipLaunchKernelGGL(out_layer_bwd_data_kernel, dim3(nb), dim3(256), 0, n->stream,
                      n->dout, n->w6, n->act[4], n->del[4], batch, H, W);
@@ -784,27 +842,19 @@ int loss_and_grad(tea_nn* n, int batch, float* loss) {
     const int nblk = (rows + rows_per - 1) / rows_per;
     hipLaunchKernelGGL(out_layer_wgrad_kernel, dim3(nblk), dim3(320), 0, n->stream,
                        n->dout, n->act[4], n->partial, batch, H, W, rows_per);
-    hipLaunchKernelGGL(partial_sum_kernel, dim3((kW6 + 1 + 255) / 256), dim3(256), 0,
-                       n->stream, n->partial, nblk, kW6 + 1, n->sums);
-    hipLaunchKernelGGL(scatter_grad6_kernel, dim3(1), dim3(320), 0, n->stream, n->sums,
-                       n->grad + w_offset(5), n->grad + b_offset(5));
+    hipLaunchKernelGGL(reduce_grad_kernel, dim3((kW6 + 1 + 63) / 64), dim3(64), 0, n->stream,
+                       n->partial, nblk, kC, kC, 1, n->grad + w_offset(5),
+                       n->grad + b_offset(5));
   }
   // Hidden layers 5..2, then layer 1.
   for (int l = 4; l >= 1; --l) {
     TEA_RETURN_IF(wgrad_layer(n, batch, l, n->del[l], n->act[l - 1]));
-    hipLaunchKernelGGL((conv_mfma_kernel<kC, 1>), rows_grid(n, batch), dim3(256), 0,
+    hipLaunchKernelGGL((conv_mfma_kernel<kC, 1>), conv_grid(n, batch), dim3(256), 0,
                        n->stream, n->del[l], n->wbh + (size_t)(l - 1) * kWh, nullptr,
                        n->act[l - 1], n->del[l - 1], H, W, batch);
   }
   TEA_RETURN_IF(wgrad_layer(n, batch, 0, n->del[0], n->in0));
   TEA_HIP_TRY(hipGetLastError());
-  std::vector<float> lp(nb);
-  TEA_HIP_TRY(hipMemcpyAsync(lp.data(), n->loss_part, nb * sizeof(float),
-                             hipMemcpyDeviceToHost, n->stream));
-  TEA_HIP_TRY(hipStreamSynchronize(n->stream));
-  double s = 0.0;
-  for (float v : lp) s += v;
-  if (loss) *loss = (float)(s / (double)cnt);
   return TEA_HIP_OK;
 }
 
@@ -835,19 +885,24 @@ int upload_batch(tea_nn* n, int batch, const float* input, const float* target) 
   return TEA_HIP_OK;
 }
 
-// Gathers samples order[0..batch) of the resident training set.
+// Gathers samples order[0..batch) of the resident training set: the packed
+// input (as pack_input_kernel) and the targets.
 __global__ __launch_bounds__(256) void gather_kernel(const float* __restrict__ ds_in,
                                                      const float* __restrict__ ds_tgt,
                                                      const int* __restrict__ order,
-                                                     float* __restrict__ in,
-                                                     float* __restrict__ tgt,
-                                                     int batch, int px) {
+                                                     bf16* __restrict__ in0,
+                                                     float* __restrict__ tgt, int batch,
+                                                     int H, int W) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  const int px = H * W;
   if (i >= (long)batch * px) return;
-  const int b = (int)(i / px), p = (int)(i % px);
+  const int b = (int)(i / px), p = (int)(i % px), y = p / W, x = p % W;
   const long src = (long)order[b] * px + p;
   tgt[i] = ds_tgt[src];
-  for (int c = 0; c < kIn; ++c) in[i * kIn + c] = ds_in[src * kIn + c];
+  bf16x8 o = bf16x8{};
+  for (int c = 0; c < kIn; ++c) o[c] = (bf16)ds_in[src * kIn + c];
+  const size_t pix = (size_t)b * (H + 2) * (W + 2) + (size_t)(y + 1) * (W + 2) + (x + 1);
+  *reinterpret_cast<bf16x8*>(in0 + pix * kC0) = o;
 }
 
 #define NN_CHECK(n) TEA_CHECK_ARG((n) != nullptr, "null network handle")
@@ -901,6 +956,7 @@ int tea_nn_create(int device, int max_batch, int height, int width, tea_nn** out
   }
   const size_t px = (size_t)max_batch * height * width;
   n->wg_blocks = 256;
+  n->loss_len = px / 256 + 2;
   n->partial_len = (size_t)n->wg_blocks * (kC * kTaps * kC + kC);
   struct {
     void** p;
@@ -921,8 +977,7 @@ int tea_nn_create(int device, int max_batch, int height, int width, tea_nn** out
       {(void**)&n->target, px * sizeof(float)},
       {(void**)&n->dout, px * sizeof(float)},
       {(void**)&n->partial, n->partial_len * sizeof(float)},
-      {(void**)&n->sums, (size_t)(kC * kTaps * kC + kC) * sizeof(float)},
-      {(void**)&n->loss_part, (px / 256 + 2) * sizeof(float)},
+      {(void**)&n->loss_part, n->loss_len * sizeof(float)},
   };
   for (auto& b : bufs) {
     const int st = nn_alloc(b.p, b.bytes, n->stream);
@@ -948,7 +1003,7 @@ int tea_nn_destroy(tea_nn* n) {
   if (n->stream) (void)hipStreamSynchronize(n->stream);
   void* ptrs[] = {n->master, n->grad, n->adam_m, n->adam_v, n->wf1, n->wfh, n->wbh,
                   n->w6, n->bias, n->in_f32, n->in0, n->out, n->target, n->dout,
-                  n->partial, n->sums, n->loss_part, n->ds_in, n->ds_tgt, n->ds_order};
+                  n->partial, n->loss_part, n->ds_in, n->ds_tgt, n->ds_order};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (int l = 0; l < 5; ++l) {
@@ -1005,12 +1060,13 @@ int tea_nn_loss_grad(tea_nn* n, int batch, const float* input, const float* targ
   TEA_CHECK_ARG(n->del[0] != nullptr, "training needs width <= 128");
   TEA_HIP_TRY(hipSetDevice(n->device));
   TEA_RETURN_IF(upload_batch(n, batch, input, target));
-  TEA_RETURN_IF(loss_and_grad(n, batch, loss));
-  if (grad) {
+  TEA_RETURN_IF(loss_and_grad(n, batch));
+  if (grad)
     TEA_HIP_TRY(hipMemcpyAsync(grad, n->grad, kNumParams * sizeof(float),
                                hipMemcpyDeviceToHost, n->stream));
-    TEA_HIP_TRY(hipStreamSynchronize(n->stream));
-  }
+  float l = 0.0f;
+  TEA_RETURN_IF(read_losses(n, batch, 1, &l));
+  if (loss) *loss = l;
   return TEA_HIP_OK;
 }
 
@@ -1082,22 +1138,30 @@ int tea_nn_train_epoch(tea_nn* n, const int* order, int count, int batch, float 
     TEA_CHECK_ARG(order[i] >= 0 && order[i] < n->ds_n, "sample index out of range");
   TEA_HIP_TRY(hipMemcpyAsync(n->ds_order, order, (size_t)count * sizeof(int),
                              hipMemcpyHostToDevice, n->stream));
-  const int px = n->H * n->W;
-  double total = 0.0;
-  int steps = 0;
-  for (int s = 0; s + batch <= count; s += batch) {
-    hipLaunchKernelGGL(gather_kernel, dim3(flat_blocks((long)batch * px)), dim3(256), 0,
-                       n->stream, n->ds_in, n->ds_tgt, n->ds_order + s, n->in_f32,
-                       n->target, batch, px);
-    hipLaunchKernelGGL(pack_input_kernel, dim3(flat_blocks((long)batch * px)), dim3(256),
-                       0, n->stream, n->in_f32, n->in0, batch, n->H, n->W);
-    float loss = 0.0f;
-    TEA_RETURN_IF(loss_and_grad(n, batch, &loss));
-    TEA_RETURN_IF(adam_step(n, lr));
-    total += loss;
-    ++steps;
+  // The batches' loss partials stay on the device until the epoch's end: a
+  // read back per batch left the GPU idle for 52 us of each 650 us step.
+  const int steps = count / batch;
+  const size_t need = (size_t)steps * loss_blocks(n, batch);
+  if (need > n->loss_len) {
+    float* more = nullptr;
+    TEA_RETURN_IF(nn_alloc((void**)&more, need * sizeof(float), n->stream));
+    (void)hipFree(n->loss_part);
+    n->loss_part = more;
+    n->loss_len = need;
   }
-  TEA_HIP_TRY(hipStreamSynchronize(n->stream));
+  const int px = n->H * n->W;
+  for (int k = 0; k < steps; ++k) {
+    hipLaunchKernelGGL(gather_kernel, dim3(flat_blocks((long)batch * px)), dim3(256), 0,
+                       n->stream, n->ds_in, n->ds_tgt, n->ds_order + (size_t)k * batch, n->in0,
+                       n->target, batch, n->H, n->W);
+    TEA_HIP_TRY(hipGetLastError());
+    TEA_RETURN_IF(loss_and_grad(n, batch, k));
+    TEA_RETURN_IF(adam_step(n, lr));
+  }
+  std::vector<float> losses(steps);
+  TEA_RETURN_IF(read_losses(n, batch, steps, losses.data()));
+  double total = 0.0;
+  for (float l : losses) total += l;
   if (mean_loss) *mean_loss = (float)(total / (steps ? steps : 1));
   return TEA_HIP_OK;
 }
