@@ -491,12 +491,6 @@ int tea_hip_chunk_destroy(tea_hip_chunk* c) {
     if (b) (void)hipFree(b);
   if (c->fcg_xsum) (void)hipFree(c->fcg_xsum);
   if (c->fcg_g) (void)hipFree(c->fcg_g);
-  if (c->fcg_side) {
-    (void)hipStreamSynchronize(c->fcg_side);
-    (void)hipStreamDestroy(c->fcg_side);
-  }
-  if (c->fcg_fork) (void)hipEventDestroy(c->fcg_fork);
-  if (c->fcg_join) (void)hipEventDestroy(c->fcg_join);
   for (FcgLevel& L : c->fcg_lv) {
     for (float* b : {L.feat, L.rbar, L.kc, L.dis, L.sig, L.y})
       if (b) (void)hipFree(b);

@@ -445,21 +445,37 @@ constexpr int kSweepR = kSweepTile + 2 * (kMaxSweeps + 1);  // staged side, at m
 // rounded to FP32 into y, T y of the rounded y in the operand order of
 // TeaLeaf's SMVP (shared.h:59-63), and the tile's partial sums of y.rbar
 // and y.T y (the block's LDS tree) at part[tile] and part[ntiles + tile],
-// tile = blockIdx.y * gridDim.x + blockIdx.x; with xsum, the sums of T y
+// tiles in row-major order; with xsum, the sums of T y
 // over the tile's 4 x 4 blocks (the level-1 cells; the cross term).
-__global__ __launch_bounds__(256) void sweeps_kernel(int hc, int wc, int sweeps,
-                                                     const float* __restrict__ kc,
-                                                     const float* __restrict__ rbar,
-                                                     float* __restrict__ y,
-                                                     double* __restrict__ part, int ntiles,
-                                                     double* __restrict__ xsum) {
+// Both levels in one launch: the first nb0 blocks take level 0's tiles.
+struct SweepLevel {
+  int hc, wc, ntiles;
+  const float* kc;
+  const float* rbar;
+  float* y;
+  double* part;
+  double* xsum;
+};
+__global__ __launch_bounds__(256) void sweeps_kernel(SweepLevel lv0, SweepLevel lv1, int nb0,
+                                                     int sweeps) {
+  const bool second = (int)blockIdx.x >= nb0;
+  const int hc = second ? lv1.hc : lv0.hc, wc = second ? lv1.wc : lv0.wc;
+  const int ntiles = second ? lv1.ntiles : lv0.ntiles;
+  const float* __restrict__ kc = second ? lv1.kc : lv0.kc;
+  const float* __restrict__ rbar = second ? lv1.rbar : lv0.rbar;
+  float* __restrict__ y = second ? lv1.y : lv0.y;
+  double* __restrict__ part = second ? lv1.part : lv0.part;
+  double* __restrict__ xsum = second ? nullptr : lv0.xsum;
+  const int tile = (int)blockIdx.x - (second ? nb0 : 0);
+  const int tiles_x = (wc + kSweepTile - 1) / kSweepTile;
+  const int by = tile / tiles_x, bx = tile - by * tiles_x;
   __shared__ float s_rb[kSweepR * kSweepR];
   __shared__ float s_kl[kSweepR * (kSweepR + 1)];  // left faces, one more column
   __shared__ float s_kb[(kSweepR + 1) * kSweepR];  // bottom faces, one more row
   __shared__ double s_y[2][kSweepR * kSweepR];
   __shared__ double s_a[256], s_b[256], s_t[256];
   const int H = sweeps + 1, R = kSweepTile + 2 * H;
-  const int X0 = blockIdx.x * kSweepTile - H, Y0 = blockIdx.y * kSweepTile - H;
+  const int X0 = bx * kSweepTile - H, Y0 = by * kSweepTile - H;
   const long n = (long)hc * wc;
   for (int q = threadIdx.x; q < (R + 1) * (R + 1); q += 256) {
     const int lx = q % (R + 1), ly = q / (R + 1);
@@ -500,7 +516,7 @@ __global__ __launch_bounds__(256) void sweeps_kernel(int hc, int wc, int sweeps,
   const double* yv = s_y[cur];
   const int tx = threadIdx.x & (kSweepTile - 1), ty = threadIdx.x / kSweepTile;
   const int lx = H + tx, ly = H + ty, k = ly * R + lx;
-  const int X = blockIdx.x * kSweepTile + tx, Y = blockIdx.y * kSweepTile + ty;
+  const int X = bx * kSweepTile + tx, Y = by * kSweepTile + ty;
   auto yr = [&](int kk) { return (double)(float)yv[kk]; };
   const double kl = s_kl[ly * (R + 1) + lx], kr = s_kl[ly * (R + 1) + lx + 1];
   const double kb = s_kb[ly * R + lx], kt = s_kb[(ly + 1) * R + lx];
@@ -525,18 +541,17 @@ __global__ __launch_bounds__(256) void sweeps_kernel(int hc, int wc, int sweeps,
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    const int tile = blockIdx.y * gridDim.x + blockIdx.x;
     part[tile] = s_a[0];
     part[ntiles + tile] = s_b[0];
   }
   if (xsum && threadIdx.x < 16) {
-    const int bx = threadIdx.x & 3, by = threadIdx.x >> 2;
-    const int X1 = blockIdx.x * 4 + bx, Y1 = blockIdx.y * 4 + by;
+    const int cx = threadIdx.x & 3, cy = threadIdx.x >> 2;
+    const int X1 = bx * 4 + cx, Y1 = by * 4 + cy;
     if (X1 < (wc >> 2) && Y1 < (hc >> 2)) {
       double rs[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const double* p = &s_t[(4 * by + j) * kSweepTile + 4 * bx];
+        const double* p = &s_t[(4 * cy + j) * kSweepTile + 4 * cx];
         rs[j] = (p[0] + p[1]) + (p[2] + p[3]);
       }
       xsum[(long)Y1 * (wc >> 2) + X1] = (rs[0] + rs[1]) + (rs[2] + rs[3]);
@@ -959,10 +974,31 @@ constexpr int kBoxC = kBoxT + 4;          // 20: sigma and input region
 constexpr int kBoxS = kBoxC + 2 * kWin;   // 32: staged region
 constexpr int kBoxStage = (2 * kBoxS * kBoxS + kBoxS * kBoxC) * 4;  // bytes
 constexpr int kBoxA1 = kBoxA * kBoxA * 5 * 16;                       // bytes
-__global__ __launch_bounds__(256) void box_conv_kernel(
-    int hc, int wc, const float* __restrict__ rbar, const float* __restrict__ dis,
-    const double* __restrict__ part, int npart, const float* __restrict__ feat,
-    float* __restrict__ sig, nn::PackedWeights wts, bf16* __restrict__ a2) {
+struct BoxLevel {
+  int hc, wc, npart;
+  const float* rbar;
+  const float* dis;
+  const double* part;
+  const float* feat;
+  float* sig;
+  nn::PackedWeights wts;
+  bf16* a2;
+};
+// Both levels in one launch: the first nb0 blocks take level 0's tiles.
+__global__ __launch_bounds__(256) void box_conv_kernel(BoxLevel lv0, BoxLevel lv1, int nb0) {
+  const bool second = (int)blockIdx.x >= nb0;
+  const int hc = second ? lv1.hc : lv0.hc, wc = second ? lv1.wc : lv0.wc;
+  const int npart = second ? lv1.npart : lv0.npart;
+  const float* __restrict__ rbar = second ? lv1.rbar : lv0.rbar;
+  const float* __restrict__ dis = second ? lv1.dis : lv0.dis;
+  const double* __restrict__ part = second ? lv1.part : lv0.part;
+  const float* __restrict__ feat = second ? lv1.feat : lv0.feat;
+  float* __restrict__ sig = second ? lv1.sig : lv0.sig;
+  const nn::PackedWeights wts = second ? lv1.wts : lv0.wts;
+  bf16* __restrict__ a2 = second ? lv1.a2 : lv0.a2;
+  const int tile = (int)blockIdx.x - (second ? nb0 : 0);
+  const int tiles_x = (wc + kBoxT - 1) / kBoxT;
+  const int by = tile / tiles_x, bx = tile - by * tiles_x;
   constexpr int kN = kBoxS * kBoxS;
   constexpr int kIt = (kN + 255) / 256;
   constexpr int kNq = (kBoxC * kBoxC + 255) / 256;
@@ -978,7 +1014,7 @@ __global__ __launch_bounds__(256) void box_conv_kernel(
   __shared__ double s_sc[256];
   __shared__ float s_floor;
   const int tid = threadIdx.x;
-  const int X0 = blockIdx.x * kBoxT, Y0 = blockIdx.y * kBoxT;
+  const int X0 = bx * kBoxT, Y0 = by * kBoxT;
   const long n = (long)hc * wc;
   auto in_grid = [&](int X, int Y) { return X >= 0 && X < wc && Y >= 0 && Y < hc; };
   // Every global load first: the first layer's weights, the RMS partials (8
@@ -1111,12 +1147,37 @@ __global__ __launch_bounds__(256) void box_conv_kernel(
 // 256-thread block per 16 x 16 tile.  (A separate output-layer launch read
 // each activation about three times from HBM and wrote N for this kernel
 // to read back: 14 + 6.7 us at 512^2.)
-__global__ __launch_bounds__(256) void out_tile_kernel(
-    int hc, int wc, const bf16* __restrict__ a5, const float* __restrict__ w6,
-    const float* __restrict__ bias, const float* __restrict__ sig,
-    const float* __restrict__ dis, const float* __restrict__ rbar,
-    const float* __restrict__ kc, float* __restrict__ y, double* __restrict__ part,
-    int ntiles, double* __restrict__ xsum) {
+struct OutLevel {
+  int hc, wc, ntiles;
+  const bf16* a5;
+  const float* w6;
+  const float* bias;
+  const float* sig;
+  const float* dis;
+  const float* rbar;
+  const float* kc;
+  float* y;
+  double* part;
+  double* xsum;
+};
+// Both levels in one launch: the first nb0 blocks take level 0's tiles.
+__global__ __launch_bounds__(256) void out_tile_kernel(OutLevel lv0, OutLevel lv1, int nb0) {
+  const bool second = (int)blockIdx.x >= nb0;
+  const int hc = second ? lv1.hc : lv0.hc, wc = second ? lv1.wc : lv0.wc;
+  const int ntiles = second ? lv1.ntiles : lv0.ntiles;
+  const bf16* __restrict__ a5 = second ? lv1.a5 : lv0.a5;
+  const float* __restrict__ w6 = second ? lv1.w6 : lv0.w6;
+  const float* __restrict__ bias = second ? lv1.bias : lv0.bias;
+  const float* __restrict__ sig = second ? lv1.sig : lv0.sig;
+  const float* __restrict__ dis = second ? lv1.dis : lv0.dis;
+  const float* __restrict__ rbar = second ? lv1.rbar : lv0.rbar;
+  const float* __restrict__ kc = second ? lv1.kc : lv0.kc;
+  float* __restrict__ y = second ? lv1.y : lv0.y;
+  double* __restrict__ part = second ? lv1.part : lv0.part;
+  double* __restrict__ xsum = second ? nullptr : lv0.xsum;
+  const int tile = (int)blockIdx.x - (second ? nb0 : 0);
+  const int tiles_x = (wc + fused::kT - 1) / fused::kT;
+  const int tby = tile / tiles_x, tbx = tile - tby * tiles_x;
   using namespace fused;
   constexpr int kSA = kSN + 2;                // 20: staged activation region
   constexpr int kChunks = kSA * kSA * 4;      // 16-byte chunks staged
@@ -1127,7 +1188,7 @@ __global__ __launch_bounds__(256) void out_tile_kernel(
   __shared__ float s_sd[kSN * kSN];
   __shared__ double s_a[256], s_b[256], s_t[256];
   const int tid = threadIdx.x;
-  const int X0 = blockIdx.x * kT, Y0 = blockIdx.y * kT;
+  const int X0 = tbx * kT, Y0 = tby * kT;
   const long n = (long)hc * wc;
   // Every global load of the kernel is issued before the first LDS store:
   // the staged activations, sigma D^-1/2 on the tile and its ring, and the
@@ -1204,7 +1265,7 @@ __global__ __launch_bounds__(256) void out_tile_kernel(
   __syncthreads();
   if (xsum && tid >= 64 && tid < 80) {
     const int bx = tid & 3, by = (tid >> 2) & 3;
-    const int X1 = blockIdx.x * 4 + bx, Y1 = blockIdx.y * 4 + by;
+    const int X1 = tbx * 4 + bx, Y1 = tby * 4 + by;
     if (X1 < (wc >> 2) && Y1 < (hc >> 2)) {
       double rs[4];
 #pragma unroll
@@ -1230,7 +1291,6 @@ __global__ __launch_bounds__(256) void out_tile_kernel(
       vb = vb + __shfl_down(vb, st);
     }
     if (tid == 0) {
-      const int tile = blockIdx.y * gridDim.x + blockIdx.x;
       part[tile] = va;
       part[ntiles + tile] = vb;
     }
@@ -1403,52 +1463,76 @@ static bool net_per_layer() {
   return v;
 }
 
-// The learned coarse solve of level l on stream st: y, the tile partials
-// and (level 0 of two) the level-1 block sums of T y.
-static int launch_net_level(tea_hip_chunk* c, int l, hipStream_t st) {
-  FcgLevel& L = c->fcg_lv[l];
-  const dim3 tiles((unsigned)(L.wc + fused::kT - 1) / fused::kT,
-                   (unsigned)(L.hc + fused::kT - 1) / fused::kT);
-  double* xs = (l == 0 && c->fcg_levels == 2) ? c->fcg_xsum : nullptr;
-  Timed t(c, K_FCG_NET, st);
+static unsigned level_tiles(const FcgLevel& L, int side) {
+  return (unsigned)((L.wc + side - 1) / side) * (unsigned)((L.hc + side - 1) / side);
+}
+
+// The learned coarse solve of every level: y, the tile partials and (level 0
+// of two) the level-1 block sums of T y.
+static int launch_net_levels(tea_hip_chunk* c) {
+  const int nl = c->fcg_levels;
+  hipStream_t st = c->stream;
+  double* xs = nl == 2 ? c->fcg_xsum : nullptr;
+  Timed t(c, K_FCG_NET);
   if (!net_per_layer()) {
     const NetShape shape = net_shape();
-    hipLaunchKernelGGL(net_level_fn(shape), tiles, dim3(shape.threads), fused::kLdsBytes, st,
-                       L.hc, L.wc, L.rbar, L.dis, L.feat, L.kc, L.rms, L.nrms,
-                       nn::packed_weights(L.net), L.y, L.tpart, L.ntiles, xs);
-  } else {
-    const dim3 boxes((unsigned)(L.wc + kBoxT - 1) / kBoxT,
-                     (unsigned)(L.hc + kBoxT - 1) / kBoxT);
-    hipLaunchKernelGGL(box_conv_kernel, boxes, dim3(256), 0, st, L.hc, L.wc, L.rbar, L.dis,
-                       L.rms, L.nrms, L.feat, L.sig, nn::packed_weights(L.net),
-                       nn::hidden(L.net, 1));
-    TEA_RETURN_IF(nn::forward_hidden_on_stream(L.net, st, 2));
-    const nn::PackedWeights wts = nn::packed_weights(L.net);
-    hipLaunchKernelGGL(out_tile_kernel, tiles, dim3(256), 0, st, L.hc, L.wc,
-                       nn::last_hidden(L.net), wts.w6, wts.bias, L.sig, L.dis, L.rbar, L.kc,
-                       L.y, L.tpart, L.ntiles, xs);
+    for (int l = 0; l < nl; ++l) {
+      FcgLevel& L = c->fcg_lv[l];
+      const dim3 tiles((unsigned)(L.wc + fused::kT - 1) / fused::kT,
+                       (unsigned)(L.hc + fused::kT - 1) / fused::kT);
+      hipLaunchKernelGGL(net_level_fn(shape), tiles, dim3(shape.threads), fused::kLdsBytes, st,
+                         L.hc, L.wc, L.rbar, L.dis, L.feat, L.kc, L.rms, L.nrms,
+                         nn::packed_weights(L.net), L.y, L.tpart, L.ntiles,
+                         l == 0 ? xs : nullptr);
+    }
+    TEA_HIP_TRY(hipGetLastError());
+    return TEA_HIP_OK;
   }
+  auto box = [&](const FcgLevel& L) {
+    return BoxLevel{L.hc, L.wc, L.nrms, L.rbar, L.dis, L.rms, L.feat, L.sig,
+                    nn::packed_weights(L.net), nn::hidden(L.net, 1)};
+  };
+  auto out = [&](const FcgLevel& L) {
+    const nn::PackedWeights w = nn::packed_weights(L.net);
+    return OutLevel{L.hc, L.wc, L.ntiles, nn::last_hidden(L.net), w.w6, w.bias, L.sig, L.dis,
+                    L.rbar, L.kc, L.y, L.tpart, xs};
+  };
+  FcgLevel& L0 = c->fcg_lv[0];
+  FcgLevel& L1 = c->fcg_lv[nl - 1];  // level 0 stands in where there is one
+  const unsigned nb = level_tiles(L0, kBoxT), nt = level_tiles(L0, fused::kT);
+  const unsigned nb1 = nl == 2 ? level_tiles(L1, kBoxT) : 0;
+  const unsigned nt1 = nl == 2 ? level_tiles(L1, fused::kT) : 0;
+  hipLaunchKernelGGL(box_conv_kernel, dim3(nb + nb1), dim3(256), 0, st, box(L0), box(L1), (int)nb);
+  TEA_HIP_TRY(hipGetLastError());
+  TEA_RETURN_IF(nl == 2 ? nn::forward_hidden_pair(L0.net, L1.net, st, 2)
+                        : nn::forward_hidden_on_stream(L0.net, st, 2));
+  hipLaunchKernelGGL(out_tile_kernel, dim3(nt + nt1), dim3(256), 0, st, out(L0), out(L1), (int)nt);
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
 }
 
-// The non-learned coarse solve of level l on stream st (same outputs).
-static int launch_sweeps_level(tea_hip_chunk* c, int l, hipStream_t st) {
-  FcgLevel& L = c->fcg_lv[l];
-  Timed t(c, K_FCG_SWEEPS, st);
-  const dim3 grid((unsigned)(L.wc + kSweepTile - 1) / kSweepTile,
-                  (unsigned)(L.hc + kSweepTile - 1) / kSweepTile);
-  hipLaunchKernelGGL(sweeps_kernel, grid, dim3(256), 0, st, L.hc, L.wc, c->fcg_sweeps,
-                     L.kc, L.rbar, L.y, L.tpart, L.ntiles,
-                     (l == 0 && c->fcg_levels == 2) ? c->fcg_xsum : nullptr);
+// The non-learned coarse solve of every level (same outputs).
+static int launch_sweeps_levels(tea_hip_chunk* c) {
+  const int nl = c->fcg_levels;
+  auto args = [&](const FcgLevel& L) {
+    return SweepLevel{L.hc, L.wc, L.ntiles, L.kc, L.rbar, L.y, L.tpart,
+                      nl == 2 ? c->fcg_xsum : nullptr};
+  };
+  const FcgLevel& L0 = c->fcg_lv[0];
+  const FcgLevel& L1 = c->fcg_lv[nl - 1];
+  const unsigned nb0 = level_tiles(L0, kSweepTile);
+  const unsigned nb1 = nl == 2 ? level_tiles(L1, kSweepTile) : 0;
+  Timed t(c, K_FCG_SWEEPS);
+  hipLaunchKernelGGL(sweeps_kernel, dim3(nb0 + nb1), dim3(256), 0, c->stream, args(L0), args(L1),
+                     (int)nb0, c->fcg_sweeps);
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
 }
 
 // The coarse part of the two-level preconditioner: the restriction of both
 // levels in one pass (with the RMS partials the network's input scale
-// needs), each level's coarse solve (level 1 on the side stream, beside
-// level 0 on the chunk's), and the factors into c->fcg_g.
+// needs), the levels' coarse solves (both in each launch), and the factors
+// into c->fcg_g.
 static int launch_coarse(tea_hip_chunk* c) {
   const int nl = c->fcg_levels;
   const bool net = c->fcg_sweeps == 0;
@@ -1465,25 +1549,7 @@ static int launch_coarse(tea_hip_chunk* c) {
                        net && nl == 2 ? L1.rms : nullptr);
     TEA_HIP_TRY(hipGetLastError());
   }
-  auto level = [&](int l, hipStream_t st) {
-    return net ? launch_net_level(c, l, st) : launch_sweeps_level(c, l, st);
-  };
-  // The network's two level chains overlap on two streams; the sweeps'
-  // single kernels are shorter than the fork and join between the streams
-  // (about 17 us at 4096^2), so they run one after the other.
-  if (nl == 2 && !net) {
-    TEA_RETURN_IF(level(0, c->stream));
-    TEA_RETURN_IF(level(1, c->stream));
-  } else if (nl == 2) {
-    TEA_HIP_TRY(hipEventRecord(c->fcg_fork, c->stream));
-    TEA_HIP_TRY(hipStreamWaitEvent(c->fcg_side, c->fcg_fork, 0));
-    TEA_RETURN_IF(level(1, c->fcg_side));
-    TEA_RETURN_IF(level(0, c->stream));
-    TEA_HIP_TRY(hipEventRecord(c->fcg_join, c->fcg_side));
-    TEA_HIP_TRY(hipStreamWaitEvent(c->stream, c->fcg_join, 0));
-  } else {
-    TEA_RETURN_IF(level(0, c->stream));
-  }
+  TEA_RETURN_IF(net ? launch_net_levels(c) : launch_sweeps_levels(c));
   Timed t(c, net ? K_FCG_NET : K_FCG_SWEEPS);
   hipLaunchKernelGGL(joint_gamma_kernel, dim3(1), dim3(kGammaThreads), 0, c->stream, nl,
                      L0.tpart,
@@ -1632,14 +1698,6 @@ static void release_levels(tea_hip_chunk* c) {
   c->fcg_sweeps = 0;
 }
 
-// The side stream and the fork / join events of a two-level coarse part.
-static int ensure_side_stream(tea_hip_chunk* c) {
-  if (!c->fcg_side) TEA_HIP_TRY(hipStreamCreateWithFlags(&c->fcg_side, hipStreamNonBlocking));
-  if (!c->fcg_fork) TEA_HIP_TRY(hipEventCreateWithFlags(&c->fcg_fork, hipEventDisableTiming));
-  if (!c->fcg_join) TEA_HIP_TRY(hipEventCreateWithFlags(&c->fcg_join, hipEventDisableTiming));
-  return TEA_HIP_OK;
-}
-
 extern "C" {
 
 int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int levels) {
@@ -1680,7 +1738,6 @@ int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int lev
   if (c->fcg_levels == 2) {
     const size_t n1 = (size_t)c->fcg_lv[1].hc * c->fcg_lv[1].wc;
     if (hipMalloc(&c->fcg_xsum, n1 * sizeof(double)) != hipSuccess) return fail();
-    TEA_RETURN_IF(ensure_side_stream(c));
   }
   c->fcg_sweeps = sweeps;
   return TEA_HIP_OK;
@@ -1743,7 +1800,6 @@ int tea_hip_fcg_attach(tea_hip_chunk* c, const float* params, size_t count,
   if (c->fcg_levels == 2) {
     const size_t n1 = (size_t)c->fcg_lv[1].hc * c->fcg_lv[1].wc;
     if (hipMalloc(&c->fcg_xsum, n1 * sizeof(double)) != hipSuccess) return fail();
-    TEA_RETURN_IF(ensure_side_stream(c));
   }
   TEA_RETURN_IF(ensure_net_lds(c->device));
   return TEA_HIP_OK;

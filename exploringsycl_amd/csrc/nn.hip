@@ -77,10 +77,10 @@ constexpr int nsteps() {
 // per hidden layer at 64 x 32 x 32); the weights a wave holds in registers
 // serve its further tiles.
 template <int CIN, int MODE>
-__global__ __launch_bounds__(256) void conv_mfma_kernel(
+__device__ inline void conv_mfma_tiles(
     const bf16* __restrict__ in, const bf16* __restrict__ wt,
     const float* __restrict__ bias, const bf16* __restrict__ mask,
-    bf16* __restrict__ out, int H, int W, int B) {
+    bf16* __restrict__ out, int H, int W, int B, int block, int blocks) {
   constexpr int NS = nsteps<CIN>();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int hf = lane >> 5, col = lane & 31;
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void conv_mfma_kernel(
   const int per_row = W / 32;
   const int tiles = B * H * per_row;
   // Contiguous tiles per XCD (xcd_span): neighbouring rows share its L2.
-  for (int tile = xcd_span(blockIdx.x, gridDim.x) * 4 + wv; tile < tiles; tile += 4 * gridDim.x) {
+  for (int tile = xcd_span(block, blocks) * 4 + wv; tile < tiles; tile += 4 * blocks) {
     const int row = tile / per_row, b = row / H, y = row - b * H;
     const bf16* inb = in + (size_t)b * plane * CIN;
     const int xo = (tile - row * per_row) * 32 + col;
@@ -147,6 +147,14 @@ __global__ __launch_bounds__(256) void conv_mfma_kernel(
   }
 }
 
+template <int CIN, int MODE>
+__global__ __launch_bounds__(256) void conv_mfma_kernel(
+    const bf16* __restrict__ in, const bf16* __restrict__ wt,
+    const float* __restrict__ bias, const bf16* __restrict__ mask,
+    bf16* __restrict__ out, int H, int W, int B) {
+  conv_mfma_tiles<CIN, MODE>(in, wt, bias, mask, out, H, W, B, blockIdx.x, gridDim.x);
+}
+
 // Stages NROWS padded input rows (from row y0) of a 130-pixel segment
 // (from padded column x0) into LDS, CPC 16-byte chunks per pixel at a pitch
 // of kPitch chunks: every thread issues all its loads before its first LDS
@@ -175,19 +183,19 @@ __device__ inline void stage_rows(bf16x8* sm, const bf16* __restrict__ inb, int 
     if (threadIdx.x + 256 * k < kTotal) sm[slot[k]] = v[k];
 }
 
-// The (segment, row group, sample) of this block in a (W / 128, H / R, B)
-// grid, numbered so that each XCD takes one contiguous range of row groups:
+// The (segment, row group, sample) of block `block` of a (W / 128, H / R, B)
+// grid in linear order, numbered so that each XCD takes one contiguous range of row groups:
 // the hardware deals blocks round-robin to the 8 XCDs, which put the row
 // groups above and below a block on other XCDs, so the input rows two
 // blocks share were fetched into two L2s (1.27x the activations per hidden
 // layer at 512^2 with four rows per block).
-__device__ inline void xcd_tile(int& seg, int& grp, int& b) {
-  const int nb = gridDim.x * gridDim.y * gridDim.z;
-  const int L = xcd_span(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z), nb);
-  seg = L % gridDim.x;
-  const int rest = L / gridDim.x;
-  grp = rest % gridDim.y;
-  b = rest / gridDim.y;
+__device__ inline void xcd_tile(int block, int segs, int groups, int samples, int& seg, int& grp,
+                                int& b) {
+  const int L = xcd_span(block, segs * groups * samples);
+  seg = L % segs;
+  const int rest = L / segs;
+  grp = rest % groups;
+  b = rest / groups;
 }
 
 // Forward layer for rows of 128 pixels or more: a block takes a 128-pixel
@@ -196,18 +204,18 @@ __device__ inline void xcd_tile(int& seg, int& grp, int& b) {
 // chunks; a pixel's chunks are padded to kPitch so that the 16 lanes of a
 // 16-byte LDS read, which take consecutive pixels, hit distinct banks),
 // and each wave computes one 32-pixel tile from LDS.  Same arithmetic and
-// output as conv_mfma_kernel<CIN, 0>.  Grid (W / 128, H, B).
+// output as conv_mfma_kernel<CIN, 0>.  W / 128 x H x B blocks.
 template <int CIN>
-__global__ __launch_bounds__(256) void conv_fwd_lds_kernel(
+__device__ inline void conv_fwd_lds_block(
     const bf16* __restrict__ in, const bf16* __restrict__ wt,
-    const float* __restrict__ bias, bf16* __restrict__ out, int H, int W) {
+    const float* __restrict__ bias, bf16* __restrict__ out, int H, int W, int B, int block) {
   constexpr int NS = nsteps<CIN>();
   constexpr int CPC = CIN / 8;                   // 16-byte chunks per pixel
   constexpr int kPitch = CPC == 1 ? 1 : CPC + 1;  // padded chunks per pixel
   constexpr int kPx = 130;
   __shared__ bf16x8 sm[3][kPx * kPitch];
   int seg, y, b;
-  xcd_tile(seg, y, b);
+  xcd_tile(block, W / 128, H, B, seg, y, b);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int hf = lane >> 5, col = lane & 31;
   const int Wp = W + 2;
@@ -257,18 +265,18 @@ __global__ __launch_bounds__(256) void conv_fwd_lds_kernel(
 // weight fragments in registers across the R rows (instead of reloading
 // them per 32-pixel tile).  Each tile's MFMA sequence, bias and ReLU are
 // those of conv_fwd_lds_kernel, so the output is bitwise the same.
-// Grid (W / 128, H / R, B).
+// W / 128 x H / R x B blocks.
 template <int CIN, int R>
-__global__ __launch_bounds__(256) void conv_fwd_rows_kernel(
+__device__ inline void conv_fwd_rows_block(
     const bf16* __restrict__ in, const bf16* __restrict__ wt,
-    const float* __restrict__ bias, bf16* __restrict__ out, int H, int W) {
+    const float* __restrict__ bias, bf16* __restrict__ out, int H, int W, int B, int block) {
   constexpr int NS = nsteps<CIN>();
   constexpr int CPC = CIN / 8;
   constexpr int kPitch = CPC == 1 ? 1 : CPC + 1;
   constexpr int kPx = 130;
   __shared__ bf16x8 sm[R + 2][kPx * kPitch];
   int seg, grp, b;
-  xcd_tile(seg, grp, b);
+  xcd_tile(block, W / 128, H / R, B, seg, grp, b);
   const int y0 = grp * R;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int hf = lane >> 5, col = lane & 31;
@@ -314,6 +322,47 @@ __global__ __launch_bounds__(256) void conv_fwd_rows_kernel(
     const size_t pix = (size_t)b * plane + (size_t)(y0 + r + 1) * Wp + (x0 + xl + 1);
     store_out_row(out + pix * kC, acc, bco, hf);
   }
+}
+
+// The forward kernel R selects: 0 a tile per wave (conv_mfma_tiles), 1 a row
+// per block, 2 or 4 rows per block.
+template <int CIN, int R>
+__device__ inline void conv_fwd_block(const bf16* in, const bf16* wt, const float* bias, bf16* out,
+                                      int H, int W, int B, int block, int blocks) {
+  if (R == 0)
+    conv_mfma_tiles<CIN, 0>(in, wt, bias, nullptr, out, H, W, B, block, blocks);
+  else if (R == 1)
+    conv_fwd_lds_block<CIN>(in, wt, bias, out, H, W, B, block);
+  else
+    conv_fwd_rows_block<CIN, R ? R : 1>(in, wt, bias, out, H, W, B, block);
+}
+
+template <int CIN, int R>
+__global__ __launch_bounds__(256) void conv_fwd_kernel(
+    const bf16* __restrict__ in, const bf16* __restrict__ wt,
+    const float* __restrict__ bias, bf16* __restrict__ out, int H, int W, int B) {
+  conv_fwd_block<CIN, R>(in, wt, bias, out, H, W, B, blockIdx.x, gridDim.x);
+}
+
+// One hidden layer of two networks of one sample each (two levels of the
+// learned preconditioner), the first nb0 blocks the first network's by R and
+// the others the second's, a tile per wave: the second level's 32 blocks ran
+// on a stream of their own before, whose fork and join cost more (about 17 us
+// per application at 4096^2) than its five short launches.
+struct ConvArgs {
+  const bf16* in;
+  const bf16* wt;
+  const float* bias;
+  bf16* out;
+  int H, W;
+};
+template <int R>
+__global__ __launch_bounds__(256) void conv_fwd_pair_kernel(ConvArgs a, ConvArgs b, int nb0) {
+  if ((int)blockIdx.x < nb0)
+    conv_fwd_block<kC, R>(a.in, a.wt, a.bias, a.out, a.H, a.W, 1, blockIdx.x, nb0);
+  else
+    conv_mfma_tiles<kC, 0>(b.in, b.wt, b.bias, nullptr, b.out, b.H, b.W, 1, blockIdx.x - nb0,
+                           gridDim.x - nb0);
 }
 
 // ---- output layer (32 -> 1), FP32 on the vector units ------------------------
@@ -725,6 +774,33 @@ dim3 conv_grid(const tea_nn* n, int batch) {
 }
 unsigned flat_blocks(long count) { return (unsigned)((count + 255) / 256); }
 
+// The forward kernel for a batch: several rows per block only while the grid
+// keeps at least 512 blocks (on small grids the one-row kernel's parallelism
+// matters more than the saved weight and row loads), a tile per wave where
+// rows are not whole 128-pixel segments.
+int fwd_variant(const tea_nn* n, int batch) {
+  const int H = n->H, W = n->W, R = n->fwd_rows;
+  if (W % 128 != 0) return 0;
+  if ((R == 2 || R == 4) && H % R == 0 && (long)(W / 128) * (H / R) * batch >= 512) return R;
+  return 1;
+}
+unsigned fwd_blocks(const tea_nn* n, int batch, int variant) {
+  return variant == 0 ? conv_grid(n, batch).x
+                      : (unsigned)((n->W / 128) * (n->H / variant) * batch);
+}
+
+template <int CIN>
+void launch_fwd(tea_nn* n, int batch, hipStream_t st, const bf16* in, const bf16* wt,
+                const float* bias, bf16* out) {
+  const int v = fwd_variant(n, batch);
+  const auto kernel = v == 0   ? conv_fwd_kernel<CIN, 0>
+                      : v == 1 ? conv_fwd_kernel<CIN, 1>
+                      : v == 2 ? conv_fwd_kernel<CIN, 2>
+                               : conv_fwd_kernel<CIN, 4>;
+  hipLaunchKernelGGL(kernel, dim3(fwd_blocks(n, batch, v)), dim3(256), 0, st, in, wt, bias, out,
+                     n->H, n->W, batch);
+}
+
 // Forward pass over `batch` samples whose packed input is in n->in0, on
 // stream `st` (the network's own, or a solver's); without the output layer
 // unless with_output (its caller then runs it on the last activations); from
@@ -733,47 +809,10 @@ unsigned flat_blocks(long count) { return (unsigned)((count + 255) / 256); }
 int forward_on(tea_nn* n, int batch, hipStream_t st, bool with_output = true,
                int first = 0) {
   const int H = n->H, W = n->W;
-  // Several rows per block only while the grid keeps at least 512 blocks:
-  // on small grids the one-row kernel's parallelism matters more than the
-  // saved weight and row loads.
-  const int R = n->fwd_rows;
-  if (W % 128 == 0 && (R == 2 || R == 4) && H % R == 0 &&
-      (long)(W / 128) * (H / R) * batch >= 512) {
-    const dim3 grid(W / 128, H / R, batch);
-    if (first > 0)
-      ;
-    else if (R == 4)
-      hipLaunchKernelGGL((conv_fwd_rows_kernel<kC0, 4>), grid, dim3(256), 0, st, n->in0,
-                         n->wf1, n->bias, n->act[0], H, W);
-    else
-      hipLaunchKernelGGL((conv_fwd_rows_kernel<kC0, 2>), grid, dim3(256), 0, st, n->in0,
-                         n->wf1, n->bias, n->act[0], H, W);
-    for (int l = first > 1 ? first : 1; l < 5; ++l) {
-      const bf16* w = n->wfh + (size_t)(l - 1) * kWh;
-      if (R == 4)
-        hipLaunchKernelGGL((conv_fwd_rows_kernel<kC, 4>), grid, dim3(256), 0, st,
-                           n->act[l - 1], w, n->bias + l * kC, n->act[l], H, W);
-      else
-        hipLaunchKernelGGL((conv_fwd_rows_kernel<kC, 2>), grid, dim3(256), 0, st,
-                           n->act[l - 1], w, n->bias + l * kC, n->act[l], H, W);
-    }
-  } else if (W % 128 == 0) {
-    const dim3 grid(W / 128, H, batch);
-    if (first == 0)
-      hipLaunchKernelGGL((conv_fwd_lds_kernel<kC0>), grid, dim3(256), 0, st, n->in0, n->wf1,
-                         n->bias, n->act[0], H, W);
-    for (int l = first > 1 ? first : 1; l < 5; ++l)
-      hipLaunchKernelGGL((conv_fwd_lds_kernel<kC>), grid, dim3(256), 0, st, n->act[l - 1],
-                         n->wfh + (size_t)(l - 1) * kWh, n->bias + l * kC, n->act[l], H, W);
-  } else {
-    if (first == 0)
-      hipLaunchKernelGGL((conv_mfma_kernel<kC0, 0>), conv_grid(n, batch), dim3(256), 0,
-                         st, n->in0, n->wf1, n->bias, nullptr, n->act[0], H, W, batch);
-    for (int l = first > 1 ? first : 1; l < 5; ++l)
-      hipLaunchKernelGGL((conv_mfma_kernel<kC, 0>), conv_grid(n, batch), dim3(256), 0,
-                         st, n->act[l - 1], n->wfh + (size_t)(l - 1) * kWh,
-                         n->bias + l * kC, nullptr, n->act[l], H, W, batch);
-  }
+  if (first == 0) launch_fwd<kC0>(n, batch, st, n->in0, n->wf1, n->bias, n->act[0]);
+  for (int l = first > 1 ? first : 1; l < 5; ++l)
+    launch_fwd<kC>(n, batch, st, n->act[l - 1], n->wfh + (size_t)(l - 1) * kWh, n->bias + l * kC,
+                   n->act[l]);
   if (with_output)
     hipLaunchKernelGGL(out_layer_kernel, dim3(flat_blocks((long)batch * H * W)), dim3(256),
                        0, st, n->act[4], n->w6, n->bias, n->out, batch, H, W);
@@ -912,9 +951,25 @@ __global__ __launch_bounds__(256) void gather_kernel(const float* __restrict__ d
 namespace tea {
 namespace nn {
 // Used by the flexible-CG preconditioner (fcg.hip).
-int forward_on_stream(tea_nn* n, hipStream_t st) { return forward_on(n, 1, st); }
 int forward_hidden_on_stream(tea_nn* n, hipStream_t st, int first) {
   return forward_on(n, 1, st, false, first);
+}
+int forward_hidden_pair(tea_nn* n0, tea_nn* n1, hipStream_t st, int first) {
+  const int v = fwd_variant(n0, 1);
+  const unsigned nb0 = fwd_blocks(n0, 1, v), nb1 = conv_grid(n1, 1).x;
+  const auto kernel = v == 0   ? conv_fwd_pair_kernel<0>
+                      : v == 1 ? conv_fwd_pair_kernel<1>
+                      : v == 2 ? conv_fwd_pair_kernel<2>
+                               : conv_fwd_pair_kernel<4>;
+  auto args = [](tea_nn* n, int l) {
+    return ConvArgs{n->act[l - 1], n->wfh + (size_t)(l - 1) * kWh, n->bias + l * kC, n->act[l],
+                    n->H, n->W};
+  };
+  for (int l = first; l < 5; ++l)
+    hipLaunchKernelGGL(kernel, dim3(nb0 + nb1), dim3(256), 0, st, args(n0, l), args(n1, l),
+                       (int)nb0);
+  TEA_HIP_TRY(hipGetLastError());
+  return TEA_HIP_OK;
 }
 const bf16* last_hidden(tea_nn* n) { return n->act[4]; }
 bf16* hidden(tea_nn* n, int l) { return n->act[l]; }

@@ -768,12 +768,14 @@ struct PackedWeights {
   const float* bias;
 };
 PackedWeights packed_weights(const tea_nn* n);
-int forward_on_stream(tea_nn* n, hipStream_t st);
 // The hidden layers alone, from layer `first` on (0-based; the caller has
 // written layer first - 1's activations at hidden(n, first - 1)); the last
 // layer's activations (padded (H + 2) x (W + 2) pixels of 32 BF16 channels,
 // zero ring) at last_hidden.
 int forward_hidden_on_stream(tea_nn* n, hipStream_t st, int first = 0);
+// The same for two networks (one sample each), their layers in one launch;
+// first >= 1.
+int forward_hidden_pair(tea_nn* n0, tea_nn* n1, hipStream_t st, int first);
 const bf16* last_hidden(tea_nn* n);
 bf16* hidden(tea_nn* n, int l);
 bf16* input_tensor(tea_nn* n);
@@ -899,11 +901,6 @@ struct tea_hip_chunk {
   int fcg_sweeps = 0;
   double* fcg_xsum = nullptr;
   float* fcg_g = nullptr;
-  // With two levels, the second level's chain runs on a side stream
-  // (default priority) between a fork after the first level's restriction
-  // and a join before the joint factors.
-  hipStream_t fcg_side = nullptr;
-  hipEvent_t fcg_fork = nullptr, fcg_join = nullptr;
 
   // Run-ahead of the fused CG iteration (cg.hip): the device forms alpha and
   // beta from its own partials and runs the next pass of the iteration into
