@@ -722,14 +722,9 @@ int sync_p_alt(tea_hip_chunk* c) {
 constexpr int kRaNone = 0, kRaR = 1, kRaWR = 2;
 constexpr int kRaW = 0, kRaRStep = 1;  // slot kinds
 
-int ra_len(const tea_hip_chunk* c) {
-  return c->nspan == 1 ? 1 : (c->nspan + kWave - 1) / kWave;
-}
-
 bool ra_possible(const tea_hip_chunk* c) {
   return c->ra_enabled && c->fused && c->poll && c->pairs && c->geo.x % 2 == 0 && c->ra_rro_known &&
-         c->ra_fail < 3 && use_pair_blocks(c, 1) && use_pair_blocks(c, 2) &&
-         ra_len(c) <= kWave * kWave;
+         c->ra_fail < 3 && use_pair_blocks(c, 1) && use_pair_blocks(c, 2);
 }
 
 double* ra_host_slot(tea_hip_chunk* c, int set, int kind) {
@@ -744,21 +739,18 @@ int ensure_ra(tea_hip_chunk* c) {
   if (c->ra_host) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(double));
   for (double** b : {&c->r_alt, &c->u_alt, &c->w_alt}) {
+    if (*b) continue;
     if (hipMalloc(b, bytes) != hipSuccess) {
       *b = nullptr;
       set_error("hipMalloc of a run-ahead buffer failed");
       return TEA_HIP_ENOMEM;
     }
   }
-  // [0..2] scalars, then the finisher's partials, then the blocks-done count.
-  const size_t nd = 3 + (size_t)ra_len(c);
-  if (hipMalloc(&c->ra_dev, (nd + 1) * sizeof(double)) != hipSuccess) {
+  if (hipMalloc(&c->ra_dev, 3 * sizeof(double)) != hipSuccess) {
     c->ra_dev = nullptr;
     set_error("hipMalloc of the run-ahead scalars failed");
     return TEA_HIP_ENOMEM;
   }
-  c->ra_count = reinterpret_cast<unsigned*>(c->ra_dev + nd);
-  TEA_HIP_TRY(hipMemsetAsync(c->ra_count, 0, sizeof(unsigned), c->stream));
   double* host = nullptr;
   if (hipHostMalloc(&host, 8 * sizeof(double),
                     hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
@@ -797,9 +789,8 @@ int ra_finish(tea_hip_chunk* c, int set, int kind, double rro, bool from_dev, Ra
     return TEA_HIP_OK;
   }
   sc->dev = c->ra_dev + (kind == kRaW ? 0 : 1);
-  const RaTail tail{rro, from_dev ? 1 : 0, kind == kRaW ? 0 : 1, c->ra_dev,
-                    ra_dev_slot(c, set, kind), c->ra_count};
-  return launch_span_finish_ra(c, c->ra_dev + 3, tail);
+  const RaTail tail{rro, from_dev ? 1 : 0, kind == kRaW ? 0 : 1, c->ra_dev};
+  return launch_span_finish_ra(c, 1, ra_dev_slot(c, set, kind), tail);
 }
 
 // The r-step behind a w-step that was just queued: alpha from its p.w (and
@@ -851,6 +842,8 @@ int ra_discard(tea_hip_chunk* c) {
 }
 
 int apply_pending(tea_hip_chunk* c) {
+  if (c->mra) TEA_RETURN_IF(mra_discard(c));
+  c->mra_synced = false;
   TEA_RETURN_IF(apply_cg_pending(c));
   return flush_held(c);
 }

@@ -72,7 +72,8 @@ int resolve_timing(tea_hip_chunk* c) {
 
 int sync_chunk(tea_hip_chunk* c) {
   TEA_HIP_TRY(hipStreamSynchronize(c->stream));
-  c->poll_len = 0;
+  c->poll_nr = 0;
+  c->ra_dirty = false;
   return resolve_timing(c);
 }
 
@@ -142,11 +143,15 @@ static int wait_values(tea_hip_chunk* c, const volatile uint64_t* v, size_t stri
 // the next scalar and launch the next kernel before the stream reports
 // completion.
 static int wait_partials(tea_hip_chunk* c) {
-  if (c->poll_len == 0) return sync_chunk(c);
-  const int len = c->poll_len, nr = c->poll_nr;
-  c->poll_len = 0;
-  return wait_values(c, reinterpret_cast<const volatile uint64_t*>(c->host_partials),
-                     (size_t)c->nspan, nr, len);
+  if (c->poll_nr == 0) return sync_chunk(c);
+  const int nr = c->poll_nr;
+  c->poll_nr = 0;
+  TEA_RETURN_IF(wait_values(c, reinterpret_cast<const volatile uint64_t*>(c->host_partials),
+                            (size_t)c->nspan, nr, 1));
+  // Every pass queued before the one waited for has ended, a dropped
+  // run-ahead too.
+  c->ra_dirty = false;
+  return TEA_HIP_OK;
 }
 
 void arm_host_values(double* host, int count) {
@@ -183,126 +188,156 @@ static double host_tree_passes(double* v, size_t len) {
   return v[0];
 }
 
-// The next tree pass over the spans from the block sums (zero past the grid,
-// as the reference pads its level-2 input with zeros).  A 512-thread block
-// covers 512 blocks = 64 spans, one group of that pass: wave w runs the tree
-// over 64 block sums (8 spans), then the eight wave sums are combined.  With
-// a single span there is no further pass and its partial is the sum (the
-// other spans' zeros add nothing).
-constexpr int kFinishBlock = kGroupBlocks;  // 512 threads = 64 spans
-
-// The host's final tree passes (host_tree_passes) over len <= 64^2 values
-// in one wave; buf is LDS of 64 doubles.  Lane 0 returns the sum.
-__device__ inline double wave_tree_passes(const double* part, int len, double* buf) {
-  const int lane = threadIdx.x & (kWave - 1);
-  if (len == 1) return part[0];
-  const int groups = (len + kWave - 1) / kWave;
-  for (int g = 0; g < groups; ++g) {
-    const int i = g * kWave + lane;
-    const double v = wave_tree(i < len ? part[i] : 0.0);
-    if (lane == 0) buf[g] = v;
+// A sum's last pass, the run-ahead's scalar and where they go (RaTail, or the
+// sums alone), by one lane.
+template <int NR, bool TAIL>
+__device__ inline void finish_out(const double (&sum)[NR], double* out, int out_stride,
+                                  const RaTail& tail) {
+  if (!TAIL) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q) out[(size_t)q * out_stride] = sum[q];
+    return;
   }
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  if (groups == 1) return buf[0];
-  return wave_tree(lane < groups ? buf[lane] : 0.0);
+  double x;
+  if (NR == 1) {
+    const double r0 = tail.from_dev ? tail.ra[2] : tail.rro;
+    x = tail.mode == 0 ? r0 / sum[0] : sum[0] / r0;
+    if (tail.mode == 1) tail.ra[2] = sum[0];
+  } else {
+    x = tail.mode == 0 ? sum[NR - 1] / sum[0] : -sum[NR - 1] / tail.ra[2];
+    if (tail.mode == 0) tail.ra[2] = sum[0];
+    out[1] = sum[NR - 1];
+  }
+  tail.ra[tail.mode] = x;
+  out[0] = sum[0];
+  out[NR] = x;
 }
 
-template <int NR, bool TAIL = false>
-__global__ __launch_bounds__(kFinishBlock) void span_finish_kernel(
-    const double* __restrict__ sub, int nblk, double* partials, int nspan,
-    RaTail tail = RaTail{}) {
-  __shared__ double lds[kWave];
-  __shared__ double ws[NR][kFinishBlock / kWave];
-  const int t = threadIdx.x;
-  const int lane = t & (kWave - 1);
-  // Every sum's loads first (a round per sum was waited for sum by sum).
-  double w[NR];
+// One group of 512 block sums (64 spans): lane l takes span l's 8 blocks.
+__device__ inline double group_sum(const double* __restrict__ p) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const double2 a = ld2(p, kSubPerSpan * lane), b = ld2(p, kSubPerSpan * lane + 2);
+  const double2 c = ld2(p, kSubPerSpan * lane + 4), d = ld2(p, kSubPerSpan * lane + 6);
+  return wave_tree_dpp(((a.x + a.y) + (b.x + b.y)) + ((c.x + c.y) + (d.x + d.y)));
+}
+
+// The rest of the tree over the block sums of at most 16 groups, a wave per
+// group in one block, wave 0 the last pass: 3.4 us at 1024^2, all latency,
+// against 4.8 us for a block per group with a last-block pass.
+constexpr int kFinishWaves = 16;
+template <int NR, bool TAIL>
+__global__ __launch_bounds__(kFinishWaves * kWave) void span_finish_kernel(
+    const double* __restrict__ sub, int nblk, double* out, int out_stride, RaTail tail) {
+  __shared__ double gs[NR][kFinishWaves];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const size_t stride = sub_stride(nblk);
+  double t[NR];
 #pragma unroll
   for (int q = 0; q < NR; ++q)
-    w[q] = sub[(size_t)q * sub_stride(nblk) + blockIdx.x * kFinishBlock + t];
+    t[q] = wv * kGroupBlocks < nblk ? group_sum(sub + q * stride + wv * kGroupBlocks) : 0.0;
 #pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const double v = wave_tree_dpp(w[q]);
-    if (lane == 0) ws[q][t / kWave] = v;
-  }
+  for (int q = 0; q < NR; ++q)
+    if (lane == 0) gs[q][wv] = t[q];
   __syncthreads();
-  if (t >= kWave) return;
+  if (wv != 0) return;
+  double sum[NR];
 #pragma unroll
-  for (int q = 0; q < NR; ++q) {
-    const double v = ((ws[q][0] + ws[q][1]) + (ws[q][2] + ws[q][3])) +
-                     ((ws[q][4] + ws[q][5]) + (ws[q][6] + ws[q][7]));
-    if (lane == 0) partials[(size_t)q * nspan + blockIdx.x] = v;
-  }
-  if (!TAIL) return;
-  // The last block to store its partial (device-scope release before the
-  // count, acquire after it) sums them all.
-  unsigned prev = 0;
-  if (lane == 0) {
-    __threadfence();
-    prev = atomicAdd(tail.count, 1u);
-  }
-  prev = __shfl(prev, 0);
-  if (prev != gridDim.x - 1) return;
-  __threadfence();
-  const int len = nspan == 1 ? 1 : (int)gridDim.x;
-  const double sum = wave_tree_passes(partials, len, lds);
-  if (lane != 0) return;
-  const double r0 = tail.from_dev ? tail.ra[2] : tail.rro;
-  double q;
-  if (tail.mode == 0) {
-    q = r0 / sum;
-    tail.ra[0] = q;
-  } else {
-    q = sum / r0;
-    tail.ra[1] = q;
-    tail.ra[2] = sum;
-  }
-  tail.out[0] = sum;
-  tail.out[1] = q;
-  *tail.count = 0u;
+  for (int q = 0; q < NR; ++q) sum[q] = wave_tree_dpp(lane < kFinishWaves ? gs[q][lane] : 0.0);
+  if (lane == 0) finish_out<NR, TAIL>(sum, out, out_stride, tail);
 }
 
-int launch_span_finish(tea_hip_chunk* c, int nr, int* len, int slot,
-                       bool poll) {
+// More groups (grids above 8192 blocks): a wave and block per group; the last
+// one to count itself done runs the remaining passes over the group sums in
+// part.  Those are stored and read at device scope (past the XCDs' own L2s),
+// and the count follows its sum's store, so no fence is needed: a release
+// fence writes back a whole L2.
+__device__ inline void st_agent(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline double ld_agent(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int NR, bool TAIL>
+__global__ __launch_bounds__(kWave) void span_finish_groups_kernel(
+    const double* __restrict__ sub, int nblk, double* part, unsigned* count, double* out,
+    int out_stride, RaTail tail) {
+  const int lane = threadIdx.x, g = blockIdx.x, ngrp = gridDim.x;
+  const size_t stride = sub_stride(nblk);
+  double t[NR];
+#pragma unroll
+  for (int q = 0; q < NR; ++q) t[q] = group_sum(sub + q * stride + (size_t)g * kGroupBlocks);
+  unsigned prev = 0;
+  if (lane == 0) {
+#pragma unroll
+    for (int q = 0; q < NR; ++q) st_agent(part + (size_t)q * ngrp + g, t[q]);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the sums are out before the count
+    prev = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  prev = __builtin_amdgcn_readfirstlane(prev);
+  if (prev != gridDim.x - 1) return;
+  // At most 8192 groups (a chunk has fewer than 2^31 cells): up to 128 sums
+  // of 64 groups, held one per lane in w[0] and w[1].
+  double sum[NR];
+#pragma unroll
+  for (int q = 0; q < NR; ++q) {
+    double w[2] = {0.0, 0.0};
+    for (int i = 0; i * kWave < ngrp; ++i) {
+      const int k = i * kWave + lane;
+      const double u = wave_tree_dpp(k < ngrp ? ld_agent(part + (size_t)q * ngrp + k) : 0.0);
+      if (lane == (i & (kWave - 1))) {
+        if (i < kWave)
+          w[0] = u;
+        else
+          w[1] = u;
+      }
+    }
+    sum[q] = wave_tree_dpp(w[0]);
+    if (ngrp > kWave * kWave) sum[q] = sum[q] + wave_tree_dpp(w[1]);
+  }
+  if (lane != 0) return;
+  __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  finish_out<NR, TAIL>(sum, out, out_stride, tail);
+}
+
+template <int NR, bool TAIL>
+static void launch_finish(tea_hip_chunk* c, const double* sub, double* out, int out_stride,
+                          const RaTail& tail) {
+  const int ngrp = sub_stride(c->nblk) / kGroupBlocks;
+  if (ngrp <= kFinishWaves)
+    hipLaunchKernelGGL((span_finish_kernel<NR, TAIL>), dim3(1), dim3(kFinishWaves * kWave), 0,
+                       c->stream, sub, c->nblk, out, out_stride, tail);
+  else
+    hipLaunchKernelGGL((span_finish_groups_kernel<NR, TAIL>), dim3(ngrp), dim3(kWave), 0,
+                       c->stream, sub,
+                       c->nblk, c->grp_sum, c->done_count, out, out_stride, tail);
+}
+
+int launch_span_finish(tea_hip_chunk* c, int nr, int* len, int slot, bool poll,
+                       const double* sub) {
   TEA_CHECK_ARG(nr >= 1 && nr <= kSubMaxNr, "span_finish: bad reduction count");
   TEA_CHECK_ARG(slot >= 0 && slot + nr <= 4, "span_finish: bad partials slot");
-  const dim3 grid((unsigned)((c->nspan + kWave - 1) / kWave));
-  double* dst = c->partials + (size_t)slot * c->nspan;
-  c->poll_len = 0;
+  if (!sub) sub = c->sub;
+  *len = 1;
+  c->poll_nr = 0;
   if (poll && c->poll && slot == 0) {
-    const int n = c->nspan == 1 ? 1 : (c->nspan + kWave - 1) / kWave;
-    uint64_t* v = reinterpret_cast<uint64_t*>(c->host_partials);
-    for (int q = 0; q < nr; ++q)
-      for (int i = 0; i < n; ++i) v[(size_t)q * c->nspan + i] = kPollSentinel;
+    for (int q = 0; q < nr; ++q) arm_host_values(c->host_partials + (size_t)q * c->nspan, 1);
     c->poll_nr = nr;
-    c->poll_len = n;
   }
-  {
-    Timed t(c, K_SPAN_FINISH);
-    if (nr == 1)
-      hipLaunchKernelGGL(span_finish_kernel<1>, grid, dim3(kFinishBlock), 0,
-                         c->stream, c->sub, c->nblk, dst, c->nspan);
-    else if (nr == 2)
-      hipLaunchKernelGGL(span_finish_kernel<2>, grid, dim3(kFinishBlock), 0,
-                         c->stream, c->sub, c->nblk, dst, c->nspan);
-    else
-      hipLaunchKernelGGL(span_finish_kernel<3>, grid, dim3(kFinishBlock), 0,
-                         c->stream, c->sub, c->nblk, dst, c->nspan);
-  }
+  Timed t(c, K_SPAN_FINISH);
+  const auto launch = nr == 1   ? launch_finish<1, false>
+                      : nr == 2 ? launch_finish<2, false>
+                                : launch_finish<3, false>;
+  launch(c, sub, c->partials + (size_t)slot * c->nspan, c->nspan, RaTail{});
   TEA_HIP_TRY(hipGetLastError());
-  *len = c->nspan == 1 ? 1 : (c->nspan + kWave - 1) / kWave;
   return TEA_HIP_OK;
 }
 
-int launch_span_finish_ra(tea_hip_chunk* c, double* dst, const RaTail& tail) {
-  const int grid = (c->nspan + kWave - 1) / kWave;
-  TEA_CHECK_ARG(grid <= kWave * kWave, "span_finish: too many partials for the run-ahead");
-  {
-    Timed t(c, K_CG_RA_FINISH);
-    hipLaunchKernelGGL((span_finish_kernel<1, true>), dim3((unsigned)grid), dim3(kFinishBlock),
-                       0, c->stream, c->sub, c->nblk, dst, c->nspan, tail);
-  }
+int launch_span_finish_ra(tea_hip_chunk* c, int nr, double* out, const RaTail& tail) {
+  TEA_CHECK_ARG(nr == 1 || nr == 2, "span_finish: bad reduction count");
+  Timed t(c, nr == 1 ? K_CG_RA_FINISH : K_SPAN_FINISH);
+  const auto launch = nr == 1 ? launch_finish<1, true> : launch_finish<2, true>;
+  launch(c, c->sub, out, 1, tail);
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
 }
@@ -436,14 +471,19 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
     set_error("hipMalloc of the second p buffer failed");
     return fail(TEA_HIP_ENOMEM);
   }
-  const size_t sbytes = (size_t)kSubMaxNr * sub_stride(c->nblk) * sizeof(double);
-  if (hipMalloc(&c->sub, 2 * sbytes) != hipSuccess) {
+  // One allocation, zero: two sets of block sums, the group sums and the
+  // finisher's counter.
+  const size_t ns = (size_t)kSubMaxNr * sub_stride(c->nblk), ng = ns / kGroupBlocks;
+  const size_t rbytes = (2 * ns + ng + 1) * sizeof(double);
+  if (hipMalloc(&c->sub, rbytes) != hipSuccess) {
     c->sub = nullptr;
-    set_error("hipMalloc of the block sums failed");
+    set_error("hipMalloc of the reduction workspace failed");
     return fail(TEA_HIP_ENOMEM);
   }
-  c->sub2 = c->sub + sbytes / sizeof(double);
-  if (hipMemsetAsync(c->sub, 0, 2 * sbytes, c->stream) != hipSuccess) {
+  c->sub2 = c->sub + ns;
+  c->grp_sum = c->sub2 + ns;
+  c->done_count = reinterpret_cast<unsigned*>(c->grp_sum + ng);
+  if (hipMemsetAsync(c->sub, 0, rbytes, c->stream) != hipSuccess) {
     set_error("hipMemsetAsync failed");
     return fail(TEA_HIP_EHIP);
   }
@@ -486,9 +526,13 @@ int tea_hip_chunk_destroy(tea_hip_chunk* c) {
   if (c->spare) (void)hipFree(c->spare);
   if (c->spare2) (void)hipFree(c->spare2);
   if (c->sub) (void)hipFree(c->sub);
-  for (float* b : {c->mp_p[0], c->mp_p[1], c->mp_p[2], c->mp_r, c->mp_w, c->mp_kx, c->mp_ky,
-                   c->fcg_z})
+  for (float* b : c->mp_p)
     if (b) (void)hipFree(b);
+  for (float* b : {c->mp_r, c->mp_w, c->mp_kx, c->mp_ky, c->fcg_z, c->mp_r_alt, c->mp_w_alt,
+                   c->fcg_z_alt})
+    if (b) (void)hipFree(b);
+  if (c->mra_dev) (void)hipFree(c->mra_dev);
+  if (c->mra_host) (void)hipHostFree(c->mra_host);
   if (c->fcg_xsum) (void)hipFree(c->fcg_xsum);
   if (c->fcg_g) (void)hipFree(c->fcg_g);
   for (FcgLevel& L : c->fcg_lv) {

@@ -1408,12 +1408,14 @@ __global__ __launch_bounds__(kGammaThreads) void joint_gamma_kernel(
 int ensure_fcg_buffers(tea_hip_chunk* c) {
   if (c->fcg_z) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
-  if (hipMalloc(&c->fcg_z, bytes) != hipSuccess) {
+  if (hipMalloc(&c->fcg_z_alt, bytes) != hipSuccess ||
+      hipMalloc(&c->fcg_z, bytes) != hipSuccess) {
     c->fcg_z = nullptr;
     set_error("hipMalloc of the FCG z buffer failed");
     return TEA_HIP_ENOMEM;
   }
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_z, 0, bytes, c->stream));
+  TEA_HIP_TRY(hipMemsetAsync(c->fcg_z_alt, 0, bytes, c->stream));
   return TEA_HIP_OK;
 }
 
@@ -1533,7 +1535,7 @@ static int launch_sweeps_levels(tea_hip_chunk* c) {
 // levels in one pass (with the RMS partials the network's input scale
 // needs), the levels' coarse solves (both in each launch), and the factors
 // into c->fcg_g.
-static int launch_coarse(tea_hip_chunk* c) {
+static int launch_coarse(tea_hip_chunk* c, const float* r) {
   const int nl = c->fcg_levels;
   const bool net = c->fcg_sweeps == 0;
   FcgLevel& L0 = c->fcg_lv[0];
@@ -1543,7 +1545,7 @@ static int launch_coarse(tea_hip_chunk* c) {
     const dim3 grid((unsigned)(L0.wc + 31) / 32, (unsigned)(L0.hc + 3) / 4);
     const bool pairs = ((c->geo.x | c->geo.h) & 1) == 0;
     hipLaunchKernelGGL(pairs ? restrict8_kernel<true> : restrict8_kernel<false>, grid,
-                       dim3(256), 0, c->stream, c->geo, L0.hc, L0.wc, c->mp_r, L0.rbar,
+                       dim3(256), 0, c->stream, c->geo, L0.hc, L0.wc, r, L0.rbar,
                        nl == 2 ? L1.rbar : nullptr, net ? L0.dis : nullptr,
                        net && nl == 2 ? L1.dis : nullptr, net ? L0.rms : nullptr,
                        net && nl == 2 ? L1.rms : nullptr);
@@ -1576,64 +1578,44 @@ static bool precondition_quads(const tea_hip_chunk* c, int use_net) {
   return quads;
 }
 
-// With sub_q >= 0 (four-cells-per-lane kernel only) the z.w subtree sums go
-// to array sub_q of c->sub and are left for the caller to finish.
-static int launch_precondition(tea_hip_chunk* c, int use_net, int slot, int* len,
-                               int sub_q = -1) {
+static CoarseTerm coarse_term(const tea_hip_chunk* c, int l, int nl) {
+  if (l >= nl) return CoarseTerm{nullptr, nullptr, 0, 0};
+  const FcgLevel& L = c->fcg_lv[l];
+  return CoarseTerm{L.y, c->fcg_g + l, log2_of(L.c), L.wc};
+}
+
+namespace tea {
+
+int launch_fcg_z(tea_hip_chunk* c, int use_net, const float* r, const float* w, float* z,
+                 double* sub) {
+  const int nl = use_net ? c->fcg_levels : 0;
+  if (nl > 0) TEA_RETURN_IF(launch_coarse(c, r));
+  Timed t(c, nl == 0 ? K_FCG_JACOBI : K_FCG_PROLONG);
+  const bool quads = precondition_quads(c, use_net);
+  const dim3 grid = quads ? quad_grid(c) : pair_grid(c), block(quads ? kQuadThreads : kBlock);
+  const auto kernel =
+      quads ? (nl == 0 ? fcg_z4_kernel<0> : nl == 1 ? fcg_z4_kernel<1> : fcg_z4_kernel<2>)
+            : (nl == 0 ? fcg_z1_kernel<0> : nl == 1 ? fcg_z1_kernel<1> : fcg_z1_kernel<2>);
+  hipLaunchKernelGGL(kernel, grid, block, 0, c->stream, c->geo, r, c->mp_kx, c->mp_ky, w,
+                     coarse_term(c, 0, nl), coarse_term(c, 1, nl), z,
+                     sub, c->nblk);
+  TEA_HIP_TRY(hipGetLastError());
+  return TEA_HIP_OK;
+}
+
+int launch_precondition(tea_hip_chunk* c, int use_net, int slot, int* len) {
+  if (use_pair_blocks(c, 2)) {
+    TEA_RETURN_IF(launch_fcg_z(c, use_net, c->mp_r, c->mp_w, c->fcg_z, c->sub));
+    return launch_span_finish(c, 1, len, slot);
+  }
   const Geo g = c->geo;
   const int sg = c->ngroup == 1 ? 1 : 0;
   const int nl = use_net ? c->fcg_levels : 0;
   double* partials = c->partials + (size_t)slot * c->nspan;
   *len = c->nspan;
-  if (nl > 0) TEA_RETURN_IF(launch_coarse(c));
-  const CoarseTerm none{nullptr, nullptr, 0, 0};
-  auto term = [&](int l) {
-    const FcgLevel& L = c->fcg_lv[l];
-    return CoarseTerm{L.y, c->fcg_g + l, log2_of(L.c), L.wc};
-  };
-  const CoarseTerm t0 = nl > 0 ? term(0) : none;
-  const CoarseTerm t1 = nl > 1 ? term(1) : none;
+  if (nl > 0) TEA_RETURN_IF(launch_coarse(c, c->mp_r));
+  const CoarseTerm t0 = coarse_term(c, 0, nl), t1 = coarse_term(c, 1, nl);
   const int kid = nl == 0 ? K_FCG_JACOBI : K_FCG_PROLONG;
-  if (precondition_quads(c, use_net)) {
-    double* sub = c->sub + (size_t)(sub_q > 0 ? sub_q : 0) * sub_stride(c->nblk);
-    {
-      Timed t(c, kid);
-      if (nl == 0)
-        hipLaunchKernelGGL((fcg_z4_kernel<0>), quad_grid(c), dim3(kQuadThreads), 0, c->stream, g,
-                           c->mp_r, c->mp_kx, c->mp_ky, c->mp_w, t0, t1, c->fcg_z, sub,
-                           c->nblk);
-      else if (nl == 1)
-        hipLaunchKernelGGL((fcg_z4_kernel<1>), quad_grid(c), dim3(kQuadThreads), 0, c->stream, g,
-                           c->mp_r, c->mp_kx, c->mp_ky, c->mp_w, t0, t1, c->fcg_z, sub,
-                           c->nblk);
-      else
-        hipLaunchKernelGGL((fcg_z4_kernel<2>), quad_grid(c), dim3(kQuadThreads), 0, c->stream, g,
-                           c->mp_r, c->mp_kx, c->mp_ky, c->mp_w, t0, t1, c->fcg_z, sub,
-                           c->nblk);
-    }
-    TEA_HIP_TRY(hipGetLastError());
-    if (sub_q >= 0) return TEA_HIP_OK;
-    return launch_span_finish(c, 1, len, slot);
-  }
-  if (use_pair_blocks(c, 2)) {
-    {
-      Timed t(c, kid);
-      if (nl == 0)
-        hipLaunchKernelGGL((fcg_z1_kernel<0>), pair_grid(c), dim3(kBlock), 0, c->stream, g,
-                           c->mp_r, c->mp_kx, c->mp_ky, c->mp_w, t0, t1, c->fcg_z, c->sub,
-                           c->nblk);
-      else if (nl == 1)
-        hipLaunchKernelGGL((fcg_z1_kernel<1>), pair_grid(c), dim3(kBlock), 0, c->stream, g,
-                           c->mp_r, c->mp_kx, c->mp_ky, c->mp_w, t0, t1, c->fcg_z, c->sub,
-                           c->nblk);
-      else
-        hipLaunchKernelGGL((fcg_z1_kernel<2>), pair_grid(c), dim3(kBlock), 0, c->stream, g,
-                           c->mp_r, c->mp_kx, c->mp_ky, c->mp_w, t0, t1, c->fcg_z, c->sub,
-                           c->nblk);
-    }
-    TEA_HIP_TRY(hipGetLastError());
-    return launch_span_finish(c, 1, len, slot);
-  }
   Timed t(c, kid);
   if (c->pairs) {
     if (nl == 0)
@@ -1664,6 +1646,8 @@ static int launch_precondition(tea_hip_chunk* c, int use_net, int slot, int* len
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
 }
+
+}  // namespace tea
 
 static void free_level(FcgLevel& L) {
   for (float* b : {L.feat, L.rbar, L.kc, L.dis, L.sig, L.y})
@@ -1843,6 +1827,8 @@ int tea_hip_fcg_precondition(tea_hip_chunk* c, int use_net, double* zw) {
   TEA_CHECK_ARG(!use_net || c->fcg_levels > 0, "no coarse correction attached");
   TEA_HIP_TRY(hipSetDevice(c->device));
   TEA_FLUSH_HELD_KEEP_U(c);
+  if (c->mra) TEA_RETURN_IF(mra_discard(c));
+  c->mra_coarse = use_net;
   int len;
   TEA_RETURN_IF(launch_precondition(c, use_net, 0, &len));
   return finish_reduction_n(c, 1, len, zw);
@@ -1856,24 +1842,7 @@ int tea_hip_fcg_calc_r_precondition(tea_hip_chunk* c, double alpha, int use_net,
   TEA_CHECK_ARG(!use_net || c->fcg_levels > 0, "no coarse correction attached");
   TEA_HIP_TRY(hipSetDevice(c->device));
   TEA_FLUSH_HELD_KEEP_U(c);
-  double out[2];
-  if (use_quad_blocks(c, 2) && precondition_quads(c, use_net)) {
-    // Both kernels leave their subtree sums in c->sub (r.r in array 0, z.w
-    // in array 1; nothing between them uses it) for one finisher launch.
-    int len;
-    TEA_RETURN_IF(launch_mp_r(c, alpha, &len, false, false));
-    TEA_RETURN_IF(launch_precondition(c, use_net, 0, &len, 1));
-    TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true));
-    TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
-  } else {
-    int lens[2] = {c->nspan, c->nspan};
-    TEA_RETURN_IF(launch_mp_r(c, alpha, &lens[0], false));
-    TEA_RETURN_IF(launch_precondition(c, use_net, 1, &lens[1]));
-    TEA_RETURN_IF(finish_reduction_lens(c, 2, lens, out));
-  }
-  *rr = out[0];
-  *zw = out[1];
-  return TEA_HIP_OK;
+  return mp_calc_r(c, true, alpha, use_net, rr, zw);
 }
 
 int tea_hip_fcg_calc_w(tea_hip_chunk* c, double alpha, int apply_u, double beta,
@@ -1885,40 +1854,7 @@ int tea_hip_fcg_calc_w(tea_hip_chunk* c, double alpha, int apply_u, double beta,
   TEA_FLUSH_HELD_KEEP_U(c);
   // p = z + beta p_old (the mixed-precision kernel with z in place of r),
   // w = A p, and the dots p.w and p.r.
-  MpArgs a{c->mp_p[c->mp_cur], c->mp_p[mp_next(c->mp_cur)], c->fcg_z,
-           c->field[TEA_FIELD_U], c->mp_w, c->mp_kx, c->mp_ky, c->mp_r,
-           alpha, beta, apply_u ? 1 : 0, 1};
-  int len = c->nspan;
-  if (use_pair_blocks(c, 1)) {
-    if (c->quads) {
-      TEA_RETURN_IF(launch_mp_w4(c, a, K_FCG_W));
-    } else {
-      if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
-      Timed t(c, K_FCG_W);
-      hipLaunchKernelGGL((mp_w1_kernel<true>), pair_grid(c), dim3(kBlock), 0,
-                         c->stream, c->geo, a, c->sub, c->nblk);
-    }
-    TEA_HIP_TRY(hipGetLastError());
-    TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true));
-  } else {
-    if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
-    Timed t(c, K_FCG_W);
-    if (c->pairs)
-      hipLaunchKernelGGL((mp_w2_kernel<true, 4>), span_grid(c), dim3(kBlock), 0,
-                         c->stream, c->geo, a, c->partials, c->nspan,
-                         c->ngroup == 1 ? 1 : 0);
-    else
-      hipLaunchKernelGGL((mp_w_kernel<4, true>), span_grid(c), dim3(kBlock), 0,
-                         c->stream, c->geo, a, c->partials, c->nspan,
-                         c->ngroup == 1 ? 1 : 0);
-  }
-  TEA_HIP_TRY(hipGetLastError());
-  c->mp_cur = mp_next(c->mp_cur);
-  double out[2];
-  TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
-  *pw = out[0];
-  *pr = out[1];
-  return TEA_HIP_OK;
+  return mp_calc_w(c, true, alpha, apply_u, beta, 1, pw, pr);
 }
 
 int tea_hip_fcg_read_z(tea_hip_chunk* c, float* host, size_t count) {

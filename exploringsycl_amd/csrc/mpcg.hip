@@ -224,11 +224,10 @@ __device__ inline void mp_pair_load(const Geo& g, const MpArgs& a, MpPair& s) {
 // the in-lane pair sums of p_new . w and, with DOT2, p_new . rdot.
 template <bool DOT2>
 __device__ inline void mp_pair_compute(const Geo& g, const MpArgs& a,
-                                       const MpPair& s, int lane,
+                                       const MpPair& s, int lane, double beta,
                                        double (&ps)[DOT2 ? 2 : 1]) {
   const int x = g.x;
   const int xl = g.h, xr = g.x - g.h - 1, yb = g.h, yt = g.y - g.h - 1;
-  const double beta = a.beta;
   const int i = s.e0;
   float pl = __shfl_up(s.P0.y, 1), pr = __shfl_down(s.P0.x, 1);
   float rl = 0.0f, rr = 0.0f;
@@ -289,14 +288,14 @@ __device__ inline void mp_pair_compute(const Geo& g, const MpArgs& a,
   if (a.apply_u) {
     ua = s.U.x + a.alpha * (double)s.P0.x;
     ub = s.U.y + a.alpha * (double)s.P0.y;
-    st2_nt(a.u, i, s.in0, s.in1, ua, ub);
+    st2_nt(a.u_out, i, s.in0, s.in1, ua, ub);
   }
   if (a.apply_p) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb);
   // Halo ring of boundary-adjacent cells (rare; per cell).
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
     if (!(c == 0 ? s.in0 : s.in1)) continue;
-    if (a.apply_u) ring_store(a.u, i + c, ka + c, row, x, xl, xr, yb, yt, c == 0 ? ua : ub);
+    if (a.apply_u) ring_store(a.u_out, i + c, ka + c, row, x, xl, xr, yb, yt, c == 0 ? ua : ub);
     if (a.apply_p) ring_store(a.p_new, i + c, ka + c, row, x, xl, xr, yb, yt, c == 0 ? ca : cb);
   }
 }
@@ -322,7 +321,7 @@ __global__ __launch_bounds__(kBlock) void mp_w2_kernel(Geo g, MpArgs a,
 #pragma unroll
     for (int j = 0; j < SB; ++j) {
       double ps[DOT2 ? 2 : 1];
-      mp_pair_compute<DOT2>(g, a, s[j], lane, ps);
+      mp_pair_compute<DOT2>(g, a, s[j], lane, a.beta, ps);
       psum[0][s0 + j] = ps[0];
       if (DOT2) psum[DOT2 ? 1 : 0][s0 + j] = ps[DOT2 ? 1 : 0];
     }
@@ -332,21 +331,36 @@ __global__ __launch_bounds__(kBlock) void mp_w2_kernel(Geo g, MpArgs a,
 
 template __global__ void mp_w2_kernel<true, 4>(Geo, MpArgs, double*, int, int);
 
+// A step's scalar (RaScalar): the host's value, the device's, or formed here
+// from the two sums the step before it left.
+template <bool CONSUME>
+__device__ inline double mp_scalar(const RaScalar& s, double value) {
+  if (!CONSUME) return s.dev ? *s.dev : value;
+  double v[2];
+  consume_sums<2>(s.sub, s.nblk, v);
+  const double q = s.inverse ? -v[1] / s.rro : v[1] / v[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    s.out[0] = v[0];
+    s.out[1] = v[1];
+    s.out[2] = q;
+  }
+  return q;
+}
+
 // One pair per thread.
-template <bool DOT2>
-__global__ __launch_bounds__(kBlock) void mp_w1_kernel(Geo g, MpArgs a,
+template <bool DOT2, bool CONSUME>
+__global__ __launch_bounds__(kBlock) void mp_w1_kernel(Geo g, MpArgs a, RaScalar sc,
                                                        double* sub, int nblk) {
   const int blk = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1);
   MpPair s;
   mp_pair_index(g, blk * kPairBlock + 2 * threadIdx.x, s);
   mp_pair_load<DOT2>(g, a, s);
+  const double beta = mp_scalar<CONSUME>(sc, a.beta);
   double ps[DOT2 ? 2 : 1];
-  mp_pair_compute<DOT2>(g, a, s, lane, ps);
+  mp_pair_compute<DOT2>(g, a, s, lane, beta, ps);
   block_sums_pairs<DOT2 ? 2 : 1>(ps, sub, nblk, blk, threadIdx.x);
 }
-
-template __global__ void mp_w1_kernel<true>(Geo, MpArgs, double*, int);
 
 // Four cells per lane (x a multiple of 4): the arithmetic of mp_w_kernel cell
 // by cell, with 16-byte loads of the FP32 operands and of u.  The
@@ -359,9 +373,9 @@ template __global__ void mp_w1_kernel<true>(Geo, MpArgs, double*, int);
 // one row apart (block c + S t, t = KS j .. KS j + KS - 1, S = x / 512;
 // blocks past the grid touch no cell), which share their rows above and
 // below in the CU's L1.
-template <bool DOT2, int UM, int KS>
-__global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs a, double* sub,
-                                                                  int nblk, int S) {
+template <bool DOT2, int UM, int KS, bool CONSUME>
+__global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs a, RaScalar sc,
+                                                                  double* sub, int nblk, int S) {
   int tid;
   const int blk = stacked_block<KS, kQuadThreads>(S, &tid);
   const int lane = threadIdx.x & (kWave - 1);
@@ -410,8 +424,6 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
     UB = ld2_nt(a.u, inB0 || inB1 ? ub : x + 2);
   }
   if (UM == 3) {
-    // p_h is the p_new buffer: each of its cells is read here by the wave
-    // that overwrites it below, and by no other.
     HA = ld2(a.p_h, inA0 || inA1 ? ua : x + 2);
     HB = ld2(a.p_h, inB0 || inB1 ? ub : x + 2);
     GA = ld2(a.p_h2, inA0 || inA1 ? ua : x + 2);
@@ -442,7 +454,7 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
     rr = RN;
     kxr = KXN;
   }
-  const double beta = a.beta;
+  const double beta = mp_scalar<CONSUME>(sc, a.beta);
   // p_new of the quad's cells, of its left and right neighbours, and of the
   // cells below and above (a halo neighbour reflects the cell itself).
   // Vector values, not arrays: an array indexed by the loop counter (pc[c - 1])
@@ -518,15 +530,15 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
                           u0[1] + a.alpha * (double)(hi ? aw : ay),
                           u0[2] + a.alpha * (double)(hi ? bz : bx),
                           u0[3] + a.alpha * (double)(hi ? bw : by)};
-    if (inA0 || inA1) st2_nt(a.u, ua, inA0, inA1, un[0], un[1]);
-    if (inB0 || inB1) st2_nt(a.u, ub, inB0, inB1, un[2], un[3]);
+    if (inA0 || inA1) st2_nt(a.u_out, ua, inA0, inA1, un[0], un[1]);
+    if (inB0 || inB1) st2_nt(a.u_out, ub, inB0, inB1, un[2], un[3]);
     // Halo ring of boundary-adjacent cells (rare; per cell).
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const bool inc = c == 0 ? inA0 : c == 1 ? inA1 : c == 2 ? inB0 : inB1;
       const int i = (c < 2 ? ua : ub) + (c & 1);
       const int kc = (c < 2 ? kA : kB) + (c & 1), rc = c < 2 ? rA : rB;
-      if (inc) ring_store(a.u, i, kc, rc, x, xl, xr, yb, yt, un[c]);
+      if (inc) ring_store(a.u_out, i, kc, rc, x, xl, xr, yb, yt, un[c]);
     }
   }
   if (any) {
@@ -577,10 +589,11 @@ __global__ __launch_bounds__(kBlock) void mp_r2_kernel(
   span_reduce_pairs_n<RW ? 2 : 1>(psum, partials, nspan, span, single_group != 0);
 }
 
-// mp_r2_kernel's arithmetic with one pair per thread.
-template <bool RW>
+// mp_r2_kernel's arithmetic with one pair per thread; the new r goes to r_out
+// (r itself, or a spare buffer when the iteration runs ahead).
+template <bool RW, bool CONSUME>
 __global__ __launch_bounds__(kBlock) void mp_r1_kernel(
-    Geo g, float* __restrict__ r, const float* __restrict__ w, double alpha,
+    Geo g, const float* r, float* r_out, const float* __restrict__ w, double value, RaScalar sc,
     double* sub, int nblk) {
   const int blk = blockIdx.x;
   const int e = blk * kPairBlock + 2 * threadIdx.x;
@@ -590,6 +603,7 @@ __global__ __launch_bounds__(kBlock) void mp_r1_kernel(
   const bool in1 = e < g.n && interior(g, kk + 1, row);
   const int i = (in0 || in1) ? e : 0;
   const float2 rv = ld2(r, i), wv = ld2(w, i);
+  const double alpha = mp_scalar<CONSUME>(sc, value);
   const float ra = (float)((double)rv.x - alpha * (double)wv.x);
   const float rb = (float)((double)rv.y - alpha * (double)wv.y);
   double v[RW ? 2 : 1];
@@ -597,14 +611,14 @@ __global__ __launch_bounds__(kBlock) void mp_r1_kernel(
   if (RW)
     v[RW ? 1 : 0] = (in0 ? (double)ra * (double)wv.x : 0.0) +
                     (in1 ? (double)rb * (double)wv.y : 0.0);
-  st2(r, e, in0, in1, ra, rb);
+  st2(r_out, e, in0, in1, ra, rb);
   block_sums_pairs<RW ? 2 : 1>(v, sub, nblk, blk, threadIdx.x);
 }
 
 // The same four cells per lane (x a multiple of 4).
-template <bool RW>
+template <bool RW, bool CONSUME>
 __global__ __launch_bounds__(kQuadThreads) void mp_r4_kernel(
-    Geo g, float* __restrict__ r, const float* __restrict__ w, double alpha,
+    Geo g, const float* r, float* r_out, const float* __restrict__ w, double value, RaScalar sc,
     double* sub, int nblk) {
   const int blk = blockIdx.x;
   const int e = blk * kQuadBlock + 4 * threadIdx.x;
@@ -616,6 +630,7 @@ __global__ __launch_bounds__(kQuadThreads) void mp_r4_kernel(
   const bool any = in[0] || in[1] || in[2] || in[3];
   const int i = any ? e : 0;
   const float4 rv = ld4(r, i), wv = ld4(w, i);
+  const double alpha = mp_scalar<CONSUME>(sc, value);
   float rn[4];
   double prod[RW ? 2 : 1][4];
 #pragma unroll
@@ -628,7 +643,7 @@ __global__ __launch_bounds__(kQuadThreads) void mp_r4_kernel(
 #pragma unroll
   for (int q = 0; q < (RW ? 2 : 1); ++q)
     v[q] = (prod[q][0] + prod[q][1]) + (prod[q][2] + prod[q][3]);
-  if (any) st4(r, e, in, rn);
+  if (any) st4(r_out, e, in, rn);
   block_sums_quads<RW ? 2 : 1>(v, sub, nblk, blk, threadIdx.x);
 }
 
@@ -699,7 +714,7 @@ __global__ __launch_bounds__(kBlock) void mp_convert_all_kernel(
     const double* __restrict__ p, const double* __restrict__ r,
     float* __restrict__ kx32, float* __restrict__ ky32,
     float* __restrict__ p32a, float* __restrict__ p32b, float* __restrict__ p32c,
-    float* __restrict__ r32) {
+    float* __restrict__ p32d, float* __restrict__ r32) {
   const int i = blockIdx.x * kBlock + threadIdx.x;
   if (i >= n) return;
   kx32[i] = (float)kx[i];
@@ -708,6 +723,7 @@ __global__ __launch_bounds__(kBlock) void mp_convert_all_kernel(
   p32a[i] = pv;
   p32b[i] = pv;
   p32c[i] = pv;
+  p32d[i] = pv;
   r32[i] = (float)r[i];
 }
 
@@ -763,8 +779,8 @@ struct MpTrueResidualBody {
 int ensure_mp_buffers(tea_hip_chunk* c) {
   if (c->mp_r) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
-  float** bufs[] = {&c->mp_p[0], &c->mp_p[1], &c->mp_p[2], &c->mp_r, &c->mp_w, &c->mp_kx,
-                    &c->mp_ky};
+  float** bufs[] = {&c->mp_p[0], &c->mp_p[1], &c->mp_p[2], &c->mp_p[3], &c->mp_w, &c->mp_kx,
+                    &c->mp_ky, &c->mp_r_alt, &c->mp_w_alt, &c->mp_r};
   for (float** b : bufs) {
     if (hipMalloc(b, bytes) != hipSuccess) {
       *b = nullptr;
@@ -779,6 +795,7 @@ int ensure_mp_buffers(tea_hip_chunk* c) {
 }  // namespace
 
 int apply_mp_hold(tea_hip_chunk* c) {
+  if (c->mra) TEA_RETURN_IF(mra_discard(c));
   const int n = c->hold;
   c->hold = 0;
   for (int i = 0; i < n; ++i) {
@@ -792,107 +809,323 @@ int apply_mp_hold(tea_hip_chunk* c) {
   return TEA_HIP_OK;
 }
 
-int launch_mp_w4(tea_hip_chunk* c, MpArgs a, int kid) {
-  const int cur = c->mp_cur, dst = mp_next(cur), prev = mp_next(dst);
-  int um = a.apply_u ? 1 : 0;
-  // Held updates are those of the two steps before this one: their p are
-  // in p_new's buffer (the older) and in the buffer before p_old's.
-  const bool ride = um == 1 && a.apply_p &&
-                    (c->hold == 0 || (c->hold == 1 && c->hold_buf[0] == prev) ||
-                     (c->hold == 2 && c->hold_buf[0] == dst && c->hold_buf[1] == prev));
-  if (c->hold && !ride) TEA_RETURN_IF(apply_mp_hold(c));
-  if (c->hold == 2) {
-    um = 3;
-    a.p_h = c->mp_p[dst];
-    a.alpha_h = c->hold_alpha[0];
-    a.p_h2 = c->mp_p[prev];
-    a.alpha_h2 = c->hold_alpha[1];
-    c->hold = 0;
-  } else if (um == 1 && a.apply_p && c->hold_ok) {
-    // Held: p_old's buffer is not written until two steps on.
-    um = 0;
-    c->hold_buf[c->hold] = cur;
-    c->hold_alpha[c->hold] = a.alpha;
-    ++c->hold;
+// ---- run-ahead of the mixed-precision and FCG iterations ------------------
+//
+// As for FP64 CG (cg.hip): the host turns p.w and p.r into alpha and the
+// r-step's sums into beta before it can ask for the next pass, two round
+// trips per iteration (about 6 us each).  So each call queues the next pass
+// behind its own before it waits for its own sums: calc_w the r-step (with
+// FCG also z = M(r)), calc_r the w-step, into spare r, z, w and u buffers and
+// a p buffer of the ring that no held update needs, with the scalar formed on
+// the device.  The host's next call takes the pass over when its arguments
+// are bitwise what the pass used; any other call drops it, and only spare
+// buffers were written.  Each scalar is formed by the next pass itself on
+// grids of at most kConsumeBlocks blocks, else by the finisher's last block.
+// A w-step is not queued where the driver refreshed after as many iterations
+// the last time (the refresh would drop it).
+
+namespace {
+
+constexpr int kMraNone = 0, kMraR = 1, kMraW = 2;
+constexpr int kMraSlotW = 0, kMraSlotR = 1;
+
+bool mra_consume(const tea_hip_chunk* c) { return c->nblk <= kConsumeBlocks; }
+
+bool mra_possible(const tea_hip_chunk* c) {
+  return c->ra_enabled && c->fused && c->poll && c->mra_fail < 3 && use_pair_blocks(c, 1) &&
+         use_pair_blocks(c, 2);
+}
+
+void mra_mismatch(tea_hip_chunk* c) {
+  c->mra = kMraNone;
+  c->ra_dirty = true;
+  c->mra_fail += 1;
+}
+
+template <class T>
+void swap_buf(T*& a, T*& b) {
+  T* t = a;
+  a = b;
+  b = t;
+}
+
+int ensure_mra(tea_hip_chunk* c) {
+  if (c->mra_host) return TEA_HIP_OK;
+  if (!c->u_alt && hipMalloc(&c->u_alt, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
+    c->u_alt = nullptr;
+    set_error("hipMalloc of a run-ahead buffer failed");
+    return TEA_HIP_ENOMEM;
   }
-  Timed t(c, kid);
+  if (!c->mra_dev && hipMalloc(&c->mra_dev, 3 * sizeof(double)) != hipSuccess) {
+    c->mra_dev = nullptr;
+    set_error("hipMalloc of the run-ahead scalars failed");
+    return TEA_HIP_ENOMEM;
+  }
+  double* host = nullptr;
+  if (hipHostMalloc(&host, 8 * sizeof(double),
+                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    set_error("hipHostMalloc of the run-ahead slots failed");
+    return TEA_HIP_ENOMEM;
+  }
+  TEA_HIP_TRY(hipHostGetDevicePointer((void**)&c->mra_host_dev, host, 0));
+  c->mra_host = host;
+  return TEA_HIP_OK;
+}
+
+// Arms a step's host slot and sets *sc to where the next pass takes the
+// step's scalar from (launching the finisher where there is one).
+int mra_finish(tea_hip_chunk* c, int slot, RaScalar* sc) {
+  if (c->ra_dirty) {
+    // A dropped pass may still be queued and write these slots.
+    TEA_HIP_TRY(hipStreamSynchronize(c->stream));
+    c->ra_dirty = false;
+  }
+  arm_host_values(c->mra_host + 4 * slot, 3);
+  *sc = RaScalar{};
+  sc->out = c->mra_host_dev + 4 * slot;
+  if (mra_consume(c)) {
+    sc->sub = slot == kMraSlotW ? c->sub : c->sub2;
+    sc->nblk = c->nblk;
+    sc->inverse = slot == kMraSlotW ? 0 : 1;
+    return TEA_HIP_OK;
+  }
+  sc->dev = c->mra_dev + slot;
+  return launch_span_finish_ra(c, 2, sc->out, RaTail{0.0, 1, slot, c->mra_dev});
+}
+
+int mra_wait(tea_hip_chunk* c, int slot, double* s0, double* s1, double* scalar) {
+  const double* h = c->mra_host + 4 * slot;
+  TEA_RETURN_IF(wait_host_values(c, h, 3));
+  *s0 = h[0];
+  *s1 = h[1];
+  *scalar = h[2];
+  return TEA_HIP_OK;
+}
+
+// The w-step of a call with these arguments.  u += alpha p_old is held back
+// over two steps (four cells per lane); held updates that cannot ride along
+// are made on their own first.  Running ahead, w and u go to the spares.
+int plan_mp_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta, int apply_p,
+              bool ahead, MpStep* s) {
+  const bool ride = c->quads && apply_u && apply_p;
+  if (c->hold && !ride) TEA_RETURN_IF(apply_mp_hold(c));
+  const int cur = c->mp_cur;
+  double* u = c->field[TEA_FIELD_U];
+  *s = MpStep{};
+  s->a = MpArgs{c->mp_p[cur], c->mp_p[mp_next(cur)], fcg ? c->fcg_z : c->mp_r, u,
+                ahead ? c->mp_w_alt : c->mp_w, c->mp_kx, c->mp_ky, c->mp_r, alpha, beta,
+                apply_u ? 1 : 0, apply_p ? 1 : 0, nullptr, nullptr, 0.0, 0.0,
+                ahead ? c->u_alt : u};
+  s->um = apply_u ? 1 : 0;
+  if (!ride || !c->hold_ok) return TEA_HIP_OK;
+  if (c->hold == 2) {
+    s->um = 3;
+    s->a.p_h = c->mp_p[c->hold_buf[0]];
+    s->a.alpha_h = c->hold_alpha[0];
+    s->a.p_h2 = c->mp_p[c->hold_buf[1]];
+    s->a.alpha_h2 = c->hold_alpha[1];
+    return TEA_HIP_OK;
+  }
+  // Held: the ring leaves p_old's buffer alone for the two steps after.
+  s->um = 0;
+  s->hold = c->hold + 1;
+  for (int i = 0; i < c->hold; ++i) {
+    s->hold_buf[i] = c->hold_buf[i];
+    s->hold_alpha[i] = c->hold_alpha[i];
+  }
+  s->hold_buf[c->hold] = cur;
+  s->hold_alpha[c->hold] = alpha;
+  return TEA_HIP_OK;
+}
+
+template <int UM, bool CONSUME>
+void launch_w4(tea_hip_chunk* c, const MpArgs& a, const RaScalar& sc) {
   // stack_factor(c) blocks one row apart per workgroup (stacked_block).
   const int S = stack_rows(c), ks = stack_factor(c);
-  const dim3 grid = stacked_grid(c, ks), block(kQuadThreads * ks);
-#define TEA_MP_W4(UMV)                                                                    \
-  do {                                                                                    \
-    if (ks == 1)                                                                          \
-      hipLaunchKernelGGL((mp_w4_kernel<true, UMV, 1>), grid, block, 0, c->stream, c->geo, \
-                         a, c->sub, c->nblk, S);                                          \
-    else if (ks == 2)                                                                     \
-      hipLaunchKernelGGL((mp_w4_kernel<true, UMV, 2>), grid, block, 0, c->stream, c->geo, \
-                         a, c->sub, c->nblk, S);                                          \
-    else                                                                                  \
-      hipLaunchKernelGGL((mp_w4_kernel<true, UMV, 4>), grid, block, 0, c->stream, c->geo, \
-                         a, c->sub, c->nblk, S);                                          \
-  } while (0)
-  if (um == 0)
-    TEA_MP_W4(0);
-  else if (um == 1)
-    TEA_MP_W4(1);
+  const auto kernel = ks == 1   ? mp_w4_kernel<true, UM, 1, CONSUME>
+                      : ks == 2 ? mp_w4_kernel<true, UM, 2, CONSUME>
+                                : mp_w4_kernel<true, UM, 4, CONSUME>;
+  hipLaunchKernelGGL(kernel, stacked_grid(c, ks), dim3(kQuadThreads * ks), 0, c->stream, c->geo, a,
+                     sc, c->sub, c->nblk, S);
+}
+
+int launch_mp_step(tea_hip_chunk* c, const MpStep& s, bool fcg, const RaScalar& sc) {
+  Timed t(c, fcg ? K_FCG_W : K_MP_W);
+  const bool consume = sc.sub != nullptr;
+  if (!c->quads)
+    hipLaunchKernelGGL((consume ? mp_w1_kernel<true, true> : mp_w1_kernel<true, false>),
+                       pair_grid(c), dim3(kBlock), 0, c->stream, c->geo, s.a, sc, c->sub, c->nblk);
+  else if (s.um == 0)
+    consume ? launch_w4<0, true>(c, s.a, sc) : launch_w4<0, false>(c, s.a, sc);
+  else if (s.um == 1)
+    consume ? launch_w4<1, true>(c, s.a, sc) : launch_w4<1, false>(c, s.a, sc);
   else
-    TEA_MP_W4(3);
-#undef TEA_MP_W4
+    consume ? launch_w4<3, true>(c, s.a, sc) : launch_w4<3, false>(c, s.a, sc);
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
 }
 
-// r -= alpha w and the partials of r.r (and, with rw, of r.w in the second
-// array) into c->partials (not waited for); *len is the number of partials
-// left to finish in each array.
-int launch_mp_r(tea_hip_chunk* c, double alpha, int* len, bool rw, bool finish) {
-  *len = c->nspan;
-  TEA_CHECK_ARG(finish || use_quad_blocks(c, 2), "launch_mp_r: unfinished sums need quads");
-  if (use_quad_blocks(c, 2)) {
-    {
-      Timed t(c, K_MP_R);
-      if (rw)
-        hipLaunchKernelGGL(mp_r4_kernel<true>, quad_grid(c), dim3(kQuadThreads), 0, c->stream,
-                           c->geo, c->mp_r, c->mp_w, alpha, c->sub, c->nblk);
-      else
-        hipLaunchKernelGGL(mp_r4_kernel<false>, quad_grid(c), dim3(kQuadThreads), 0, c->stream,
-                           c->geo, c->mp_r, c->mp_w, alpha, c->sub, c->nblk);
-    }
-    TEA_HIP_TRY(hipGetLastError());
-    if (!finish) return TEA_HIP_OK;
-    return launch_span_finish(c, rw ? 2 : 1, len, 0, rw);
+// The chunk's state once a w-step has been asked for (or taken over).
+void commit_mp_step(tea_hip_chunk* c, const MpStep& s) {
+  c->hold = s.hold;
+  for (int i = 0; i < s.hold; ++i) {
+    c->hold_buf[i] = s.hold_buf[i];
+    c->hold_alpha[i] = s.hold_alpha[i];
   }
-  if (use_pair_blocks(c, 2)) {
-    {
-      Timed t(c, K_MP_R);
-      if (rw)
-        hipLaunchKernelGGL(mp_r1_kernel<true>, pair_grid(c), dim3(kBlock), 0, c->stream,
-                           c->geo, c->mp_r, c->mp_w, alpha, c->sub, c->nblk);
-      else
-        hipLaunchKernelGGL(mp_r1_kernel<false>, pair_grid(c), dim3(kBlock), 0, c->stream,
-                           c->geo, c->mp_r, c->mp_w, alpha, c->sub, c->nblk);
-    }
-    TEA_HIP_TRY(hipGetLastError());
-    return launch_span_finish(c, rw ? 2 : 1, len, 0, rw);
+  if (s.um && s.a.u_out != s.a.u) swap_buf(c->field[TEA_FIELD_U], c->u_alt);
+  if (s.a.w != c->mp_w) swap_buf(c->mp_w, c->mp_w_alt);
+  if (s.a.apply_p) c->mp_cur = mp_next(c->mp_cur);
+}
+
+// Queues the r-step (with FCG also z = M(r)) behind the w-step whose sums are
+// in c->sub, then waits for that w-step's sums.
+int mra_queue_r(tea_hip_chunk* c, bool fcg, double* pw, double* pr) {
+  RaScalar sc;
+  TEA_RETURN_IF(mra_finish(c, kMraSlotW, &sc));
+  double* sub = mra_consume(c) ? c->sub2 : c->sub;
+  TEA_RETURN_IF(launch_mp_r(c, MpRStep{c->mp_r, c->mp_r_alt, c->mp_w, 0.0, sc}, !fcg, sub));
+  if (fcg)
+    TEA_RETURN_IF(launch_fcg_z(c, c->mra_coarse, c->mp_r_alt, c->mp_w, c->fcg_z_alt,
+                               sub + sub_stride(c->nblk)));
+  TEA_RETURN_IF(mra_finish(c, kMraSlotR, &c->mra_next));
+  c->mra = kMraR;
+  c->mra_fcg = fcg;
+  TEA_RETURN_IF(mra_wait(c, kMraSlotW, pw, pr, &c->mra_alpha));
+  c->mra_pw = *pw;
+  return TEA_HIP_OK;
+}
+
+}  // namespace
+
+int mra_discard(tea_hip_chunk* c) {
+  if (c->mra != kMraNone) {
+    c->mra = kMraNone;
+    c->ra_dirty = true;
   }
-  Timed t(c, K_MP_R);
-  const int sg = c->ngroup == 1 ? 1 : 0;
-  if (c->pairs) {
-    if (rw)
-      hipLaunchKernelGGL(mp_r2_kernel<true>, span_grid(c), dim3(kBlock), 0, c->stream,
-                         c->geo, c->mp_r, c->mp_w, alpha, c->partials, c->nspan, sg);
-    else
-      hipLaunchKernelGGL(mp_r2_kernel<false>, span_grid(c), dim3(kBlock), 0, c->stream,
-                         c->geo, c->mp_r, c->mp_w, alpha, c->partials, c->nspan, sg);
+  return TEA_HIP_OK;
+}
+
+int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta, int apply_p,
+              double* pw, double* pr) {
+  if (c->mra == kMraW && c->mra_fcg == fcg && apply_u && apply_p &&
+      alpha == c->mra_step.a.alpha && beta == c->mra_beta) {
+    commit_mp_step(c, c->mra_step);
+    c->mra = kMraNone;
+    c->mra_fail = 0;
+    return mra_queue_r(c, fcg, pw, pr);
+  }
+  if (c->mra) mra_mismatch(c);
+  int len = c->nspan;
+  if (use_pair_blocks(c, 1)) {
+    const bool ahead = mra_possible(c);
+    if (ahead) TEA_RETURN_IF(ensure_mra(c));
+    MpStep s;
+    TEA_RETURN_IF(plan_mp_w(c, fcg, alpha, apply_u, beta, apply_p, false, &s));
+    TEA_RETURN_IF(launch_mp_step(c, s, fcg, RaScalar{}));
+    commit_mp_step(c, s);
+    if (ahead) return mra_queue_r(c, fcg, pw, pr);
+    TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true));
   } else {
-    if (rw)
-      hipLaunchKernelGGL(mp_r_kernel<true>, span_grid(c), dim3(kBlock), 0, c->stream,
-                         c->geo, c->mp_r, c->mp_w, alpha, c->partials, c->nspan, sg);
-    else
-      hipLaunchKernelGGL(mp_r_kernel<false>, span_grid(c), dim3(kBlock), 0, c->stream,
-                         c->geo, c->mp_r, c->mp_w, alpha, c->partials, c->nspan, sg);
+    if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
+    const int cur = c->mp_cur, sg = c->ngroup == 1 ? 1 : 0;
+    const MpArgs a{c->mp_p[cur], c->mp_p[mp_next(cur)], fcg ? c->fcg_z : c->mp_r,
+                   c->field[TEA_FIELD_U], c->mp_w, c->mp_kx, c->mp_ky, c->mp_r, alpha, beta,
+                   apply_u ? 1 : 0, apply_p ? 1 : 0, nullptr, nullptr, 0.0, 0.0,
+                   c->field[TEA_FIELD_U]};
+    {
+      Timed t(c, fcg ? K_FCG_W : K_MP_W);
+      if (c->pairs)
+        hipLaunchKernelGGL((mp_w2_kernel<true, 4>), span_grid(c), dim3(kBlock), 0, c->stream,
+                           c->geo, a, c->partials, c->nspan, sg);
+      else
+        hipLaunchKernelGGL((mp_w_kernel<4, true>), span_grid(c), dim3(kBlock), 0, c->stream,
+                           c->geo, a, c->partials, c->nspan, sg);
+    }
+    TEA_HIP_TRY(hipGetLastError());
+    if (apply_p) c->mp_cur = mp_next(cur);
+  }
+  double out[2];
+  TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
+  *pw = out[0];
+  *pr = out[1];
+  return TEA_HIP_OK;
+}
+
+int launch_mp_r(tea_hip_chunk* c, const MpRStep& s, bool rw, double* sub) {
+  Timed t(c, K_MP_R);
+  if (use_pair_blocks(c, 2)) {
+    const bool quads = use_quad_blocks(c, 2), consume = s.sc.sub != nullptr;
+    const dim3 grid = quads ? quad_grid(c) : pair_grid(c), block(quads ? kQuadThreads : kBlock);
+    const auto kernel =
+        quads ? (rw ? (consume ? mp_r4_kernel<true, true> : mp_r4_kernel<true, false>)
+                    : (consume ? mp_r4_kernel<false, true> : mp_r4_kernel<false, false>))
+              : (rw ? (consume ? mp_r1_kernel<true, true> : mp_r1_kernel<true, false>)
+                    : (consume ? mp_r1_kernel<false, true> : mp_r1_kernel<false, false>));
+    hipLaunchKernelGGL(kernel, grid, block, 0, c->stream, c->geo, s.r, s.r_out, s.w, s.alpha,
+                       s.sc, sub, c->nblk);
+  } else {
+    const int sg = c->ngroup == 1 ? 1 : 0;
+    const auto kernel = c->pairs ? (rw ? mp_r2_kernel<true> : mp_r2_kernel<false>)
+                                 : (rw ? mp_r_kernel<true> : mp_r_kernel<false>);
+    hipLaunchKernelGGL(kernel, span_grid(c), dim3(kBlock), 0, c->stream, c->geo, s.r_out, s.w,
+                       s.alpha, c->partials, c->nspan, sg);
   }
   TEA_HIP_TRY(hipGetLastError());
+  return TEA_HIP_OK;
+}
+
+int mp_calc_r(tea_hip_chunk* c, bool fcg, double alpha, int use_net, double* rr, double* rx) {
+  c->mra_since += 1;
+  if (c->mra == kMraR && c->mra_fcg == fcg && alpha == c->mra_alpha &&
+      (!fcg || use_net == c->mra_coarse)) {
+    swap_buf(c->mp_r, c->mp_r_alt);
+    if (fcg) swap_buf(c->fcg_z, c->fcg_z_alt);
+    c->mra = kMraNone;
+    c->mra_fail = 0;
+    if (mra_possible(c) && c->mra_since != c->mra_period) {
+      if (!c->mra_synced) {
+        // The spare u takes the cells outside the interior that no step writes.
+        TEA_HIP_TRY(hipMemcpyAsync(c->u_alt, c->field[TEA_FIELD_U],
+                                   (size_t)c->geo.n * sizeof(double), hipMemcpyDeviceToDevice,
+                                   c->stream));
+        c->mra_synced = true;
+      }
+      TEA_RETURN_IF(plan_mp_w(c, fcg, alpha, 1, 0.0, 1, true, &c->mra_step));
+      RaScalar sc = c->mra_next;
+      sc.rro = c->mra_pw;
+      TEA_RETURN_IF(launch_mp_step(c, c->mra_step, fcg, sc));
+      c->mra = kMraW;
+      return mra_wait(c, kMraSlotR, rr, rx, &c->mra_beta);
+    }
+    if (!mra_consume(c)) return mra_wait(c, kMraSlotR, rr, rx, &c->mra_beta);
+    int len;
+    double out[2];
+    TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true, c->sub2));
+    TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
+    *rr = out[0];
+    *rx = out[1];
+    return TEA_HIP_OK;
+  }
+  if (c->mra) mra_mismatch(c);
+  if (fcg) c->mra_coarse = use_net;
+  const MpRStep s{c->mp_r, c->mp_r, c->mp_w, alpha, RaScalar{}};
+  double out[2];
+  if (use_pair_blocks(c, 2)) {
+    TEA_RETURN_IF(launch_mp_r(c, s, !fcg, c->sub));
+    if (fcg)
+      TEA_RETURN_IF(launch_fcg_z(c, use_net, c->mp_r, c->mp_w, c->fcg_z,
+                                 c->sub + sub_stride(c->nblk)));
+    int len;
+    TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true));
+    TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
+  } else {
+    int lens[2] = {c->nspan, c->nspan};
+    TEA_RETURN_IF(launch_mp_r(c, s, !fcg, nullptr));
+    if (fcg) TEA_RETURN_IF(launch_precondition(c, use_net, 1, &lens[1]));
+    TEA_RETURN_IF(finish_reduction_lens(c, 2, lens, out));
+  }
+  *rr = out[0];
+  *rx = out[1];
   return TEA_HIP_OK;
 }
 
@@ -925,7 +1158,7 @@ int tea_hip_mpcg_init(tea_hip_chunk* c, int coefficient, double rx, double ry,
     hipLaunchKernelGGL(mp_convert_all_kernel, flat_grid(g.n), dim3(kBlock), 0,
                        c->stream, g.n, f[TEA_FIELD_KX], f[TEA_FIELD_KY],
                        f[TEA_FIELD_P], f[TEA_FIELD_R], c->mp_kx, c->mp_ky,
-                       c->mp_p[0], c->mp_p[1], c->mp_p[2], c->mp_r);
+                       c->mp_p[0], c->mp_p[1], c->mp_p[2], c->mp_p[3], c->mp_r);
     MpConvertBody body{f[TEA_FIELD_R], f[TEA_FIELD_U0]};
     hipLaunchKernelGGL((span_kernel<2, MpConvertBody>), span_grid(c),
                        dim3(kBlock), 0, c->stream, g, body, c->partials,
@@ -933,6 +1166,8 @@ int tea_hip_mpcg_init(tea_hip_chunk* c, int coefficient, double rx, double ry,
   }
   TEA_HIP_TRY(hipGetLastError());
   c->mp_cur = 0;
+  c->mra_synced = false;
+  c->mra_fail = c->mra_since = 0;
   double out[2];
   TEA_RETURN_IF(finish_reduction(c, 2, out));
   *rr = out[0];
@@ -947,42 +1182,7 @@ int tea_hip_mpcg_calc_w(tea_hip_chunk* c, double alpha, int apply_u,
   TEA_CHECK_ARG(pw != nullptr && pr != nullptr, "null outputs");
   TEA_HIP_TRY(hipSetDevice(c->device));
   TEA_FLUSH_HELD_KEEP_U(c);
-  // The two-dot kernel of flexible CG with z = r: p = r + beta p_old,
-  // w = A p, p.w and p.r.
-  MpArgs a{c->mp_p[c->mp_cur], c->mp_p[mp_next(c->mp_cur)], c->mp_r,
-           c->field[TEA_FIELD_U], c->mp_w, c->mp_kx, c->mp_ky, c->mp_r,
-           alpha, beta, apply_u ? 1 : 0, apply_p ? 1 : 0};
-  int len = c->nspan;
-  if (use_pair_blocks(c, 1)) {
-    if (c->quads) {
-      TEA_RETURN_IF(launch_mp_w4(c, a, K_MP_W));
-    } else {
-      if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
-      Timed t(c, K_MP_W);
-      hipLaunchKernelGGL((mp_w1_kernel<true>), pair_grid(c), dim3(kBlock), 0,
-                         c->stream, c->geo, a, c->sub, c->nblk);
-    }
-    TEA_HIP_TRY(hipGetLastError());
-    TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true));
-  } else {
-    if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
-    Timed t(c, K_MP_W);
-    if (c->pairs)
-      hipLaunchKernelGGL((mp_w2_kernel<true, 4>), span_grid(c), dim3(kBlock), 0,
-                         c->stream, c->geo, a, c->partials, c->nspan,
-                         c->ngroup == 1 ? 1 : 0);
-    else
-      hipLaunchKernelGGL((mp_w_kernel<4, true>), span_grid(c), dim3(kBlock), 0,
-                         c->stream, c->geo, a, c->partials, c->nspan,
-                         c->ngroup == 1 ? 1 : 0);
-  }
-  TEA_HIP_TRY(hipGetLastError());
-  if (apply_p) c->mp_cur = mp_next(c->mp_cur);
-  double out[2];
-  TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
-  *pw = out[0];
-  *pr = out[1];
-  return TEA_HIP_OK;
+  return mp_calc_w(c, false, alpha, apply_u, beta, apply_p, pw, pr);
 }
 
 int tea_hip_mpcg_calc_r(tea_hip_chunk* c, double alpha, double* rr, double* rw) {
@@ -991,13 +1191,7 @@ int tea_hip_mpcg_calc_r(tea_hip_chunk* c, double alpha, double* rr, double* rw) 
   TEA_CHECK_ARG(rr != nullptr && rw != nullptr, "null outputs");
   TEA_HIP_TRY(hipSetDevice(c->device));
   TEA_FLUSH_HELD_KEEP_U(c);
-  int len;
-  TEA_RETURN_IF(launch_mp_r(c, alpha, &len, true));
-  double out[2];
-  TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
-  *rr = out[0];
-  *rw = out[1];
-  return TEA_HIP_OK;
+  return mp_calc_r(c, false, alpha, 0, rr, rw);
 }
 
 int tea_hip_mpcg_refresh(tea_hip_chunk* c, double alpha, int apply_u,
@@ -1007,6 +1201,8 @@ int tea_hip_mpcg_refresh(tea_hip_chunk* c, double alpha, int apply_u,
   TEA_CHECK_ARG(rr && rr_true && rw, "null outputs");
   TEA_HIP_TRY(hipSetDevice(c->device));
   TEA_FLUSH_HELD(c);
+  c->mra_period = c->mra_since;
+  c->mra_since = 0;
   double** f = c->field;
   const Geo g = c->geo;
   if (apply_u) {

@@ -479,7 +479,7 @@ __device__ inline void block_sums_quads(const double (&v)[NR], double* sub, int 
 }
 
 // The sums a pass before this one left in sub, formed by every block of this
-// pass for itself (the first 256 threads load, every thread gets the sums):
+// pass for itself (up to four waves load, every thread gets the sums):
 // with up to 2048 blocks (4 groups) the reference's remaining passes are one
 // pairwise tree over the zero-padded block sums.  It saves the finisher's
 // launch (3.4-4.2 us) between two dependent passes: an FP64 CG iteration at
@@ -493,20 +493,24 @@ template <int NR>
 __device__ inline void consume_sums(const double* __restrict__ sub, int nblk,
                                     double (&sum)[NR]) {
   __shared__ double gs[NR][4];
-  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-  const int stride = sub_stride(nblk);
-  if (wv < 4) {
-    const int i0 = kGroupBlocks * wv + kSubPerSpan * lane;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int stride = sub_stride(nblk), waves = blockDim.x / kWave;
+  for (int g = threadIdx.x / kWave; g < 4; g += waves) {
+    const int i0 = kGroupBlocks * g + kSubPerSpan * lane;
+    double t[NR];
 #pragma unroll
     for (int q = 0; q < NR; ++q) {
-      double t = 0.0;
+      t[q] = 0.0;
       if (i0 < stride) {
         const double* p = sub + (size_t)q * stride + i0;
         const double2 a = ld2(p, 0), b = ld2(p, 2), c = ld2(p, 4), d = ld2(p, 6);
-        t = ((a.x + a.y) + (b.x + b.y)) + ((c.x + c.y) + (d.x + d.y));
+        t[q] = ((a.x + a.y) + (b.x + b.y)) + ((c.x + c.y) + (d.x + d.y));
       }
-      t = wave_tree_dpp(t);
-      if (lane == 0) gs[q][wv] = t;
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const double s = wave_tree_dpp(t[q]);
+      if (lane == 0) gs[q][g] = s;
     }
   }
   __syncthreads();
@@ -664,11 +668,31 @@ struct MpArgs {
   double alpha, beta;
   int apply_u, apply_p;
   // Held updates applied first (mp_w4_kernel, UM 3): u += alpha_h p_h,
-  // then u += alpha_h2 p_h2; p_h is p_new's buffer, read before it is
-  // overwritten.
+  // then u += alpha_h2 p_h2.
   const float* p_h;
   const float* p_h2;
   double alpha_h, alpha_h2;
+  // Pair-per-thread and four-cell kernels: the new u goes to u_out (u, or a
+  // spare buffer when the iteration runs ahead).
+  double* u_out;
+};
+
+// Where a pass of the iteration takes its scalar from: the host's value
+// (dev null), the device's (dev: a finisher of the run-ahead left it there),
+// or, with CONSUME, the block sums sub of the pass before it, which every
+// block reduces for itself; the first block then leaves the scalar and the
+// sum for the next pass and the host.  alpha = rro / sum (r-step), beta =
+// sum / rro (w-step); rro is *rro_dev where that is set, else the value.
+// Mixed-precision CG and FCG take two sums: (p.w, p.r) give alpha = p.r /
+// p.w, (r.r, r.w or z.w) give beta = -r.w / p.w with p.w in rro.
+struct RaScalar {
+  const double* dev = nullptr;
+  const double* sub = nullptr;
+  int nblk = 0, inverse = 0;
+  double rro = 0.0;
+  const double* rro_dev = nullptr;
+  double* sum_dev = nullptr;  // set by the w-step: r.r, the next alpha's rro
+  double* out = nullptr;      // host slot {sum(s), scalar}
 };
 
 template <int kBatch, bool DOT2>
@@ -680,29 +704,6 @@ __global__ void mp_r_kernel(Geo g, float* r, const float* w, double alpha,
 template <bool DOT2, int SB>
 __global__ void mp_w2_kernel(Geo g, MpArgs a, double* partials, int nspan,
                              int single_group);
-template <bool DOT2>
-__global__ void mp_w1_kernel(Geo g, MpArgs a, double* sub, int nblk);
-// UM: 0 leaves u alone, 1 adds alpha p_old, 3 adds alpha_h p_h, alpha_h2
-// p_h2 and then alpha p_old.
-template <bool DOT2, int UM, int KS>
-__global__ void mp_w4_kernel(Geo g, MpArgs a, double* sub, int nblk, int S);
-
-// Where a pass of the iteration takes its scalar from: the host's value
-// (dev null), the device's (dev: a finisher of the run-ahead left it there),
-// or, with CONSUME, the block sums sub of the pass before it, which every
-// block reduces for itself; the first block then leaves the scalar and the
-// sum for the next pass and the host.  alpha = rro / sum (r-step), beta =
-// sum / rro (w-step); rro is *rro_dev where that is set, else the value.
-struct RaScalar {
-  const double* dev = nullptr;
-  const double* sub = nullptr;
-  int nblk = 0, inverse = 0;
-  double rro = 0.0;
-  const double* rro_dev = nullptr;
-  double* sum_dev = nullptr;  // set by the w-step: r.r, the next alpha's rro
-  double* out = nullptr;      // host slot {sum, scalar}
-};
-
 }  // namespace tea
 
 struct tea_nn;
@@ -786,11 +787,22 @@ const float* output(tea_nn* n);
 // ---------------------------------------------------------------------------
 // The chunk handle.
 
-// The mixed-precision p buffers: a ring of three, so that a w-step can
-// hold the u updates of two steps back (their p are the two buffers it
-// does not write).
-constexpr int kMpRing = 3;
+// The mixed-precision p buffers: a ring of four, so that a w-step can hold
+// the u updates of two steps back and a w-step that runs ahead writes a
+// buffer no update still needs.
+constexpr int kMpRing = 4;
 inline int mp_next(int i) { return i + 1 == kMpRing ? 0 : i + 1; }
+
+// One mixed-precision (or FCG) w-step on the pair or four-cell kernels: its
+// arguments, the u update it makes (um: none, its own, or the two held ones
+// and its own) and the updates held once it is taken over.
+struct MpStep {
+  tea::MpArgs a;
+  int um = 0;
+  int hold = 0;
+  int hold_buf[2] = {0, 0};
+  double hold_alpha[2] = {0.0, 0.0};
+};
 
 // One coarse level of the learned preconditioner.
 struct FcgLevel {
@@ -836,6 +848,10 @@ struct tea_hip_chunk {
   int nblk = 0;                     // 512-cell blocks covering x*y
   double* sub = nullptr;
   double* sub2 = nullptr;
+  // Sums of the groups of 512 blocks and the finisher's count of blocks done
+  // (zero between launches), for grids of more than 16 groups.
+  double* grp_sum = nullptr;
+  unsigned* done_count = nullptr;
   int pair_blocks = 3;              // pair-per-thread kernels: bit 0 fused_w,
                                     // bit 1 fused_r
 
@@ -869,15 +885,15 @@ struct tea_hip_chunk {
   bool pend_u = false, pend_p = false, pend_halo = false;
   double pend_alpha = 0.0, pend_beta = 0.0;
 
-  // Mixed-precision CG: FP32 p (a ring of three buffers, mp_cur is
+  // Mixed-precision CG: FP32 p (a ring of buffers, mp_cur is
   // current; each w-step writes the next), r, w and
   // face coefficients; allocated by the first tea_hip_mpcg_init.
-  float* mp_p[kMpRing] = {nullptr, nullptr, nullptr};
+  float* mp_p[kMpRing] = {};
   int mp_cur = 0;
   // Up to two updates u += hold_alpha[i] p, p in mp_p[hold_buf[i]] (oldest
   // first), reported done to the host but held back (TEA_HIP_HOLD_U=0 turns
-  // this off): the four-cells-per-lane w-step that overwrites the oldest's
-  // p buffer reads both held p first and makes the held updates and its own
+  // this off): the third four-cells-per-lane w-step reads both held p and
+  // makes the held updates and its own
   // in one pass over u; any other entry point makes them first.
   bool hold_ok = true;
   int hold = 0;
@@ -927,18 +943,38 @@ struct tea_hip_chunk {
   double* w_alt = nullptr;
   tea::RaScalar ra_next;      // where the w-step after the r-step in flight
                               // takes its beta from
-  double* ra_dev = nullptr;   // device: [0] alpha, [1] beta, [2] r.r, then the
-                              // finisher's partials and its blocks-done count
-  unsigned* ra_count = nullptr;
+  double* ra_dev = nullptr;   // device: [0] alpha, [1] beta, [2] r.r
   double* ra_host = nullptr;  // pinned: 2 sets x {w-step, r-step} x {sum, ratio}
   double* ra_host_dev = nullptr;  // device view of ra_host
 
+  // Run-ahead of mixed-precision CG and FCG (mpcg.hip): one pass in flight
+  // beyond the one the host asked for (kMraNone, kMraR: the r-step, with FCG
+  // also z = M(r); kMraW: the w-step), into spare buffers.
+  int mra = 0;
+  bool mra_fcg = false;        // the pass belongs to FCG
+  int mra_coarse = 0;          // use_net of the last preconditioner call
+  int mra_fail = 0;            // consecutive mismatches (3 turn it off)
+  int mra_since = 0, mra_period = 0;  // r-steps since the last refresh, and
+                                      // how many the last two were apart
+  bool mra_synced = false;     // u_alt equals u outside the interior
+  double mra_alpha = 0.0;      // kMraR: the device's alpha
+  double mra_beta = 0.0;       // kMraW: the device's beta ...
+  double mra_pw = 0.0;         // the p.w the host was last given
+  MpStep mra_step;             // ... and the w-step in flight
+  tea::RaScalar mra_next;      // where the next w-step takes beta from
+  float* mp_r_alt = nullptr;
+  float* mp_w_alt = nullptr;
+  float* fcg_z_alt = nullptr;
+  double* mra_dev = nullptr;   // [0] alpha, [1] beta, [2] p.w
+  double* mra_host = nullptr;  // pinned: {w-step, r-step} x {sum, sum, scalar}
+  double* mra_host_dev = nullptr;
+
   // Waiting for a reduction by its values: launch_span_finish(..., poll)
-  // fills the first poll_len partials of arrays 0 .. poll_nr-1 with a
-  // sentinel, and the finish waits until the finisher has overwritten them
-  // all (or the stream is idle).
+  // fills the first partial of arrays 0 .. poll_nr-1 with a sentinel, and the
+  // finish waits until the finisher has overwritten them all (or the stream
+  // is idle).
   bool poll = true;
-  int poll_nr = 0, poll_len = 0;
+  int poll_nr = 0;
 
   // A depth-1 reflective update also copies the cells of its face lines
   // beyond the ring (e.g. column h-1 at rows below h-1) from other cells
@@ -988,34 +1024,29 @@ int resolve_ready(tea_hip_chunk* c);
 // partials; results go to out[0..nr).
 int finish_reduction(tea_hip_chunk* c, int nr, double* out);
 
-// Combines the 8 block sums of each span in c->sub (nr dot products) into
-// the span's level-2 partials and runs the next tree pass over them, leaving
-// *len partials per dot product in c->partials.
-// The partials go to arrays slot .. slot + nr - 1 of c->partials.  With
-// poll (slot 0), the next finish waits for the values themselves instead of
-// the stream; only for a finish that follows with no other kernel writing
-// the partials in between.
-// The run-ahead's scalar, formed by the last block of the finisher once
-// every block's partial is in: the host's final tree passes (zero-padded
-// groups of 64, each by the reference's pairwise tree) over the grid's
-// partials give the sum; mode 0 (after a w-step) alpha = rro / sum into
-// ra[0]; mode 1 (after an r-step) beta = sum / rro into ra[1] and sum into
-// ra[2].  rro is ra[2] when from_dev, else the value.  The sum and the
-// scalar also go to out[0], out[1] (pinned host memory the host polls).
-// count is the blocks-done counter, zero between launches.
+// Finishes nr sums from their block sums (the first nr arrays of sub, c->sub
+// unless given), sum q into the first value of array slot + q of c->partials
+// (*len = 1).  With poll (slot 0), the next finish waits for the values
+// themselves instead of the stream; only for a finish that follows with no
+// other kernel writing the partials in between.
+// The run-ahead's scalar, formed by the finisher: mode 0 (after a w-step)
+// alpha = rro / sum into ra[0]; mode 1 (after an r-step) beta = sum / rro into
+// ra[1] and sum into ra[2].  rro is ra[2] when from_dev, else the value.  The
+// sum and the scalar also go to out[0], out[1] (pinned host memory the host
+// polls).
+// With two sums (mixed-precision CG, FCG): mode 0 alpha = sum1 / sum0 into
+// ra[0] and sum0 (p.w) into ra[2]; mode 1 beta = -sum1 / ra[2] into ra[1];
+// out holds both sums and the scalar.
 struct RaTail {
   double rro;
   int from_dev, mode;
   double* ra;
-  double* out;
-  unsigned* count;
 };
-// The finisher of one reduction (array 0 of sub) into dst, device memory
-// (ceil(nspan / 64) partials, 1 with a single span), with the run-ahead's
-// scalar (at most 64^2 partials); not waited for.
-int launch_span_finish_ra(tea_hip_chunk* c, double* dst, const RaTail& tail);
+// The finisher of nr sums (1 or 2) of c->sub with the run-ahead's scalar, into
+// out; not waited for.
+int launch_span_finish_ra(tea_hip_chunk* c, int nr, double* out, const RaTail& tail);
 int launch_span_finish(tea_hip_chunk* c, int nr, int* len, int slot = 0,
-                       bool poll = false);
+                       bool poll = false, const double* sub = nullptr);
 
 // finish_reduction over the first len partials of each array (len is what
 // launch_span_finish leaves).
@@ -1058,19 +1089,29 @@ int apply_pre_halo(tea_hip_chunk* c);
 // update before a step (pre_halo), a held-back PPCG inner step or Chebyshev
 // step and its held-back halo update (solvers.hip).
 int flush_held(tea_hip_chunk* c);
-// Mixed-precision residual update r -= alpha w with the partials of r.r
-// (and, with rw, of r.w as a second array) written to c->partials
-// (mpcg.hip); *len is the number left to finish in each.  Without finish
-// (four-cells-per-lane kernel only) the subtree sums stay in c->sub for the
-// caller's finisher.
-int launch_mp_r(tea_hip_chunk* c, double alpha, int* len, bool rw, bool finish = true);
-// The four-cells-per-lane w-step for the arguments a (p_old in
-// mp_p[mp_cur], p_new in mp_p[mp_next(mp_cur)]), timed as kernel kid, with
-// u += alpha p_old held back over two steps: held while fewer than two
-// are, made with the two held updates when the oldest one's p is this
-// step's p_new buffer; held updates that cannot ride along run first on
-// their own (mpcg.hip).
-int launch_mp_w4(tea_hip_chunk* c, MpArgs a, int kid);
+// A mixed-precision residual step: r_out = r - alpha w, r.r and, with rw, r.w.
+struct MpRStep {
+  const float* r;
+  float* r_out;
+  const float* w;
+  double alpha;
+  RaScalar sc;
+};
+// Launches it, its sums left in `sub` (pair and four-cell kernels; the first
+// two arrays) or, on the span kernels, its partials in c->partials (mpcg.hip).
+int launch_mp_r(tea_hip_chunk* c, const MpRStep& s, bool rw, double* sub);
+// The w-step and r-step of mixed-precision CG, and of FCG (fcg), with the
+// run-ahead (mpcg.hip).  The r-step returns r.r and r.w (z.w).
+int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta, int apply_p,
+              double* pw, double* pr);
+int mp_calc_r(tea_hip_chunk* c, bool fcg, double alpha, int use_net, double* rr, double* rx);
+// FCG's z = M(r) and z.w, the block sums in `sub` (pair and four-cell kernels;
+// fcg.hip).
+int launch_fcg_z(tea_hip_chunk* c, int use_net, const float* r, const float* w, float* z,
+                 double* sub);
+// The same on any kernels with the partials of z.w in array `slot` of
+// c->partials; *len is the number left to finish (fcg.hip).
+int launch_precondition(tea_hip_chunk* c, int use_net, int slot, int* len);
 // Makes the held-back u updates on their own, oldest first (mpcg.hip).
 int apply_mp_hold(tea_hip_chunk* c);
 
@@ -1081,6 +1122,8 @@ int launch_halos(tea_hip_chunk* c, int depth, const int neighbours[4],
 // Drops a run-ahead of the fused CG iteration (cg.hip): it wrote only
 // spare buffers and device scalars, so nothing is undone.
 int ra_discard(tea_hip_chunk* c);
+// The same for a pass of mixed-precision CG or FCG in flight (mpcg.hip).
+int mra_discard(tea_hip_chunk* c);
 
 // Checks the handle and makes its device current, leaving a run-ahead in
 // flight (the CG entry points that can take it over); applies a held-back
@@ -1088,6 +1131,8 @@ int ra_discard(tea_hip_chunk* c);
 #define TEA_ENTER_RA(c)                                   \
   TEA_CHECK_ARG((c) != nullptr, "null chunk handle");     \
   TEA_HIP_TRY(hipSetDevice((c)->device));                 \
+  if ((c)->mra) TEA_RETURN_IF(::tea::mra_discard(c));     \
+  (c)->mra_synced = false;                                \
   if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c))
 
 // Checks the handle and makes its device current (entry points); drops a
@@ -1101,11 +1146,13 @@ int ra_discard(tea_hip_chunk* c);
 // and apply a held-back mixed-precision u update.
 #define TEA_FLUSH_HELD(c)                                                  \
   do {                                                                     \
+    if ((c)->mra) TEA_RETURN_IF(::tea::mra_discard(c));                    \
     if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c));                 \
     TEA_FLUSH_HELD_KEEP_U(c);                                              \
   } while (0)
 
-// TEA_FLUSH_HELD leaving a held-back mixed-precision u update held: for the
+// TEA_FLUSH_HELD leaving a held-back mixed-precision u update held and a
+// mixed-precision pass in flight: for the
 // mixed-precision and FCG steps, which touch neither u nor the held p.
 #define TEA_FLUSH_HELD_KEEP_U(c)                                           \
   do {                                                                     \
