@@ -671,14 +671,7 @@ int launch_each(tea_hip_chunk* c, int kid, const Body& body) {
 
 template <class Body>
 int launch_span1(tea_hip_chunk* c, int kid, const Body& body, double* out) {
-  {
-    Timed t(c, kid);
-    hipLaunchKernelGGL((span_kernel<1, Body>), span_grid(c), dim3(kBlock), 0,
-                       c->stream, c->geo, body, c->partials, c->nspan,
-                       c->ngroup == 1 ? 1 : 0);
-  }
-  TEA_HIP_TRY(hipGetLastError());
-  return finish_reduction(c, 1, out);
+  return sum_over_cells<1>(c, kid, body, out);
 }
 
 // Makes the second p buffer's cells outside the interior and the halo ring

@@ -327,7 +327,8 @@ int launch_span_finish(tea_hip_chunk* c, int nr, int* len, int slot, bool poll,
   Timed t(c, K_SPAN_FINISH);
   const auto launch = nr == 1   ? launch_finish<1, false>
                       : nr == 2 ? launch_finish<2, false>
-                                : launch_finish<3, false>;
+                      : nr == 3 ? launch_finish<3, false>
+                                : launch_finish<4, false>;
   launch(c, sub, c->partials + (size_t)slot * c->nspan, c->nspan, RaTail{});
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;

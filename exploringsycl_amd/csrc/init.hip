@@ -427,15 +427,8 @@ int tea_hip_field_summary(tea_hip_chunk* c, double* vol, double* mass,
   double** f = c->field;
   SummaryBody body{f[TEA_FIELD_VOLUME], f[TEA_FIELD_DENSITY],
                    f[TEA_FIELD_ENERGY0], f[TEA_FIELD_U]};
-  {
-    Timed t(c, K_FIELD_SUMMARY);
-    hipLaunchKernelGGL((span_kernel<4, SummaryBody>), span_grid(c),
-                       dim3(kBlock), 0, c->stream, c->geo, body, c->partials,
-                       c->nspan, c->ngroup == 1 ? 1 : 0);
-  }
-  TEA_HIP_TRY(hipGetLastError());
   double out[4];
-  TEA_RETURN_IF(finish_reduction(c, 4, out));
+  TEA_RETURN_IF(sum_over_cells<4>(c, K_FIELD_SUMMARY, body, out));
   *vol = out[0];
   *mass = out[1];
   *ie = out[2];

@@ -1159,17 +1159,14 @@ int tea_hip_mpcg_init(tea_hip_chunk* c, int coefficient, double rx, double ry,
                        c->stream, g.n, f[TEA_FIELD_KX], f[TEA_FIELD_KY],
                        f[TEA_FIELD_P], f[TEA_FIELD_R], c->mp_kx, c->mp_ky,
                        c->mp_p[0], c->mp_p[1], c->mp_p[2], c->mp_p[3], c->mp_r);
-    MpConvertBody body{f[TEA_FIELD_R], f[TEA_FIELD_U0]};
-    hipLaunchKernelGGL((span_kernel<2, MpConvertBody>), span_grid(c),
-                       dim3(kBlock), 0, c->stream, g, body, c->partials,
-                       c->nspan, c->ngroup == 1 ? 1 : 0);
   }
   TEA_HIP_TRY(hipGetLastError());
   c->mp_cur = 0;
   c->mra_synced = false;
   c->mra_fail = c->mra_since = 0;
   double out[2];
-  TEA_RETURN_IF(finish_reduction(c, 2, out));
+  TEA_RETURN_IF(sum_over_cells<2>(c, K_MP_CONVERT,
+                                  MpConvertBody{f[TEA_FIELD_R], f[TEA_FIELD_U0]}, out));
   *rr = out[0];
   *bb = out[1];
   return TEA_HIP_OK;

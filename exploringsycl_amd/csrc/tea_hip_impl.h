@@ -356,7 +356,7 @@ __device__ inline void st2_nt(float* p, int i, bool in0, bool in1, float v0,
 
 constexpr int kPairBlock = 2 * kBlock;              // 512 cells
 constexpr int kSubPerSpan = kSpan / kPairBlock;     // 8
-constexpr int kSubMaxNr = 3;                        // dot products per launch
+constexpr int kSubMaxNr = 4;                        // dot products per launch
 
 // Length of one dot product's block sums: the blocks rounded up to whole
 // groups of 512 (64 spans), the cells past the grid's blocks zero for good.
@@ -524,6 +524,7 @@ struct PairAt {
   int e;          // first cell
   bool valid;     // e < x*y
   bool in0, in1;  // interior cells
+  int kk, row;    // column and row of e
   int ic;         // e if valid, else a safe even index (safe_pair)
   int ir;         // e if either cell is interior, else the safe index
 };
@@ -532,10 +533,10 @@ __device__ inline PairAt pair_at(const Geo& g, int e) {
   PairAt q;
   q.e = e;
   q.valid = e < g.n;
-  const int row = q.valid ? (int)g.dx.div((uint32_t)e) : 0;
-  const int kk = e - row * g.x;
-  q.in0 = q.valid && interior(g, kk, row);
-  q.in1 = q.valid && interior(g, kk + 1, row);
+  q.row = q.valid ? (int)g.dx.div((uint32_t)e) : 0;
+  q.kk = e - q.row * g.x;
+  q.in0 = q.valid && interior(g, q.kk, q.row);
+  q.in1 = q.valid && interior(g, q.kk + 1, q.row);
   q.ic = q.valid ? e : safe_pair(g.x);
   q.ir = (q.in0 || q.in1) ? e : safe_pair(g.x);
   return q;
@@ -584,6 +585,24 @@ __global__ __launch_bounds__(kBlock) void span_kernel(Geo g, Body body,
     for (int q = 0; q < NR; ++q) v[q][k] = out[q];
   }
   span_reduce<NR>(v, partials, nspan, span, single_group != 0);
+}
+
+// The same sums with one cell pair per thread and the block's sums in sub (for
+// a finisher): 16 cells' values of four sums per thread did not fit in
+// registers (528 bytes of scratch per lane: 290 us for the field summary at
+// 4096^2, and a 140 us wait for the scratch memory before it at any size).
+template <int NR, class Body>
+__global__ __launch_bounds__(kBlock) void pair_sum_kernel(Geo g, Body body, double* sub,
+                                                          int nblk) {
+  const PairAt q = pair_at(g, blockIdx.x * kPairBlock + 2 * threadIdx.x);
+  double a[NR], b[NR];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) a[k] = b[k] = 0.0;
+  if (q.in0) body(q.e, q.kk, q.row, a);
+  if (q.in1) body(q.e + 1, q.kk + 1, q.row, b);
+#pragma unroll
+  for (int k = 0; k < NR; ++k) a[k] = a[k] + b[k];
+  block_sums_pairs<NR>(a, sub, nblk, blockIdx.x, threadIdx.x);
 }
 
 // One thread per cell of the padded x*y range.
@@ -1071,6 +1090,31 @@ inline bool use_pair_blocks(const tea_hip_chunk* c, int kernel_bit) {
 // results bit for bit) apply where those do and x is a multiple of 4.
 inline bool use_quad_blocks(const tea_hip_chunk* c, int kernel_bit) {
   return c->quads && use_pair_blocks(c, kernel_bit);
+}
+
+// A body's NR sums over the interior, to out: one pair per thread and a
+// finisher where the pair kernels apply, else one block per span and the
+// host's passes.
+template <int NR, class Body>
+int sum_over_cells(tea_hip_chunk* c, int kid, const Body& body, double* out) {
+  if (use_pair_blocks(c, 1)) {
+    {
+      Timed t(c, kid);
+      hipLaunchKernelGGL((pair_sum_kernel<NR, Body>), dim3(c->nblk), dim3(kBlock), 0, c->stream,
+                         c->geo, body, c->sub, c->nblk);
+    }
+    TEA_HIP_TRY(hipGetLastError());
+    int len;
+    TEA_RETURN_IF(launch_span_finish(c, NR, &len, 0, true));
+    return finish_reduction_n(c, NR, len, out);
+  }
+  {
+    Timed t(c, kid);
+    hipLaunchKernelGGL((span_kernel<NR, Body>), dim3(c->nspan), dim3(kBlock), 0, c->stream,
+                       c->geo, body, c->partials, c->nspan, c->ngroup == 1 ? 1 : 0);
+  }
+  TEA_HIP_TRY(hipGetLastError());
+  return finish_reduction(c, NR, out);
 }
 
 // Kinds of held-back step.
