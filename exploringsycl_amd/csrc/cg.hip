@@ -835,7 +835,7 @@ int ra_discard(tea_hip_chunk* c) {
 }
 
 int apply_pending(tea_hip_chunk* c) {
-  if (c->mra) TEA_RETURN_IF(mra_discard(c));
+  TEA_RETURN_IF(mra_discard(c));
   c->mra_synced = false;
   TEA_RETURN_IF(apply_cg_pending(c));
   return flush_held(c);

@@ -1827,7 +1827,7 @@ int tea_hip_fcg_precondition(tea_hip_chunk* c, int use_net, double* zw) {
   TEA_CHECK_ARG(!use_net || c->fcg_levels > 0, "no coarse correction attached");
   TEA_HIP_TRY(hipSetDevice(c->device));
   TEA_FLUSH_HELD_KEEP_U(c);
-  if (c->mra) TEA_RETURN_IF(mra_discard(c));
+  TEA_RETURN_IF(mra_discard(c));
   c->mra_coarse = use_net;
   int len;
   TEA_RETURN_IF(launch_precondition(c, use_net, 0, &len));

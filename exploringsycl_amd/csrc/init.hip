@@ -301,7 +301,7 @@ int launch_halos(tea_hip_chunk* c, int depth, const int neighbours[4],
     c->faces_ok_u |= fields[TEA_HALO_U] != 0;
     c->faces_ok_p |= fields[TEA_HALO_P] != 0;
   }
-  if (c->mra) TEA_RETURN_IF(mra_discard(c));
+  TEA_RETURN_IF(mra_discard(c));
   c->mra_synced = false;
   const long items = 2L * g.y * depth + 2L * g.x * depth;
   {

@@ -286,8 +286,9 @@ __device__ inline void mp_pair_compute(const Geo& g, const MpArgs& a,
   st2(a.w, i, s.in0, s.in1, sa, sb);
   double ua = 0.0, ub = 0.0;
   if (a.apply_u) {
-    ua = s.U.x + a.alpha * (double)s.P0.x;
-    ub = s.U.y + a.alpha * (double)s.P0.y;
+    const double alpha = a.alpha_dev ? *a.alpha_dev : a.alpha;
+    ua = s.U.x + alpha * (double)s.P0.x;
+    ub = s.U.y + alpha * (double)s.P0.y;
     st2_nt(a.u_out, i, s.in0, s.in1, ua, ub);
   }
   if (a.apply_p) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb);
@@ -338,8 +339,12 @@ __device__ inline double mp_scalar(const RaScalar& s, double value) {
   if (!CONSUME) return s.dev ? *s.dev : value;
   double v[2];
   consume_sums<2>(s.sub, s.nblk, v);
-  const double q = s.inverse ? -v[1] / s.rro : v[1] / v[0];
+  const double q = s.inverse ? -v[1] / *s.rro_dev : v[1] / v[0];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (s.sum_dev) {
+      s.sum_dev[0] = q;
+      s.sum_dev[2] = v[0];
+    }
     s.out[0] = v[0];
     s.out[1] = v[1];
     s.out[2] = q;
@@ -526,10 +531,11 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
       u0[2] = u0[2] + a.alpha_h2 * (double)GB.x;
       u0[3] = u0[3] + a.alpha_h2 * (double)GB.y;
     }
-    const double un[4] = {u0[0] + a.alpha * (double)(hi ? az : ax),
-                          u0[1] + a.alpha * (double)(hi ? aw : ay),
-                          u0[2] + a.alpha * (double)(hi ? bz : bx),
-                          u0[3] + a.alpha * (double)(hi ? bw : by)};
+    const double alpha = a.alpha_dev ? *a.alpha_dev : a.alpha;
+    const double un[4] = {u0[0] + alpha * (double)(hi ? az : ax),
+                          u0[1] + alpha * (double)(hi ? aw : ay),
+                          u0[2] + alpha * (double)(hi ? bz : bx),
+                          u0[3] + alpha * (double)(hi ? bw : by)};
     if (inA0 || inA1) st2_nt(a.u_out, ua, inA0, inA1, un[0], un[1]);
     if (inB0 || inB1) st2_nt(a.u_out, ub, inB0, inB1, un[2], un[3]);
     // Halo ring of boundary-adjacent cells (rare; per cell).
@@ -795,7 +801,7 @@ int ensure_mp_buffers(tea_hip_chunk* c) {
 }  // namespace
 
 int apply_mp_hold(tea_hip_chunk* c) {
-  if (c->mra) TEA_RETURN_IF(mra_discard(c));
+  TEA_RETURN_IF(mra_discard(c));
   const int n = c->hold;
   c->hold = 0;
   for (int i = 0; i < n; ++i) {
@@ -813,20 +819,20 @@ int apply_mp_hold(tea_hip_chunk* c) {
 //
 // As for FP64 CG (cg.hip): the host turns p.w and p.r into alpha and the
 // r-step's sums into beta before it can ask for the next pass, two round
-// trips per iteration (about 6 us each).  So each call queues the next pass
-// behind its own before it waits for its own sums: calc_w the r-step (with
-// FCG also z = M(r)), calc_r the w-step, into spare r, z, w and u buffers and
-// a p buffer of the ring that no held update needs, with the scalar formed on
-// the device.  The host's next call takes the pass over when its arguments
-// are bitwise what the pass used; any other call drops it, and only spare
-// buffers were written.  Each scalar is formed by the next pass itself on
-// grids of at most kConsumeBlocks blocks, else by the finisher's last block.
-// A w-step is not queued where the driver refreshed after as many iterations
-// the last time (the refresh would drop it).
+// trips per iteration (about 6 us each).  So calc_w leaves the r-step (with FCG
+// also z = M(r)) and the next w-step queued behind its own pass, and calc_r
+// the r-step after that: two passes, because a pass of a small grid (3-6 us)
+// is over before the host has seen its scalar and launched another.  They
+// write spare r, z, w and u buffers and a p buffer of the ring that no held
+// update needs, and take alpha and beta from the device.  The host's next
+// call takes a pass over when its arguments are bitwise what the pass used;
+// any other call drops both, and only spare buffers were written.  Each scalar
+// is formed by the next pass itself on grids of at most kConsumeBlocks
+// blocks, else by a finisher.  Nothing is queued past the r-step after which
+// the driver refreshed the last time (the refresh would drop it).
 
 namespace {
 
-constexpr int kMraNone = 0, kMraR = 1, kMraW = 2;
 constexpr int kMraSlotW = 0, kMraSlotR = 1;
 
 bool mra_consume(const tea_hip_chunk* c) { return c->nblk <= kConsumeBlocks; }
@@ -837,7 +843,7 @@ bool mra_possible(const tea_hip_chunk* c) {
 }
 
 void mra_mismatch(tea_hip_chunk* c) {
-  c->mra = kMraNone;
+  c->mra_r = c->mra_w = false;
   c->ra_dirty = true;
   c->mra_fail += 1;
 }
@@ -862,7 +868,7 @@ int ensure_mra(tea_hip_chunk* c) {
     return TEA_HIP_ENOMEM;
   }
   double* host = nullptr;
-  if (hipHostMalloc(&host, 8 * sizeof(double),
+  if (hipHostMalloc(&host, 16 * sizeof(double),
                     hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
     set_error("hipHostMalloc of the run-ahead slots failed");
     return TEA_HIP_ENOMEM;
@@ -872,29 +878,46 @@ int ensure_mra(tea_hip_chunk* c) {
   return TEA_HIP_OK;
 }
 
-// Arms a step's host slot and sets *sc to where the next pass takes the
-// step's scalar from (launching the finisher where there is one).
-int mra_finish(tea_hip_chunk* c, int slot, RaScalar* sc) {
+// Offset of a slot in mra_host.
+int mra_slot(int kind, int i) { return 4 * (2 * kind + i); }
+
+// Arms a step's host slot for the pass or finisher about to be launched.
+int mra_arm(tea_hip_chunk* c, int kind, int i) {
   if (c->ra_dirty) {
     // A dropped pass may still be queued and write these slots.
     TEA_HIP_TRY(hipStreamSynchronize(c->stream));
     c->ra_dirty = false;
   }
-  arm_host_values(c->mra_host + 4 * slot, 3);
-  *sc = RaScalar{};
-  sc->out = c->mra_host_dev + 4 * slot;
-  if (mra_consume(c)) {
-    sc->sub = slot == kMraSlotW ? c->sub : c->sub2;
-    sc->nblk = c->nblk;
-    sc->inverse = slot == kMraSlotW ? 0 : 1;
-    return TEA_HIP_OK;
-  }
-  sc->dev = c->mra_dev + slot;
-  return launch_span_finish_ra(c, 2, sc->out, RaTail{0.0, 1, slot, c->mra_dev});
+  arm_host_values(c->mra_host + mra_slot(kind, i), 3);
+  return TEA_HIP_OK;
 }
 
-int mra_wait(tea_hip_chunk* c, int slot, double* s0, double* s1, double* scalar) {
-  const double* h = c->mra_host + 4 * slot;
+// Where the pass after a w-step (kind W) or r-step takes its scalar from.
+RaScalar mra_scalar(const tea_hip_chunk* c, int kind, int i) {
+  RaScalar sc;
+  sc.out = c->mra_host_dev + mra_slot(kind, i);
+  if (!mra_consume(c)) {
+    sc.dev = c->mra_dev + kind;
+    return sc;
+  }
+  sc.sub = kind == kMraSlotW ? c->sub : c->sub2;
+  sc.nblk = c->nblk;
+  sc.inverse = kind == kMraSlotW ? 0 : 1;
+  sc.rro_dev = c->mra_dev + 2;
+  sc.sum_dev = kind == kMraSlotW ? c->mra_dev : nullptr;
+  return sc;
+}
+
+// The finisher of a w-step or r-step just queued (larger grids).
+int mra_finish(tea_hip_chunk* c, int kind, int i) {
+  if (mra_consume(c)) return TEA_HIP_OK;
+  TEA_RETURN_IF(mra_arm(c, kind, i));
+  return launch_span_finish_ra(c, 2, c->mra_host_dev + mra_slot(kind, i),
+                               RaTail{0.0, 1, kind, c->mra_dev});
+}
+
+int mra_wait(tea_hip_chunk* c, int kind, int i, double* s0, double* s1, double* scalar) {
+  const double* h = c->mra_host + mra_slot(kind, i);
   TEA_RETURN_IF(wait_host_values(c, h, 3));
   *s0 = h[0];
   *s1 = h[1];
@@ -904,7 +927,9 @@ int mra_wait(tea_hip_chunk* c, int slot, double* s0, double* s1, double* scalar)
 
 // The w-step of a call with these arguments.  u += alpha p_old is held back
 // over two steps (four cells per lane); held updates that cannot ride along
-// are made on their own first.  Running ahead, w and u go to the spares.
+// are made on their own first.  Running ahead (behind the r-step in flight),
+// it reads the spare r or z, writes the spare w and u, and takes alpha from
+// the device; commit_mp_step is given it.
 int plan_mp_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta, int apply_p,
               bool ahead, MpStep* s) {
   const bool ride = c->quads && apply_u && apply_p;
@@ -912,10 +937,12 @@ int plan_mp_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
   const int cur = c->mp_cur;
   double* u = c->field[TEA_FIELD_U];
   *s = MpStep{};
-  s->a = MpArgs{c->mp_p[cur], c->mp_p[mp_next(cur)], fcg ? c->fcg_z : c->mp_r, u,
-                ahead ? c->mp_w_alt : c->mp_w, c->mp_kx, c->mp_ky, c->mp_r, alpha, beta,
+  const float* r = ahead ? c->mp_r_alt : c->mp_r;
+  const float* z = ahead ? c->fcg_z_alt : c->fcg_z;
+  s->a = MpArgs{c->mp_p[cur], c->mp_p[mp_next(cur)], fcg ? z : r, u,
+                ahead ? c->mp_w_alt : c->mp_w, c->mp_kx, c->mp_ky, r, alpha, beta,
                 apply_u ? 1 : 0, apply_p ? 1 : 0, nullptr, nullptr, 0.0, 0.0,
-                ahead ? c->u_alt : u};
+                ahead ? c->u_alt : u, ahead ? c->mra_dev : nullptr};
   s->um = apply_u ? 1 : 0;
   if (!ride || !c->hold_ok) return TEA_HIP_OK;
   if (c->hold == 2) {
@@ -934,7 +961,6 @@ int plan_mp_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
     s->hold_alpha[i] = c->hold_alpha[i];
   }
   s->hold_buf[c->hold] = cur;
-  s->hold_alpha[c->hold] = alpha;
   return TEA_HIP_OK;
 }
 
@@ -965,41 +991,61 @@ int launch_mp_step(tea_hip_chunk* c, const MpStep& s, bool fcg, const RaScalar& 
   return TEA_HIP_OK;
 }
 
-// The chunk's state once a w-step has been asked for (or taken over).
-void commit_mp_step(tea_hip_chunk* c, const MpStep& s) {
+// The chunk's state once a w-step has been asked for (or taken over) with
+// this alpha.
+void commit_mp_step(tea_hip_chunk* c, const MpStep& s, double alpha) {
+  const bool holds = s.um == 0 && s.hold > 0;
   c->hold = s.hold;
   for (int i = 0; i < s.hold; ++i) {
     c->hold_buf[i] = s.hold_buf[i];
-    c->hold_alpha[i] = s.hold_alpha[i];
+    c->hold_alpha[i] = holds && i == s.hold - 1 ? alpha : s.hold_alpha[i];
   }
   if (s.um && s.a.u_out != s.a.u) swap_buf(c->field[TEA_FIELD_U], c->u_alt);
   if (s.a.w != c->mp_w) swap_buf(c->mp_w, c->mp_w_alt);
   if (s.a.apply_p) c->mp_cur = mp_next(c->mp_cur);
 }
 
-// Queues the r-step (with FCG also z = M(r)) behind the w-step whose sums are
-// in c->sub, then waits for that w-step's sums.
-int mra_queue_r(tea_hip_chunk* c, bool fcg, double* pw, double* pr) {
-  RaScalar sc;
-  TEA_RETURN_IF(mra_finish(c, kMraSlotW, &sc));
+// Queues the r-step (with FCG also z = M(r)) behind the newest w-step.
+int mra_queue_r(tea_hip_chunk* c, bool fcg) {
   double* sub = mra_consume(c) ? c->sub2 : c->sub;
-  TEA_RETURN_IF(launch_mp_r(c, MpRStep{c->mp_r, c->mp_r_alt, c->mp_w, 0.0, sc}, !fcg, sub));
+  const float* w = c->mra_w ? c->mp_w_alt : c->mp_w;
+  if (mra_consume(c)) TEA_RETURN_IF(mra_arm(c, kMraSlotW, c->mra_wi));
+  const RaScalar sc = mra_scalar(c, kMraSlotW, c->mra_wi);
+  TEA_RETURN_IF(launch_mp_r(c, MpRStep{c->mp_r, c->mp_r_alt, w, 0.0, sc}, !fcg, sub));
   if (fcg)
-    TEA_RETURN_IF(launch_fcg_z(c, c->mra_coarse, c->mp_r_alt, c->mp_w, c->fcg_z_alt,
+    TEA_RETURN_IF(launch_fcg_z(c, c->mra_coarse, c->mp_r_alt, w, c->fcg_z_alt,
                                sub + sub_stride(c->nblk)));
-  TEA_RETURN_IF(mra_finish(c, kMraSlotR, &c->mra_next));
-  c->mra = kMraR;
+  c->mra_ri ^= 1;
+  TEA_RETURN_IF(mra_finish(c, kMraSlotR, c->mra_ri));
+  c->mra_r = true;
   c->mra_fcg = fcg;
-  TEA_RETURN_IF(mra_wait(c, kMraSlotW, pw, pr, &c->mra_alpha));
-  c->mra_pw = *pw;
+  return TEA_HIP_OK;
+}
+
+// Queues the next w-step behind the r-step in flight.
+int mra_queue_w(tea_hip_chunk* c, bool fcg) {
+  if (!c->mra_synced) {
+    // The spare u takes the cells outside the interior that no step writes.
+    TEA_HIP_TRY(hipMemcpyAsync(c->u_alt, c->field[TEA_FIELD_U],
+                               (size_t)c->geo.n * sizeof(double), hipMemcpyDeviceToDevice,
+                               c->stream));
+    c->mra_synced = true;
+  }
+  TEA_RETURN_IF(plan_mp_w(c, fcg, 0.0, 1, 0.0, 1, true, &c->mra_step));
+  if (mra_consume(c)) TEA_RETURN_IF(mra_arm(c, kMraSlotR, c->mra_ri));
+  TEA_RETURN_IF(
+      launch_mp_step(c, c->mra_step, fcg, mra_scalar(c, kMraSlotR, c->mra_ri)));
+  c->mra_wi ^= 1;
+  TEA_RETURN_IF(mra_finish(c, kMraSlotW, c->mra_wi));
+  c->mra_w = true;
   return TEA_HIP_OK;
 }
 
 }  // namespace
 
 int mra_discard(tea_hip_chunk* c) {
-  if (c->mra != kMraNone) {
-    c->mra = kMraNone;
+  if (c->mra_r || c->mra_w) {
+    c->mra_r = c->mra_w = false;
     c->ra_dirty = true;
   }
   return TEA_HIP_OK;
@@ -1007,31 +1053,34 @@ int mra_discard(tea_hip_chunk* c) {
 
 int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta, int apply_p,
               double* pw, double* pr) {
-  if (c->mra == kMraW && c->mra_fcg == fcg && apply_u && apply_p &&
-      alpha == c->mra_step.a.alpha && beta == c->mra_beta) {
-    commit_mp_step(c, c->mra_step);
-    c->mra = kMraNone;
-    c->mra_fail = 0;
-    return mra_queue_r(c, fcg, pw, pr);
-  }
-  if (c->mra) mra_mismatch(c);
+  const bool taken = c->mra_w && c->mra_fcg == fcg && apply_u && apply_p &&
+                     alpha == c->mra_alpha && beta == c->mra_beta;
+  if ((c->mra_r || c->mra_w) && !taken) mra_mismatch(c);
+  bool ahead = taken;
   int len = c->nspan;
-  if (use_pair_blocks(c, 1)) {
-    const bool ahead = mra_possible(c);
+  if (taken) {
+    commit_mp_step(c, c->mra_step, alpha);
+    c->mra_w = false;
+    c->mra_fail = 0;
+  } else if (use_pair_blocks(c, 1)) {
+    ahead = mra_possible(c);
     if (ahead) TEA_RETURN_IF(ensure_mra(c));
     MpStep s;
     TEA_RETURN_IF(plan_mp_w(c, fcg, alpha, apply_u, beta, apply_p, false, &s));
     TEA_RETURN_IF(launch_mp_step(c, s, fcg, RaScalar{}));
-    commit_mp_step(c, s);
-    if (ahead) return mra_queue_r(c, fcg, pw, pr);
-    TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true));
+    commit_mp_step(c, s, alpha);
+    if (!ahead) TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true));
+    if (ahead) {
+      c->mra_wi ^= 1;
+      TEA_RETURN_IF(mra_finish(c, kMraSlotW, c->mra_wi));
+    }
   } else {
     if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
     const int cur = c->mp_cur, sg = c->ngroup == 1 ? 1 : 0;
     const MpArgs a{c->mp_p[cur], c->mp_p[mp_next(cur)], fcg ? c->fcg_z : c->mp_r,
                    c->field[TEA_FIELD_U], c->mp_w, c->mp_kx, c->mp_ky, c->mp_r, alpha, beta,
                    apply_u ? 1 : 0, apply_p ? 1 : 0, nullptr, nullptr, 0.0, 0.0,
-                   c->field[TEA_FIELD_U]};
+                   c->field[TEA_FIELD_U], nullptr};
     {
       Timed t(c, fcg ? K_FCG_W : K_MP_W);
       if (c->pairs)
@@ -1043,6 +1092,12 @@ int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
     }
     TEA_HIP_TRY(hipGetLastError());
     if (apply_p) c->mp_cur = mp_next(cur);
+  }
+  if (ahead) {
+    const int slot = c->mra_wi;
+    if (!c->mra_r) TEA_RETURN_IF(mra_queue_r(c, fcg));
+    if (c->mra_since + 1 != c->mra_period) TEA_RETURN_IF(mra_queue_w(c, fcg));
+    return mra_wait(c, kMraSlotW, slot, pw, pr, &c->mra_alpha);
   }
   double out[2];
   TEA_RETURN_IF(finish_reduction_n(c, 2, len, out));
@@ -1076,28 +1131,17 @@ int launch_mp_r(tea_hip_chunk* c, const MpRStep& s, bool rw, double* sub) {
 
 int mp_calc_r(tea_hip_chunk* c, bool fcg, double alpha, int use_net, double* rr, double* rx) {
   c->mra_since += 1;
-  if (c->mra == kMraR && c->mra_fcg == fcg && alpha == c->mra_alpha &&
+  if (c->mra_r && c->mra_fcg == fcg && alpha == c->mra_alpha &&
       (!fcg || use_net == c->mra_coarse)) {
     swap_buf(c->mp_r, c->mp_r_alt);
     if (fcg) swap_buf(c->fcg_z, c->fcg_z_alt);
-    c->mra = kMraNone;
+    c->mra_r = false;
     c->mra_fail = 0;
-    if (mra_possible(c) && c->mra_since != c->mra_period) {
-      if (!c->mra_synced) {
-        // The spare u takes the cells outside the interior that no step writes.
-        TEA_HIP_TRY(hipMemcpyAsync(c->u_alt, c->field[TEA_FIELD_U],
-                                   (size_t)c->geo.n * sizeof(double), hipMemcpyDeviceToDevice,
-                                   c->stream));
-        c->mra_synced = true;
-      }
-      TEA_RETURN_IF(plan_mp_w(c, fcg, alpha, 1, 0.0, 1, true, &c->mra_step));
-      RaScalar sc = c->mra_next;
-      sc.rro = c->mra_pw;
-      TEA_RETURN_IF(launch_mp_step(c, c->mra_step, fcg, sc));
-      c->mra = kMraW;
-      return mra_wait(c, kMraSlotR, rr, rx, &c->mra_beta);
-    }
-    if (!mra_consume(c)) return mra_wait(c, kMraSlotR, rr, rx, &c->mra_beta);
+    const int slot = c->mra_ri;
+    if (c->mra_w) TEA_RETURN_IF(mra_queue_r(c, fcg));
+    if (c->mra_w || !mra_consume(c))
+      return mra_wait(c, kMraSlotR, slot, rr, rx, &c->mra_beta);
+    // No w-step behind it to form the sums.
     int len;
     double out[2];
     TEA_RETURN_IF(launch_span_finish(c, 2, &len, 0, true, c->sub2));
@@ -1106,7 +1150,7 @@ int mp_calc_r(tea_hip_chunk* c, bool fcg, double alpha, int use_net, double* rr,
     *rx = out[1];
     return TEA_HIP_OK;
   }
-  if (c->mra) mra_mismatch(c);
+  if (c->mra_r || c->mra_w) mra_mismatch(c);
   if (fcg) c->mra_coarse = use_net;
   const MpRStep s{c->mp_r, c->mp_r, c->mp_w, alpha, RaScalar{}};
   double out[2];

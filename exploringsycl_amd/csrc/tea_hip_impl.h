@@ -694,6 +694,8 @@ struct MpArgs {
   // Pair-per-thread and four-cell kernels: the new u goes to u_out (u, or a
   // spare buffer when the iteration runs ahead).
   double* u_out;
+  // Those kernels only: the alpha of u's update, where the device has it.
+  const double* alpha_dev;
 };
 
 // Where a pass of the iteration takes its scalar from: the host's value
@@ -711,6 +713,7 @@ struct RaScalar {
   double rro = 0.0;
   const double* rro_dev = nullptr;
   double* sum_dev = nullptr;  // set by the w-step: r.r, the next alpha's rro
+                              // (two sums: set by the r-step, alpha and p.w)
   double* out = nullptr;      // host slot {sum(s), scalar}
 };
 
@@ -966,26 +969,27 @@ struct tea_hip_chunk {
   double* ra_host = nullptr;  // pinned: 2 sets x {w-step, r-step} x {sum, ratio}
   double* ra_host_dev = nullptr;  // device view of ra_host
 
-  // Run-ahead of mixed-precision CG and FCG (mpcg.hip): one pass in flight
-  // beyond the one the host asked for (kMraNone, kMraR: the r-step, with FCG
-  // also z = M(r); kMraW: the w-step), into spare buffers.
-  int mra = 0;
-  bool mra_fcg = false;        // the pass belongs to FCG
+  // Run-ahead of mixed-precision CG and FCG (mpcg.hip): up to two passes in
+  // flight beyond what the host asked for, the next r-step (mra_r; with FCG
+  // also z = M(r)) and the next w-step (mra_w), into spare buffers.
+  bool mra_r = false, mra_w = false;
+  bool mra_fcg = false;        // the passes belong to FCG
   int mra_coarse = 0;          // use_net of the last preconditioner call
   int mra_fail = 0;            // consecutive mismatches (3 turn it off)
   int mra_since = 0, mra_period = 0;  // r-steps since the last refresh, and
                                       // how many the last two were apart
+  int mra_wi = 0, mra_ri = 0;  // host slots of the newest w-step and r-step
   bool mra_synced = false;     // u_alt equals u outside the interior
-  double mra_alpha = 0.0;      // kMraR: the device's alpha
-  double mra_beta = 0.0;       // kMraW: the device's beta ...
-  double mra_pw = 0.0;         // the p.w the host was last given
-  MpStep mra_step;             // ... and the w-step in flight
-  tea::RaScalar mra_next;      // where the next w-step takes beta from
+  double mra_alpha = 0.0;      // the device's alpha of the last w-step the
+                               // host asked for
+  double mra_beta = 0.0;       // its beta of the last r-step
+  MpStep mra_step;             // the w-step in flight
   float* mp_r_alt = nullptr;
   float* mp_w_alt = nullptr;
   float* fcg_z_alt = nullptr;
   double* mra_dev = nullptr;   // [0] alpha, [1] beta, [2] p.w
-  double* mra_host = nullptr;  // pinned: {w-step, r-step} x {sum, sum, scalar}
+  double* mra_host = nullptr;  // pinned: {w-step, r-step} x 2 slots x {sum,
+                               // sum, scalar}
   double* mra_host_dev = nullptr;
 
   // Waiting for a reduction by its values: launch_span_finish(..., poll)
@@ -1175,7 +1179,7 @@ int mra_discard(tea_hip_chunk* c);
 #define TEA_ENTER_RA(c)                                   \
   TEA_CHECK_ARG((c) != nullptr, "null chunk handle");     \
   TEA_HIP_TRY(hipSetDevice((c)->device));                 \
-  if ((c)->mra) TEA_RETURN_IF(::tea::mra_discard(c));     \
+  TEA_RETURN_IF(::tea::mra_discard(c));                   \
   (c)->mra_synced = false;                                \
   if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c))
 
@@ -1190,7 +1194,7 @@ int mra_discard(tea_hip_chunk* c);
 // and apply a held-back mixed-precision u update.
 #define TEA_FLUSH_HELD(c)                                                  \
   do {                                                                     \
-    if ((c)->mra) TEA_RETURN_IF(::tea::mra_discard(c));                    \
+    TEA_RETURN_IF(::tea::mra_discard(c));                                  \
     if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c));                 \
     TEA_FLUSH_HELD_KEEP_U(c);                                              \
   } while (0)
