@@ -133,21 +133,6 @@ struct CalcPBody {  // cg.cpp:257-281
 // Together 11 words = 88 bytes per cell per iteration against the
 // reference's 13 (calc_w 4 + calc_ur 6 + calc_p 3).
 
-struct FusedWArgs {
-  const double* p_old;
-  double* p_new;
-  const double* r;
-  double* u;
-  double* w;
-  const double* kx;
-  const double* ky;
-  double alpha, beta;
-  int apply_u, ring;
-  // Pair-per-thread kernel only: the new u goes to u_out (u itself for the
-  // iteration the host asked for, a spare buffer when it runs ahead).
-  double* u_out;
-};
-
 template <bool CONSUME>
 __device__ inline double ra_scalar(const RaScalar& s, double value) {
   if (!CONSUME) return s.dev ? *s.dev : value;
@@ -156,7 +141,7 @@ __device__ inline double ra_scalar(const RaScalar& s, double value) {
   consume_sums<1>(s.sub, s.nblk, sum);
   const double q = s.inverse ? sum[0] / rro : rro / sum[0];
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    if (s.sum_dev) *s.sum_dev = sum[0];
+    if (s.sum_dev) *s.sum_dev = s.inverse ? sum[0] : q;
     s.out[0] = sum[0];
     s.out[1] = q;
   }
@@ -306,7 +291,7 @@ __device__ inline void span_reduce_pairs(double (&v)[kSlots], double* partials,
 struct FusedPair {
   int e0, kk, jj;
   bool in0, in1, any;
-  double2 P0, Pt, Pb, R0, Rt, Rb, KX, KY, KYt, U;
+  double2 P0, Pt, Pb, R0, Rt, Rb, KX, KY, KYt, U, H, H2;
   // Wave-edge neighbours: lane 0 holds p and r at e0 - 1, lane 63 p, r and
   // kx at e0 + 2 (the other lanes take theirs from adjacent lanes).
   double PN, RN, KXN;
@@ -325,7 +310,7 @@ __device__ inline void fused_pair_index(const Geo& g, int e, FusedPair& s) {
 // The pair's own p, r and kx are also the left/right neighbours the adjacent
 // lanes take by shuffle, so they are read whenever the pair is in range; the
 // rows above and below only for interior pairs.
-template <bool APPLY_P>
+template <bool APPLY_P, int UM>
 __device__ inline void fused_pair_load(const Geo& g, const FusedWArgs& a,
                                        FusedPair& s) {
   const int x = g.x;
@@ -344,7 +329,11 @@ __device__ inline void fused_pair_load(const Geo& g, const FusedWArgs& a,
   s.KX = ld2(a.kx, ic);
   s.KY = ld2(a.ky, ir);
   s.KYt = ld2u(a.ky, ir + x);
-  if (a.apply_u) s.U = ld2_nt(a.u, ir);
+  if (UM == 3 || (UM == 1 && a.apply_u)) s.U = ld2_nt(a.u, ir);
+  if (UM == 3) {
+    s.H = ld2_nt(a.p_h, ir);
+    s.H2 = ld2_nt(a.p_h2, ir);
+  }
   // Issued with the pair's own loads so the wave waits once; ir - 1 and
   // ir + 2 are in range (ir is an interior pair's index or the safe one).
   // Lanes 0 and 63 share each load instruction, at their own addresses
@@ -360,7 +349,7 @@ __device__ inline void fused_pair_load(const Geo& g, const FusedWArgs& a,
 
 // Computes and stores the pair (w, u, p_new and their halo ring) and returns
 // the in-lane pair sum of p_new . w (the first level of the reduction tree).
-template <bool APPLY_P>
+template <bool APPLY_P, int UM>
 __device__ inline double fused_pair_compute(const Geo& g, const FusedWArgs& a,
                                             const FusedPair& s, int lane, double beta) {
   const int x = g.x;
@@ -420,9 +409,17 @@ __device__ inline double fused_pair_compute(const Geo& g, const FusedWArgs& a,
   if (!s.any) return psum;
   st2(a.w, i, s.in0, s.in1, sa, sb);
   double ua = 0.0, ub = 0.0;
-  if (a.apply_u) {
-    ua = s.U.x + a.alpha * s.P0.x;
-    ub = s.U.y + a.alpha * s.P0.y;
+  const bool apply_u = UM == 3 || (UM == 1 && a.apply_u);
+  if (apply_u) {
+    const double alpha = a.alpha_dev ? *a.alpha_dev : a.alpha;
+    ua = s.U.x;
+    ub = s.U.y;
+    if (UM == 3) {
+      ua = (ua + a.alpha_h * s.H.x) + a.alpha_h2 * s.H2.x;
+      ub = (ub + a.alpha_h * s.H.y) + a.alpha_h2 * s.H2.y;
+    }
+    ua = ua + alpha * s.P0.x;
+    ub = ub + alpha * s.P0.y;
     st2_nt(a.u_out, i, s.in0, s.in1, ua, ub);
   }
   if (APPLY_P) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb);
@@ -434,7 +431,7 @@ __device__ inline double fused_pair_compute(const Geo& g, const FusedWArgs& a,
     const int ic = i + c, kc = ka + c;
     if (!(c == 0 ? s.in0 : s.in1) || !(kc == xl || kc == xr || row == yb || row == yt)) continue;
     if (a.ring) {
-      if (a.apply_u) ring_store(a.u_out, ic, kc, row, x, xl, xr, yb, yt, c == 0 ? ua : ub);
+      if (apply_u) ring_store(a.u_out, ic, kc, row, x, xl, xr, yb, yt, c == 0 ? ua : ub);
       if (APPLY_P) ring_store(a.p_new, ic, kc, row, x, xl, xr, yb, yt, c == 0 ? ca : cb);
       continue;
     }
@@ -442,7 +439,7 @@ __device__ inline double fused_pair_compute(const Geo& g, const FusedWArgs& a,
       for (int dk = kc == xl ? -1 : 0; dk <= (kc == xr ? 1 : 0); ++dk) {
         if (dj == 0 && dk == 0) continue;
         const int q = ic + dj * x + dk;
-        if (a.apply_u && a.u_out != a.u) a.u_out[q] = a.u[q];
+        if (apply_u && a.u_out != a.u) a.u_out[q] = a.u[q];
         if (APPLY_P) a.p_new[q] = P[q];
       }
   }
@@ -466,10 +463,10 @@ __global__ __launch_bounds__(kBlock) void fused_w2_kernel(Geo g, FusedWArgs a,
     for (int j = 0; j < SB; ++j)
       fused_pair_index(g, base + (s0 + j) * (2 * kBlock) + 2 * threadIdx.x, s[j]);
 #pragma unroll
-    for (int j = 0; j < SB; ++j) fused_pair_load<APPLY_P>(g, a, s[j]);
+    for (int j = 0; j < SB; ++j) fused_pair_load<APPLY_P, 1>(g, a, s[j]);
 #pragma unroll
     for (int j = 0; j < SB; ++j)
-      psum[s0 + j] = fused_pair_compute<APPLY_P>(g, a, s[j], lane, a.beta);
+      psum[s0 + j] = fused_pair_compute<APPLY_P, 1>(g, a, s[j], lane, a.beta);
   }
   span_reduce_pairs(psum, partials, nspan, span, single_group != 0);
 }
@@ -478,7 +475,12 @@ __global__ __launch_bounds__(kBlock) void fused_w2_kernel(Geo g, FusedWArgs a,
 // reduction tree) and stores their 8-leaf subtree sum.  Small blocks
 // keep 4x more waves per SIMD in flight than the span-per-block kernel.
 // With CONSUME beta is formed from the sums of the r-step before it.
-template <bool APPLY_P, int KS, bool CONSUME = false>
+// UM: 0 leaves u alone, 1 adds alpha p_old where a.apply_u, 3 the two held
+// updates and its own, each rounded as when made one by one.  u's read and
+// write are 16 of the pass's 64 bytes per cell; with two passes of three
+// leaving it to the third they move 48, 48 and 80 (the third also reads the
+// two held p).
+template <bool APPLY_P, int KS, int UM, bool CONSUME>
 __global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs a, RaScalar sc,
                                                                double* sub, int nblk, int S) {
   int tid;
@@ -486,9 +488,9 @@ __global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs
   const int lane = threadIdx.x & (kWave - 1);
   FusedPair s;
   fused_pair_index(g, blk < nblk ? blk * kPairBlock + 2 * tid : g.n, s);
-  fused_pair_load<APPLY_P>(g, a, s);
+  fused_pair_load<APPLY_P, UM>(g, a, s);
   const double beta = ra_scalar<CONSUME>(sc, a.beta);
-  const double v[1] = {fused_pair_compute<APPLY_P>(g, a, s, lane, beta)};
+  const double v[1] = {fused_pair_compute<APPLY_P, UM>(g, a, s, lane, beta)};
   block_sums_pairs<1, KS>(v, sub, nblk, blk, tid);
 }
 
@@ -497,18 +499,32 @@ __global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs
 // mostly from the CU's L1.  At 4096^2 two blocks per workgroup take the FP64
 // iteration from 269.2 to 267.6 us and the mixed-precision w-step from 83.2
 // to 79.0 us (four: 270.6 us).
-template <bool APPLY_P>
-void launch_fused_w1(tea_hip_chunk* c, const FusedWArgs& a, const RaScalar& sc = {}) {
+template <bool APPLY_P, int UM, bool CONSUME>
+void launch_fused_w1(tea_hip_chunk* c, const FusedWArgs& a, const RaScalar& sc) {
   const int S = stack_rows(c), ks = stack_factor(c);
-  const auto kernel =
-      sc.sub ? (ks == 1   ? fused_w1_kernel<APPLY_P, 1, true>
-                : ks == 2 ? fused_w1_kernel<APPLY_P, 2, true>
-                          : fused_w1_kernel<APPLY_P, 4, true>)
-             : (ks == 1   ? fused_w1_kernel<APPLY_P, 1>
-                : ks == 2 ? fused_w1_kernel<APPLY_P, 2>
-                          : fused_w1_kernel<APPLY_P, 4>);
+  const auto kernel = ks == 1   ? fused_w1_kernel<APPLY_P, 1, UM, CONSUME>
+                      : ks == 2 ? fused_w1_kernel<APPLY_P, 2, UM, CONSUME>
+                                : fused_w1_kernel<APPLY_P, 4, UM, CONSUME>;
   hipLaunchKernelGGL(kernel, stacked_grid(c, ks), dim3(ks * kBlock), 0, c->stream, c->geo, a, sc,
                      c->sub, c->nblk, S);
+}
+
+int launch_cg_step(tea_hip_chunk* c, const CgStep& s, const RaScalar& sc) {
+  Timed t(c, K_CG_FUSED_W);
+  const bool consume = sc.sub != nullptr;
+  if (!s.apply_p)
+    launch_fused_w1<false, 1, false>(c, s.a, sc);
+  else if (s.um == 0)
+    consume ? launch_fused_w1<true, 0, true>(c, s.a, sc)
+            : launch_fused_w1<true, 0, false>(c, s.a, sc);
+  else if (s.um == 1)
+    consume ? launch_fused_w1<true, 1, true>(c, s.a, sc)
+            : launch_fused_w1<true, 1, false>(c, s.a, sc);
+  else
+    consume ? launch_fused_w1<true, 3, true>(c, s.a, sc)
+            : launch_fused_w1<true, 3, false>(c, s.a, sc);
+  TEA_HIP_TRY(hipGetLastError());
+  return TEA_HIP_OK;
 }
 
 __global__ __launch_bounds__(kBlock) void fused_r2_kernel(
@@ -674,15 +690,68 @@ int launch_span1(tea_hip_chunk* c, int kid, const Body& body, double* out) {
   return sum_over_cells<1>(c, kid, body, out);
 }
 
-// Makes the second p buffer's cells outside the interior and the halo ring
-// equal to p's (the fused kernel writes only the interior and the ring).
+// The cells outside the interior of up to kFrames buffers from others
+// (blockIdx.y the pair): the h rows below and above it, then its rows' h cells
+// left and right of it.
+constexpr int kFrames = 6;
+struct FramePairs {
+  const double* src[kFrames];
+  double* dst[kFrames];
+};
+__global__ __launch_bounds__(kBlock) void copy_frame_kernel(Geo g, FramePairs f) {
+  const int rows = 2 * g.h * g.x, sides = 2 * g.h * (g.y - 2 * g.h);
+  int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= rows + sides) return;
+  int i;
+  if (k < rows) {
+    i = k < rows / 2 ? k : k + (g.y - 2 * g.h) * g.x;
+  } else {
+    k -= rows;
+    const int row = k / (2 * g.h), q = k - row * (2 * g.h);
+    i = (g.h + row) * g.x + (q < g.h ? q : g.x - 2 * g.h + q);
+  }
+  f.dst[blockIdx.y][i] = f.src[blockIdx.y][i];
+}
+
+int copy_frames(tea_hip_chunk* c, const FramePairs& f, int n) {
+  if (n == 0) return TEA_HIP_OK;
+  const Geo& g = c->geo;
+  const long cells = 2L * g.h * g.x + 2L * g.h * (g.y - 2 * g.h);
+  hipLaunchKernelGGL(copy_frame_kernel, dim3((unsigned)((cells + kBlock - 1) / kBlock), n),
+                     dim3(kBlock), 0, c->stream, g, f);
+  TEA_HIP_TRY(hipGetLastError());
+  return TEA_HIP_OK;
+}
+
+// Makes the spare p buffers' cells outside the interior equal to p's (the
+// fused kernel writes only the interior and the ring).
 int sync_p_alt(tea_hip_chunk* c) {
   if (c->p_alt_synced) return TEA_HIP_OK;
-  TEA_HIP_TRY(hipMemcpyAsync(c->p_alt, c->field[TEA_FIELD_P],
-                             (size_t)c->geo.n * sizeof(double),
-                             hipMemcpyDeviceToDevice, c->stream));
+  FramePairs f{};
+  int n = 0;
+  for (double* b : c->p_alt)
+    if (b) {
+      f.src[n] = c->field[TEA_FIELD_P];
+      f.dst[n++] = b;
+    }
+  TEA_RETURN_IF(copy_frames(c, f, n));
   c->p_alt_synced = true;
   return TEA_HIP_OK;
+}
+
+// The spare p buffers that held updates need (none: updates are not held).
+void ensure_p_ring(tea_hip_chunk* c) {
+  if (!c->hold_ok || c->p_alt[2]) return;
+  for (int i = 1; i < 3; ++i) {
+    if (c->p_alt[i]) continue;
+    if (hipMalloc(&c->p_alt[i], pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
+      c->p_alt[i] = nullptr;
+      (void)hipGetLastError();
+      c->hold_ok = false;
+      return;
+    }
+    c->p_alt_synced = false;
+  }
 }
 
 // ---- run-ahead of the fused CG iteration ----------------------------------
@@ -699,10 +768,12 @@ int sync_p_alt(tea_hip_chunk* c) {
 // of at most kConsumeBlocks blocks there is no finisher: the next pass itself
 // sums and divides, see RaScalar, and its first block hands the host the
 // values):
-//   after cg_calc_w  (the r-step): r - alpha w into r_alt, and r.r;
-//   after cg_calc_ur (the w-step): u + alpha p into u_alt, p = beta p + r
-//     into p_alt with the U/P halo ring, w = A p into w_alt, p.w; then the
-//     next r-step.
+//   the r-step: r - alpha w into r_alt, and r.r;
+//   the w-step: u + alpha p into u_alt (or held), p = beta p + r into a spare
+//     p with the U/P halo ring, w = A p into w_alt, p.w.
+// cg_calc_w leaves the r-step and the w-step behind its own pass queued,
+// cg_calc_ur the r-step after that: two passes ahead, as a pass of a small
+// grid (4-6 us) is over before the host has seen its scalar.
 // The host's next call takes a pass over (exchanging the buffers) when its
 // scalar is bitwise the one the device used (read back with the sums) and,
 // for the w-step, the deferred work is exactly the u and p updates and the
@@ -712,7 +783,6 @@ int sync_p_alt(tea_hip_chunk* c) {
 // sum and scalar go to one of two host slot sets, alternating, so the next
 // step is queued before the host has read the last one.
 
-constexpr int kRaNone = 0, kRaR = 1, kRaWR = 2;
 constexpr int kRaW = 0, kRaRStep = 1;  // slot kinds
 
 bool ra_possible(const tea_hip_chunk* c) {
@@ -720,13 +790,8 @@ bool ra_possible(const tea_hip_chunk* c) {
          c->ra_fail < 3 && use_pair_blocks(c, 1) && use_pair_blocks(c, 2);
 }
 
-double* ra_host_slot(tea_hip_chunk* c, int set, int kind) {
-  return c->ra_host + 2 * (2 * set + kind);
-}
-
-double* ra_dev_slot(tea_hip_chunk* c, int set, int kind) {
-  return c->ra_host_dev + 2 * (2 * set + kind);
-}
+// Offset of a slot in ra_host.
+int ra_slot(int kind, int i) { return 2 * (2 * kind + i); }
 
 int ensure_ra(tea_hip_chunk* c) {
   if (c->ra_host) return TEA_HIP_OK;
@@ -758,61 +823,59 @@ int ensure_ra(tea_hip_chunk* c) {
 // The next pass forms the scalar of the pass before it (RaScalar::sub).
 bool ra_consume(const tea_hip_chunk* c) { return c->nblk <= kConsumeBlocks; }
 
-// Arms host slot (set, kind) for the pass just queued, a w-step (kRaW) or
-// an r-step, and sets *sc to where the pass after it takes its scalar: the
-// device's, left there by a finisher launched here, or the pass's block
-// sums.  Either counts as one cg_ra_finish launch in the statistics.
-int ra_finish(tea_hip_chunk* c, int set, int kind, double rro, bool from_dev, RaScalar* sc) {
+// Arms a step's host slot for the pass or finisher about to be launched.
+int ra_arm(tea_hip_chunk* c, int kind, int i) {
   if (c->ra_dirty) {
     // A dropped run-ahead may still be queued and write these slots.
     TEA_HIP_TRY(hipStreamSynchronize(c->stream));
     c->ra_dirty = false;
   }
-  arm_host_values(ra_host_slot(c, set, kind), 2);
-  *sc = RaScalar{};
+  arm_host_values(c->ra_host + ra_slot(kind, i), 2);
+  return TEA_HIP_OK;
+}
+
+// Where the pass after a w-step (kind kRaW) or r-step takes its scalar from;
+// rro is the value, or what the w-step before left on the device.
+RaScalar ra_scalar_of(const tea_hip_chunk* c, int kind, int i, double rro, bool from_dev) {
+  RaScalar sc;
+  sc.out = c->ra_host_dev + ra_slot(kind, i);
+  if (!ra_consume(c)) {
+    sc.dev = c->ra_dev + kind;
+    return sc;
+  }
+  sc.sub = kind == kRaW ? c->sub : c->sub2;
+  sc.nblk = c->nblk;
+  sc.inverse = kind == kRaW ? 0 : 1;
+  sc.rro = rro;
+  sc.rro_dev = from_dev ? c->ra_dev + 2 : nullptr;
+  sc.sum_dev = c->ra_dev + (kind == kRaW ? 0 : 2);
+  return sc;
+}
+
+// The finisher of a w-step or r-step just queued (grids above kConsumeBlocks
+// blocks).  Either way the step counts as one cg_ra_finish launch in the
+// statistics.
+int ra_finish(tea_hip_chunk* c, int kind, int i, double rro, bool from_dev) {
   if (ra_consume(c)) {
-    sc->sub = kind == kRaW ? c->sub : c->sub2;
-    sc->nblk = c->nblk;
-    sc->inverse = kind == kRaW ? 0 : 1;
-    sc->rro = rro;
-    sc->rro_dev = from_dev ? c->ra_dev + 2 : nullptr;
-    sc->sum_dev = kind == kRaW ? nullptr : c->ra_dev + 2;
-    sc->out = ra_dev_slot(c, set, kind);
     if (c->timing && c->time_kernel[K_CG_RA_FINISH]) c->launches[K_CG_RA_FINISH] += 1;
     return TEA_HIP_OK;
   }
-  sc->dev = c->ra_dev + (kind == kRaW ? 0 : 1);
-  const RaTail tail{rro, from_dev ? 1 : 0, kind == kRaW ? 0 : 1, c->ra_dev};
-  return launch_span_finish_ra(c, 1, ra_dev_slot(c, set, kind), tail);
-}
-
-// The r-step behind a w-step that was just queued: alpha from its p.w (and
-// rro), r_alt = r - alpha w, r.r; c->ra_next is where the next w-step will
-// take beta from.
-int ra_launch_r(tea_hip_chunk* c, int set, const double* w, double rro, bool from_dev) {
-  RaScalar sc;
-  TEA_RETURN_IF(ra_finish(c, set, kRaW, rro, from_dev, &sc));
-  {
-    Timed t(c, K_CG_FUSED_R);
-    hipLaunchKernelGGL(sc.sub ? fused_r1_kernel<true> : fused_r1_kernel<false>, pair_grid(c),
-                       dim3(kBlock), 0, c->stream, c->geo, c->field[TEA_FIELD_R], c->r_alt, w,
-                       0.0, sc, sc.sub ? c->sub2 : c->sub, c->nblk);
-  }
-  TEA_HIP_TRY(hipGetLastError());
-  return ra_finish(c, set, kRaRStep, rro, from_dev, &c->ra_next);
+  TEA_RETURN_IF(ra_arm(c, kind, i));
+  return launch_span_finish_ra(c, 1, c->ra_host_dev + ra_slot(kind, i),
+                               RaTail{rro, from_dev ? 1 : 0, kind, c->ra_dev});
 }
 
 // Waits for a slot's sum and scalar.
-int ra_wait(tea_hip_chunk* c, int set, int kind, double* sum, double* ratio) {
-  const double* h = ra_host_slot(c, set, kind);
+int ra_wait(tea_hip_chunk* c, int kind, int i, double* sum, double* scalar) {
+  const double* h = c->ra_host + ra_slot(kind, i);
   TEA_RETURN_IF(wait_host_values(c, h, 2));
   *sum = h[0];
-  *ratio = h[1];
+  *scalar = h[1];
   return TEA_HIP_OK;
 }
 
 void ra_mismatch(tea_hip_chunk* c) {
-  c->ra = kRaNone;
+  c->ra_r = c->ra_w = false;
   c->ra_dirty = true;
   c->ra_fail += 1;
 }
@@ -824,14 +887,136 @@ void swap_ptr(T*& a, T*& b) {
   b = t;
 }
 
+// The w-step for the deferred work (ahead: behind the r-step in flight, for
+// the whole of an iteration's deferred work, its alpha and beta on the
+// device).  With all of it deferred, u's update is held over two steps.
+int plan_cg_w(tea_hip_chunk* c, bool ahead, CgStep* s) {
+  double** f = c->field;
+  const bool ride = c->hold_ok && c->p_alt[2] &&
+                    (ahead || (c->pend_u && c->pend_p && c->pend_halo));
+  if (c->uh && !ride) TEA_RETURN_IF(apply_held_u(c));
+  *s = CgStep{};
+  s->apply_p = ahead || c->pend_p;
+  if (s->apply_p) TEA_RETURN_IF(sync_p_alt(c));
+  double* p_new = c->p_alt[0];
+  for (double* b : c->p_alt) {
+    if (!b || (c->uh > 0 && b == c->uh_p[0]) || (c->uh > 1 && b == c->uh_p[1])) continue;
+    p_new = b;
+    break;
+  }
+  s->a = FusedWArgs{f[TEA_FIELD_P], p_new, ahead ? c->r_alt : f[TEA_FIELD_R], f[TEA_FIELD_U],
+                    ahead ? c->w_alt : f[TEA_FIELD_W], f[TEA_FIELD_KX], f[TEA_FIELD_KY],
+                    c->pend_alpha, c->pend_beta, ahead || c->pend_u ? 1 : 0,
+                    ahead || c->pend_halo ? 1 : 0, ahead ? c->u_alt : f[TEA_FIELD_U],
+                    ahead ? c->ra_dev : nullptr, nullptr, nullptr, 0.0, 0.0};
+  if (!ride) return TEA_HIP_OK;
+  if (c->uh == 2) {
+    s->um = 3;
+    s->a.p_h = c->uh_p[0];
+    s->a.alpha_h = c->uh_alpha[0];
+    s->a.p_h2 = c->uh_p[1];
+    s->a.alpha_h2 = c->uh_alpha[1];
+    return TEA_HIP_OK;
+  }
+  s->um = 0;
+  s->hold = c->uh + 1;
+  for (int i = 0; i < c->uh; ++i) {
+    s->hold_p[i] = c->uh_p[i];
+    s->hold_alpha[i] = c->uh_alpha[i];
+  }
+  s->hold_p[c->uh] = f[TEA_FIELD_P];
+  return TEA_HIP_OK;
+}
+
+// The chunk's state once a w-step has been asked for (or taken over), its u
+// update's factor alpha.
+void commit_cg_step(tea_hip_chunk* c, const CgStep& s, double alpha) {
+  double** f = c->field;
+  c->pend_u = c->pend_p = c->pend_halo = false;
+  c->uh = s.hold;
+  for (int i = 0; i < s.hold; ++i) {
+    c->uh_p[i] = s.hold_p[i];
+    c->uh_alpha[i] = i == s.hold - 1 ? alpha : s.hold_alpha[i];
+  }
+  if (s.um && s.a.apply_u && s.a.u_out != s.a.u) swap_ptr(f[TEA_FIELD_U], c->u_alt);
+  if (s.a.w != f[TEA_FIELD_W]) swap_ptr(f[TEA_FIELD_W], c->w_alt);
+  if (!s.apply_p) return;
+  for (double*& b : c->p_alt)
+    if (b == s.a.p_new) {
+      swap_ptr(f[TEA_FIELD_P], b);
+      break;
+    }
+}
+
+// Queues the r-step behind the newest w-step.  rro: r.r before it, the value
+// where the host has it.
+int ra_queue_r(tea_hip_chunk* c, double rro, bool from_dev) {
+  if (ra_consume(c)) TEA_RETURN_IF(ra_arm(c, kRaW, c->ra_wi));
+  const RaScalar sc = ra_scalar_of(c, kRaW, c->ra_wi, rro, from_dev);
+  {
+    Timed t(c, K_CG_FUSED_R);
+    hipLaunchKernelGGL(sc.sub ? fused_r1_kernel<true> : fused_r1_kernel<false>, pair_grid(c),
+                       dim3(kBlock), 0, c->stream, c->geo, c->field[TEA_FIELD_R], c->r_alt,
+                       c->ra_w ? c->w_alt : c->field[TEA_FIELD_W], 0.0, sc,
+                       sc.sub ? c->sub2 : c->sub, c->nblk);
+  }
+  TEA_HIP_TRY(hipGetLastError());
+  c->ra_ri ^= 1;
+  TEA_RETURN_IF(ra_finish(c, kRaRStep, c->ra_ri, rro, from_dev));
+  c->ra_r = true;
+  return TEA_HIP_OK;
+}
+
+// Queues the next w-step behind the r-step in flight (r.r before that step:
+// ra_rro).
+int ra_queue_w(tea_hip_chunk* c) {
+  TEA_RETURN_IF(plan_cg_w(c, true, &c->ra_step));
+  if (ra_consume(c)) TEA_RETURN_IF(ra_arm(c, kRaRStep, c->ra_ri));
+  TEA_RETURN_IF(
+      launch_cg_step(c, c->ra_step, ra_scalar_of(c, kRaRStep, c->ra_ri, c->ra_rro, false)));
+  c->ra_wi ^= 1;
+  TEA_RETURN_IF(ra_finish(c, kRaW, c->ra_wi, 0.0, true));
+  c->ra_w = true;
+  return TEA_HIP_OK;
+}
+
+struct HeldUBody {
+  double* __restrict__ u;
+  const double* __restrict__ p0;
+  const double* __restrict__ p1;
+  double a0, a1;
+  int n;
+  Geo g;
+  __device__ void operator()(int i, int kk, int jj) const {
+    if (!interior(g, kk, jj)) return;
+    double v = u[i] + a0 * p0[i];
+    if (n == 2) v = v + a1 * p1[i];
+    u[i] = v;
+  }
+};
+
 }  // namespace
 
 int ra_discard(tea_hip_chunk* c) {
-  if (c->ra != kRaNone) {
-    c->ra = kRaNone;
+  if (c->ra_r || c->ra_w) {
+    c->ra_r = c->ra_w = false;
     c->ra_dirty = true;
   }
   return TEA_HIP_OK;
+}
+
+int apply_held_u(tea_hip_chunk* c) {
+  if (c->uh == 0) return TEA_HIP_OK;
+  TEA_RETURN_IF(ra_discard(c));
+  const int n = c->uh;
+  c->uh = 0;
+  TEA_RETURN_IF(launch_each(c, K_CG_APPLY_PENDING,
+                            HeldUBody{c->field[TEA_FIELD_U], c->uh_p[0], c->uh_p[n - 1],
+                                      c->uh_alpha[0], c->uh_alpha[n - 1], n, c->geo}));
+  static const int ext[4] = {-1, -1, -1, -1};
+  int fields[TEA_HALO_NUM] = {0};
+  fields[TEA_HALO_U] = 1;
+  return launch_halos(c, 1, ext, fields);
 }
 
 int apply_pending(tea_hip_chunk* c) {
@@ -842,8 +1027,9 @@ int apply_pending(tea_hip_chunk* c) {
 }
 
 int apply_cg_pending(tea_hip_chunk* c) {
-  if (c->ra) TEA_RETURN_IF(ra_discard(c));
+  TEA_RETURN_IF(ra_discard(c));
   if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
+  TEA_RETURN_IF(apply_held_u(c));
   if (!c->pend_u && !c->pend_p && !c->pend_halo) return TEA_HIP_OK;
   double** f = c->field;
   const bool halo_u = c->pend_u;  // the deferred ring update includes U
@@ -911,25 +1097,17 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
   TEA_CHECK_ARG(pw != nullptr, "null pw");
   double** f = c->field;
   const Geo g = c->geo;
-  if (c->ra == kRaWR) {
+  if (c->ra_r || c->ra_w) {
     // The w-step in flight applied exactly the deferred work: take it over.
-    if (c->pend_u && c->pend_p && c->pend_halo && !c->held && c->pre_halo < 0 &&
-        c->pend_alpha == c->ra_w_alpha && c->pend_beta == c->ra_beta) {
-      swap_ptr(f[TEA_FIELD_P], c->p_alt);
-      swap_ptr(f[TEA_FIELD_U], c->u_alt);
-      swap_ptr(f[TEA_FIELD_W], c->w_alt);
-      c->pend_u = c->pend_p = c->pend_halo = false;
-      c->ra = kRaR;  // its r-step is queued behind it
-      c->ra_commits += 1;
+    if (c->ra_w && c->pend_u && c->pend_p && c->pend_halo && !c->held && c->pre_halo < 0 &&
+        c->pend_alpha == c->ra_alpha && c->pend_beta == c->ra_beta) {
+      commit_cg_step(c, c->ra_step, c->pend_alpha);
+      c->ra_w = false;
       c->ra_fail = 0;
-      double sum = 0.0, alpha = 0.0;
-      TEA_RETURN_IF(ra_wait(c, c->ra_set, kRaW, &sum, &alpha));
-      c->ra_alpha = alpha;
-      *pw = sum;
-      return TEA_HIP_OK;
+      const int slot = c->ra_wi;
+      TEA_RETURN_IF(ra_queue_w(c));  // its r-step is queued already
+      return ra_wait(c, kRaW, slot, pw, &c->ra_alpha);
     }
-    ra_mismatch(c);
-  } else if (c->ra != kRaNone) {
     ra_mismatch(c);
   }
   TEA_FLUSH_HELD(c);
@@ -940,49 +1118,34 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
                                   f[TEA_FIELD_KY], f[TEA_FIELD_W], g.x},
                         pw);
   }
-  const bool apply_p = c->pend_p;
-  if (apply_p) TEA_RETURN_IF(sync_p_alt(c));
-  FusedWArgs args{f[TEA_FIELD_P], c->p_alt,        f[TEA_FIELD_R],
-                  f[TEA_FIELD_U], f[TEA_FIELD_W],  f[TEA_FIELD_KX],
-                  f[TEA_FIELD_KY], c->pend_alpha,  c->pend_beta,
-                  c->pend_u ? 1 : 0, c->pend_halo ? 1 : 0, f[TEA_FIELD_U]};
-  c->pend_u = c->pend_p = c->pend_halo = false;
+  const bool pair_blocks = use_pair_blocks(c, 1), ahead = pair_blocks && ra_possible(c);
+  if (pair_blocks) ensure_p_ring(c);
+  const double alpha = c->pend_alpha;
+  CgStep s;
+  TEA_RETURN_IF(plan_cg_w(c, false, &s));
+  const bool apply_p = s.apply_p;
+  const FusedWArgs& args = s.a;
   int plen = c->nspan;
-  if (use_pair_blocks(c, 1)) {
-    const bool ahead = ra_possible(c);
+  if (pair_blocks) {
     if (ahead) {
       // Start a run-ahead: the spare buffers take the cells outside the
       // interior (and the ring) that no pass writes.
       TEA_RETURN_IF(ensure_ra(c));
-      const size_t bytes = (size_t)g.n * sizeof(double);
-      TEA_HIP_TRY(hipMemcpyAsync(c->r_alt, f[TEA_FIELD_R], bytes, hipMemcpyDeviceToDevice,
-                                 c->stream));
-      TEA_HIP_TRY(hipMemcpyAsync(c->u_alt, f[TEA_FIELD_U], bytes, hipMemcpyDeviceToDevice,
-                                 c->stream));
-      TEA_HIP_TRY(hipMemcpyAsync(c->w_alt, f[TEA_FIELD_W], bytes, hipMemcpyDeviceToDevice,
-                                 c->stream));
+      TEA_RETURN_IF(copy_frames(c, FramePairs{{f[TEA_FIELD_R], f[TEA_FIELD_U], f[TEA_FIELD_W]},
+                                              {c->r_alt, c->u_alt, c->w_alt}}, 3));
     }
-    {
-      Timed t(c, K_CG_FUSED_W);
-      if (apply_p)
-        launch_fused_w1<true>(c, args);
-      else
-        launch_fused_w1<false>(c, args);
-    }
-    TEA_HIP_TRY(hipGetLastError());
+    TEA_RETURN_IF(launch_cg_step(c, s, RaScalar{}));
+    commit_cg_step(c, s, alpha);
     if (ahead) {
-      const int set = c->ra_set ^ 1;
-      TEA_RETURN_IF(ra_launch_r(c, set, f[TEA_FIELD_W], c->ra_rro, false));
-      if (apply_p) swap_ptr(f[TEA_FIELD_P], c->p_alt);
-      c->ra = kRaR;
-      c->ra_set = set;
-      double sum = 0.0, alpha = 0.0;
-      TEA_RETURN_IF(ra_wait(c, set, kRaW, &sum, &alpha));
-      c->ra_alpha = alpha;
-      *pw = sum;
-      return TEA_HIP_OK;
+      c->ra_wi ^= 1;
+      TEA_RETURN_IF(ra_finish(c, kRaW, c->ra_wi, c->ra_rro, false));
+      TEA_RETURN_IF(ra_queue_r(c, c->ra_rro, false));
+      const int slot = c->ra_wi;
+      TEA_RETURN_IF(ra_queue_w(c));
+      return ra_wait(c, kRaW, slot, pw, &c->ra_alpha);
     }
     TEA_RETURN_IF(launch_span_finish(c, 1, &plen, 0, true));
+    return finish_reduction_n(c, 1, plen, pw);
   } else {
     Timed t(c, K_CG_FUSED_W);
     const int sg = c->ngroup == 1 ? 1 : 0;
@@ -1007,11 +1170,7 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
 #undef TEA_FUSED_W2
   }
   TEA_HIP_TRY(hipGetLastError());
-  if (apply_p) {
-    double* t = f[TEA_FIELD_P];
-    f[TEA_FIELD_P] = c->p_alt;
-    c->p_alt = t;
-  }
+  commit_cg_step(c, s, alpha);
   return finish_reduction_n(c, 1, plen, pw);
 }
 
@@ -1019,52 +1178,28 @@ int tea_hip_cg_calc_ur(tea_hip_chunk* c, double alpha, double* rrn) {
   TEA_ENTER_RA(c);
   TEA_CHECK_ARG(rrn != nullptr, "null rrn");
   double** f = c->field;
-  if (c->ra == kRaR) {
+  if (c->ra_r || c->ra_w) {
     // The r-step in flight used the device's alpha: take it over when the
     // host's is the same.
-    if (alpha == c->ra_alpha && !c->pend_u && !c->pend_p && !c->pend_halo && !c->held &&
-        c->pre_halo < 0 && ra_possible(c)) {
+    if (c->ra_r && c->ra_w && alpha == c->ra_alpha && !c->pend_u && !c->pend_p &&
+        !c->pend_halo && !c->held && c->pre_halo < 0) {
       swap_ptr(f[TEA_FIELD_R], c->r_alt);
       c->pend_u = true;
       c->pend_alpha = alpha;
-      const int set = c->ra_set;
-      c->ra = kRaNone;
-      // Queue the next w-step (its beta from the device) and r-step
-      // before waiting for this r.r.
-      TEA_RETURN_IF(sync_p_alt(c));
-      const int next = set ^ 1;
-      FusedWArgs a{f[TEA_FIELD_P], c->p_alt,  f[TEA_FIELD_R], f[TEA_FIELD_U],
-                   c->w_alt,       f[TEA_FIELD_KX], f[TEA_FIELD_KY], alpha,
-                   0.0,            1,         1,              c->u_alt};
-      // beta's rro is the r.r the host was last given (a consuming pass
-      // overwrites the device's copy).
-      RaScalar sc = c->ra_next;
-      sc.rro = c->ra_rro;
-      sc.rro_dev = nullptr;
-      {
-        Timed t(c, K_CG_FUSED_W);
-        launch_fused_w1<true>(c, a, sc);
-      }
-      TEA_HIP_TRY(hipGetLastError());
-      TEA_RETURN_IF(ra_launch_r(c, next, c->w_alt, 0.0, true));
-      c->ra = kRaWR;
-      c->ra_set = next;
-      c->ra_w_alpha = alpha;
-      double sum = 0.0, beta = 0.0;
-      TEA_RETURN_IF(ra_wait(c, set, kRaRStep, &sum, &beta));
-      c->ra_beta = beta;
-      c->ra_rro = sum;
-      c->ra_commits += 1;
+      c->ra_r = false;
+      const int slot = c->ra_ri;
+      // The r-step of the w-step in flight, before waiting for this r.r.
+      TEA_RETURN_IF(ra_queue_r(c, 0.0, true));
+      TEA_RETURN_IF(ra_wait(c, kRaRStep, slot, rrn, &c->ra_beta));
+      c->ra_rro = *rrn;
       c->ra_fail = 0;
-      *rrn = sum;
       return TEA_HIP_OK;
     }
     ra_mismatch(c);
-  } else if (c->ra != kRaNone) {
-    ra_mismatch(c);
   }
   TEA_FLUSH_HELD(c);
-  TEA_RETURN_IF(apply_pending(c));
+  // Held u updates alone may stay held: this step leaves u and p alone.
+  if (!c->fused || c->pend_u || c->pend_p || c->pend_halo) TEA_RETURN_IF(apply_pending(c));
   if (!c->fused)
     return launch_span1(c, K_CG_CALC_UR,
                         CalcURBody{f[TEA_FIELD_U], f[TEA_FIELD_R],

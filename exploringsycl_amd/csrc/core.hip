@@ -467,8 +467,8 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
       return fail(TEA_HIP_EHIP);
     }
   }
-  if (hipMalloc(&c->p_alt, pair_bytes(n, sizeof(double))) != hipSuccess) {
-    c->p_alt = nullptr;
+  if (hipMalloc(&c->p_alt[0], pair_bytes(n, sizeof(double))) != hipSuccess) {
+    c->p_alt[0] = nullptr;
     set_error("hipMalloc of the second p buffer failed");
     return fail(TEA_HIP_ENOMEM);
   }
@@ -520,7 +520,8 @@ int tea_hip_chunk_destroy(tea_hip_chunk* c) {
   for (auto e : c->event_pool) (void)hipEventDestroy(e);
   for (int f = 0; f < TEA_NUM_FIELDS; ++f)
     if (c->field[f]) (void)hipFree(c->field[f]);
-  if (c->p_alt) (void)hipFree(c->p_alt);
+  for (double* b : c->p_alt)
+    if (b) (void)hipFree(b);
   for (double* b : {c->r_alt, c->u_alt, c->w_alt, c->ra_dev})
     if (b) (void)hipFree(b);
   if (c->ra_host) (void)hipHostFree(c->ra_host);

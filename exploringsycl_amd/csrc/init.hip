@@ -303,6 +303,7 @@ int launch_halos(tea_hip_chunk* c, int depth, const int neighbours[4],
   }
   TEA_RETURN_IF(mra_discard(c));
   c->mra_synced = false;
+  if (fields[TEA_HALO_P]) c->p_alt_synced = false;
   const long items = 2L * g.y * depth + 2L * g.x * depth;
   {
     Timed t(c, K_LOCAL_HALOS);
@@ -352,7 +353,7 @@ int tea_hip_local_halos(tea_hip_chunk* c, int depth, const int neighbours[4],
         ++count;
       }
     if (count == 1 && (only == TEA_HALO_SD || only == TEA_HALO_U) &&
-        !(only == TEA_HALO_U && (c->pend_u || c->pend_halo))) {
+        !(only == TEA_HALO_U && (c->pend_u || c->pend_halo || c->uh))) {
       c->pre_halo = only;
       return TEA_HIP_OK;
     }

@@ -1242,6 +1242,7 @@ int tea_hip_mpcg_refresh(tea_hip_chunk* c, double alpha, int apply_u,
   TEA_CHECK_ARG(rr && rr_true && rw, "null outputs");
   TEA_HIP_TRY(hipSetDevice(c->device));
   TEA_FLUSH_HELD(c);
+  TEA_RETURN_IF(apply_held_u(c));
   c->mra_period = c->mra_since;
   c->mra_since = 0;
   double** f = c->field;

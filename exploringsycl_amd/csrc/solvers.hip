@@ -1067,6 +1067,7 @@ int tea_hip_ppcg_init(tea_hip_chunk* c, double theta) {
   // sd = r / theta reads neither u nor p: u += alpha p, left pending by
   // cg_calc_ur, stays pending for the first inner pass to apply.
   if (c->pend_p || c->pend_halo) TEA_RETURN_IF(apply_pending(c));
+  TEA_RETURN_IF(apply_held_u(c));
   double** f = c->field;
   return launch_each_cell(
       c, K_PPCG_INIT, DivideBody{f[TEA_FIELD_SD], f[TEA_FIELD_R], theta, c->geo});
@@ -1075,6 +1076,7 @@ int tea_hip_ppcg_init(tea_hip_chunk* c, double theta) {
 int tea_hip_ppcg_inner_iteration(tea_hip_chunk* c, double alpha,
                                  double beta) {
   TEA_ENTER_HELD(c);
+  TEA_RETURN_IF(apply_held_u(c));
   if (c->fused) {
     // Held back until the next inner step: with the SD halo update between
     // them (all faces external), both steps run as one pass.

@@ -698,6 +698,28 @@ struct MpArgs {
   const double* alpha_dev;
 };
 
+// Arguments of the FP64 w-step kernels (cg.hip).
+struct FusedWArgs {
+  const double* p_old;
+  double* p_new;
+  const double* r;
+  double* u;
+  double* w;
+  const double* kx;
+  const double* ky;
+  double alpha, beta;
+  int apply_u, ring;
+  // Pair-per-thread kernel only: the new u goes to u_out (u itself for the
+  // iteration the host asked for, a spare buffer when it runs ahead); its
+  // alpha is *alpha_dev where that is set; held updates made first (UM 3):
+  // u += alpha_h p_h, then u += alpha_h2 p_h2.
+  double* u_out;
+  const double* alpha_dev;
+  const double* p_h;
+  const double* p_h2;
+  double alpha_h, alpha_h2;
+};
+
 // Where a pass of the iteration takes its scalar from: the host's value
 // (dev null), the device's (dev: a finisher of the run-ahead left it there),
 // or, with CONSUME, the block sums sub of the pass before it, which every
@@ -712,8 +734,9 @@ struct RaScalar {
   int nblk = 0, inverse = 0;
   double rro = 0.0;
   const double* rro_dev = nullptr;
-  double* sum_dev = nullptr;  // set by the w-step: r.r, the next alpha's rro
-                              // (two sums: set by the r-step, alpha and p.w)
+  double* sum_dev = nullptr;  // left for the next passes: by the w-step r.r (the
+                              // next alpha's rro), by the r-step alpha (with
+                              // two sums alpha and p.w)
   double* out = nullptr;      // host slot {sum(s), scalar}
 };
 
@@ -815,6 +838,18 @@ const float* output(tea_nn* n);
 constexpr int kMpRing = 4;
 inline int mp_next(int i) { return i + 1 == kMpRing ? 0 : i + 1; }
 
+// One FP64 CG w-step on the pair kernels: its arguments, the u update it makes
+// (um: none, its own where a.apply_u, or the two held ones and its own) and
+// the updates held once it is taken over.
+struct CgStep {
+  tea::FusedWArgs a{};
+  bool apply_p = false;
+  int um = 1;
+  int hold = 0;
+  double* hold_p[2] = {};
+  double hold_alpha[2] = {0.0, 0.0};
+};
+
 // One mixed-precision (or FCG) w-step on the pair or four-cell kernels: its
 // arguments, the u update it makes (um: none, its own, or the two held ones
 // and its own) and the updates held once it is taken over.
@@ -855,9 +890,11 @@ struct tea_hip_chunk {
   double* field[TEA_NUM_FIELDS] = {};
   size_t field_len[TEA_NUM_FIELDS] = {};
 
-  // Second p buffer for the fused iteration (p is read as a stencil while
-  // the new p is written).  p_alt_synced: its non-interior cells equal p's.
-  double* p_alt = nullptr;
+  // Spare p buffers for the fused iteration (p is read as a stencil while the
+  // new p is written; the first at creation, the others with the first
+  // iteration, for the held updates below).  p_alt_synced: their cells
+  // outside the interior and its ring equal p's.
+  double* p_alt[3] = {};
   bool p_alt_synced = false;
 
   // Reduction workspace: up to 4 x nspan level-2 partials in pinned,
@@ -906,6 +943,14 @@ struct tea_hip_chunk {
   bool quads = false;  // four-cells-per-lane mixed-precision kernels (x % 4 == 0)
   bool pend_u = false, pend_p = false, pend_halo = false;
   double pend_alpha = 0.0, pend_beta = 0.0;
+  // Up to two updates u += uh_alpha[i] uh_p[i] (oldest first, uh_p among
+  // p_alt), each with the U halo update after it, that passes of the fused
+  // iteration have left to a later one (TEA_HIP_HOLD_U=0 turns this off):
+  // the third pass makes both and its own in one pass over u.  Older than
+  // the deferred work above; any other entry point makes them first.
+  int uh = 0;
+  double* uh_p[2] = {};
+  double uh_alpha[2] = {0.0, 0.0};
 
   // Mixed-precision CG: FP32 p (a ring of buffers, mp_cur is
   // current; each w-step writes the next), r, w and
@@ -941,10 +986,12 @@ struct tea_hip_chunk {
   float* fcg_g = nullptr;
 
   // Run-ahead of the fused CG iteration (cg.hip): the device forms alpha and
-  // beta from its own partials and runs the next pass of the iteration into
-  // spare buffers before the host asks for it; the host's call commits it
-  // when its scalar is bitwise the device's.
-  int ra = 0;                 // kRaNone, kRaR (r-step in flight), kRaWR
+  // beta from its own sums and runs the next passes of the iteration, the
+  // r-step (ra_r) and the w-step behind it (ra_w), into spare buffers before
+  // the host asks for them; the host's call takes a pass over when its scalar
+  // is bitwise the device's.
+  bool ra_r = false, ra_w = false;
+  CgStep ra_step;             // the w-step in flight
   bool ra_enabled = true;     // TEA_HIP_RUN_AHEAD=0 turns it off
   // Blocks one row apart per workgroup of the stencil passes mp_w4_kernel,
   // fused_w1_kernel and jacobi_pair_kernel: 1, 2 (the default) or 4
@@ -953,20 +1000,17 @@ struct tea_hip_chunk {
   int stack = 2;
   bool ra_dirty = false;      // a discarded run-ahead may still be writing ra_host
   int ra_fail = 0;            // consecutive mismatches (3 turn it off)
-  int ra_set = 0;             // host slot set of the step in flight
-  long ra_commits = 0;        // run-ahead passes taken over (statistics)
+  int ra_wi = 0, ra_ri = 0;   // host slots of the newest w-step and r-step
   double ra_rro = 0.0;        // r.r the host was last given (its rro)
   bool ra_rro_known = false;
-  double ra_alpha = 0.0;      // alpha of the r-step in flight (the device's)
-  double ra_beta = 0.0;       // beta of the w-step in flight (the device's)
-  double ra_w_alpha = 0.0;    // alpha whose u update the w-step in flight applies
+  double ra_alpha = 0.0;      // the device's alpha of the last w-step the
+                              // host asked for
+  double ra_beta = 0.0;       // its beta of the last r-step
   double* r_alt = nullptr;    // spare r, u and w (x*y each)
   double* u_alt = nullptr;
   double* w_alt = nullptr;
-  tea::RaScalar ra_next;      // where the w-step after the r-step in flight
-                              // takes its beta from
   double* ra_dev = nullptr;   // device: [0] alpha, [1] beta, [2] r.r
-  double* ra_host = nullptr;  // pinned: 2 sets x {w-step, r-step} x {sum, ratio}
+  double* ra_host = nullptr;  // pinned: {w-step, r-step} x 2 slots x {sum, scalar}
   double* ra_host_dev = nullptr;  // device view of ra_host
 
   // Run-ahead of mixed-precision CG and FCG (mpcg.hip): up to two passes in
@@ -1131,6 +1175,8 @@ enum { kHeldNone = 0, kHeldPpcg = 1, kHeldCheby = 2 };
 int apply_pending(tea_hip_chunk* c);
 // The deferred CG work alone (cg.hip).
 int apply_cg_pending(tea_hip_chunk* c);
+// The held FP64 u updates alone, with their U halo update (cg.hip).
+int apply_held_u(tea_hip_chunk* c);
 // A held-back halo update before a step, alone (solvers.hip).
 int apply_pre_halo(tea_hip_chunk* c);
 // Runs what is held back, oldest first: deferred CG work, a held-back halo
@@ -1187,7 +1233,7 @@ int mra_discard(tea_hip_chunk* c);
 // run-ahead of the CG iteration.
 #define TEA_ENTER_HELD(c)                                 \
   TEA_ENTER_RA(c);                                        \
-  if ((c)->ra) TEA_RETURN_IF(::tea::ra_discard(c))
+  TEA_RETURN_IF(::tea::ra_discard(c))
 
 // Entry points other than the PPCG inner step and the halo update first run
 // a held-back halo update and PPCG or Chebyshev step (and drop a run-ahead)
@@ -1204,7 +1250,7 @@ int mra_discard(tea_hip_chunk* c);
 // mixed-precision and FCG steps, which touch neither u nor the held p.
 #define TEA_FLUSH_HELD_KEEP_U(c)                                           \
   do {                                                                     \
-    if ((c)->ra) TEA_RETURN_IF(::tea::ra_discard(c));                      \
+    TEA_RETURN_IF(::tea::ra_discard(c));                                   \
     if ((c)->held || (c)->pre_halo >= 0) TEA_RETURN_IF(::tea::flush_held(c)); \
   } while (0)
 
