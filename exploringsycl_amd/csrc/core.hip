@@ -535,6 +535,7 @@ int tea_hip_chunk_destroy(tea_hip_chunk* c) {
     if (b) (void)hipFree(b);
   if (c->mra_dev) (void)hipFree(c->mra_dev);
   if (c->mra_host) (void)hipHostFree(c->mra_host);
+  if (c->j_host) (void)hipHostFree(c->j_host);
   if (c->fcg_xsum) (void)hipFree(c->fcg_xsum);
   if (c->fcg_g) (void)hipFree(c->fcg_g);
   for (FcgLevel& L : c->fcg_lv) {

@@ -277,6 +277,18 @@ int tea_hip_store_energy(tea_hip_chunk* c) {
 
 namespace tea {
 
+int launch_halo_of(tea_hip_chunk* c, double* field) {
+  const Geo g = c->geo;
+  const long items = 2L * g.y + 2L * g.x;
+  HaloFields hf{};
+  hf.f[0] = field;
+  Timed t(c, K_LOCAL_HALOS);
+  hipLaunchKernelGGL(halo_kernel, dim3((unsigned)((items + kBlock - 1) / kBlock), 1),
+                     dim3(kBlock), 0, c->stream, g, 1, 1, 1, 1, 1, hf);
+  TEA_HIP_TRY(hipGetLastError());
+  return TEA_HIP_OK;
+}
+
 // Launches one reflective-halo pass; used by tea_hip_local_halos and by the
 // flush of deferred CG halos.
 int launch_halos(tea_hip_chunk* c, int depth, const int neighbours[4],

@@ -255,28 +255,93 @@ __device__ inline void st2_all(double* p, const PairAt& q, double v0,
   if (q.valid) st2_nt(p, q.e, true, true, v0, v1);
 }
 
-template <int KS>
+// The sum of the block sums in sub (at most 16 groups of 512 blocks), by one
+// block of at least four waves; thread 0 returns it.
+constexpr int kJacobiGroups = 16;
+__device__ inline double block_total(const double* __restrict__ sub, int nblk) {
+  __shared__ double gs[kJacobiGroups];
+  const int lane = threadIdx.x & (kWave - 1), waves = blockDim.x / kWave;
+  const int stride = sub_stride(nblk);
+  for (int g = threadIdx.x / kWave; g < kJacobiGroups; g += waves) {
+    const int i0 = kGroupBlocks * g + kSubPerSpan * lane;
+    double t = 0.0;
+    if (i0 < stride) {
+      const double2 a = ld2(sub, i0), b = ld2(sub, i0 + 2), c = ld2(sub, i0 + 4),
+                    d = ld2(sub, i0 + 6);
+      t = ((a.x + a.y) + (b.x + b.y)) + ((c.x + c.y) + (d.x + d.y));
+    }
+    t = wave_tree_dpp(t);
+    if (lane == 0) gs[g] = t;
+  }
+  __syncthreads();
+  double s[kJacobiGroups];
+#pragma unroll
+  for (int g = 0; g < kJacobiGroups; ++g) s[g] = gs[g];
+#pragma unroll
+  for (int m = 1; m < kJacobiGroups; m *= 2)
+#pragma unroll
+    for (int g = 0; g + m < kJacobiGroups; g += 2 * m) s[g] = s[g] + s[g + m];
+  return s[0];
+}
+
+// One sweep: 40 bytes per cell (u, u0, the two faces, the new u), bound by HBM
+// beyond the caches' size and by the cache and the launch below: 1000^2 (40 MB,
+// in the last-level cache) 12.4 us.  A sweep was 24.9 us there with the halo
+// update (3.5), the finisher (3.4) and the host's round trip between sweeps;
+// it is 12.9 us without them.
+// With HALO the depth-1 U halo update that precedes it is folded in: a neighbour on the ring is the cell's own mirror image, and the ring of
+// the new u gets what that update leaves (the old values); the ring of the
+// old u is left to jacobi_settle.  With prev the first block also finishes
+// the sum of the sweep before (its block sums in prev) into out.
+template <int KS, bool HALO>
 __global__ __launch_bounds__(kBlock * KS) void jacobi_pair_kernel(
     Geo g, const double* __restrict__ u_old, double* __restrict__ u_new,
     const double* __restrict__ u0, const double* __restrict__ kx,
-    const double* __restrict__ ky, double* sub, int nblk, int S) {
+    const double* __restrict__ ky, double* sub, int nblk, int S,
+    const double* __restrict__ prev, double* out) {
   int tid;
   const int blk = stacked_block<KS, kBlock>(S, &tid);
   const int lane = threadIdx.x & (kWave - 1);
   const PairAt q = pair_at(g, blk < nblk ? blk * kPairBlock + 2 * tid : g.n);
-  const Operand o = load_operand(u_old, q, g.x, lane);
+  Operand o = load_operand(u_old, q, g.x, lane);
   const Faces f = load_faces(kx, ky, q, g.x, lane);
   const double2 s = ld2_nt(u0, q.ir);
-  const double n0 = q.in0 ? jacobi_cell(s.x, o.l, o.c.y, o.b.x, o.t.x, f.kx.x,
+  double ra = o.c.y, lb = o.c.x;  // the pair's inner neighbours
+  bool st0 = q.valid, st1 = q.valid;
+  const int x = g.x, xl = g.h, xr = g.x - g.h - 1, yb = g.h, yt = g.y - g.h - 1;
+  if (HALO) {
+    if (q.kk == xl) o.l = o.c.x;
+    if (q.kk == xr) ra = o.c.x;
+    if (q.kk + 1 == xl) lb = o.c.y;
+    if (q.kk + 1 == xr) o.r = o.c.y;
+    if (q.row == yb) o.b = o.c;
+    if (q.row == yt) o.t = o.c;
+    // Ring cells are written by the cells they mirror.
+    auto ring = [&](int kk, int row) {
+      return kk >= xl - 1 && kk <= xr + 1 && row >= yb - 1 && row <= yt + 1;
+    };
+    const bool wrap = q.kk + 1 == x;  // the second cell begins the next row
+    st0 = q.valid && (q.in0 || !ring(q.kk, q.row));
+    st1 = q.valid && (q.in1 || !ring(wrap ? 0 : q.kk + 1, wrap ? q.row + 1 : q.row));
+  }
+  const double n0 = q.in0 ? jacobi_cell(s.x, o.l, ra, o.b.x, o.t.x, f.kx.x,
                                         f.kx.y, f.ky.x, f.kyt.x)
                           : o.c.x;
-  const double n1 = q.in1 ? jacobi_cell(s.y, o.c.x, o.r, o.b.y, o.t.y, f.kx.y,
+  const double n1 = q.in1 ? jacobi_cell(s.y, lb, o.r, o.b.y, o.t.y, f.kx.y,
                                         f.kx2, f.ky.y, f.kyt.y)
                           : o.c.y;
-  st2_all(u_new, q, n0, n1);
+  st2_nt(u_new, q.e, st0, st1, n0, n1);
+  if (HALO) {
+    if (q.in0) ring_store(u_new, q.e, q.kk, q.row, x, xl, xr, yb, yt, o.c.x);
+    if (q.in1) ring_store(u_new, q.e + 1, q.kk + 1, q.row, x, xl, xr, yb, yt, o.c.y);
+  }
   const double v[1] = {(q.in0 ? fabs(n0 - o.c.x) : 0.0) +
                        (q.in1 ? fabs(n1 - o.c.y) : 0.0)};
   block_sums_pairs<1, KS>(v, sub, nblk, blk, tid);
+  if (prev && blockIdx.x == 0) {
+    const double total = block_total(prev, nblk);
+    if (threadIdx.x == 0) *out = total;
+  }
 }
 
 __global__ __launch_bounds__(kBlock) void cheby_pair_kernel(
@@ -337,6 +402,17 @@ int ensure_spare(tea_hip_chunk* c) {
   if (hipMalloc(&c->spare, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
     c->spare = nullptr;
     set_error("hipMalloc of the spare field buffer failed");
+    return TEA_HIP_ENOMEM;
+  }
+  return TEA_HIP_OK;
+}
+
+// The second spare buffer, allocated on first use.
+int ensure_spare2(tea_hip_chunk* c) {
+  if (c->spare2) return TEA_HIP_OK;
+  if (hipMalloc(&c->spare2, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
+    c->spare2 = nullptr;
+    set_error("hipMalloc of the second spare field buffer failed");
     return TEA_HIP_ENOMEM;
   }
   return TEA_HIP_OK;
@@ -805,13 +881,81 @@ __global__ __launch_bounds__(kTSBlock) void cheby_two_step_kernel(
   }
 }
 
-// The second spare buffer, allocated on first use.
-int ensure_spare2(tea_hip_chunk* c) {
-  if (c->spare2) return TEA_HIP_OK;
-  if (hipMalloc(&c->spare2, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
-    c->spare2 = nullptr;
-    set_error("hipMalloc of the second spare field buffer failed");
-    return TEA_HIP_ENOMEM;
+// ---- Jacobi sweeps ahead of the host ----------------------------------------
+//
+// The host only tests the error a sweep returns, so the next sweeps do not wait
+// for it: each call leaves up to two more queued (a sweep of a small grid is
+// over before the host has seen its error), each with the U halo update that
+// the driver makes before it, into the spare buffers, and takes one over; any
+// other call drops them.  A sweep's error is summed by the first block of the
+// sweep after it.  No sweep is queued past the one after which the driver
+// left the sequence the last time (its every-50th residual).  Up to 16 groups
+// (4.2 M cells): the sums of more are too much for one block, and a round trip
+// (about 6 us) is little of such a sweep.
+
+bool jacobi_ahead_possible(const tea_hip_chunk* c) {
+  return c->ra_enabled && c->fused && c->poll && !c->j_off && use_pair_blocks(c, 1) &&
+         sub_stride(c->nblk) <= kJacobiGroups * kGroupBlocks;
+}
+
+// Whether the buffers of sweeps ahead are there (else there are none).
+bool ensure_jacobi_ahead(tea_hip_chunk* c) {
+  if (c->j_host) return true;
+  double* host = nullptr;
+  if (ensure_spare(c) == TEA_HIP_OK && ensure_spare2(c) == TEA_HIP_OK &&
+      hipHostMalloc(&host, 2 * sizeof(double),
+                    hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
+    if (hipHostGetDevicePointer((void**)&c->j_host_dev, host, 0) == hipSuccess) {
+      c->j_host = host;
+      return true;
+    }
+    (void)hipHostFree(host);
+  }
+  (void)hipGetLastError();
+  c->j_off = true;
+  return false;
+}
+
+// A sweep from u_old into u_new, its block sums in sub; with prev the sum of
+// the sweep before goes to out.  Workgroups of stack_factor(c) blocks one row
+// apart (tea_hip_impl.h).
+int launch_jacobi(tea_hip_chunk* c, const double* u_old, double* u_new, bool halo, double* sub,
+                  const double* prev, double* out) {
+  Timed t(c, K_JACOBI_FUSED);
+  double** f = c->field;
+  const int ks = stack_factor(c), S = stack_rows(c);
+  const auto kernel =
+      halo ? (ks == 1   ? jacobi_pair_kernel<1, true>
+              : ks == 2 ? jacobi_pair_kernel<2, true>
+                        : jacobi_pair_kernel<4, true>)
+           : (ks == 1   ? jacobi_pair_kernel<1, false>
+              : ks == 2 ? jacobi_pair_kernel<2, false>
+                        : jacobi_pair_kernel<4, false>);
+  hipLaunchKernelGGL(kernel, stacked_grid(c, ks), dim3(kBlock * ks), 0, c->stream, c->geo, u_old,
+                     u_new, f[TEA_FIELD_U0], f[TEA_FIELD_KX], f[TEA_FIELD_KY], sub, c->nblk, S,
+                     prev, out);
+  TEA_HIP_TRY(hipGetLastError());
+  return TEA_HIP_OK;
+}
+
+// Queues sweeps behind the one just asked for, up to two.
+int jacobi_queue(tea_hip_chunk* c) {
+  while (c->jra < 2 && (c->j_period == 0 || c->j_since + c->jra < c->j_period)) {
+    if (c->ra_dirty) {
+      // A dropped pass may still be queued and write the slots.
+      TEA_HIP_TRY(hipStreamSynchronize(c->stream));
+      c->ra_dirty = false;
+    }
+    const double* from = c->jra ? *c->j_buf[c->jra - 1] : c->field[TEA_FIELD_U];
+    double** to = c->jra ? (c->j_buf[c->jra - 1] == &c->spare ? &c->spare2 : &c->spare)
+                         : &c->spare;
+    double* sums[2] = {c->sub, c->sub2};
+    const int slot = c->j_slot ^ (c->jra & 1);
+    arm_host_values(c->j_host + slot, 1);
+    TEA_RETURN_IF(launch_jacobi(c, from, *to, true, sums[c->j_sub ^ 1], sums[c->j_sub],
+                                c->j_host_dev + slot));
+    c->j_sub ^= 1;
+    c->j_buf[c->jra++] = to;
   }
   return TEA_HIP_OK;
 }
@@ -921,6 +1065,16 @@ int ppcg_two_steps(tea_hip_chunk* c, double a0, double b0, double a1,
 
 }  // namespace
 
+int jacobi_settle(tea_hip_chunk* c) {
+  if (c->jra) {
+    c->jra = 0;
+    c->ra_dirty = true;
+  }
+  if (!c->j_ring) return TEA_HIP_OK;
+  c->j_ring = false;
+  return launch_halo_of(c, c->field[TEA_FIELD_R]);
+}
+
 int apply_pre_halo(tea_hip_chunk* c) {
   if (c->pre_halo < 0) return TEA_HIP_OK;
   static const int ext[4] = {-1, -1, -1, -1};
@@ -974,50 +1128,65 @@ int tea_hip_jacobi_init(tea_hip_chunk* c, int coefficient, double rx,
 }
 
 int tea_hip_jacobi_iterate(tea_hip_chunk* c, double* error) {
-  TEA_ENTER(c);
+  TEA_CHECK_ARG(c != nullptr, "null chunk handle");
   TEA_CHECK_ARG(error != nullptr, "null error");
-  TEA_RETURN_IF(apply_pending(c));
+  TEA_HIP_TRY(hipSetDevice(c->device));
   double** f = c->field;
-  const Geo g = c->geo;
-  if (!(c->fused && use_pair_blocks(c, 1))) {
-    TEA_RETURN_IF(launch_each_cell(c, K_JACOBI_COPY_U,
-                                   CopyAllBody{f[TEA_FIELD_U], f[TEA_FIELD_R]}));
-    {
-      Timed t(c, K_JACOBI_ITERATE);
-      hipLaunchKernelGGL(
-          (span_kernel<1, JacobiBody>), span_grid(c), dim3(kBlock), 0,
-          c->stream, g,
-          JacobiBody{f[TEA_FIELD_U], f[TEA_FIELD_U0], f[TEA_FIELD_R],
-                     f[TEA_FIELD_KX], f[TEA_FIELD_KY], g.x},
-          c->partials, c->nspan, c->ngroup == 1 ? 1 : 0);
+  // The U halo update that came just before: folded into the sweep.
+  const bool folded = c->pre_halo == TEA_HALO_U && !c->held && c->faces_ok_u && c->fused &&
+                      use_pair_blocks(c, 1);
+  if (c->jra && folded) {
+    c->pre_halo = -1;
+    // The queued sweep made the new u in a spare buffer; the old u is r now
+    // and r's buffer is spare.
+    double* t = *c->j_buf[0];
+    *c->j_buf[0] = f[TEA_FIELD_R];
+    f[TEA_FIELD_R] = f[TEA_FIELD_U];
+    f[TEA_FIELD_U] = t;
+    c->j_buf[0] = c->j_buf[1];
+    c->jra -= 1;
+    c->j_ring = true;
+    c->j_since += 1;
+    c->j_slot ^= 1;
+    TEA_RETURN_IF(jacobi_queue(c));
+  } else {
+    // The sequence goes on, past the sweep that was to be its last: the guess
+    // is dropped.
+    const bool goes_on = folded && c->j_ring;
+    if (folded) {
+      c->pre_halo = -1;
+      c->j_ring = false;  // r is about to be replaced
     }
-    TEA_HIP_TRY(hipGetLastError());
-    return finish_reduction(c, 1, error);
+    TEA_ENTER(c);
+    TEA_RETURN_IF(apply_pending(c));
+    if (!(c->fused && use_pair_blocks(c, 1))) {
+      TEA_RETURN_IF(launch_each_cell(c, K_JACOBI_COPY_U,
+                                     CopyAllBody{f[TEA_FIELD_U], f[TEA_FIELD_R]}));
+      return sum_over_cells<1>(c, K_JACOBI_ITERATE,
+                               JacobiBody{f[TEA_FIELD_U], f[TEA_FIELD_U0], f[TEA_FIELD_R],
+                                          f[TEA_FIELD_KX], f[TEA_FIELD_KY], c->geo.x},
+                               error);
+    }
+    const bool ahead = jacobi_ahead_possible(c) && ensure_jacobi_ahead(c);
+    TEA_RETURN_IF(launch_jacobi(c, f[TEA_FIELD_U], f[TEA_FIELD_R], folded, c->sub, nullptr,
+                                nullptr));
+    // The new u is in r's buffer; the old u becomes r (the reference's copy).
+    std::swap(f[TEA_FIELD_U], f[TEA_FIELD_R]);
+    c->j_ring = folded;
+    c->j_sub = 0;
+    c->j_period = goes_on ? 0 : c->j_since;
+    c->j_since = goes_on ? c->j_since + 1 : 1;
+    if (ahead) TEA_RETURN_IF(jacobi_queue(c));
   }
-  {
-    Timed t(c, K_JACOBI_FUSED);
-    // Workgroups of stack_factor(c) blocks one row apart (tea_hip_impl.h).
-    const int ks = stack_factor(c), S = stack_rows(c);
-    const dim3 grid = stacked_grid(c, ks), block(kBlock * ks);
-    if (ks == 1)
-      hipLaunchKernelGGL(jacobi_pair_kernel<1>, grid, block, 0, c->stream, g, f[TEA_FIELD_U],
-                         f[TEA_FIELD_R], f[TEA_FIELD_U0], f[TEA_FIELD_KX], f[TEA_FIELD_KY],
-                         c->sub, c->nblk, S);
-    else if (ks == 2)
-      hipLaunchKernelGGL(jacobi_pair_kernel<2>, grid, block, 0, c->stream, g, f[TEA_FIELD_U],
-                         f[TEA_FIELD_R], f[TEA_FIELD_U0], f[TEA_FIELD_KX], f[TEA_FIELD_KY],
-                         c->sub, c->nblk, S);
-    else
-      hipLaunchKernelGGL(jacobi_pair_kernel<4>, grid, block, 0, c->stream, g, f[TEA_FIELD_U],
-                         f[TEA_FIELD_R], f[TEA_FIELD_U0], f[TEA_FIELD_KX], f[TEA_FIELD_KY],
-                         c->sub, c->nblk, S);
+  if (c->jra == 0) {
+    // No sweep behind it to sum its error.
+    int len;
+    TEA_RETURN_IF(launch_span_finish(c, 1, &len, 0, true, c->j_sub ? c->sub2 : c->sub));
+    return finish_reduction_n(c, 1, len, error);
   }
-  TEA_HIP_TRY(hipGetLastError());
-  // The new u is in r's buffer; the old u becomes r (the reference's copy).
-  std::swap(f[TEA_FIELD_U], f[TEA_FIELD_R]);
-  int len = c->nspan;
-  TEA_RETURN_IF(launch_span_finish(c, 1, &len, 0, true));
-  return finish_reduction_n(c, 1, len, error);
+  TEA_RETURN_IF(wait_host_values(c, c->j_host + c->j_slot, 1));
+  *error = c->j_host[c->j_slot];
+  return TEA_HIP_OK;
 }
 
 int tea_hip_cheby_init(tea_hip_chunk* c, double theta) {

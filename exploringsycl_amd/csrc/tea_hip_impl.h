@@ -1036,6 +1036,21 @@ struct tea_hip_chunk {
                                // sum, scalar}
   double* mra_host_dev = nullptr;
 
+  // Run-ahead of the Jacobi sweeps (solvers.hip): up to two sweeps queued
+  // beyond the one the host asked for, the first into j_buf[0] (one of the
+  // spare buffers), each with the U halo update before it; and whether the
+  // ring of r, the u of before the last sweep, still lacks that update.
+  int jra = 0;
+  bool j_off = false;          // a buffer it needs could not be allocated
+  double** j_buf[2] = {};
+  bool j_ring = false;
+  int j_sub = 0;               // the block sums (sub or sub2) of the newest sweep
+  int j_slot = 0;              // host slot of the last sweep the host asked for
+  int j_since = 0, j_period = 0;  // sweeps since the last restart, and between
+                                  // the last two
+  double* j_host = nullptr;    // pinned, 2 slots
+  double* j_host_dev = nullptr;
+
   // Waiting for a reduction by its values: launch_span_finish(..., poll)
   // fills the first partial of arrays 0 .. poll_nr-1 with a sentinel, and the
   // finish waits until the finisher has overwritten them all (or the stream
@@ -1173,6 +1188,9 @@ enum { kHeldNone = 0, kHeldPpcg = 1, kHeldCheby = 2 };
 // older than a held step: a step is held with at most u += alpha p pending,
 // and the CG entry points run a held step before they defer new work.
 int apply_pending(tea_hip_chunk* c);
+// Drops Jacobi sweeps in flight and makes r's ring what the halo update of the
+// u it was leaves (solvers.hip).
+int jacobi_settle(tea_hip_chunk* c);
 // The deferred CG work alone (cg.hip).
 int apply_cg_pending(tea_hip_chunk* c);
 // The held FP64 u updates alone, with their U halo update (cg.hip).
@@ -1209,6 +1227,8 @@ int launch_precondition(tea_hip_chunk* c, int use_net, int slot, int* len);
 // Makes the held-back u updates on their own, oldest first (mpcg.hip).
 int apply_mp_hold(tea_hip_chunk* c);
 
+// The depth-1 reflective update of one field's x*y array, all faces external.
+int launch_halo_of(tea_hip_chunk* c, double* field);
 // One reflective-halo launch (all flagged fields and external faces).
 int launch_halos(tea_hip_chunk* c, int depth, const int neighbours[4],
                  const int fields[6]);
@@ -1226,6 +1246,7 @@ int mra_discard(tea_hip_chunk* c);
   TEA_CHECK_ARG((c) != nullptr, "null chunk handle");     \
   TEA_HIP_TRY(hipSetDevice((c)->device));                 \
   TEA_RETURN_IF(::tea::mra_discard(c));                   \
+  TEA_RETURN_IF(::tea::jacobi_settle(c));                 \
   (c)->mra_synced = false;                                \
   if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c))
 
@@ -1241,6 +1262,7 @@ int mra_discard(tea_hip_chunk* c);
 #define TEA_FLUSH_HELD(c)                                                  \
   do {                                                                     \
     TEA_RETURN_IF(::tea::mra_discard(c));                                  \
+    TEA_RETURN_IF(::tea::jacobi_settle(c));                                \
     if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c));                 \
     TEA_FLUSH_HELD_KEEP_U(c);                                              \
   } while (0)

@@ -1,0 +1,94 @@
+"""Jacobi sweeps with the U halo update folded in and two sweeps queued ahead,
+against sweeps on their own: without either (TEA_HIP_PAIRS=0) and with the
+update folded in only (TEA_HIP_RUN_AHEAD=0).  The same errors and fields bit
+for bit, also where other calls come between the sweeps."""
+
+import os
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _chunk(x, y, h, env):
+    from exploringsycl_amd.chunk import DeviceChunk
+    old = {n: os.environ.get(n) for n in env}
+    os.environ.update(env)
+    try:
+        return DeviceChunk(x, y, h)
+    finally:
+        for n in env:
+            if old[n] is None:
+                del os.environ[n]
+            else:
+                os.environ[n] = old[n]
+
+
+def _between(c, what, seen):
+    if what == "read":
+        seen.extend(c.read(n) for n in ("u", "r"))
+    elif what == "residual":
+        c.calculate_residual()
+        seen.append(np.array([c.calculate_2norm("r")]))
+        c.local_halos(1, ["u"])
+    elif what == "halo2":
+        c.local_halos(2, ["u"])
+    elif what == "twice":
+        c.local_halos(1, ["u"])
+    elif what == "other halos":
+        c.local_halos(1, ["energy1"])
+    elif what == "cheby":
+        c.cheby_init(3.0)
+        c.local_halos(1, ["u"])
+        for _ in range(3):
+            c.cheby_iterate(0.3, 0.4)
+            c.local_halos(1, ["u"])
+    elif what == "write":
+        c.write("u", np.full(c.x * c.y, 2.5))
+    elif what == "init":
+        c.jacobi_init(1, 0.8, 1.3)
+        c.copy_u()
+        c.local_halos(1, ["u"])
+
+
+def _run(x, y, h, sweeps, between, env):
+    rng = np.random.default_rng(x + y)
+    errors, seen = [], []
+    with _chunk(x, y, h, env) as c:
+        c.set_chunk_data(0.0, 0.0, 0.1, 0.1)
+        c.write("density", rng.uniform(0.1, 100.0, x * y))
+        c.write("energy", rng.uniform(0.1, 25.0, x * y))
+        c.jacobi_init(1, 0.8, 1.3)
+        c.copy_u()
+        c.local_halos(1, ["u"])
+        for it in range(sweeps):
+            errors.append(c.jacobi_iterate())
+            c.local_halos(1, ["u"])
+            if it % 5 == 4 and it // 5 < len(between):
+                _between(c, between[it // 5], seen)
+        seen.extend(c.read(n) for n in ("u", "r"))
+        seen.append(np.array(c.field_summary()))
+    return np.array(errors), seen
+
+
+BETWEEN = ("read", "residual", "halo2", "twice", "other halos", "cheby", "write", "init")
+
+
+@pytest.mark.parametrize("x,y,h,between", [
+    (20, 12, 2, BETWEEN),          # less than a block
+    (64, 33, 3, BETWEEN), (65, 33, 2, BETWEEN),
+    (1025, 67, 2, ("residual", "read")),   # odd, rows of two blocks
+    (1024, 130, 2, ("residual",)),         # stacked blocks
+    (2048, 2048, 2, ()),           # 16 groups: the most that one block sums
+    (2050, 2048, 2, ("read",)),    # one more: no sweep ahead
+])
+def test_jacobi_ahead(x, y, h, between):
+    sweeps = 5 * len(between) + 7
+    want = _run(x, y, h, sweeps, between, {"TEA_HIP_PAIRS": "0"})
+    for env in ({"TEA_HIP_RUN_AHEAD": "0"}, {"TEA_HIP_RUN_AHEAD": "1"}):
+        got = _run(x, y, h, sweeps, between, env)
+        assert np.array_equal(want[0], got[0])
+        assert len(want[1]) == len(got[1])
+        for a, b in zip(want[1], got[1]):
+            assert np.array_equal(a, b, equal_nan=True)
