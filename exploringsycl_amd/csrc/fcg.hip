@@ -1408,13 +1408,18 @@ __global__ __launch_bounds__(kGammaThreads) void joint_gamma_kernel(
 int ensure_fcg_buffers(tea_hip_chunk* c) {
   if (c->fcg_z) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
-  if (hipMalloc(&c->fcg_z_alt, bytes) != hipSuccess ||
-      hipMalloc(&c->fcg_z, bytes) != hipSuccess) {
+  if (hipMalloc(&c->fcg_z, bytes) != hipSuccess) {
     c->fcg_z = nullptr;
     set_error("hipMalloc of the FCG z buffer failed");
     return TEA_HIP_ENOMEM;
   }
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_z, 0, bytes, c->stream));
+  if (hipMalloc(&c->fcg_z_alt, bytes) != hipSuccess) {
+    c->fcg_z_alt = nullptr;
+    (void)hipGetLastError();
+    c->mra_off = true;  // no run-ahead without it
+    return TEA_HIP_OK;
+  }
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_z_alt, 0, bytes, c->stream));
   return TEA_HIP_OK;
 }

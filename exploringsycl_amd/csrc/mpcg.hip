@@ -729,7 +729,7 @@ __global__ __launch_bounds__(kBlock) void mp_convert_all_kernel(
   p32a[i] = pv;
   p32b[i] = pv;
   p32c[i] = pv;
-  p32d[i] = pv;
+  if (p32d) p32d[i] = pv;
   r32[i] = (float)r[i];
 }
 
@@ -785,11 +785,18 @@ struct MpTrueResidualBody {
 int ensure_mp_buffers(tea_hip_chunk* c) {
   if (c->mp_r) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
-  float** bufs[] = {&c->mp_p[0], &c->mp_p[1], &c->mp_p[2], &c->mp_p[3], &c->mp_w, &c->mp_kx,
-                    &c->mp_ky, &c->mp_r_alt, &c->mp_w_alt, &c->mp_r};
+  // The last three, for the run-ahead alone, may be missing.
+  float** bufs[] = {&c->mp_p[0], &c->mp_p[1], &c->mp_p[2], &c->mp_w, &c->mp_kx, &c->mp_ky,
+                    &c->mp_r, &c->mp_p[3], &c->mp_r_alt, &c->mp_w_alt};
   for (float** b : bufs) {
+    if (*b) continue;
     if (hipMalloc(b, bytes) != hipSuccess) {
       *b = nullptr;
+      (void)hipGetLastError();
+      if (c->mp_r) {
+        c->mra_off = true;
+        break;
+      }
       set_error("hipMalloc of an FP32 CG buffer failed");
       return TEA_HIP_ENOMEM;
     }
@@ -838,7 +845,7 @@ constexpr int kMraSlotW = 0, kMraSlotR = 1;
 bool mra_consume(const tea_hip_chunk* c) { return c->nblk <= kConsumeBlocks; }
 
 bool mra_possible(const tea_hip_chunk* c) {
-  return c->ra_enabled && c->fused && c->poll && c->mra_fail < 3 && use_pair_blocks(c, 1) &&
+  return c->ra_enabled && c->fused && c->poll && !c->mra_off && c->mra_fail < 3 && use_pair_blocks(c, 1) &&
          use_pair_blocks(c, 2);
 }
 
@@ -855,27 +862,26 @@ void swap_buf(T*& a, T*& b) {
   b = t;
 }
 
-int ensure_mra(tea_hip_chunk* c) {
-  if (c->mra_host) return TEA_HIP_OK;
-  if (!c->u_alt && hipMalloc(&c->u_alt, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
+// Whether the run-ahead's buffers are there (else there is no run-ahead).
+bool ensure_mra(tea_hip_chunk* c) {
+  if (c->mra_host) return true;
+  if (!c->u_alt && hipMalloc(&c->u_alt, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess)
     c->u_alt = nullptr;
-    set_error("hipMalloc of a run-ahead buffer failed");
-    return TEA_HIP_ENOMEM;
-  }
-  if (!c->mra_dev && hipMalloc(&c->mra_dev, 3 * sizeof(double)) != hipSuccess) {
+  if (!c->mra_dev && hipMalloc(&c->mra_dev, 3 * sizeof(double)) != hipSuccess)
     c->mra_dev = nullptr;
-    set_error("hipMalloc of the run-ahead scalars failed");
-    return TEA_HIP_ENOMEM;
-  }
   double* host = nullptr;
-  if (hipHostMalloc(&host, 16 * sizeof(double),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-    set_error("hipHostMalloc of the run-ahead slots failed");
-    return TEA_HIP_ENOMEM;
+  if (c->u_alt && c->mra_dev &&
+      hipHostMalloc(&host, 16 * sizeof(double),
+                    hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
+    if (hipHostGetDevicePointer((void**)&c->mra_host_dev, host, 0) == hipSuccess) {
+      c->mra_host = host;
+      return true;
+    }
+    (void)hipHostFree(host);
   }
-  TEA_HIP_TRY(hipHostGetDevicePointer((void**)&c->mra_host_dev, host, 0));
-  c->mra_host = host;
-  return TEA_HIP_OK;
+  (void)hipGetLastError();
+  c->mra_off = true;
+  return false;
 }
 
 // Offset of a slot in mra_host.
@@ -939,7 +945,7 @@ int plan_mp_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
   *s = MpStep{};
   const float* r = ahead ? c->mp_r_alt : c->mp_r;
   const float* z = ahead ? c->fcg_z_alt : c->fcg_z;
-  s->a = MpArgs{c->mp_p[cur], c->mp_p[mp_next(cur)], fcg ? z : r, u,
+  s->a = MpArgs{c->mp_p[cur], c->mp_p[mp_next(c, cur)], fcg ? z : r, u,
                 ahead ? c->mp_w_alt : c->mp_w, c->mp_kx, c->mp_ky, r, alpha, beta,
                 apply_u ? 1 : 0, apply_p ? 1 : 0, nullptr, nullptr, 0.0, 0.0,
                 ahead ? c->u_alt : u, ahead ? c->mra_dev : nullptr};
@@ -1002,7 +1008,7 @@ void commit_mp_step(tea_hip_chunk* c, const MpStep& s, double alpha) {
   }
   if (s.um && s.a.u_out != s.a.u) swap_buf(c->field[TEA_FIELD_U], c->u_alt);
   if (s.a.w != c->mp_w) swap_buf(c->mp_w, c->mp_w_alt);
-  if (s.a.apply_p) c->mp_cur = mp_next(c->mp_cur);
+  if (s.a.apply_p) c->mp_cur = mp_next(c, c->mp_cur);
 }
 
 // Queues the r-step (with FCG also z = M(r)) behind the newest w-step.
@@ -1063,8 +1069,7 @@ int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
     c->mra_w = false;
     c->mra_fail = 0;
   } else if (use_pair_blocks(c, 1)) {
-    ahead = mra_possible(c);
-    if (ahead) TEA_RETURN_IF(ensure_mra(c));
+    ahead = mra_possible(c) && ensure_mra(c);
     MpStep s;
     TEA_RETURN_IF(plan_mp_w(c, fcg, alpha, apply_u, beta, apply_p, false, &s));
     TEA_RETURN_IF(launch_mp_step(c, s, fcg, RaScalar{}));
@@ -1077,7 +1082,7 @@ int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
   } else {
     if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
     const int cur = c->mp_cur, sg = c->ngroup == 1 ? 1 : 0;
-    const MpArgs a{c->mp_p[cur], c->mp_p[mp_next(cur)], fcg ? c->fcg_z : c->mp_r,
+    const MpArgs a{c->mp_p[cur], c->mp_p[mp_next(c, cur)], fcg ? c->fcg_z : c->mp_r,
                    c->field[TEA_FIELD_U], c->mp_w, c->mp_kx, c->mp_ky, c->mp_r, alpha, beta,
                    apply_u ? 1 : 0, apply_p ? 1 : 0, nullptr, nullptr, 0.0, 0.0,
                    c->field[TEA_FIELD_U], nullptr};
@@ -1091,7 +1096,7 @@ int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
                            c->geo, a, c->partials, c->nspan, sg);
     }
     TEA_HIP_TRY(hipGetLastError());
-    if (apply_p) c->mp_cur = mp_next(cur);
+    if (apply_p) c->mp_cur = mp_next(c, cur);
   }
   if (ahead) {
     const int slot = c->mra_wi;

@@ -834,9 +834,9 @@ const float* output(tea_nn* n);
 
 // The mixed-precision p buffers: a ring of four, so that a w-step can hold
 // the u updates of two steps back and a w-step that runs ahead writes a
-// buffer no update still needs.
+// buffer no update still needs (three, without the run-ahead, where there is
+// no memory for the fourth).
 constexpr int kMpRing = 4;
-inline int mp_next(int i) { return i + 1 == kMpRing ? 0 : i + 1; }
 
 // One FP64 CG w-step on the pair kernels: its arguments, the u update it makes
 // (um: none, its own where a.apply_u, or the two held ones and its own) and
@@ -1020,6 +1020,7 @@ struct tea_hip_chunk {
   bool mra_fcg = false;        // the passes belong to FCG
   int mra_coarse = 0;          // use_net of the last preconditioner call
   int mra_fail = 0;            // consecutive mismatches (3 turn it off)
+  bool mra_off = false;        // a buffer it needs could not be allocated
   int mra_since = 0, mra_period = 0;  // r-steps since the last refresh, and
                                       // how many the last two were apart
   int mra_wi = 0, mra_ri = 0;  // host slots of the newest w-step and r-step
@@ -1279,6 +1280,10 @@ int mra_discard(tea_hip_chunk* c);
 #define TEA_ENTER(c)   \
   TEA_ENTER_HELD(c);   \
   TEA_FLUSH_HELD(c)
+
+inline int mp_next(const tea_hip_chunk* c, int i) {
+  return i + 1 == kMpRing || !c->mp_p[i + 1] ? 0 : i + 1;
+}
 
 inline dim3 span_grid(const tea_hip_chunk* c) { return dim3(c->nspan); }
 inline dim3 pair_grid(const tea_hip_chunk* c) { return dim3(c->nblk); }
