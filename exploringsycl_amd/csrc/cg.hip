@@ -484,7 +484,7 @@ template <bool APPLY_P, int KS, int UM, bool CONSUME>
 __global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs a, RaScalar sc,
                                                                double* sub, int nblk, int S) {
   int tid;
-  const int blk = stacked_block<KS, kBlock>(S, &tid);
+  const int blk = stacked_block<KS, kBlock>(S, &tid, g.bands);
   const int lane = threadIdx.x & (kWave - 1);
   FusedPair s;
   fused_pair_index(g, blk < nblk ? blk * kPairBlock + 2 * tid : g.n, s);
@@ -563,7 +563,7 @@ template <bool CONSUME>
 __global__ __launch_bounds__(kBlock) void fused_r1_kernel(
     Geo g, const double* r, double* r_out, const double* __restrict__ w, double value,
     RaScalar sc, double* sub, int nblk) {
-  const int blk = blockIdx.x;
+  const int blk = band_index(g.bands);
   const int e = blk * kPairBlock + 2 * threadIdx.x;
   const int row = e < g.n ? (int)g.dx.div((uint32_t)e) : 0;
   const int kk = e - row * g.x;
@@ -658,10 +658,11 @@ struct NormBody {
 // The 2-norm over cell pairs, one pair per lane (more than one group): 8 bytes per cell, the sum tree's first level in-lane.
 __global__ __launch_bounds__(kBlock) void norm_pair_kernel(
     Geo g, const double* __restrict__ b, double* sub, int nblk) {
-  const PairAt q = pair_at(g, blockIdx.x * kPairBlock + 2 * threadIdx.x);
+  const int blk = band_index(g.bands);
+  const PairAt q = pair_at(g, blk * kPairBlock + 2 * threadIdx.x);
   const double2 v = ld2_nt(b, q.ic);
   const double s[1] = {(q.in0 ? v.x * v.x : 0.0) + (q.in1 ? v.y * v.y : 0.0)};
-  block_sums_pairs<1>(s, sub, nblk, blockIdx.x, threadIdx.x);
+  block_sums_pairs<1>(s, sub, nblk, blk, threadIdx.x);
 }
 
 struct FinaliseBody {

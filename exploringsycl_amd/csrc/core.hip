@@ -402,6 +402,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   tea_hip_chunk* c = new tea_hip_chunk();
   c->device = device;
   c->geo.x = x;
+  c->geo.bands = bands_for(x);
   c->geo.y = y;
   c->geo.h = halo_depth;
   c->geo.n = (int)n;

@@ -157,7 +157,7 @@ __global__ __launch_bounds__(kBlock) void fcg_z1_kernel(
     Geo g, const float* __restrict__ r, const float* __restrict__ kx,
     const float* __restrict__ ky, const float* __restrict__ w, CoarseTerm t0,
     CoarseTerm t1, float* __restrict__ z, double* sub, int nblk) {
-  const int blk = blockIdx.x;
+  const int blk = band_index();
   const int lane = threadIdx.x & (kWave - 1);
   const int x = g.x;
   const int e = blk * kPairBlock + 2 * threadIdx.x;
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(kQuadThreads) void fcg_z4_kernel(
     Geo g, const float* __restrict__ r, const float* __restrict__ kx,
     const float* __restrict__ ky, const float* __restrict__ w, CoarseTerm t0,
     CoarseTerm t1, float* __restrict__ z, double* sub, int nblk) {
-  const int blk = blockIdx.x;
+  const int blk = band_index();
   const int lane = threadIdx.x & (kWave - 1);
   const int x = g.x;
   const int e = blk * kQuadBlock + 4 * threadIdx.x;

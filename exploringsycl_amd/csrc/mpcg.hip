@@ -356,7 +356,7 @@ __device__ inline double mp_scalar(const RaScalar& s, double value) {
 template <bool DOT2, bool CONSUME>
 __global__ __launch_bounds__(kBlock) void mp_w1_kernel(Geo g, MpArgs a, RaScalar sc,
                                                        double* sub, int nblk) {
-  const int blk = blockIdx.x;
+  const int blk = band_index();
   const int lane = threadIdx.x & (kWave - 1);
   MpPair s;
   mp_pair_index(g, blk * kPairBlock + 2 * threadIdx.x, s);
@@ -601,7 +601,7 @@ template <bool RW, bool CONSUME>
 __global__ __launch_bounds__(kBlock) void mp_r1_kernel(
     Geo g, const float* r, float* r_out, const float* __restrict__ w, double value, RaScalar sc,
     double* sub, int nblk) {
-  const int blk = blockIdx.x;
+  const int blk = band_index();
   const int e = blk * kPairBlock + 2 * threadIdx.x;
   const int row = e < g.n ? (int)g.dx.div((uint32_t)e) : 0;
   const int kk = e - row * g.x;
@@ -626,7 +626,7 @@ template <bool RW, bool CONSUME>
 __global__ __launch_bounds__(kQuadThreads) void mp_r4_kernel(
     Geo g, const float* r, float* r_out, const float* __restrict__ w, double value, RaScalar sc,
     double* sub, int nblk) {
-  const int blk = blockIdx.x;
+  const int blk = band_index();
   const int e = blk * kQuadBlock + 4 * threadIdx.x;
   const int row = e < g.n ? (int)g.dx.div((uint32_t)e) : 0;
   const int kk = e - row * g.x;
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(kBlock) void mp_residual1_kernel(
     Geo g, const double* __restrict__ u, const double* __restrict__ u0,
     const double* __restrict__ kx, const double* __restrict__ ky, float* __restrict__ r32,
     const float* __restrict__ w, double* sub, int nblk) {
-  const int blk = blockIdx.x;
+  const int blk = band_index();
   const int lane = threadIdx.x & (kWave - 1);
   const int x = g.x;
   const int e = blk * kPairBlock + 2 * threadIdx.x;

@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kBlock * KS) void jacobi_pair_kernel(
     const double* __restrict__ ky, double* sub, int nblk, int S,
     const double* __restrict__ prev, double* out) {
   int tid;
-  const int blk = stacked_block<KS, kBlock>(S, &tid);
+  const int blk = stacked_block<KS, kBlock>(S, &tid, g.bands);
   const int lane = threadIdx.x & (kWave - 1);
   const PairAt q = pair_at(g, blk < nblk ? blk * kPairBlock + 2 * tid : g.n);
   Operand o = load_operand(u_old, q, g.x, lane);
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(kBlock) void cheby_pair_kernel(
     const double* __restrict__ kx, const double* __restrict__ ky,
     double alpha, double beta) {
   const int lane = threadIdx.x & (kWave - 1);
-  const PairAt q = pair_at(g, blockIdx.x * kPairBlock + 2 * threadIdx.x);
+  const PairAt q = pair_at(g, band_index(g.bands) * kPairBlock + 2 * threadIdx.x);
   const Operand o = load_operand(u_old, q, g.x, lane);
   const Faces f = load_faces(kx, ky, q, g.x, lane);
   const double2 s0 = ld2_nt(u0, q.ir);
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(kBlock) void ppcg_pair_kernel(
     const double* __restrict__ kx, const double* __restrict__ ky,
     double alpha, double beta) {
   const int lane = threadIdx.x & (kWave - 1);
-  const PairAt q = pair_at(g, blockIdx.x * kPairBlock + 2 * threadIdx.x);
+  const PairAt q = pair_at(g, band_index(g.bands) * kPairBlock + 2 * threadIdx.x);
   const Operand o = load_operand(sd_old, q, g.x, lane);
   const Faces f = load_faces(kx, ky, q, g.x, lane);
   const double2 rv = ld2_nt(r, q.ir);

@@ -70,6 +70,7 @@ struct Geo {
   int x, y, h;
   int n;      // x*y
   FastDiv dx; // division by x
+  int bands = 0;  // FP64 passes in XCD bands (band_index)
 };
 
 __device__ inline bool interior(const Geo& g, int kk, int jj) {
@@ -99,6 +100,33 @@ __device__ inline int xcd_span(int b, int nb) {
   const int per = nb / kNumXcd, rem = nb % kNumXcd;
   return xcd * per + (xcd < rem ? xcd : rem) + idx;
 }
+
+// The workgroup's place in a pair- or quad-per-thread pass: in segments of
+// 8 * kBandBlocks blocks each XCD takes kBandBlocks consecutive blocks, so a
+// row is re-read, as the row above or below, from the L2 that read it first,
+// passes find in it what the pass before wrote, and the chip still streams
+// through memory as one front (one band per XCD over the whole grid: 4-7%
+// slower from 4096^2 on).  In launch order each row comes into up to three
+// L2s.  FP64 CG per iteration, launch order against bands of 128 blocks (64
+// and 256 within 1%): 1000^2 24.6 -> 21.5 us, 1500^2 50.9 -> 39.8, 3000^2 166.6
+// -> 138.6, 6000^2 612 -> 534; Jacobi sweeps 2048^2 44.5 -> 38.7; mixed
+// precision 1024^2 22.8 -> 20.9, 3001x2999 119.1 -> 105.2, 4096^2 158.1 ->
+// 156.4.
+// KS: blocks per workgroup (stacked_block).
+constexpr int kBandBlocks = 128;
+template <int KS = 1>
+__device__ inline int band_index(bool bands = true) {
+  if (!bands) return (int)blockIdx.x;
+  constexpr int seg_len = kNumXcd * kBandBlocks / KS;
+  const int seg = (int)blockIdx.x / seg_len * seg_len, left = (int)gridDim.x - seg;
+  return seg + xcd_span((int)blockIdx.x - seg, left < seg_len ? left : seg_len);
+}
+// FP64 passes keep the launch order where rows are 8 blocks (or a multiple)
+// and up to 48 cells long: the rows above and below then lie on the same XCD
+// anyway, and the plain front is 1% faster (4096^2 249.6 against 251.5 us,
+// x = 4124 185.9 against 188.2; even at x = 4156, where a fifth of the cells
+// above is on another XCD; x = 4060 193.2 against 182.1).
+inline int bands_for(int x) { return x < kNumXcd * 512 || x % (kNumXcd * 512) > 48; }
 
 // Cross-lane moves on the VALU's data-parallel-primitive (DPP) path instead
 // of LDS permutes.  CTRL is a DPP control: 0x130 wave_shl:1 (lane l takes
@@ -348,11 +376,7 @@ __device__ inline void st2_nt(float* p, int i, bool in0, bool in1, float v0,
 // store it in sub[q * sub_stride + block], and span_finish_kernel (or, for
 // small grids, the next pass itself: consume_sums) combines them.
 //
-// These kernels keep the launch order of blocks (no xcd_span renumbering):
-// the hardware deals consecutive blocks round-robin to the 8 XCDs, so the
-// whole chip streams through memory as one front, and rows re-read above and
-// below a block were fetched moments earlier (measured at 4096^2: 8% faster
-// than one contiguous range per XCD for 512-cell blocks).
+// Which block a workgroup takes: band_index.
 
 constexpr int kPairBlock = 2 * kBlock;              // 512 cells
 constexpr int kSubPerSpan = kSpan / kPairBlock;     // 8
@@ -409,12 +433,9 @@ __device__ inline void block_sums_pairs(const double (&v)[NR], double* sub, int 
 // A 128-thread block over one 512-cell pair block, four cells per lane (x a
 // multiple of 4, so a quad never straddles a row and every quad, and the
 // quads one row up and down, are 16-byte aligned).  The block covers the
-// cells of a pair block so that, as there, the rows above and below a block
-// at x = 4100 lie 8 blocks back and ahead: on the same XCD, whose L2 has
-// them (with 1024-cell blocks they lie 4 blocks away, on another XCD: the
-// prolongation, which reads ky one row up, took 12-22% longer at 4096^2).  The in-lane sum ((v0 + v1) +
-// (v2 + v3)) is tree steps 1 and 2; the four DPP steps of wave_tree_dpp
-// then finish a 64-cell group in each 16-lane row, and (g0 + g1) + (g2 + g3)
+// cells of a pair block, so that the same XCD has them in both kinds of pass.
+// The in-lane sum ((v0 + v1) + (v2 + v3)) is tree steps 1 and 2; the four DPP
+// steps of wave_tree_dpp then finish a 64-cell group in each 16-lane row, and (g0 + g1) + (g2 + g3)
 // is the sum pair waves 2w and 2w + 1 combine to: the same tree, bit for bit.
 
 constexpr int kQuadThreads = kPairBlock / 4;  // 128
@@ -594,7 +615,8 @@ __global__ __launch_bounds__(kBlock) void span_kernel(Geo g, Body body,
 template <int NR, class Body>
 __global__ __launch_bounds__(kBlock) void pair_sum_kernel(Geo g, Body body, double* sub,
                                                           int nblk) {
-  const PairAt q = pair_at(g, blockIdx.x * kPairBlock + 2 * threadIdx.x);
+  const int blk = band_index(g.bands);
+  const PairAt q = pair_at(g, blk * kPairBlock + 2 * threadIdx.x);
   double a[NR], b[NR];
 #pragma unroll
   for (int k = 0; k < NR; ++k) a[k] = b[k] = 0.0;
@@ -602,7 +624,7 @@ __global__ __launch_bounds__(kBlock) void pair_sum_kernel(Geo g, Body body, doub
   if (q.in1) body(q.e + 1, q.kk + 1, q.row, b);
 #pragma unroll
   for (int k = 0; k < NR; ++k) a[k] = a[k] + b[k];
-  block_sums_pairs<NR>(a, sub, nblk, blockIdx.x, threadIdx.x);
+  block_sums_pairs<NR>(a, sub, nblk, blk, threadIdx.x);
 }
 
 // One thread per cell of the padded x*y range.
@@ -1310,10 +1332,11 @@ inline dim3 stacked_grid(const tea_hip_chunk* c, int ks) {
 // The block and thread index of the calling thread in a workgroup of KS
 // blocks of T threads (blk >= nblk for the unused blocks of the last row).
 template <int KS, int T>
-__device__ inline int stacked_block(int S, int* tid) {
+__device__ inline int stacked_block(int S, int* tid, bool bands = true) {
   *tid = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x % T;
-  if (KS == 1) return (int)blockIdx.x;
-  return (int)(blockIdx.x % S) + S * ((int)(blockIdx.x / S) * KS + (int)threadIdx.x / T);
+  const int b = band_index<KS>(bands);
+  if (KS == 1) return b;
+  return b % S + S * (b / S * KS + (int)threadIdx.x / T);
 }
 
 }  // namespace tea
