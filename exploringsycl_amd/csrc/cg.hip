@@ -329,10 +329,10 @@ __device__ inline void fused_pair_load(const Geo& g, const FusedWArgs& a,
   s.KX = ld2(a.kx, ic);
   s.KY = ld2(a.ky, ir);
   s.KYt = ld2u(a.ky, ir + x);
-  if (UM == 3 || (UM == 1 && a.apply_u)) s.U = ld2_nt(a.u, ir);
+  if (UM == 3 || (UM == 1 && a.apply_u)) s.U = ld2_nt(a.u, ir, g.nt);
   if (UM == 3) {
-    s.H = ld2_nt(a.p_h, ir);
-    s.H2 = ld2_nt(a.p_h2, ir);
+    s.H = ld2_nt(a.p_h, ir, g.nt);
+    s.H2 = ld2_nt(a.p_h2, ir, g.nt);
   }
   // Issued with the pair's own loads so the wave waits once; ir - 1 and
   // ir + 2 are in range (ir is an interior pair's index or the safe one).
@@ -420,9 +420,9 @@ __device__ inline double fused_pair_compute(const Geo& g, const FusedWArgs& a,
     }
     ua = ua + alpha * s.P0.x;
     ub = ub + alpha * s.P0.y;
-    st2_nt(a.u_out, i, s.in0, s.in1, ua, ub);
+    st2_nt(a.u_out, i, s.in0, s.in1, ua, ub, g.nt);
   }
-  if (APPLY_P) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb);
+  if (APPLY_P) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb, g.nt);
   // Halo ring of boundary-adjacent cells (rare; per cell).  With the halo
   // refresh folded in it takes the new values; without, p (and u, where it
   // goes to another buffer) keeps its old ring.
@@ -570,12 +570,12 @@ __global__ __launch_bounds__(kBlock) void fused_r1_kernel(
   const bool in0 = e < g.n && interior(g, kk, row);
   const bool in1 = e < g.n && interior(g, kk + 1, row);
   const int i = (in0 || in1) ? e : 0;
-  const double2 rv = ld2_nt(r, i), wv = ld2_nt(w, i);
+  const double2 rv = ld2_nt(r, i, g.nt), wv = ld2_nt(w, i, g.nt);
   const double alpha = ra_scalar<CONSUME>(sc, value);
   const double ra = rv.x - alpha * wv.x;
   const double rb = rv.y - alpha * wv.y;
   const double v[1] = {(in0 ? ra * ra : 0.0) + (in1 ? rb * rb : 0.0)};
-  st2_nt(r_out, e, in0, in1, ra, rb);
+  st2_nt(r_out, e, in0, in1, ra, rb, g.nt);
   block_sums_pairs<1>(v, sub, nblk, blk, threadIdx.x);
 }
 
@@ -660,7 +660,7 @@ __global__ __launch_bounds__(kBlock) void norm_pair_kernel(
     Geo g, const double* __restrict__ b, double* sub, int nblk) {
   const int blk = band_index(g.bands);
   const PairAt q = pair_at(g, blk * kPairBlock + 2 * threadIdx.x);
-  const double2 v = ld2_nt(b, q.ic);
+  const double2 v = ld2_nt(b, q.ic, g.nt);
   const double s[1] = {(q.in0 ? v.x * v.x : 0.0) + (q.in1 ? v.y * v.y : 0.0)};
   block_sums_pairs<1>(s, sub, nblk, blk, threadIdx.x);
 }

@@ -402,10 +402,12 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   tea_hip_chunk* c = new tea_hip_chunk();
   c->device = device;
   c->geo.x = x;
-  c->geo.bands = bands_for(x);
   c->geo.y = y;
   c->geo.h = halo_depth;
   c->geo.n = (int)n;
+  c->geo.nt = n > kStreamCells;
+  c->geo.nt_half = n > kStreamCellsHalf;
+  c->geo.bands = bands_for(x);
   c->geo.dx = FastDiv((uint32_t)x);
   c->ngroup = (int)((n + kWave - 1) / kWave);
   c->nspan = (int)((n + kSpan - 1) / kSpan);

@@ -207,7 +207,7 @@ __device__ inline void mp_pair_load(const Geo& g, const MpArgs& a, MpPair& s) {
   s.KX = ld2(a.kx, ic);
   s.KY = ld2(a.ky, ir);
   s.KYt = ld2u(a.ky, ir + x);
-  s.U = ld2_nt(a.u, ir);
+  s.U = ld2_nt(a.u, ir, g.nt_half);
   if (DOT2) s.RD = ld2(a.rdot, ir);
   // Lanes 0 and 63 share each load instruction, at their own addresses
   // (lane 0's kx value is not used).
@@ -289,9 +289,9 @@ __device__ inline void mp_pair_compute(const Geo& g, const MpArgs& a,
     const double alpha = a.alpha_dev ? *a.alpha_dev : a.alpha;
     ua = s.U.x + alpha * (double)s.P0.x;
     ub = s.U.y + alpha * (double)s.P0.y;
-    st2_nt(a.u_out, i, s.in0, s.in1, ua, ub);
+    st2_nt(a.u_out, i, s.in0, s.in1, ua, ub, g.nt_half);
   }
-  if (a.apply_p) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb);
+  if (a.apply_p) st2_nt(a.p_new, i, s.in0, s.in1, ca, cb, g.nt_half);
   // Halo ring of boundary-adjacent cells (rare; per cell).
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
@@ -425,8 +425,8 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
   double2 UA = {}, UB = {};
   float2 HA = {}, HB = {}, GA = {}, GB = {};
   if (UM > 0) {
-    UA = ld2_nt(a.u, inA0 || inA1 ? ua : x + 2);
-    UB = ld2_nt(a.u, inB0 || inB1 ? ub : x + 2);
+    UA = ld2_nt(a.u, inA0 || inA1 ? ua : x + 2, g.nt_half);
+    UB = ld2_nt(a.u, inB0 || inB1 ? ub : x + 2, g.nt_half);
   }
   if (UM == 3) {
     HA = ld2(a.p_h, inA0 || inA1 ? ua : x + 2);
@@ -536,8 +536,8 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
                           u0[1] + alpha * (double)(hi ? aw : ay),
                           u0[2] + alpha * (double)(hi ? bz : bx),
                           u0[3] + alpha * (double)(hi ? bw : by)};
-    if (inA0 || inA1) st2_nt(a.u_out, ua, inA0, inA1, un[0], un[1]);
-    if (inB0 || inB1) st2_nt(a.u_out, ub, inB0, inB1, un[2], un[3]);
+    if (inA0 || inA1) st2_nt(a.u_out, ua, inA0, inA1, un[0], un[1], g.nt_half);
+    if (inB0 || inB1) st2_nt(a.u_out, ub, inB0, inB1, un[2], un[3], g.nt_half);
     // Halo ring of boundary-adjacent cells (rare; per cell).
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
@@ -550,7 +550,7 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
   if (any) {
     st4(a.w, e, in, s);
     if (a.apply_p) {
-      st4_nt(a.p_new, e, in, pc);
+      st4_nt(a.p_new, e, in, pc, g.nt_half);
 #pragma unroll
       for (int c = 0; c < 4; ++c)
         if (in[c]) ring_store(a.p_new, e + c, kk + c, row, x, xl, xr, yb, yt, pc[c]);
@@ -673,7 +673,7 @@ __global__ __launch_bounds__(kBlock) void mp_residual1_kernel(
   const int ir = any ? e : safe_pair(x);
   const double2 U = ld2(u, ic), Ut = ld2u(u, ir + x), Ub = ld2u(u, ir - x);
   const double2 KX = ld2(kx, ic), KY = ld2(ky, ir), KYt = ld2u(ky, ir + x);
-  const double2 B = ld2_nt(u0, ir);
+  const double2 B = ld2_nt(u0, ir, g.nt_half);
   const float2 W = ld2(w, ir);
   double UN = 0.0, KXN = 0.0;
   if (lane == 0 || lane == kWave - 1) {

@@ -251,44 +251,36 @@ __device__ inline double op5_hi(const Operand& o, const Faces& f) {
 // Stores both cells of a valid pair with one 16-byte streaming store (the
 // buffers hold room for the last pair of an odd number of cells).
 __device__ inline void st2_all(double* p, const PairAt& q, double v0,
-                               double v1) {
-  if (q.valid) st2_nt(p, q.e, true, true, v0, v1);
+                               double v1, int nt) {
+  if (q.valid) st2_nt(p, q.e, true, true, v0, v1, nt);
 }
 
-// The sum of the block sums in sub (at most 16 groups of 512 blocks), by one
-// block of at least four waves; thread 0 returns it.
-constexpr int kJacobiGroups = 16;
+// The sum of the block sums in sub (at most 128 groups of 512 blocks) by one
+// block, which thread 0 returns: each wave sums whole groups, the first the
+// groups (the reference's passes: 64 groups a tree, then the two trees).
+constexpr int kJacobiGroups = 2 * kWave;
 __device__ inline double block_total(const double* __restrict__ sub, int nblk) {
   __shared__ double gs[kJacobiGroups];
   const int lane = threadIdx.x & (kWave - 1), waves = blockDim.x / kWave;
-  const int stride = sub_stride(nblk);
-  for (int g = threadIdx.x / kWave; g < kJacobiGroups; g += waves) {
+  const int groups = sub_stride(nblk) / kGroupBlocks;
+  if ((int)threadIdx.x < kJacobiGroups && (int)threadIdx.x >= groups) gs[threadIdx.x] = 0.0;
+  for (int g = threadIdx.x / kWave; g < groups; g += waves) {
     const int i0 = kGroupBlocks * g + kSubPerSpan * lane;
-    double t = 0.0;
-    if (i0 < stride) {
-      const double2 a = ld2(sub, i0), b = ld2(sub, i0 + 2), c = ld2(sub, i0 + 4),
-                    d = ld2(sub, i0 + 6);
-      t = ((a.x + a.y) + (b.x + b.y)) + ((c.x + c.y) + (d.x + d.y));
-    }
-    t = wave_tree_dpp(t);
+    const double2 a = ld2(sub, i0), b = ld2(sub, i0 + 2), c = ld2(sub, i0 + 4),
+                  d = ld2(sub, i0 + 6);
+    const double t = wave_tree_dpp(((a.x + a.y) + (b.x + b.y)) + ((c.x + c.y) + (d.x + d.y)));
     if (lane == 0) gs[g] = t;
   }
   __syncthreads();
-  double s[kJacobiGroups];
-#pragma unroll
-  for (int g = 0; g < kJacobiGroups; ++g) s[g] = gs[g];
-#pragma unroll
-  for (int m = 1; m < kJacobiGroups; m *= 2)
-#pragma unroll
-    for (int g = 0; g + m < kJacobiGroups; g += 2 * m) s[g] = s[g] + s[g + m];
-  return s[0];
+  if ((int)threadIdx.x >= kWave) return 0.0;
+  return wave_tree_dpp(gs[lane]) + wave_tree_dpp(gs[kWave + lane]);
 }
 
 // One sweep: 40 bytes per cell (u, u0, the two faces, the new u), bound by HBM
 // beyond the caches' size and by the cache and the launch below: 1000^2 (40 MB,
-// in the last-level cache) 12.4 us.  A sweep was 24.9 us there with the halo
-// update (3.5), the finisher (3.4) and the host's round trip between sweeps;
-// it is 12.9 us without them.
+// in the last-level cache) 12.4 us in launch order, 8.8 in bands and kept in that
+// cache.  A sweep was 24.9 us there with the halo update (3.5), the finisher
+// (3.4) and the host's round trip between sweeps.
 // With HALO the depth-1 U halo update that precedes it is folded in: a neighbour on the ring is the cell's own mirror image, and the ring of
 // the new u gets what that update leaves (the old values); the ring of the
 // old u is left to jacobi_settle.  With prev the first block also finishes
@@ -305,7 +297,7 @@ __global__ __launch_bounds__(kBlock * KS) void jacobi_pair_kernel(
   const PairAt q = pair_at(g, blk < nblk ? blk * kPairBlock + 2 * tid : g.n);
   Operand o = load_operand(u_old, q, g.x, lane);
   const Faces f = load_faces(kx, ky, q, g.x, lane);
-  const double2 s = ld2_nt(u0, q.ir);
+  const double2 s = ld2_nt(u0, q.ir, g.nt_half);
   double ra = o.c.y, lb = o.c.x;  // the pair's inner neighbours
   bool st0 = q.valid, st1 = q.valid;
   const int x = g.x, xl = g.h, xr = g.x - g.h - 1, yb = g.h, yt = g.y - g.h - 1;
@@ -330,7 +322,7 @@ __global__ __launch_bounds__(kBlock * KS) void jacobi_pair_kernel(
   const double n1 = q.in1 ? jacobi_cell(s.y, lb, o.r, o.b.y, o.t.y, f.kx.y,
                                         f.kx2, f.ky.y, f.kyt.y)
                           : o.c.y;
-  st2_nt(u_new, q.e, st0, st1, n0, n1);
+  st2_nt(u_new, q.e, st0, st1, n0, n1, g.nt_half);
   if (HALO) {
     if (q.in0) ring_store(u_new, q.e, q.kk, q.row, x, xl, xr, yb, yt, o.c.x);
     if (q.in1) ring_store(u_new, q.e + 1, q.kk + 1, q.row, x, xl, xr, yb, yt, o.c.y);
@@ -354,16 +346,16 @@ __global__ __launch_bounds__(kBlock) void cheby_pair_kernel(
   const PairAt q = pair_at(g, band_index(g.bands) * kPairBlock + 2 * threadIdx.x);
   const Operand o = load_operand(u_old, q, g.x, lane);
   const Faces f = load_faces(kx, ky, q, g.x, lane);
-  const double2 s0 = ld2_nt(u0, q.ir);
-  const double2 pv = ld2_nt(p, q.ir);
+  const double2 s0 = ld2_nt(u0, q.ir, g.nt);
+  const double2 pv = ld2_nt(p, q.ir, g.nt);
   if (!q.valid) return;
   const double w0 = op5_lo(o, f), w1 = op5_hi(o, f);
   const double r0 = s0.x - w0, r1 = s0.y - w1;
   const double p0 = alpha * pv.x + beta * r0, p1 = alpha * pv.y + beta * r1;
-  st2_nt(w, q.e, q.in0, q.in1, w0, w1);
-  st2_nt(r, q.e, q.in0, q.in1, r0, r1);
-  st2_nt(p, q.e, q.in0, q.in1, p0, p1);
-  st2_all(u_new, q, q.in0 ? o.c.x + p0 : o.c.x, q.in1 ? o.c.y + p1 : o.c.y);
+  st2_nt(w, q.e, q.in0, q.in1, w0, w1, g.nt);
+  st2_nt(r, q.e, q.in0, q.in1, r0, r1, g.nt);
+  st2_nt(p, q.e, q.in0, q.in1, p0, p1, g.nt);
+  st2_all(u_new, q, q.in0 ? o.c.x + p0 : o.c.x, q.in1 ? o.c.y + p1 : o.c.y, g.nt);
 }
 
 __global__ __launch_bounds__(kBlock) void ppcg_pair_kernel(
@@ -375,14 +367,14 @@ __global__ __launch_bounds__(kBlock) void ppcg_pair_kernel(
   const PairAt q = pair_at(g, band_index(g.bands) * kPairBlock + 2 * threadIdx.x);
   const Operand o = load_operand(sd_old, q, g.x, lane);
   const Faces f = load_faces(kx, ky, q, g.x, lane);
-  const double2 rv = ld2_nt(r, q.ir);
-  const double2 uv = ld2_nt(u, q.ir);
+  const double2 rv = ld2_nt(r, q.ir, g.nt);
+  const double2 uv = ld2_nt(u, q.ir, g.nt);
   if (!q.valid) return;
   const double r0 = rv.x - op5_lo(o, f), r1 = rv.y - op5_hi(o, f);
-  st2_nt(r, q.e, q.in0, q.in1, r0, r1);
-  st2_nt(u, q.e, q.in0, q.in1, uv.x + o.c.x, uv.y + o.c.y);
+  st2_nt(r, q.e, q.in0, q.in1, r0, r1, g.nt);
+  st2_nt(u, q.e, q.in0, q.in1, uv.x + o.c.x, uv.y + o.c.y, g.nt);
   st2_all(sd_new, q, q.in0 ? alpha * o.c.x + beta * r0 : o.c.x,
-          q.in1 ? alpha * o.c.y + beta * r1 : o.c.y);
+          q.in1 ? alpha * o.c.y + beta * r1 : o.c.y, g.nt);
 }
 
 template <class Body>
@@ -889,9 +881,9 @@ __global__ __launch_bounds__(kTSBlock) void cheby_two_step_kernel(
 // the driver makes before it, into the spare buffers, and takes one over; any
 // other call drops them.  A sweep's error is summed by the first block of the
 // sweep after it.  No sweep is queued past the one after which the driver
-// left the sequence the last time (its every-50th residual).  Up to 16 groups
-// (4.2 M cells): the sums of more are too much for one block, and a round trip
-// (about 6 us) is little of such a sweep.
+// left the sequence the last time (its every-50th residual).  Up to 128 groups
+// of blocks (33.5 M cells), whose sums one block can add while the rest of
+// its pass runs.
 
 bool jacobi_ahead_possible(const tea_hip_chunk* c) {
   return c->ra_enabled && c->fused && c->poll && !c->j_off && use_pair_blocks(c, 1) &&

@@ -70,6 +70,7 @@ struct Geo {
   int x, y, h;
   int n;      // x*y
   FastDiv dx; // division by x
+  int nt = 1, nt_half = 1;  // streaming access (kStreamCells)
   int bands = 0;  // FP64 passes in XCD bands (band_index)
 };
 
@@ -100,6 +101,15 @@ __device__ inline int xcd_span(int b, int nb) {
   const int per = nb / kNumXcd, rem = nb % kNumXcd;
   return xcd * per + (xcd < rem ? xcd : rem) + idx;
 }
+
+// From how many cells on the passes stream (ld2_nt): where an iteration's
+// arrays outgrow the 256 MB Infinity Cache.  FP64 CG (about 80 bytes per cell)
+// per iteration, streaming against plain: 1000^2 22.1, 20.3 us, 1700^2 47.8,
+// 46.0, 1800^2 52.5, 52.2, 1900^2 56.6, 57.7, 3000^2 137.4, 149.8.  Jacobi and
+// the FP32 passes (half): Jacobi 1000^2 10.5, 8.8, 2400^2 47.2, 44.1, 2800^2
+// 60.1, 65.6; mixed precision 1400^2 27.9, 25.9, 2400^2 57.8, 56.6, 2800^2
+// 76.4, 79.0.
+constexpr int kStreamCells = 3200000, kStreamCellsHalf = 6200000;
 
 // The workgroup's place in a pair- or quad-per-thread pass: in segments of
 // 8 * kBandBlocks blocks each XCD takes kBandBlocks consecutive blocks, so a
@@ -333,10 +343,12 @@ __device__ inline void span_reduce_pairs_n(double (&v)[NR][kSlots], double* part
 // pass's r); stencil operands (p, r, kx, ky) use ld2 so the neighbouring rows
 // can reuse them from L2, and w, which the residual pass reads next, is
 // stored normally so that it can stay in the 256 MB Infinity Cache (storing
-// it streaming made that pass 1-12% slower).
+// it streaming made that pass 1-12% slower).  With nt = 0 they are plain:
+// an iteration's arrays that fit in that cache are read back from it.
 typedef double dvec2 __attribute__((ext_vector_type(2)));
 
-__device__ inline double2 ld2_nt(const double* p, int i) {
+__device__ inline double2 ld2_nt(const double* p, int i, int nt = 1) {
+  if (!nt) return ld2(p, i);
   const dvec2 v = __builtin_nontemporal_load(reinterpret_cast<const dvec2*>(p + i));
   return double2{v.x, v.y};
 }
@@ -344,7 +356,16 @@ __device__ inline double2 ld2_nt(const double* p, int i) {
 // Stores a cell pair with one 16-byte streaming store, or the interior
 // member alone.
 __device__ inline void st2_nt(double* p, int i, bool in0, bool in1, double v0,
-                              double v1) {
+                              double v1, int nt = 1) {
+  if (!nt) {
+    if (in0 && in1) {
+      *reinterpret_cast<dvec2*>(p + i) = dvec2{v0, v1};
+    } else {
+      if (in0) p[i] = v0;
+      if (in1) p[i + 1] = v1;
+    }
+    return;
+  }
   if (in0 && in1) {
     __builtin_nontemporal_store(dvec2{v0, v1}, reinterpret_cast<dvec2*>(p + i));
   } else {
@@ -357,7 +378,16 @@ __device__ inline void st2_nt(double* p, int i, bool in0, bool in1, double v0,
 typedef float fvec2 __attribute__((ext_vector_type(2)));
 
 __device__ inline void st2_nt(float* p, int i, bool in0, bool in1, float v0,
-                              float v1) {
+                              float v1, int nt = 1) {
+  if (!nt) {
+    if (in0 && in1) {
+      *reinterpret_cast<fvec2*>(p + i) = fvec2{v0, v1};
+    } else {
+      if (in0) p[i] = v0;
+      if (in1) p[i + 1] = v1;
+    }
+    return;
+  }
   if (in0 && in1) {
     __builtin_nontemporal_store(fvec2{v0, v1}, reinterpret_cast<fvec2*>(p + i));
   } else {
@@ -473,7 +503,9 @@ __device__ inline void st4(float* p, int i, const bool (&in)[4], fvec4 v) {
 }
 
 // The same with streaming stores.
-__device__ inline void st4_nt(float* p, int i, const bool (&in)[4], fvec4 v) {
+__device__ inline void st4_nt(float* p, int i, const bool (&in)[4], fvec4 v,
+                              int nt = 1) {
+  if (!nt) return st4(p, i, in, v);
   if (in[0] && in[1] && in[2] && in[3]) {
     __builtin_nontemporal_store(v, reinterpret_cast<fvec4*>(p + i));
   } else {
@@ -483,7 +515,9 @@ __device__ inline void st4_nt(float* p, int i, const bool (&in)[4], fvec4 v) {
   }
 }
 
-__device__ inline void st4_nt(float* p, int i, const bool (&in)[4], const float (&v)[4]) {
+__device__ inline void st4_nt(float* p, int i, const bool (&in)[4], const float (&v)[4],
+                              int nt = 1) {
+  if (!nt) return st4(p, i, in, v);
   if (in[0] && in[1] && in[2] && in[3]) {
     __builtin_nontemporal_store(fvec4{v[0], v[1], v[2], v[3]}, reinterpret_cast<fvec4*>(p + i));
   } else {

@@ -80,8 +80,13 @@ BETWEEN = ("read", "residual", "halo2", "twice", "other halos", "cheby", "write"
     (64, 33, 3, BETWEEN), (65, 33, 2, BETWEEN),
     (1025, 67, 2, ("residual", "read")),   # odd, rows of two blocks
     (1024, 130, 2, ("residual",)),         # stacked blocks
-    (2048, 2048, 2, ()),           # 16 groups: the most that one block sums
-    (2050, 2048, 2, ("read",)),    # one more: no sweep ahead
+    (2048, 2048, 2, ()),           # 16 groups of 512 blocks
+    (2050, 2048, 2, ("read",)),    # 17
+    (3200, 2001, 2, ()),           # streaming (more than 6.2 M cells)
+    (4096, 4096, 2, ()),           # 64 groups: one tree
+    (4100, 4100, 2, ()),           # 65
+    (8192, 4096, 2, ()),           # 128: the most that one block sums
+    (8192, 4097, 2, ("read",)),    # one more: no sweep ahead
 ])
 def test_jacobi_ahead(x, y, h, between):
     sweeps = 5 * len(between) + 7
