@@ -616,14 +616,9 @@ struct LayerFrag {
   float bco[16];
   __device__ inline void load(const bf16* __restrict__ wt, const float* __restrict__ bias) {
     const int lane = threadIdx.x & (kWave - 1);
-    const int hf = lane >> 5, col = lane & 31;
+    const int hf = lane >> 5;
 #pragma unroll
-    for (int t = 0; t < NS; ++t) {
-      const int tap = kCin == fused::kCh ? t >> 1 : 2 * t + hf;
-      const int ci = kCin == fused::kCh ? ((t & 1) << 4) + 8 * hf : 0;
-      A[t] = tap < 9 ? *reinterpret_cast<const bf16x8*>(wt + ((size_t)col * 9 + tap) * kCin + ci)
-                     : bf16x8{};
-    }
+    for (int t = 0; t < NS; ++t) A[t] = nn::weight_frag(wt, t, lane);
 #pragma unroll
     for (int v = 0; v < 16; ++v) bco[v] = bias[8 * (v >> 2) + 4 * hf + (v & 3)];
   }

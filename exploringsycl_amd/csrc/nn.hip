@@ -39,6 +39,7 @@ constexpr int kFwdRows = 4;  // output rows per block of the multi-row forward k
 // (32,32,3,3) with b2..b5 (32), W6 (1,32,3,3), b6 (1); W[co][ci][ky][kx].
 constexpr int kW1 = kC * kIn * kTaps;  // 864
 constexpr int kWh = kC * kC * kTaps;   // 9216
+constexpr int kWf1 = 5 * 64 * 8;       // layer 1 in fragment order, taps and channels padded
 constexpr int kW6 = kC * kTaps;        // 288
 constexpr int kNumParams = (kW1 + kC) + 4 * (kWh + kC) + (kW6 + 1);  // 38177
 constexpr int kWgradMaxW = 128;  // widest row the weight-gradient kernel stages
@@ -88,14 +89,7 @@ __device__ inline void conv_mfma_tiles(
   const size_t plane = (size_t)(H + 2) * Wp;
   bf16x8 A[NS];
 #pragma unroll
-  for (int t = 0; t < NS; ++t) {
-    int tap, ci;
-    kmap<CIN>(t, hf, tap, ci);
-    if (tap < kTaps)
-      A[t] = *reinterpret_cast<const bf16x8*>(wt + ((size_t)col * kTaps + tap) * CIN + ci);
-    else
-      A[t] = bf16x8{};
-  }
+  for (int t = 0; t < NS; ++t) A[t] = weight_frag(wt, t, lane);
   float bco[16];
   if (MODE == 0) {
 #pragma unroll
@@ -121,28 +115,28 @@ __device__ inline void conv_mfma_tiles(
         Bv[t] = bf16x8{};
       }
     }
+    const size_t pix = (size_t)b * plane + (size_t)(y + 1) * Wp + (xo + 1);
+    bf16x4 m[4];
+    if (MODE == 1) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        m[g] = *reinterpret_cast<const bf16x4*>(mask + pix * kC + 8 * g + 4 * hf);
+    }
     f32x16 acc = {};
 #pragma unroll
     for (int t = 0; t < NS; ++t)
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[t], Bv[t], acc, 0, 0, 0);
-    const size_t pix = (size_t)b * plane + (size_t)(y + 1) * Wp + (xo + 1);
+    if (MODE == 0) {
+      store_out_row(out + pix * kC, acc, bco, hf);
+    } else {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int co0 = 8 * g + 4 * hf;
-      bf16x4 o;
-      if (MODE == 0) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const float vv = acc[4 * g + q] + bco[4 * g + q];
-          o[q] = (bf16)(vv > 0.0f ? vv : 0.0f);
-        }
-      } else {
-        const bf16x4 m = *reinterpret_cast<const bf16x4*>(mask + pix * kC + co0);
+      for (int g = 0; g < 4; ++g) {
+        bf16x4 o;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          o[q] = (bf16)((float)m[q] > 0.0f ? acc[4 * g + q] : 0.0f);
+          o[q] = (bf16)((float)m[g][q] > 0.0f ? acc[4 * g + q] : 0.0f);
+        *reinterpret_cast<bf16x4*>(out + pix * kC + 8 * g + 4 * hf) = o;
       }
-      *reinterpret_cast<bf16x4*>(out + pix * kC + co0) = o;
     }
   }
 }
@@ -226,14 +220,7 @@ __device__ inline void conv_fwd_lds_block(
   // were a second global-memory latency before the first MFMA.
   bf16x8 A[NS];
 #pragma unroll
-  for (int t = 0; t < NS; ++t) {
-    int tap, ci;
-    kmap<CIN>(t, hf, tap, ci);
-    if (tap < kTaps)
-      A[t] = *reinterpret_cast<const bf16x8*>(wt + ((size_t)col * kTaps + tap) * CIN + ci);
-    else
-      A[t] = bf16x8{};
-  }
+  for (int t = 0; t < NS; ++t) A[t] = weight_frag(wt, t, lane);
   float bco[16];
 #pragma unroll
   for (int v = 0; v < 16; ++v) bco[v] = bias[8 * (v >> 2) + 4 * hf + (v & 3)];
@@ -287,14 +274,7 @@ __device__ inline void conv_fwd_rows_block(
   // Weights and biases first (as conv_fwd_lds_kernel).
   bf16x8 A[NS];
 #pragma unroll
-  for (int t = 0; t < NS; ++t) {
-    int tap, ci;
-    kmap<CIN>(t, hf, tap, ci);
-    if (tap < kTaps)
-      A[t] = *reinterpret_cast<const bf16x8*>(wt + ((size_t)col * kTaps + tap) * CIN + ci);
-    else
-      A[t] = bf16x8{};
-  }
+  for (int t = 0; t < NS; ++t) A[t] = weight_frag(wt, t, lane);
   float bco[16];
 #pragma unroll
   for (int v = 0; v < 16; ++v) bco[v] = bias[8 * (v >> 2) + 4 * hf + (v & 3)];
@@ -644,34 +624,30 @@ __global__ __launch_bounds__(64) void reduce_grad_kernel(
 
 // ---- parameters ------------------------------------------------------------
 
-// BF16 kernel layouts from the FP32 master: forward Wf[co][tap][ci_pad],
-// backward-data Wb[ci][tap][co] = W[co][ci][flip(tap)], output-layer w6
-// [tap][ci] (FP32) and the biases.
+// BF16 kernel layouts from the FP32 master: the hidden layers' forward and
+// backward-data weights and the first layer's in fragment order (weight_frag),
+// output-layer w6 [tap][ci] (FP32) and the biases.  Row col and K-value k of
+// the forward fragments are output channel and (tap, input channel), of the
+// backward ones input channel and (flipped tap, output channel).
 __global__ __launch_bounds__(256) void pack_params_kernel(
     const float* __restrict__ master, bf16* __restrict__ wf1,
     bf16* __restrict__ wfh, bf16* __restrict__ wbh, float* __restrict__ w6,
     float* __restrict__ bias) {
   const int i = blockIdx.x * 256 + threadIdx.x;
-  // Layer 1: [co][ci<3][ky][kx] -> wf1[co][tap][ci pad 8].
-  if (i < kC * kTaps * kC0) {
-    const int co = i / (kTaps * kC0), rem = i % (kTaps * kC0);
-    const int tap = rem / kC0, ci = rem % kC0;
-    wf1[i] = (bf16)(ci < kIn ? master[(co * kIn + ci) * kTaps + tap] : 0.0f);
+  const int j = i & 7, hf = (i >> 8) & 1, col = (i >> 3) & 31;
+  if (i < kWf1) {
+    int tap, ci;
+    kmap<kC0>(i >> 9, hf, tap, ci);
+    wf1[i] = (bf16)(j < kIn && tap < kTaps ? master[(col * kIn + j) * kTaps + tap] : 0.0f);
   }
   // Hidden layers 2..5.
   if (i < 4 * kWh) {
-    const int l = i / kWh, rem = i % kWh;
+    const int l = i / kWh;
     const float* W = master + w_offset(l + 1);
-    {
-      const int co = rem / (kTaps * kC), r2 = rem % (kTaps * kC);
-      const int tap = r2 / kC, ci = r2 % kC;
-      wfh[i] = (bf16)W[(co * kC + ci) * kTaps + tap];
-    }
-    {
-      const int ci = rem / (kTaps * kC), r2 = rem % (kTaps * kC);
-      const int tap = r2 / kC, co = r2 % kC;
-      wbh[i] = (bf16)W[(co * kC + ci) * kTaps + (kTaps - 1 - tap)];
-    }
+    int tap, c0;
+    kmap<kC>((i - l * kWh) >> 9, hf, tap, c0);
+    wfh[i] = (bf16)W[(col * kC + c0 + j) * kTaps + tap];
+    wbh[i] = (bf16)W[((c0 + j) * kC + col) * kTaps + (kTaps - 1 - tap)];
   }
   if (i < kW6) {
     const int tap = i / kC, ci = i % kC;
@@ -1021,7 +997,7 @@ int tea_nn_create(int device, int max_batch, int height, int width, tea_nn** out
       {(void**)&n->grad, kNumParams * sizeof(float)},
       {(void**)&n->adam_m, kNumParams * sizeof(float)},
       {(void**)&n->adam_v, kNumParams * sizeof(float)},
-      {(void**)&n->wf1, (size_t)kC * kTaps * kC0 * sizeof(bf16)},
+      {(void**)&n->wf1, (size_t)kWf1 * sizeof(bf16)},
       {(void**)&n->wfh, (size_t)4 * kWh * sizeof(bf16)},
       {(void**)&n->wbh, (size_t)4 * kWh * sizeof(bf16)},
       {(void**)&n->w6, kW6 * sizeof(float)},

@@ -859,10 +859,18 @@ __device__ inline void store_out_row(bf16* px, const f32x16& acc, const float (&
   *reinterpret_cast<bf16x8*>(px + 16 * hf + 8) = hi.v;
 }
 
+// The A operand of a layer's K-step t (lane l: output channel l % 32, the
+// step's K-values 8 (l / 32) .. + 7), stored as the lanes take it: each load is
+// one KiB in a row.  (From [co][tap][ci] a load touched 32 cache lines, and a
+// hidden layer's 18 of them a wave: 64 x 32 x 32 8.9 us per layer.)
+__device__ inline bf16x8 weight_frag(const bf16* __restrict__ wt, int t, int lane) {
+  return *reinterpret_cast<const bf16x8*>(wt + (size_t)(t * kWave + lane) * 8);
+}
+
 // The network's device copies of its parameters, in the layouts of its
-// forward kernels: layer 1 wf1[co][tap][8] (3 channels used) and the hidden
-// layers wfh[layer][co][tap][ci] in BF16, the output layer w6[tap][ci]
-// (BF16 values in FP32) and the biases bias[layer * 32 + co], bias[160].
+// forward kernels: layer 1 and the hidden layers in BF16 in fragment order
+// (weight_frag), the output layer w6[tap][ci] (BF16 values in FP32) and the
+// biases bias[layer * 32 + co], bias[160].
 struct PackedWeights {
   const bf16* wf1;
   const bf16* wfh;
