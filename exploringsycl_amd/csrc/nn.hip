@@ -440,9 +440,9 @@ __global__ __launch_bounds__(256) void out_layer_bwd_data_kernel(
 }
 
 // Partial dW6[tap][ci] and db6 per block of rows: thread t < 288 handles
-// (tap, ci) = (t / 32, t % 32); thread 288 accumulates db6.  Grid: nblk
-// blocks, each handling rows [blk*rows_per, ...) of the B*H rows.
-__global__ __launch_bounds__(320) void out_layer_wgrad_kernel(
+// (tap, ci) = (t / 32, t % 32); thread 288 accumulates db6.  Block blk of nblk
+// handles rows [blk*rows_per, ...) of the B*H rows.
+__device__ inline void out_layer_wgrad_rows(
     const float* __restrict__ dout, const bf16* __restrict__ a5,
     float* __restrict__ partial, int B, int H, int W, int rows_per) {
   const int t = threadIdx.x;
@@ -486,31 +486,34 @@ __global__ __launch_bounds__(320) void out_layer_wgrad_kernel(
 // then each wave accumulates its share of the 32-wide n blocks over all
 // pixels with MFMA steps of 16 pixels (A: lane co, 8 pixels; B: lane n,
 // the same 8 pixels).  Per-block partials are summed by reduce_grad_kernel.
+constexpr int kWgradThreads = 320;     // 5 waves: 9 n blocks as 2, 2, 2, 2, 1
 template <int CIN>
-__global__ __launch_bounds__(256) void wgrad_mfma_kernel(
-    const bf16* __restrict__ delta, const bf16* __restrict__ in,
-    float* __restrict__ partial, int B, int H, int W, int rows_per) {
+__device__ inline void wgrad_rows(
+    bf16* __restrict__ sd, bf16* __restrict__ sa, const bf16* __restrict__ delta,
+    const bf16* __restrict__ in, float* __restrict__ partial, int B, int H, int W,
+    int rows_per) {
+  constexpr int kT = kWgradThreads, kWv = kT / 64;
+  constexpr int kQ = CIN == kC ? 2 : 1;  // n blocks per wave
   constexpr int N = kTaps * CIN;         // 288 or 72
   constexpr int NB = (N + 31) / 32;      // 9 or 3 blocks of 32
   constexpr int kMaxW = kWgradMaxW;      // staged row width limit
-  __shared__ bf16 sd[kMaxW * kC];        // delta row
-  __shared__ bf16 sa[3 * (kMaxW + 2) * CIN];  // input rows y-1..y+1
+  // sd: delta row; sa: input rows y-1..y+1.
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int hf = lane >> 5, col = lane & 31;
   const int Wp = W + 2;
   const size_t plane = (size_t)(H + 2) * Wp;
-  f32x16 acc[3];
+  f32x16 acc[kQ];
 #pragma unroll
-  for (int q = 0; q < 3; ++q) acc[q] = f32x16{};
+  for (int q = 0; q < kQ; ++q) acc[q] = f32x16{};
   float dbias = 0.0f;
   const int r0 = blockIdx.x * rows_per;
   const int r1 = min(r0 + rows_per, B * H);
   // delta[b][y+1][1..W][*] and in[b][y..y+2][0..W+1][*] of one row, in 16-byte
   // chunks: row r + 1's are loaded into registers while row r is computed
   // from LDS (waiting for each row's loads in turn took 17.6 us per hidden
-  // layer at 64 x 32 x 32; 13.0 us now).
-  constexpr int kD = (kMaxW * kC / 8 + 255) / 256;
-  constexpr int kA = (3 * (kMaxW + 2) * CIN / 8 + 255) / 256;
+  // layer at 64 x 32 x 32, 13.0 us without).
+  constexpr int kD = (kMaxW * kC / 8 + kT - 1) / kT;
+  constexpr int kA = (3 * (kMaxW + 2) * CIN / 8 + kT - 1) / kT;
   const int nd = W * kC / 8, na = 3 * Wp * CIN / 8;
   bf16x8 vd[kD], va[kA];
   auto load_row = [&](int row) {
@@ -519,12 +522,12 @@ __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
     const bf16* a = in + ((size_t)b * plane + (size_t)y * Wp) * CIN;
 #pragma unroll
     for (int k = 0; k < kD; ++k) {
-      const int i = threadIdx.x + 256 * k;
+      const int i = threadIdx.x + kT * k;
       if (i < nd) vd[k] = *reinterpret_cast<const bf16x8*>(d + 8 * i);
     }
 #pragma unroll
     for (int k = 0; k < kA; ++k) {
-      const int i = threadIdx.x + 256 * k;
+      const int i = threadIdx.x + kT * k;
       if (i < na) va[k] = *reinterpret_cast<const bf16x8*>(a + 8 * i);
     }
   };
@@ -533,12 +536,12 @@ __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kD; ++k) {
-      const int i = threadIdx.x + 256 * k;
+      const int i = threadIdx.x + kT * k;
       if (i < nd) *reinterpret_cast<bf16x8*>(sd + 8 * i) = vd[k];
     }
 #pragma unroll
     for (int k = 0; k < kA; ++k) {
-      const int i = threadIdx.x + 256 * k;
+      const int i = threadIdx.x + kT * k;
       if (i < na) *reinterpret_cast<bf16x8*>(sa + 8 * i) = va[k];
     }
     __syncthreads();
@@ -552,8 +555,8 @@ __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
         for (int s = 0; s < 8; ++s) dbias += (float)a[s];
       }
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const int nb = wv + 4 * q;
+      for (int q = 0; q < kQ; ++q) {
+        const int nb = wv + kWv * q;
         if (nb >= NB) break;
         const int n = nb * 32 + col;
         bf16x8 bv;
@@ -573,8 +576,8 @@ __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
   // D[co][n]: lane l holds n = nb*32 + l%32 and co = 8*(v/4) + 4*hf + v%4.
   float* pb = partial + (size_t)blockIdx.x * (kC * N + kC);
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const int nb = wv + 4 * q;
+  for (int q = 0; q < kQ; ++q) {
+    const int nb = wv + kWv * q;
     if (nb >= NB) break;
     const int n = nb * 32 + col;
     if (n >= N) continue;
@@ -591,17 +594,58 @@ __global__ __launch_bounds__(256) void wgrad_mfma_kernel(
   }
 }
 
-// Sums a layer's nblk partial rows ([co][tap][ci_pad] then db) in block order
-// into the master-layout gradient ([co][ci][ky][kx], then b).  One column per
-// thread; kReduceBatch rows are loaded before any is added, or each load's
+// A layer's input gradients' and activations' pointers (0 the first layer).
+struct WgradArgs {
+  const bf16* delta[5];
+  const bf16* in[5];
+  const float* dout;  // output layer
+  const bf16* a5;
+  float* partial;
+};
+
+// Length of a block's partial row of layer l (5: the output layer), and the
+// rows of the layers before it per block.
+__host__ __device__ inline int wgrad_len(int l) {
+  return l == 0 ? kC * kTaps * kC0 + kC : l < 5 ? kC * kTaps * kC + kC : kW6 + 1;
+}
+__host__ __device__ inline int wgrad_offset(int l) {
+  return l == 0 ? 0 : wgrad_len(0) + (l - 1) * wgrad_len(1);
+}
+
+// The weight gradients of all six layers in one launch, after the backward
+// data pass, which none of them waits for: a layer alone is one four-wave
+// block per CU whose rows are a chain of load, LDS and MFMA latencies (64 x 32
+// x 32: 13.1 us per hidden layer, 14.0 and 7.9 us the last and first, 74 us in
+// all); together they fill the chip.
+// Grid (nblk, 6), the longest layers first.
+__global__ __launch_bounds__(kWgradThreads) void wgrad_kernel(WgradArgs a, int B, int H, int W,
+                                                              int rows_per) {
+  __shared__ bf16 sd[kWgradMaxW * kC];
+  __shared__ bf16 sa[3 * (kWgradMaxW + 2) * kC];
+  const int l = blockIdx.y < 4 ? 4 - blockIdx.y : blockIdx.y == 4 ? 5 : 0;
+  float* part = a.partial + (size_t)gridDim.x * wgrad_offset(l);
+  if (l == 5)
+    out_layer_wgrad_rows(a.dout, a.a5, part, B, H, W, rows_per);
+  else if (l == 0)
+    wgrad_rows<kC0>(sd, sa, a.delta[0], a.in[0], part, B, H, W, rows_per);
+  else
+    wgrad_rows<kC>(sd, sa, a.delta[l], a.in[l], part, B, H, W, rows_per);
+}
+
+// Sums each layer's nblk partial rows ([co][tap][ci_pad] then db) in block
+// order into the master-layout gradient ([co][ci][ky][kx], then b).  One column
+// per thread; kReduceBatch rows are loaded before any is added, or each load's
 // latency would be waited for in turn (a plain loop took 60 us for 256 rows
-// of 9248 columns, 9.5 MB; this takes 5 us on average over the layers).
+// of 9248 columns, 9.5 MB).  All layers in one launch: blockIdx.y is the layer.
 constexpr int kReduceBatch = 64;
-__global__ __launch_bounds__(64) void reduce_grad_kernel(
-    const float* __restrict__ partial, int nblk, int cin_pad, int cin, int cout,
-    float* __restrict__ gw, float* __restrict__ gb) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
+__global__ __launch_bounds__(64) void reduce_grad_kernel(const float* __restrict__ partials,
+                                                         int nblk, float* __restrict__ grad) {
+  const int i = blockIdx.x * 64 + threadIdx.x, l = blockIdx.y;
+  const int cin_pad = l == 0 ? kC0 : kC, cin = l == 0 ? kIn : kC, cout = l == 5 ? 1 : kC;
   const int nw = cout * kTaps * cin_pad, len = nw + cout;
+  const float* __restrict__ partial = partials + (size_t)nblk * wgrad_offset(l);
+  float* gw = grad + w_offset(l);
+  float* gb = grad + b_offset(l);
   if (i >= len) return;
   float s = 0.0f;
   int b = 0;
@@ -798,25 +842,6 @@ int forward_on(tea_nn* n, int batch, hipStream_t st, bool with_output = true,
 
 int forward(tea_nn* n, int batch) { return forward_on(n, batch, n->stream); }
 
-int wgrad_layer(tea_nn* n, int batch, int layer, const bf16* delta, const bf16* in) {
-  const int rows = batch * n->H;
-  const int rows_per = (rows + n->wg_blocks - 1) / n->wg_blocks;
-  const int nblk = (rows + rows_per - 1) / rows_per;
-  const int cin_pad = layer == 0 ? kC0 : kC;
-  const int len = kC * kTaps * cin_pad + kC;
-  if (layer == 0)
-    hipLaunchKernelGGL((wgrad_mfma_kernel<kC0>), dim3(nblk), dim3(256), 0, n->stream,
-                       delta, in, n->partial, batch, n->H, n->W, rows_per);
-  else
-    hipLaunchKernelGGL((wgrad_mfma_kernel<kC>), dim3(nblk), dim3(256), 0, n->stream,
-                       delta, in, n->partial, batch, n->H, n->W, rows_per);
-  hipLaunchKernelGGL(reduce_grad_kernel, dim3((len + 63) / 64), dim3(64), 0, n->stream,
-                     n->partial, nblk, cin_pad, layer == 0 ? kIn : kC, kC,
-                     n->grad + w_offset(layer), n->grad + b_offset(layer));
-  TEA_HIP_TRY(hipGetLastError());
-  return TEA_HIP_OK;
-}
-
 // Blocks of mse_kernel, each leaving one partial of a batch's squared error.
 unsigned loss_blocks(const tea_nn* n, int batch) {
   return flat_blocks((long)batch * n->H * n->W);
@@ -848,27 +873,29 @@ int loss_and_grad(tea_nn* n, int batch, int k = 0) {
   const unsigned nb = loss_blocks(n, batch);
   hipLaunchKernelGGL(mse_kernel, dim3(nb), dim3(256), 0, n->stream, n->out, n->target,
                      n->dout, n->loss_part + (size_t)k * nb, cnt);
-  // Output layer.
+  // Backward data, output layer to layer 1.
   hipLaunchKernelGGL(out_layer_bwd_data_kernel, dim3(nb), dim3(256), 0, n->stream,
                      n->dout, n->w6, n->act[4], n->del[4], batch, H, W);
-  {
-    const int rows = batch * H;
-    const int rows_per = (rows + n->wg_blocks - 1) / n->wg_blocks;
-    const int nblk = (rows + rows_per - 1) / rows_per;
-    hipLaunchKernelGGL(out_layer_wgrad_kernel, dim3(nblk), dim3(320), 0, n->stream,
-                       n->dout, n->act[4], n->partial, batch, H, W, rows_per);
-    hipLaunchKernelGGL(reduce_grad_kernel, dim3((kW6 + 1 + 63) / 64), dim3(64), 0, n->stream,
-                       n->partial, nblk, kC, kC, 1, n->grad + w_offset(5),
-                       n->grad + b_offset(5));
-  }
-  // Hidden layers 5..2, then layer 1.
-  for (int l = 4; l >= 1; --l) {
-    TEA_RETURN_IF(wgrad_layer(n, batch, l, n->del[l], n->act[l - 1]));
+  for (int l = 4; l >= 1; --l)
     hipLaunchKernelGGL((conv_mfma_kernel<kC, 1>), conv_grid(n, batch), dim3(256), 0,
                        n->stream, n->del[l], n->wbh + (size_t)(l - 1) * kWh, nullptr,
                        n->act[l - 1], n->del[l - 1], H, W, batch);
+  // Weight gradients.
+  const int rows = batch * H;
+  const int rows_per = (rows + n->wg_blocks - 1) / n->wg_blocks;
+  const int nblk = (rows + rows_per - 1) / rows_per;
+  WgradArgs a{};
+  for (int l = 0; l < 5; ++l) {
+    a.delta[l] = n->del[l];
+    a.in[l] = l == 0 ? n->in0 : n->act[l - 1];
   }
-  TEA_RETURN_IF(wgrad_layer(n, batch, 0, n->del[0], n->in0));
+  a.dout = n->dout;
+  a.a5 = n->act[4];
+  a.partial = n->partial;
+  hipLaunchKernelGGL(wgrad_kernel, dim3(nblk, 6), dim3(kWgradThreads), 0, n->stream, a, batch, H,
+                     W, rows_per);
+  hipLaunchKernelGGL(reduce_grad_kernel, dim3((wgrad_len(1) + 63) / 64, 6), dim3(64), 0,
+                     n->stream, n->partial, nblk, n->grad);
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
 }
@@ -988,7 +1015,7 @@ int tea_nn_create(int device, int max_batch, int height, int width, tea_nn** out
   const size_t px = (size_t)max_batch * height * width;
   n->wg_blocks = 256;
   n->loss_len = px / 256 + 2;
-  n->partial_len = (size_t)n->wg_blocks * (kC * kTaps * kC + kC);
+  n->partial_len = (size_t)n->wg_blocks * (wgrad_offset(5) + wgrad_len(5));
   struct {
     void** p;
     size_t bytes;
