@@ -967,7 +967,7 @@ constexpr int kBoxT = 16;
 constexpr int kBoxA = kBoxT + 2;          // 18: layer-1 region
 constexpr int kBoxC = kBoxT + 4;          // 20: sigma and input region
 constexpr int kBoxS = kBoxC + 2 * kWin;   // 32: staged region
-constexpr int kBoxStage = (2 * kBoxS * kBoxS + kBoxS * kBoxC) * 4;  // bytes
+constexpr int kBoxStage = (4 * kBoxS * kBoxS + kBoxS * kBoxC) * 4;  // bytes
 constexpr int kBoxA1 = kBoxA * kBoxA * 5 * 16;                       // bytes
 struct BoxLevel {
   int hc, wc, npart;
@@ -979,8 +979,12 @@ struct BoxLevel {
   nn::PackedWeights wts;
   bf16* a2;
 };
-// Both levels in one launch: the first nb0 blocks take level 0's tiles.
-__global__ __launch_bounds__(256) void box_conv_kernel(BoxLevel lv0, BoxLevel lv1, int nb0) {
+// Both levels in one launch: the first nb0 blocks take level 0's tiles.  Four
+// blocks per CU, so that the 1088 blocks of 512^2 and 128^2 are about one
+// round of the chip: with layer 2's weights loaded before layer 1 (172
+// registers, two blocks per CU, three rounds) it took 31 us at 4096^2, 21 us
+// now.  The squares of the window sums are formed once per staged cell.
+__global__ __launch_bounds__(256, 4) void box_conv_kernel(BoxLevel lv0, BoxLevel lv1, int nb0) {
   const bool second = (int)blockIdx.x >= nb0;
   const int hc = second ? lv1.hc : lv0.hc, wc = second ? lv1.wc : lv0.wc;
   const int npart = second ? lv1.npart : lv0.npart;
@@ -1001,7 +1005,8 @@ __global__ __launch_bounds__(256) void box_conv_kernel(BoxLevel lv0, BoxLevel lv
   // activations (act_slot layout) take its place.
   __shared__ __attribute__((aligned(16)))
   unsigned char s_u[kBoxStage > kBoxA1 ? kBoxStage : kBoxA1];
-  float* s_rb = reinterpret_cast<float*>(s_u);
+  double* s_w2 = reinterpret_cast<double*>(s_u);  // (D^-1/2 rbar)^2, 0 outside the grid
+  float* s_rb = reinterpret_cast<float*>(s_w2 + kN);
   float* s_ds = s_rb + kN;
   float* s_tmp = s_ds + kN;
   bf16x8* s_a1 = reinterpret_cast<bf16x8*>(s_u);
@@ -1017,15 +1022,6 @@ __global__ __launch_bounds__(256) void box_conv_kernel(BoxLevel lv0, BoxLevel lv
   // input pixels.
   LayerFrag<8> w1;
   w1.load(wts.wf1, wts.bias);
-  double v = 0.0;
-  for (int i0 = tid; i0 < npart; i0 += 256 * 8) {
-    double t8[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t8[j] = part[i0 + 256 * j < npart ? i0 + 256 * j : 0];
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (i0 + 256 * j < npart) v += t8[j];
-  }
   // Staged cell q: (X0 - 2 - kWin + q % kBoxS, Y0 - 2 - kWin + q / kBoxS).
   float rb[kIt], ds[kIt];
 #pragma unroll
@@ -1047,24 +1043,31 @@ __global__ __launch_bounds__(256) void box_conv_kernel(BoxLevel lv0, BoxLevel lv
     f0[k] = feat[j];
     f1[k] = feat[n + j];
   }
+  double v = 0.0;
+  for (int i0 = tid; i0 < npart; i0 += 256 * 8) {
+    double t8[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) t8[j] = part[i0 + 256 * j < npart ? i0 + 256 * j : 0];
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      if (i0 + 256 * j < npart) v += t8[j];
+  }
   s_sc[tid] = v;
 #pragma unroll
   for (int k = 0; k < kIt; ++k)
     if (tid + 256 * k < kN) {
       s_rb[tid + 256 * k] = rb[k];
       s_ds[tid + 256 * k] = ds[k];
+      const double w = (double)rb[k] * (double)ds[k];
+      s_w2[tid + 256 * k] = w * w;
     }
   __syncthreads();
   // Row pass: staged row r, region column c (staged column c + kWin).
   for (int q = tid; q < kBoxS * kBoxC; q += 256) {
     const int r = q / kBoxC, c = q - r * kBoxC + kWin;
-    const int Xc = X0 - 2 - kWin + c;
     double s = 0.0;
 #pragma unroll
-    for (int d = -kWin; d <= kWin; ++d) {
-      const double w = (double)s_rb[r * kBoxS + c + d] * (double)s_ds[r * kBoxS + c + d];
-      s += Xc + d < 0 || Xc + d >= wc ? 0.0 : w * w;
-    }
+    for (int d = -kWin; d <= kWin; ++d) s += s_w2[r * kBoxS + c + d];
     s_tmp[q] = (float)s;
   }
   // The LDS tree of the RMS sum (element t adds element t + st): steps 128
@@ -1091,7 +1094,7 @@ __global__ __launch_bounds__(256) void box_conv_kernel(BoxLevel lv0, BoxLevel lv
       double s = 0.0;
 #pragma unroll
       for (int d = -kWin; d <= kWin; ++d)
-        s += Y + d < 0 || Y + d >= hc ? 0.0 : (double)s_tmp[(r + kWin + d) * kBoxC + c];
+        s += (double)s_tmp[(r + kWin + d) * kBoxC + c];
       const float sg =
           fmaxf((float)sqrt(s / (double)((2 * kWin + 1) * (2 * kWin + 1))), floor_s);
       const long i = (long)Y * wc + X;
@@ -1103,12 +1106,12 @@ __global__ __launch_bounds__(256) void box_conv_kernel(BoxLevel lv0, BoxLevel lv
     }
     s_in[q] = o;
   }
-  // Layer 2's weights, loaded before the barrier that waits for the input.
-  LayerFrag<fused::kCh> w2;
-  w2.load(wts.wfh, wts.bias + fused::kCh);
   __syncthreads();
   // Layer 1 on the 18 x 18 region (the stage's LDS is dead now).
   fused_conv<8, 1>(s_in, s_a1, kBoxC, w1, X0 - 1, Y0 - 1, hc, wc, kWaves);
+  // Layer 2's weights, loaded before the barrier that waits for layer 1.
+  LayerFrag<fused::kCh> w2;
+  w2.load(wts.wfh, wts.bias + fused::kCh);
   __syncthreads();
   // Layer 2 on the tile: wave w takes 32-pixel tiles w and w + 4 (tile rows
   // 2j, 2j + 1).

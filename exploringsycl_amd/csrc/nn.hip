@@ -77,6 +77,22 @@ constexpr int nsteps() {
   return CIN == kC ? 18 : 5;
 }
 
+// LDS place (in 16-byte chunks) of chunk ch of staged pixel px.  The chunks of
+// a pixel are swapped by px / 4 % 4, so that one chunk of 16 consecutive
+// pixels, a 16-lane part of an LDS read, lies in 16 distinct bank groups
+// (a padded fifth chunk did the same with a quarter more LDS: two instead of
+// three blocks of the four-row kernel per CU).
+template <int CPC>
+__device__ inline int px_slot(int px, int ch) {
+  return CPC == 1 ? px : px * CPC + (ch ^ ((px >> 2) & 3));
+}
+
+// 16-byte LDS chunks of a forward block by R (conv_fwd_block).
+template <int CIN, int R>
+constexpr int conv_lds() {
+  return CIN / 8 * (R == 0 ? 4 * 3 * 34 : (R + 2) * 130);
+}
+
 // MODE 0: out = relu(D + bias).  MODE 1: out = D * (mask > 0).
 // One 32-pixel tile per wave and round, the tiles of all rows and samples
 // numbered in one sequence, so that every wave of a block has work at any
@@ -88,16 +104,14 @@ constexpr int nsteps() {
 // 6.6 -> 5.6 us forward, 8.4 -> 6.1 backward).
 template <int CIN, int MODE>
 __device__ inline void conv_mfma_tiles(
-    const bf16* __restrict__ in, const bf16* __restrict__ wt,
+    bf16x8* sm, const bf16* __restrict__ in, const bf16* __restrict__ wt,
     const float* __restrict__ bias, const bf16* __restrict__ mask,
     bf16* __restrict__ out, int H, int W, int B, int block, int blocks) {
   constexpr int NS = nsteps<CIN>();
-  constexpr int CPC = CIN / 8;                    // 16-byte chunks per pixel
-  constexpr int kPitch = CPC == 1 ? 1 : CPC + 1;  // in LDS (act_slot's reason)
+  constexpr int CPC = CIN / 8;  // 16-byte chunks per pixel
   constexpr int kPx = 34, kChunks = 3 * kPx * CPC, kIt = (kChunks + 63) / 64;
-  __shared__ bf16x8 sm[4][3 * kPx * kPitch];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  bf16x8* sw = sm[wv];
+  bf16x8* sw = sm + wv * kChunks;
   const int hf = lane >> 5, col = lane & 31;
   const int Wp = W + 2;
   const size_t plane = (size_t)(H + 2) * Wp;
@@ -133,7 +147,7 @@ __device__ inline void conv_mfma_tiles(
 #pragma unroll
     for (int k = 0; k < kIt; ++k) {
       const int q = lane + 64 * k;
-      if (q < kChunks) sw[q / CPC * kPitch + q % CPC] = v[k];
+      if (q < kChunks) sw[px_slot<CPC>(q / CPC, q % CPC)] = v[k];
     }
     wave_lds_fence();
     bf16x8 Bv[NS];
@@ -142,7 +156,7 @@ __device__ inline void conv_mfma_tiles(
       int tap, ci;
       kmap<CIN>(t, hf, tap, ci);
       if (tap < kTaps)
-        Bv[t] = sw[(tap / 3 * kPx + col + tap % 3) * kPitch + ci / 8];
+        Bv[t] = sw[px_slot<CPC>(tap / 3 * kPx + col + tap % 3, ci / 8)];
       else
         Bv[t] = bf16x8{};
     }
@@ -170,15 +184,16 @@ __global__ __launch_bounds__(256) void conv_mfma_kernel(
     const bf16* __restrict__ in, const bf16* __restrict__ wt,
     const float* __restrict__ bias, const bf16* __restrict__ mask,
     bf16* __restrict__ out, int H, int W, int B) {
-  conv_mfma_tiles<CIN, MODE>(in, wt, bias, mask, out, H, W, B, blockIdx.x, gridDim.x);
+  __shared__ bf16x8 sm[conv_lds<CIN, 0>()];
+  conv_mfma_tiles<CIN, MODE>(sm, in, wt, bias, mask, out, H, W, B, blockIdx.x, gridDim.x);
 }
 
 // Stages NROWS padded input rows (from row y0) of a 130-pixel segment
-// (from padded column x0) into LDS, CPC 16-byte chunks per pixel at a pitch
-// of kPitch chunks: every thread issues all its loads before its first LDS
+// (from padded column x0) into LDS, CPC 16-byte chunks per pixel (px_slot):
+// every thread issues all its loads before its first LDS
 // store (a load-store loop waited for each load in turn: 13 global-memory
 // latencies per thread of the four-row kernel).
-template <int NROWS, int CPC, int kPx, int kPitch>
+template <int NROWS, int CPC, int kPx>
 __device__ inline void stage_rows(bf16x8* sm, const bf16* __restrict__ inb, int y0, int Wp,
                                   int x0) {
   constexpr int kTotal = NROWS * kPx * CPC;
@@ -192,7 +207,7 @@ __device__ inline void stage_rows(bf16x8* sm, const bf16* __restrict__ inb, int 
     const int qq = q < kTotal ? q : 0;
     const int row = qq / (kPx * CPC), rem = qq - row * (kPx * CPC);
     const int px = rem / CPC, ch = rem - px * CPC;
-    slot[k] = row * (kPx * kPitch) + px * kPitch + ch;
+    slot[k] = row * (kPx * CPC) + px_slot<CPC>(px, ch);
     v[k] = *reinterpret_cast<const bf16x8*>(inb + ((size_t)(y0 + row) * Wp + (x0 + px)) * CIN +
                                             ch * 8);
   }
@@ -219,19 +234,16 @@ __device__ inline void xcd_tile(int block, int segs, int groups, int samples, in
 // Forward layer for rows of 128 pixels or more: a block takes a 128-pixel
 // segment of row y, stages input rows y-1..y+1 over the segment plus its
 // 1-pixel ring in LDS once (130 pixels x CIN channels x 3 rows, in 16-byte
-// chunks; a pixel's chunks are padded to kPitch so that the 16 lanes of a
-// 16-byte LDS read, which take consecutive pixels, hit distinct banks),
+// chunks),
 // and each wave computes one 32-pixel tile from LDS.  Same arithmetic and
 // output as conv_mfma_kernel<CIN, 0>.  W / 128 x H x B blocks.
 template <int CIN>
 __device__ inline void conv_fwd_lds_block(
-    const bf16* __restrict__ in, const bf16* __restrict__ wt,
+    bf16x8* sm, const bf16* __restrict__ in, const bf16* __restrict__ wt,
     const float* __restrict__ bias, bf16* __restrict__ out, int H, int W, int B, int block) {
   constexpr int NS = nsteps<CIN>();
-  constexpr int CPC = CIN / 8;                   // 16-byte chunks per pixel
-  constexpr int kPitch = CPC == 1 ? 1 : CPC + 1;  // padded chunks per pixel
+  constexpr int CPC = CIN / 8;  // 16-byte chunks per pixel
   constexpr int kPx = 130;
-  __shared__ bf16x8 sm[3][kPx * kPitch];
   int seg, y, b;
   xcd_tile(block, W / 128, H, B, seg, y, b);
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -248,7 +260,7 @@ __device__ inline void conv_fwd_lds_block(
   float bco[16];
 #pragma unroll
   for (int v = 0; v < 16; ++v) bco[v] = bias[8 * (v >> 2) + 4 * hf + (v & 3)];
-  stage_rows<3, CPC, kPx, kPitch>(&sm[0][0], inb, y, Wp, x0);
+  stage_rows<3, CPC, kPx>(sm, inb, y, Wp, x0);
   __syncthreads();
   const int xl = wv * 32 + col;  // pixel within the segment
   bf16x8 Bv[NS];
@@ -258,7 +270,7 @@ __device__ inline void conv_fwd_lds_block(
     kmap<CIN>(t, hf, tap, ci);
     if (tap < kTaps) {
       const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-      Bv[t] = sm[dy + 1][(xl + 1 + dx) * kPitch + ci / 8];
+      Bv[t] = sm[(dy + 1) * kPx * CPC + px_slot<CPC>(xl + 1 + dx, ci / 8)];
     } else {
       Bv[t] = bf16x8{};
     }
@@ -279,13 +291,11 @@ __device__ inline void conv_fwd_lds_block(
 // W / 128 x H / R x B blocks.
 template <int CIN, int R>
 __device__ inline void conv_fwd_rows_block(
-    const bf16* __restrict__ in, const bf16* __restrict__ wt,
+    bf16x8* sm, const bf16* __restrict__ in, const bf16* __restrict__ wt,
     const float* __restrict__ bias, bf16* __restrict__ out, int H, int W, int B, int block) {
   constexpr int NS = nsteps<CIN>();
   constexpr int CPC = CIN / 8;
-  constexpr int kPitch = CPC == 1 ? 1 : CPC + 1;
   constexpr int kPx = 130;
-  __shared__ bf16x8 sm[R + 2][kPx * kPitch];
   int seg, grp, b;
   xcd_tile(block, W / 128, H / R, B, seg, grp, b);
   const int y0 = grp * R;
@@ -302,7 +312,7 @@ __device__ inline void conv_fwd_rows_block(
   float bco[16];
 #pragma unroll
   for (int v = 0; v < 16; ++v) bco[v] = bias[8 * (v >> 2) + 4 * hf + (v & 3)];
-  stage_rows<R + 2, CPC, kPx, kPitch>(&sm[0][0], inb, y0, Wp, x0);
+  stage_rows<R + 2, CPC, kPx>(sm, inb, y0, Wp, x0);
   __syncthreads();
   const int xl = wv * 32 + col;
 #pragma unroll 1
@@ -314,7 +324,7 @@ __device__ inline void conv_fwd_rows_block(
       kmap<CIN>(t, hf, tap, ci);
       if (tap < kTaps) {
         const int dy = tap / 3 - 1, dx = tap % 3 - 1;
-        Bv[t] = sm[r + dy + 1][(xl + 1 + dx) * kPitch + ci / 8];
+        Bv[t] = sm[(r + dy + 1) * kPx * CPC + px_slot<CPC>(xl + 1 + dx, ci / 8)];
       } else {
         Bv[t] = bf16x8{};
       }
@@ -331,28 +341,31 @@ __device__ inline void conv_fwd_rows_block(
 // The forward kernel R selects: 0 a tile per wave (conv_mfma_tiles), 1 a row
 // per block, 2 or 4 rows per block.
 template <int CIN, int R>
-__device__ inline void conv_fwd_block(const bf16* in, const bf16* wt, const float* bias, bf16* out,
+__device__ inline void conv_fwd_block(bf16x8* sm, const bf16* in, const bf16* wt, const float* bias, bf16* out,
                                       int H, int W, int B, int block, int blocks) {
   if (R == 0)
-    conv_mfma_tiles<CIN, 0>(in, wt, bias, nullptr, out, H, W, B, block, blocks);
+    conv_mfma_tiles<CIN, 0>(sm, in, wt, bias, nullptr, out, H, W, B, block, blocks);
   else if (R == 1)
-    conv_fwd_lds_block<CIN>(in, wt, bias, out, H, W, B, block);
+    conv_fwd_lds_block<CIN>(sm, in, wt, bias, out, H, W, B, block);
   else
-    conv_fwd_rows_block<CIN, R ? R : 1>(in, wt, bias, out, H, W, B, block);
+    conv_fwd_rows_block<CIN, R ? R : 1>(sm, in, wt, bias, out, H, W, B, block);
 }
 
 template <int CIN, int R>
-__global__ __launch_bounds__(256) void conv_fwd_kernel(
+__global__ __launch_bounds__(256, 3) void conv_fwd_kernel(
     const bf16* __restrict__ in, const bf16* __restrict__ wt,
     const float* __restrict__ bias, bf16* __restrict__ out, int H, int W, int B) {
-  conv_fwd_block<CIN, R>(in, wt, bias, out, H, W, B, blockIdx.x, gridDim.x);
+  __shared__ bf16x8 sm[conv_lds<CIN, R>()];
+  conv_fwd_block<CIN, R>(sm, in, wt, bias, out, H, W, B, blockIdx.x, gridDim.x);
 }
 
 // One hidden layer of two networks of one sample each (two levels of the
 // learned preconditioner), the first nb0 blocks the first network's by R and
 // the others the second's, a tile per wave: the second level's 32 blocks ran
 // on a stream of their own before, whose fork and join cost more (about 17 us
-// per application at 4096^2) than its five short launches.
+// per application at 4096^2) than its five short launches.  Three blocks per
+// CU (px_slot, 168 registers): the 640 blocks of 512^2 and 128^2 are one round
+// (14.2 us with two per CU, 12.4 now).
 struct ConvArgs {
   const bf16* in;
   const bf16* wt;
@@ -361,11 +374,13 @@ struct ConvArgs {
   int H, W;
 };
 template <int R>
-__global__ __launch_bounds__(256) void conv_fwd_pair_kernel(ConvArgs a, ConvArgs b, int nb0) {
+__global__ __launch_bounds__(256, 3) void conv_fwd_pair_kernel(ConvArgs a, ConvArgs b, int nb0) {
+  __shared__ bf16x8 sm[conv_lds<kC, R>() > conv_lds<kC, 0>() ? conv_lds<kC, R>()
+                                                             : conv_lds<kC, 0>()];
   if ((int)blockIdx.x < nb0)
-    conv_fwd_block<kC, R>(a.in, a.wt, a.bias, a.out, a.H, a.W, 1, blockIdx.x, nb0);
+    conv_fwd_block<kC, R>(sm, a.in, a.wt, a.bias, a.out, a.H, a.W, 1, blockIdx.x, nb0);
   else
-    conv_mfma_tiles<kC, 0>(b.in, b.wt, b.bias, nullptr, b.out, b.H, b.W, 1, blockIdx.x - nb0,
+    conv_mfma_tiles<kC, 0>(sm, b.in, b.wt, b.bias, nullptr, b.out, b.H, b.W, 1, blockIdx.x - nb0,
                            gridDim.x - nb0);
 }
 
