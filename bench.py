@@ -19,9 +19,10 @@ drawn at 8192 x 8192 is then solved by plain FP64 CG and learned FCG.
 
 Printed (one JSON line): effective HBM throughput of the timed solve,
   value = 88 B x N^2 x (CG iterations executed) / t_solve,
-88 B being the algorithmic FP64 traffic per cell per iteration (11 words),
+88 B being the FP64 traffic per cell per iteration with each update in its own
+pass (11 words, the metric's convention; u's updates held back move 82.7),
 plus time-to-solution, iterations/s, cell-updates/s, the roofline of the
-dominant kernel (cg_fused_w: 8 words = 64 B per cell per launch, timed with
+dominant kernel (cg_fused_w: 48, 48 and 80 B per cell in turn, timed with
 HIP events on the library's stream; also set against a measured 16-byte
 device-copy rate) and a CPU baseline (the OpenMP CPU restatement of the
 reference kernels, unfused 13-word dataflow, timed on a bounded sample of the
@@ -41,8 +42,11 @@ sys.path.insert(0, REPO)
 METRIC = ("time-to-solution @4096², 1e-10 rel. residual: learned FCG vs plain CG; "
           "HBM GB/s")
 HBM_PEAK_GBS = 8000.0
-BYTES_PER_CELL_ITER = 88      # fused FP64 iteration, algorithmic
-BYTES_FUSED_W = 64            # cg_fused_w: p_old, r, u, kx, ky read; p, u, w written
+BYTES_PER_CELL_ITER = 88      # fused FP64 iteration, the metric's convention
+# cg_fused_w reads p_old, r, kx, ky and writes p, w (48); every third w-step also
+# reads and writes u and reads the two held p (80).  The mean of the three, or
+# 64 where each w-step updates u itself.
+BYTES_FUSED_W = 64 if os.environ.get("TEA_HIP_HOLD_U") == "0" else 176 / 3
 BYTES_FUSED_R = 24            # cg_fused_r: r, w read; r written
 PROFILE_TRAFFIC = os.path.join(REPO, "profiles", "cg_fused_w_4096_traffic.json")
 
@@ -300,7 +304,7 @@ def other_solvers(n, jacobi_iters=2000, max_iters=0, timeout=900):
             "temp": rec["summaries"][-1]["temp"],
             "kernel": {"name": kname, "launches": k["launches"],
                        "avg_us": round(avg_ms * 1e3, 2),
-                       "algorithmic_bytes_per_cell": kbytes,
+                       "algorithmic_bytes_per_cell": round(kbytes, 2),
                        "achieved_gbs": round(gbs, 1),
                        "frac_of_hbm_peak": round(gbs / HBM_PEAK_GBS, 4)},
         }
@@ -356,7 +360,7 @@ def main():
     roofline = {"bound": "hbm", "kernel": kname, "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                "algorithmic_bytes_per_launch": kbytes * n * n,
+                "algorithmic_bytes_per_launch": round(kbytes * n * n),
                 "avg_launch_ms": round(avg_ms, 5)}
 
     line = {

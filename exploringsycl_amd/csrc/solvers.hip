@@ -393,6 +393,7 @@ int ensure_spare(tea_hip_chunk* c) {
   if (c->spare) return TEA_HIP_OK;
   if (hipMalloc(&c->spare, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
     c->spare = nullptr;
+    (void)hipGetLastError();
     set_error("hipMalloc of the spare field buffer failed");
     return TEA_HIP_ENOMEM;
   }
@@ -404,6 +405,7 @@ int ensure_spare2(tea_hip_chunk* c) {
   if (c->spare2) return TEA_HIP_OK;
   if (hipMalloc(&c->spare2, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
     c->spare2 = nullptr;
+    (void)hipGetLastError();
     set_error("hipMalloc of the second spare field buffer failed");
     return TEA_HIP_ENOMEM;
   }
@@ -956,7 +958,7 @@ int jacobi_queue(tea_hip_chunk* c) {
 int cheby_step(tea_hip_chunk* c, double alpha, double beta) {
   double** f = c->field;
   const Geo g = c->geo;
-  if (!fused_pairs(c)) {
+  if (!fused_pairs(c) || ensure_spare(c) != TEA_HIP_OK) {
     TEA_RETURN_IF(launch_each_cell(
         c, K_CHEBY_ITERATE,
         ChebyIterateBody{f[TEA_FIELD_P], f[TEA_FIELD_R], f[TEA_FIELD_U],
@@ -965,7 +967,6 @@ int cheby_step(tea_hip_chunk* c, double alpha, double beta) {
     return launch_each_cell(c, K_CHEBY_CALC_U,
                             AddBody{f[TEA_FIELD_U], f[TEA_FIELD_P], g});
   }
-  TEA_RETURN_IF(ensure_spare(c));
   {
     Timed t(c, K_CHEBY_FUSED);
     hipLaunchKernelGGL(cheby_pair_kernel, pair_grid(c), dim3(kBlock), 0,
@@ -1007,7 +1008,7 @@ int cheby_two_steps(tea_hip_chunk* c, double a0, double b0, double a1,
 int ppcg_step(tea_hip_chunk* c, double alpha, double beta) {
   double** f = c->field;
   const Geo g = c->geo;
-  if (!fused_pairs(c)) {
+  if (!fused_pairs(c) || ensure_spare(c) != TEA_HIP_OK) {
     TEA_RETURN_IF(launch_each_cell(
         c, K_PPCG_CALC_UR,
         PpcgCalcURBody{f[TEA_FIELD_SD], f[TEA_FIELD_R], f[TEA_FIELD_U],
@@ -1016,7 +1017,6 @@ int ppcg_step(tea_hip_chunk* c, double alpha, double beta) {
         c, K_PPCG_CALC_SD,
         PpcgCalcSDBody{f[TEA_FIELD_SD], f[TEA_FIELD_R], alpha, beta, g});
   }
-  TEA_RETURN_IF(ensure_spare(c));
   {
     Timed t(c, K_PPCG_FUSED);
     hipLaunchKernelGGL(ppcg_pair_kernel, pair_grid(c), dim3(kBlock), 0,

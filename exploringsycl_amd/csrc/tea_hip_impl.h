@@ -1376,9 +1376,12 @@ inline dim3 stacked_grid(const tea_hip_chunk* c, int ks) {
 template <int KS, int T>
 __device__ inline int stacked_block(int S, int* tid, bool bands = true) {
   *tid = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x % T;
-  const int b = band_index<KS>(bands);
-  if (KS == 1) return b;
-  return b % S + S * (b / S * KS + (int)threadIdx.x / T);
+  if (KS == 1) return band_index(bands);
+  // Workgroup w in launch order or, in bands, in place w of the pass.
+  if (!bands)
+    return (int)(blockIdx.x % S) + S * ((int)(blockIdx.x / S) * KS + (int)threadIdx.x / T);
+  const int w = band_index<KS>();
+  return w % S + S * (w / S * KS + (int)threadIdx.x / T);
 }
 
 }  // namespace tea

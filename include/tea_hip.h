@@ -207,11 +207,16 @@ int tea_hip_cg_init(tea_hip_chunk* chunk, int coefficient, double rx,
  * Run-ahead (fused mode, x even, all reductions polled): after this call
  * the device forms alpha = rro / pw itself (rro: the value the last
  * tea_hip_cg_init or tea_hip_cg_calc_ur returned) and already runs
- * r - alpha w into a spare buffer; after tea_hip_cg_calc_ur it forms beta
- * and runs the next w = A p likewise.  The next call takes that work over
- * when its alpha (and, for tea_hip_cg_calc_w, the deferred beta, u update
- * and U/P halo update) is bitwise what the device used; any other call
- * drops it.  Results are bitwise those without it (TEA_HIP_RUN_AHEAD=0). */
+ * r - alpha w and then the next w = A p into spare buffers; after
+ * tea_hip_cg_calc_ur the r-step after that, so that two passes are queued.
+ * The next call takes such a pass over when its alpha (and, for
+ * tea_hip_cg_calc_w, the deferred beta, u update and U/P halo update) is
+ * bitwise what the device used; any other call drops both.  Results are
+ * bitwise those without it (TEA_HIP_RUN_AHEAD=0).
+ * Two calls in turn hold their deferred u update back and the third makes all
+ * three in one pass over u, rounded as if made one by one (TEA_HIP_HOLD_U=0
+ * makes each at once); entry points that read or write u make held updates
+ * first, tea_hip_flush all of them. */
 int tea_hip_cg_calc_w(tea_hip_chunk* chunk, double* pw);
 
 /* u += alpha p, r -= alpha w, *rrn = r.r.  Replaces run_cg_calc_ur
@@ -312,7 +317,8 @@ int tea_hip_mpcg_init(tea_hip_chunk* chunk, int coefficient, double rx,
                       double ry, double* rr, double* bb);
 
 /* If apply_u: u += alpha p_old (FP64).  If apply_p: p = beta p_old + r.
- * Then w = A p (FP32), *pw = p.w and *pr = p.r.  With four cells per lane
+ * Then w = A p (FP32), *pw = p.w and *pr = p.r.  Passes run ahead of the host
+ * as in tea_hip_cg_calc_w, at any x.  With four cells per lane
  * (x a multiple of 4) two calls in turn hold their u update back and the
  * third makes all three in one pass over u, rounded as if made one by one
  * (TEA_HIP_HOLD_U=0 makes each at once); every other entry point except
