@@ -496,9 +496,8 @@ __global__ __launch_bounds__(kBlock * KS) void fused_w1_kernel(Geo g, FusedWArgs
 
 // Launches fused_w1_kernel with stack_factor(c) blocks one row apart per
 // workgroup (stacked_block, tea_hip_impl.h): their rows above and below come
-// mostly from the CU's L1.  At 4096^2 two blocks per workgroup take the FP64
-// iteration from 269.2 to 267.6 us and the mixed-precision w-step from 83.2
-// to 79.0 us (four: 270.6 us).
+// mostly from the CU's L1.  FP64 iteration with one, two and four blocks per
+// workgroup: 4096^2 252.2, 250.3, 261.6 us; 1000^2 20.4, 20.1, 23.0.
 template <bool APPLY_P, int UM, bool CONSUME>
 void launch_fused_w1(tea_hip_chunk* c, const FusedWArgs& a, const RaScalar& sc) {
   const int S = stack_rows(c), ks = stack_factor(c);
