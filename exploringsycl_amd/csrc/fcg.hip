@@ -456,8 +456,15 @@ struct SweepLevel {
   double* part;
   double* xsum;
 };
-__global__ __launch_bounds__(256) void sweeps_kernel(SweepLevel lv0, SweepLevel lv1, int nb0,
-                                                     int sweeps) {
+// T = 1024 threads take a sweep's cells (784 to 324 with six) in one round of
+// divides and LDS latencies instead of up to four; 256 leave four blocks per CU
+// instead of two.  1024 on up to 512 tiles, two per CU: FCG iteration at 2048x1536
+// (204 tiles) 69.8 us with 256 and 68.0 with 1024 (kernel 9.7 and 7.2), 1024^2
+// 45.0 and 44.4, 4096^2 (1088 tiles) 255.0 and 256.9.
+constexpr int kSweepWideTiles = 512;
+template <int T>
+__global__ __launch_bounds__(T) void sweeps_kernel(SweepLevel lv0, SweepLevel lv1, int nb0,
+                                                   int sweeps) {
   const bool second = (int)blockIdx.x >= nb0;
   const int hc = second ? lv1.hc : lv0.hc, wc = second ? lv1.wc : lv0.wc;
   const int ntiles = second ? lv1.ntiles : lv0.ntiles;
@@ -477,7 +484,7 @@ __global__ __launch_bounds__(256) void sweeps_kernel(SweepLevel lv0, SweepLevel 
   const int H = sweeps + 1, R = kSweepTile + 2 * H;
   const int X0 = bx * kSweepTile - H, Y0 = by * kSweepTile - H;
   const long n = (long)hc * wc;
-  for (int q = threadIdx.x; q < (R + 1) * (R + 1); q += 256) {
+  for (int q = threadIdx.x; q < (R + 1) * (R + 1); q += T) {
     const int lx = q % (R + 1), ly = q / (R + 1);
     const int X = X0 + lx, Y = Y0 + ly;
     const bool in = X >= 0 && X < wc && Y >= 0 && Y < hc;
@@ -501,7 +508,7 @@ __global__ __launch_bounds__(256) void sweeps_kernel(SweepLevel lv0, SweepLevel 
     const int lo = s, w = R - 2 * s;
     const double* yp = s_y[cur];
     double* yn = s_y[cur ^ 1];
-    for (int q = threadIdx.x; q < w * w; q += 256) {
+    for (int q = threadIdx.x; q < w * w; q += T) {
       const int lx = lo + q % w, ly = lo + q / w;
       const int k = ly * R + lx;
       const double kl = s_kl[ly * (R + 1) + lx], kr = s_kl[ly * (R + 1) + lx + 1];
@@ -513,25 +520,27 @@ __global__ __launch_bounds__(256) void sweeps_kernel(SweepLevel lv0, SweepLevel 
     __syncthreads();
     cur ^= 1;
   }
-  const double* yv = s_y[cur];
-  const int tx = threadIdx.x & (kSweepTile - 1), ty = threadIdx.x / kSweepTile;
-  const int lx = H + tx, ly = H + ty, k = ly * R + lx;
-  const int X = bx * kSweepTile + tx, Y = by * kSweepTile + ty;
-  auto yr = [&](int kk) { return (double)(float)yv[kk]; };
-  const double kl = s_kl[ly * (R + 1) + lx], kr = s_kl[ly * (R + 1) + lx + 1];
-  const double kb = s_kb[ly * R + lx], kt = s_kb[(ly + 1) * R + lx];
-  const double yc = yr(k);
-  const double tyv = (((1.0 + (kr + kl)) + (kt + kb)) * yc - (kr * yr(k + 1) + kl * yr(k - 1))) -
-                     (kt * yr(k + R) + kb * yr(k - R));
-  double a = 0.0, b = 0.0;
-  if (X < wc && Y < hc) {
-    y[(long)Y * wc + X] = (float)yv[k];
-    a = yc * (double)s_rb[k];
-    b = yc * tyv;
+  if (threadIdx.x < kSweepTile * kSweepTile) {
+    const double* yv = s_y[cur];
+    const int tx = threadIdx.x & (kSweepTile - 1), ty = threadIdx.x / kSweepTile;
+    const int lx = H + tx, ly = H + ty, k = ly * R + lx;
+    const int X = bx * kSweepTile + tx, Y = by * kSweepTile + ty;
+    auto yr = [&](int kk) { return (double)(float)yv[kk]; };
+    const double kl = s_kl[ly * (R + 1) + lx], kr = s_kl[ly * (R + 1) + lx + 1];
+    const double kb = s_kb[ly * R + lx], kt = s_kb[(ly + 1) * R + lx];
+    const double yc = yr(k);
+    const double tyv = (((1.0 + (kr + kl)) + (kt + kb)) * yc - (kr * yr(k + 1) + kl * yr(k - 1))) -
+                       (kt * yr(k + R) + kb * yr(k - R));
+    double a = 0.0, b = 0.0;
+    if (X < wc && Y < hc) {
+      y[(long)Y * wc + X] = (float)yv[k];
+      a = yc * (double)s_rb[k];
+      b = yc * tyv;
+    }
+    s_a[threadIdx.x] = a;
+    s_b[threadIdx.x] = b;
+    s_t[threadIdx.x] = tyv;
   }
-  s_a[threadIdx.x] = a;
-  s_b[threadIdx.x] = b;
-  s_t[threadIdx.x] = tyv;
   __syncthreads();
   for (int st = 128; st > 0; st >>= 1) {
     if (threadIdx.x < st) {
@@ -1528,7 +1537,9 @@ static int launch_sweeps_levels(tea_hip_chunk* c) {
   const unsigned nb0 = level_tiles(L0, kSweepTile);
   const unsigned nb1 = nl == 2 ? level_tiles(L1, kSweepTile) : 0;
   Timed t(c, K_FCG_SWEEPS);
-  hipLaunchKernelGGL(sweeps_kernel, dim3(nb0 + nb1), dim3(256), 0, c->stream, args(L0), args(L1),
+  const bool wide = nb0 + nb1 <= kSweepWideTiles;
+  hipLaunchKernelGGL(wide ? sweeps_kernel<1024> : sweeps_kernel<256>, dim3(nb0 + nb1),
+                     dim3(wide ? 1024 : 256), 0, c->stream, args(L0), args(L1),
                      (int)nb0, c->fcg_sweeps);
   TEA_HIP_TRY(hipGetLastError());
   return TEA_HIP_OK;
