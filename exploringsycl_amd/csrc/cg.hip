@@ -1020,8 +1020,7 @@ int apply_held_u(tea_hip_chunk* c) {
 }
 
 int apply_pending(tea_hip_chunk* c) {
-  TEA_RETURN_IF(mra_discard(c));
-  TEA_RETURN_IF(jacobi_settle(c));
+  TEA_RETURN_IF(drop_ahead(c, kAheadNone));
   c->mra_synced = false;
   TEA_RETURN_IF(apply_cg_pending(c));
   return flush_held(c);

@@ -1840,7 +1840,7 @@ int tea_hip_fcg_precondition(tea_hip_chunk* c, int use_net, double* zw) {
   TEA_CHECK_ARG(zw != nullptr, "null zw");
   TEA_CHECK_ARG(!use_net || c->fcg_levels > 0, "no coarse correction attached");
   TEA_HIP_TRY(hipSetDevice(c->device));
-  TEA_FLUSH_HELD_KEEP_U(c);
+  TEA_FLUSH_HELD_KEEP_MP(c);
   TEA_RETURN_IF(mra_discard(c));
   c->mra_coarse = use_net;
   int len;
@@ -1855,7 +1855,7 @@ int tea_hip_fcg_calc_r_precondition(tea_hip_chunk* c, double alpha, int use_net,
   TEA_CHECK_ARG(rr != nullptr && zw != nullptr, "null outputs");
   TEA_CHECK_ARG(!use_net || c->fcg_levels > 0, "no coarse correction attached");
   TEA_HIP_TRY(hipSetDevice(c->device));
-  TEA_FLUSH_HELD_KEEP_U(c);
+  TEA_FLUSH_HELD_KEEP_MP(c);
   return mp_calc_r(c, true, alpha, use_net, rr, zw);
 }
 
@@ -1865,7 +1865,7 @@ int tea_hip_fcg_calc_w(tea_hip_chunk* c, double alpha, int apply_u, double beta,
   TEA_CHECK_ARG(c->fcg_z != nullptr && c->mp_r != nullptr, "FCG not initialised");
   TEA_CHECK_ARG(pw && pr, "null outputs");
   TEA_HIP_TRY(hipSetDevice(c->device));
-  TEA_FLUSH_HELD_KEEP_U(c);
+  TEA_FLUSH_HELD_KEEP_MP(c);
   // p = z + beta p_old (the mixed-precision kernel with z in place of r),
   // w = A p, and the dots p.w and p.r.
   return mp_calc_w(c, true, alpha, apply_u, beta, 1, pw, pr);

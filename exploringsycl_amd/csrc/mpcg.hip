@@ -1227,7 +1227,7 @@ int tea_hip_mpcg_calc_w(tea_hip_chunk* c, double alpha, int apply_u,
   TEA_CHECK_ARG(c->mp_r != nullptr, "tea_hip_mpcg_init has not been called");
   TEA_CHECK_ARG(pw != nullptr && pr != nullptr, "null outputs");
   TEA_HIP_TRY(hipSetDevice(c->device));
-  TEA_FLUSH_HELD_KEEP_U(c);
+  TEA_FLUSH_HELD_KEEP_MP(c);
   return mp_calc_w(c, false, alpha, apply_u, beta, apply_p, pw, pr);
 }
 
@@ -1236,7 +1236,7 @@ int tea_hip_mpcg_calc_r(tea_hip_chunk* c, double alpha, double* rr, double* rw) 
   TEA_CHECK_ARG(c->mp_r != nullptr, "tea_hip_mpcg_init has not been called");
   TEA_CHECK_ARG(rr != nullptr && rw != nullptr, "null outputs");
   TEA_HIP_TRY(hipSetDevice(c->device));
-  TEA_FLUSH_HELD_KEEP_U(c);
+  TEA_FLUSH_HELD_KEEP_MP(c);
   return mp_calc_r(c, false, alpha, 0, rr, rw);
 }
 

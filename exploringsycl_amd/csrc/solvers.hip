@@ -1128,6 +1128,7 @@ int tea_hip_jacobi_iterate(tea_hip_chunk* c, double* error) {
   const bool folded = c->pre_halo == TEA_HALO_U && !c->held && c->faces_ok_u && c->fused &&
                       use_pair_blocks(c, 1);
   if (c->jra && folded) {
+    TEA_RETURN_IF(drop_ahead(c, kAheadJacobi));
     c->pre_halo = -1;
     // The queued sweep made the new u in a spare buffer; the old u is r now
     // and r's buffer is spare.

@@ -1304,14 +1304,25 @@ int ra_discard(tea_hip_chunk* c);
 // The same for a pass of mixed-precision CG or FCG in flight (mpcg.hip).
 int mra_discard(tea_hip_chunk* c);
 
+// Drops the passes in flight of every solver but `keep`, whose entry points
+// may take theirs over.  The solvers' passes share the block sums, the spare
+// u and the fields themselves, so a call that launches anything, or changes
+// what they read, leaves at most its own in flight.
+enum { kAheadNone, kAheadCg, kAheadMp, kAheadJacobi };
+inline int drop_ahead(tea_hip_chunk* c, int keep) {
+  if (keep != kAheadCg) TEA_RETURN_IF(ra_discard(c));
+  if (keep != kAheadMp) TEA_RETURN_IF(mra_discard(c));
+  if (keep != kAheadJacobi) TEA_RETURN_IF(jacobi_settle(c));
+  return TEA_HIP_OK;
+}
+
 // Checks the handle and makes its device current, leaving a run-ahead in
 // flight (the CG entry points that can take it over); applies a held-back
 // mixed-precision u update.
 #define TEA_ENTER_RA(c)                                   \
   TEA_CHECK_ARG((c) != nullptr, "null chunk handle");     \
   TEA_HIP_TRY(hipSetDevice((c)->device));                 \
-  TEA_RETURN_IF(::tea::mra_discard(c));                   \
-  TEA_RETURN_IF(::tea::jacobi_settle(c));                 \
+  TEA_RETURN_IF(::tea::drop_ahead(c, ::tea::kAheadCg));   \
   (c)->mra_synced = false;                                \
   if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c))
 
@@ -1319,25 +1330,24 @@ int mra_discard(tea_hip_chunk* c);
 // run-ahead of the CG iteration.
 #define TEA_ENTER_HELD(c)                                 \
   TEA_ENTER_RA(c);                                        \
-  TEA_RETURN_IF(::tea::ra_discard(c))
+  TEA_RETURN_IF(::tea::drop_ahead(c, ::tea::kAheadNone))
 
 // Entry points other than the PPCG inner step and the halo update first run
 // a held-back halo update and PPCG or Chebyshev step (and drop a run-ahead)
 // and apply a held-back mixed-precision u update.
 #define TEA_FLUSH_HELD(c)                                                  \
   do {                                                                     \
-    TEA_RETURN_IF(::tea::mra_discard(c));                                  \
-    TEA_RETURN_IF(::tea::jacobi_settle(c));                                \
+    TEA_RETURN_IF(::tea::drop_ahead(c, ::tea::kAheadNone));                \
     if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c));                 \
-    TEA_FLUSH_HELD_KEEP_U(c);                                              \
+    TEA_FLUSH_HELD_KEEP_MP(c);                                             \
   } while (0)
 
-// TEA_FLUSH_HELD leaving a held-back mixed-precision u update held and a
-// mixed-precision pass in flight: for the
-// mixed-precision and FCG steps, which touch neither u nor the held p.
-#define TEA_FLUSH_HELD_KEEP_U(c)                                           \
+// TEA_FLUSH_HELD for the mixed-precision and FCG steps: leaves their own held
+// u updates held (the w-step makes them with its own) and their own passes in
+// flight.
+#define TEA_FLUSH_HELD_KEEP_MP(c)                                          \
   do {                                                                     \
-    TEA_RETURN_IF(::tea::ra_discard(c));                                   \
+    TEA_RETURN_IF(::tea::drop_ahead(c, ::tea::kAheadMp));                  \
     if ((c)->held || (c)->pre_halo >= 0) TEA_RETURN_IF(::tea::flush_held(c)); \
   } while (0)
 

@@ -50,6 +50,25 @@ def _between(c, what, seen):
         c.jacobi_init(1, 0.8, 1.3)
         c.copy_u()
         c.local_halos(1, ["u"])
+    elif what == "mixed w":          # adds 1e-3 p to u
+        seen.append(np.array(c.mpcg_calc_w(1e-3, 1, 0.5, 1)))
+        c.local_halos(1, ["u"])
+    elif what == "mixed r":
+        seen.append(np.array(c.mpcg_calc_r(1e-3)))
+    elif what == "mixed iteration":  # a sweep between w- and r-step
+        pw, pr = c.mpcg_calc_w(0.0, 0, 0.5, 1)
+        c.local_halos(1, ["u"])
+        seen.append(np.array([pw, pr, c.jacobi_iterate(), *c.mpcg_calc_r(pr / pw)]))
+        c.local_halos(1, ["u"])
+    elif what == "precondition":
+        seen.append(np.array([c.fcg_precondition(0)]))
+    elif what == "fcg":              # a sweep between r- and w-step
+        pw, pr = c.fcg_calc_w(1e-3, 1, 0.5)
+        rr, zw = c.fcg_calc_r_precondition(pr / pw, 0)
+        c.local_halos(1, ["u"])
+        seen.append(np.array([pw, pr, rr, zw, c.jacobi_iterate()]))
+        seen.append(np.array(c.fcg_calc_w(pr / pw, 1, -zw / pw)))
+        c.local_halos(1, ["u"])
 
 
 def _run(x, y, h, sweeps, between, env):
@@ -59,6 +78,10 @@ def _run(x, y, h, sweeps, between, env):
         c.set_chunk_data(0.0, 0.0, 0.1, 0.1)
         c.write("density", rng.uniform(0.1, 100.0, x * y))
         c.write("energy", rng.uniform(0.1, 25.0, x * y))
+        if set(between) & set(MIXED):
+            c.fcg_attach()
+            c.fcg_init(1, 0.8, 1.3)
+            c.fcg_precondition(0)
         c.jacobi_init(1, 0.8, 1.3)
         c.copy_u()
         c.local_halos(1, ["u"])
@@ -72,6 +95,7 @@ def _run(x, y, h, sweeps, between, env):
     return np.array(errors), seen
 
 
+MIXED = ("mixed w", "mixed r", "mixed iteration", "precondition", "fcg")
 BETWEEN = ("read", "residual", "halo2", "twice", "other halos", "cheby", "write", "init")
 
 
@@ -89,6 +113,17 @@ BETWEEN = ("read", "residual", "halo2", "twice", "other halos", "cheby", "write"
     (8192, 4097, 2, ("read",)),    # one more: no sweep ahead
 ])
 def test_jacobi_ahead(x, y, h, between):
+    _check(x, y, h, between)
+
+
+@pytest.mark.parametrize("x,y", [(20, 12), (64, 33), (65, 33), (1026, 1030)])
+@pytest.mark.parametrize("between", [MIXED, *((m, m) for m in MIXED)])
+def test_sweeps_in_flight_end_at_a_mixed_precision_or_fcg_step(x, y, between):
+    """A step that writes u, or the sums' workspace, between the sweeps."""
+    _check(x, y, 2, between)
+
+
+def _check(x, y, h, between):
     sweeps = 5 * len(between) + 7
     want = _run(x, y, h, sweeps, between, {"TEA_HIP_PAIRS": "0"})
     for env in ({"TEA_HIP_RUN_AHEAD": "0"}, {"TEA_HIP_RUN_AHEAD": "1"}):
