@@ -1339,16 +1339,17 @@ inline int drop_ahead(tea_hip_chunk* c, int keep) {
   do {                                                                     \
     TEA_RETURN_IF(::tea::drop_ahead(c, ::tea::kAheadNone));                \
     if ((c)->hold) TEA_RETURN_IF(::tea::apply_mp_hold(c));                 \
-    TEA_FLUSH_HELD_KEEP_MP(c);                                             \
+    TEA_RETURN_IF(::tea::flush_held(c));                                   \
   } while (0)
 
 // TEA_FLUSH_HELD for the mixed-precision and FCG steps: leaves their own held
 // u updates held (the w-step makes them with its own) and their own passes in
-// flight.
+// flight, and makes the FP64 iteration's held updates, which are older.
 #define TEA_FLUSH_HELD_KEEP_MP(c)                                          \
   do {                                                                     \
     TEA_RETURN_IF(::tea::drop_ahead(c, ::tea::kAheadMp));                  \
-    if ((c)->held || (c)->pre_halo >= 0) TEA_RETURN_IF(::tea::flush_held(c)); \
+    TEA_RETURN_IF(::tea::apply_held_u(c));                                 \
+    TEA_RETURN_IF(::tea::flush_held(c));                                   \
   } while (0)
 
 #define TEA_ENTER(c)   \

@@ -58,6 +58,10 @@ def _between(c, what, seen):
         seen.append(np.array(c.field_summary()))
     elif what == "mixed":
         seen.append(np.array(c.mpcg_refresh(1e-3, 1)))
+    elif what == "mixed_w":
+        seen.append(np.array(c.mpcg_calc_w(1e-3, 1, 0.5, 1)))
+    elif what == "fcg_w":
+        seen.append(np.array(c.fcg_calc_w(1e-3, 1, 0.5)))
 
 
 def _run(x, y, h, on, iters, between=(), where="end"):
@@ -67,8 +71,10 @@ def _run(x, y, h, on, iters, between=(), where="end"):
         c.set_chunk_data(0.0, 0.0, 0.1, 0.1)
         c.write("density", rng.uniform(0.1, 100.0, x * y))
         c.write("energy", rng.uniform(0.1, 25.0, x * y))
-        if "mixed" in between:
-            c.mpcg_init(2, 0.8, 1.3)
+        if set(between) & {"mixed", "mixed_w", "fcg_w"}:
+            c.fcg_attach()
+            c.fcg_init(2, 0.8, 1.3)
+            c.fcg_precondition(0)
         rro = c.cg_init(2, 0.8, 1.3)
         c.local_halos(1, ["u", "p"])
         c.copy_u()
@@ -120,3 +126,10 @@ def test_held_updates_are_the_steps_one_by_one(x, y, h, iters):
     ("mixed", "mixed", "mixed")])
 def test_held_updates_are_made_before_other_calls(between, where):
     _check(128, 64, 2, 14, between=between, where=where)
+
+
+@pytest.mark.parametrize("where", ["after_w", "after_ur", "end"])
+@pytest.mark.parametrize("x", [128, 127])
+@pytest.mark.parametrize("between", [("mixed_w",) * 3, ("fcg_w",) * 3])
+def test_held_updates_are_made_before_a_mixed_precision_one(between, x, where):
+    _check(x, 64, 2, 14, between=between, where=where)
