@@ -832,11 +832,12 @@ int apply_mp_hold(tea_hip_chunk* c) {
 // is over before the host has seen its scalar and launched another.  They
 // write spare r, z, w and u buffers and a p buffer of the ring that no held
 // update needs, and take alpha and beta from the device.  The host's next
-// call takes a pass over when its arguments are bitwise what the pass used;
-// any other call drops both, and only spare buffers were written.  Each scalar
-// is formed by the next pass itself on grids of at most kConsumeBlocks
-// blocks, else by a finisher.  Nothing is queued past the r-step after which
-// the driver refreshed the last time (the refresh would drop it).
+// call takes a pass over when it is the first of those in flight (mra_turn:
+// a host may ask for the same step twice) and its arguments are bitwise what
+// the pass used; any other call drops both, and only spare buffers were
+// written.  Each scalar is formed by the next pass itself on grids of at most
+// kConsumeBlocks blocks, else by a finisher.  Nothing is queued past the r-step
+// after which the driver refreshed the last time (the refresh would drop it).
 
 namespace {
 
@@ -1059,8 +1060,9 @@ int mra_discard(tea_hip_chunk* c) {
 
 int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta, int apply_p,
               double* pw, double* pr) {
-  const bool taken = c->mra_w && c->mra_fcg == fcg && apply_u && apply_p &&
-                     alpha == c->mra_alpha && beta == c->mra_beta;
+  // The w-step in flight is next only once its r-step has been taken over.
+  const bool taken = c->mra_w && c->mra_turn == kMraSlotW && c->mra_fcg == fcg && apply_u &&
+                     apply_p && alpha == c->mra_alpha && beta == c->mra_beta;
   if ((c->mra_r || c->mra_w) && !taken) mra_mismatch(c);
   bool ahead = taken;
   int len = c->nspan;
@@ -1100,6 +1102,7 @@ int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
   }
   if (ahead) {
     const int slot = c->mra_wi;
+    c->mra_turn = kMraSlotR;
     if (!c->mra_r) TEA_RETURN_IF(mra_queue_r(c, fcg));
     if (c->mra_since + 1 != c->mra_period) TEA_RETURN_IF(mra_queue_w(c, fcg));
     return mra_wait(c, kMraSlotW, slot, pw, pr, &c->mra_alpha);
@@ -1136,11 +1139,13 @@ int launch_mp_r(tea_hip_chunk* c, const MpRStep& s, bool rw, double* sub) {
 
 int mp_calc_r(tea_hip_chunk* c, bool fcg, double alpha, int use_net, double* rr, double* rx) {
   c->mra_since += 1;
-  if (c->mra_r && c->mra_fcg == fcg && alpha == c->mra_alpha &&
+  // With a w-step in flight before it the r-step is that one's.
+  if (c->mra_r && c->mra_turn == kMraSlotR && c->mra_fcg == fcg && alpha == c->mra_alpha &&
       (!fcg || use_net == c->mra_coarse)) {
     swap_buf(c->mp_r, c->mp_r_alt);
     if (fcg) swap_buf(c->fcg_z, c->fcg_z_alt);
     c->mra_r = false;
+    c->mra_turn = kMraSlotW;
     c->mra_fail = 0;
     const int slot = c->mra_ri;
     if (c->mra_w) TEA_RETURN_IF(mra_queue_r(c, fcg));

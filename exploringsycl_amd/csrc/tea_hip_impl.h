@@ -1081,6 +1081,7 @@ struct tea_hip_chunk {
   // flight beyond what the host asked for, the next r-step (mra_r; with FCG
   // also z = M(r)) and the next w-step (mra_w), into spare buffers.
   bool mra_r = false, mra_w = false;
+  int mra_turn = 0;            // kind of the first one (kMraSlotW or R)
   bool mra_fcg = false;        // the passes belong to FCG
   int mra_coarse = 0;          // use_net of the last preconditioner call
   int mra_fail = 0;            // consecutive mismatches (3 turn it off)

@@ -64,6 +64,7 @@ def _solve(cells, coarse, ahead, iters, refresh, stray=None):
                 pw, pr = c.mpcg_calc_w(alpha, pu, beta, pp)
             alpha = pr / pw
             if stray:
+                stray.beta = beta
                 alpha, use = stray(c, it, alpha, use)
             if fcg:
                 rr, rx = c.fcg_calc_r_precondition(alpha, use)
@@ -134,6 +135,24 @@ def test_run_ahead_is_dropped_when_the_host_strays(coarse):
         return alpha, use
 
     _check((128, 64), coarse, iters=18, refresh=50, stray=stray)
+
+
+@pytest.mark.parametrize("cells,coarse", [((128, 64), None), ((121, 50), None),
+                                          ((1100, 1000), None), ((128, 64), "sweeps")])
+def test_a_pass_in_flight_is_taken_over_only_in_its_turn(cells, coarse):
+    """The r-step (4) and the w-step (6) asked for twice in a row, with the
+    scalars that the passes in flight behind them were made with."""
+    def stray(c, it, alpha, use):
+        if it == 4:
+            (c.fcg_calc_r_precondition(alpha, use) if coarse else c.mpcg_calc_r(alpha))
+        if it == 6:
+            beta = stray.beta
+            pw, pr = (c.fcg_calc_w(alpha, True, beta) if coarse
+                      else c.mpcg_calc_w(alpha, True, beta, True))
+            alpha = pr / pw
+        return alpha, use
+
+    _check(cells, coarse, iters=9, refresh=50, stray=stray)
 
 
 def test_init_of_a_second_solve_drops_a_pass_in_flight():
