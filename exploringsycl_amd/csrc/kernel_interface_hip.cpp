@@ -46,8 +46,9 @@ double* field_ptr(tea_hip_chunk* h, int field) {
   return p;
 }
 
-// p, u, r, w and sd are double-buffered by the fused iterations (CG and
-// its run-ahead, Jacobi, Chebyshev, PPCG): republish their addresses after
+// p, u, r, w and sd are double-buffered by the fused iterations (CG,
+// mixed-precision CG and FCG with their run-ahead, Jacobi, Chebyshev, PPCG),
+// and any call may first run a step held back: republish their addresses after
 // every call that can swap them.
 void refresh_fields(Chunk* chunk) {
   tea_hip_chunk* h = H(chunk);
@@ -132,6 +133,7 @@ void run_set_chunk_data(Chunk* chunk, Settings* settings) {
       settings->grid_y_min + settings->dy * (double)chunk->bottom;
   HIP_CALL(tea_hip_set_chunk_data(H(chunk), x_min, y_min, settings->dx,
                                   settings->dy));
+  refresh_fields(chunk);
 }
 
 void run_set_chunk_state(Chunk* chunk, Settings* settings, State* states) {
@@ -156,6 +158,7 @@ void run_set_chunk_state(Chunk* chunk, Settings* settings, State* states) {
   }
   HIP_CALL(tea_hip_set_chunk_state(H(chunk), n, density, energy, x_min, y_min,
                                    x_max, y_max, radius, geometry));
+  refresh_fields(chunk);
   delete[] buf;
   delete[] geometry;
 }
@@ -179,6 +182,7 @@ void run_pack_or_unpack(Chunk* chunk, Settings* settings, int depth, int face,
 void run_store_energy(Chunk* chunk, Settings* settings) {
   (void)settings;
   HIP_CALL(tea_hip_store_energy(H(chunk)));
+  refresh_fields(chunk);
 }
 
 void run_field_summary(Chunk* chunk, Settings* settings, double* vol,
@@ -300,6 +304,7 @@ void run_mpcg_calc_w(Chunk* chunk, Settings* settings, double alpha,
   (void)settings;
   double a, b;
   HIP_CALL(tea_hip_mpcg_calc_w(H(chunk), alpha, apply_u, beta, apply_p, &a, &b));
+  refresh_fields(chunk);
   *pw += a;
   *pr += b;
 }
@@ -309,6 +314,7 @@ void run_mpcg_calc_r(Chunk* chunk, Settings* settings, double alpha,
   (void)settings;
   double a, b;
   HIP_CALL(tea_hip_mpcg_calc_r(H(chunk), alpha, &a, &b));
+  refresh_fields(chunk);
   *rr += a;
   *rw += b;
 }
@@ -318,6 +324,7 @@ void run_mpcg_refresh(Chunk* chunk, Settings* settings, double alpha,
   (void)settings;
   double a, b, w;
   HIP_CALL(tea_hip_mpcg_refresh(H(chunk), alpha, apply_u, &a, &b, &w));
+  refresh_fields(chunk);
   *rr += a;
   *rr_true += b;
   *rw += w;
@@ -327,18 +334,21 @@ void run_read_u(Chunk* chunk, Settings* settings, double* host) {
   (void)settings;
   HIP_CALL(tea_hip_field_read(H(chunk), TEA_FIELD_U, host,
                               (size_t)chunk->x * chunk->y));
+  refresh_fields(chunk);
 }
 
 void run_fcg_attach(Chunk* chunk, Settings* settings, const float* params,
                     size_t count, const float* norm, int coarsen, int levels) {
   (void)settings;
   HIP_CALL(tea_hip_fcg_attach(H(chunk), params, count, norm, coarsen, levels));
+  refresh_fields(chunk);
 }
 
 void run_fcg_attach_sweeps(Chunk* chunk, Settings* settings, int sweeps, int coarsen,
                            int levels) {
   (void)settings;
   HIP_CALL(tea_hip_fcg_attach_sweeps(H(chunk), sweeps, coarsen, levels));
+  refresh_fields(chunk);
 }
 
 void run_fcg_init(Chunk* chunk, Settings* settings, double rx, double ry,
@@ -358,6 +368,7 @@ void run_fcg_precondition(Chunk* chunk, Settings* settings, int use_net,
   (void)settings;
   double v;
   HIP_CALL(tea_hip_fcg_precondition(H(chunk), use_net, &v));
+  refresh_fields(chunk);
   *zw += v;
 }
 
@@ -367,6 +378,7 @@ void run_fcg_calc_r_precondition(Chunk* chunk, Settings* settings,
   (void)settings;
   double a, b;
   HIP_CALL(tea_hip_fcg_calc_r_precondition(H(chunk), alpha, use_net, &a, &b));
+  refresh_fields(chunk);
   *rr += a;
   *zw += b;
 }
@@ -376,6 +388,7 @@ void run_fcg_calc_w(Chunk* chunk, Settings* settings, double alpha,
   (void)settings;
   double a, b;
   HIP_CALL(tea_hip_fcg_calc_w(H(chunk), alpha, apply_u, beta, &a, &b));
+  refresh_fields(chunk);
   *pw += a;
   *pr += b;
 }

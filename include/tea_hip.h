@@ -95,9 +95,10 @@ int tea_hip_chunk_destroy(tea_hip_chunk* chunk);
 /* Device address and element count of a field.  The addresses of
  * TEA_FIELD_P, TEA_FIELD_U, TEA_FIELD_R, TEA_FIELD_W and TEA_FIELD_SD can
  * change after solver calls (the fused CG, Jacobi, Chebyshev and PPCG
- * iterations and the CG run-ahead write the new p, u, r, w or sd into a
- * second buffer and exchange the two); ask again after each call instead
- * of caching them.  The address is returned as
+ * iterations and the run-ahead of CG, mixed-precision CG and FCG write the
+ * new p, u, r, w or sd into a second buffer and exchange the two; other calls
+ * may first run a step held back); ask again after each call instead of
+ * caching them.  The address is returned as
  * is: deferred updates (see tea_hip_set_fused and tea_hip_local_halos) may
  * not have reached the field yet; call tea_hip_flush before reading or
  * writing through it. */
