@@ -741,17 +741,14 @@ int sync_p_alt(tea_hip_chunk* c) {
 
 // The spare p buffers that held updates need (none: updates are not held).
 void ensure_p_ring(tea_hip_chunk* c) {
-  if (!c->hold_ok || c->p_alt[2]) return;
-  for (int i = 1; i < 3; ++i) {
-    if (c->p_alt[i]) continue;
-    if (hipMalloc(&c->p_alt[i], pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
-      c->p_alt[i] = nullptr;
-      (void)hipGetLastError();
-      c->hold_ok = false;
-      return;
-    }
-    c->p_alt_synced = false;
+  if (!c->hold_ok || c->p_ring_off || c->p_alt[2]) return;
+  const size_t bytes = pair_bytes(c->geo.n, sizeof(double));
+  if (!dev_alloc(c, &c->p_alt[1], bytes) || !dev_alloc(c, &c->p_alt[2], bytes)) {
+    dev_free(c, c->p_alt[1]);
+    c->p_ring_off = true;
+    return;
   }
+  c->p_alt_synced = false;
 }
 
 // ---- run-ahead of the fused CG iteration ----------------------------------
@@ -786,38 +783,27 @@ void ensure_p_ring(tea_hip_chunk* c) {
 constexpr int kRaW = 0, kRaRStep = 1;  // slot kinds
 
 bool ra_possible(const tea_hip_chunk* c) {
-  return c->ra_enabled && c->fused && c->poll && c->pairs && c->geo.x % 2 == 0 && c->ra_rro_known &&
-         c->ra_fail < 3 && use_pair_blocks(c, 1) && use_pair_blocks(c, 2);
+  return c->ra_enabled && !c->ra_off && c->fused && c->poll && c->pairs && c->geo.x % 2 == 0 &&
+         c->ra_rro_known && c->ra_fail < 3 && use_pair_blocks(c, 1) && use_pair_blocks(c, 2);
 }
 
 // Offset of a slot in ra_host.
 int ra_slot(int kind, int i) { return 2 * (2 * kind + i); }
 
-int ensure_ra(tea_hip_chunk* c) {
-  if (c->ra_host) return TEA_HIP_OK;
+// Whether the run-ahead's buffers are there (else there is no run-ahead).
+bool ensure_ra(tea_hip_chunk* c) {
+  if (c->ra_host) return true;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(double));
-  for (double** b : {&c->r_alt, &c->u_alt, &c->w_alt}) {
-    if (*b) continue;
-    if (hipMalloc(b, bytes) != hipSuccess) {
-      *b = nullptr;
-      set_error("hipMalloc of a run-ahead buffer failed");
-      return TEA_HIP_ENOMEM;
-    }
-  }
-  if (hipMalloc(&c->ra_dev, 3 * sizeof(double)) != hipSuccess) {
-    c->ra_dev = nullptr;
-    set_error("hipMalloc of the run-ahead scalars failed");
-    return TEA_HIP_ENOMEM;
-  }
-  double* host = nullptr;
-  if (hipHostMalloc(&host, 8 * sizeof(double),
-                    hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
-    set_error("hipHostMalloc of the run-ahead slots failed");
-    return TEA_HIP_ENOMEM;
-  }
-  TEA_HIP_TRY(hipHostGetDevicePointer((void**)&c->ra_host_dev, host, 0));
-  c->ra_host = host;
-  return TEA_HIP_OK;
+  bool ok = true;
+  for (double** b : {&c->r_alt, &c->w_alt, &c->u_alt}) ok = ok && (*b || dev_alloc(c, b, bytes));
+  ok = ok && (c->ra_dev || dev_alloc(c, &c->ra_dev, 3 * sizeof(double)));
+  if (ok) c->ra_host = host_slots(8, &c->ra_host_dev);
+  if (c->ra_host) return true;
+  dev_free(c, c->r_alt);
+  dev_free(c, c->w_alt);
+  if (!c->mra_host) dev_free(c, c->u_alt);
+  c->ra_off = true;
+  return false;
 }
 
 // The next pass forms the scalar of the pass before it (RaScalar::sub).
@@ -1118,7 +1104,9 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
                                   f[TEA_FIELD_KY], f[TEA_FIELD_W], g.x},
                         pw);
   }
-  const bool pair_blocks = use_pair_blocks(c, 1), ahead = pair_blocks && ra_possible(c);
+  // The run-ahead's buffers before those of the held updates, which gain less.
+  const bool pair_blocks = use_pair_blocks(c, 1);
+  const bool ahead = pair_blocks && ra_possible(c) && ensure_ra(c);
   if (pair_blocks) ensure_p_ring(c);
   const double alpha = c->pend_alpha;
   CgStep s;
@@ -1130,7 +1118,6 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
     if (ahead) {
       // Start a run-ahead: the spare buffers take the cells outside the
       // interior (and the ring) that no pass writes.
-      TEA_RETURN_IF(ensure_ra(c));
       TEA_RETURN_IF(copy_frames(c, FramePairs{{f[TEA_FIELD_R], f[TEA_FIELD_U], f[TEA_FIELD_W]},
                                               {c->r_alt, c->u_alt, c->w_alt}}, 3));
     }

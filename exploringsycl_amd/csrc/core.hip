@@ -343,6 +343,40 @@ int launch_span_finish_ra(tea_hip_chunk* c, int nr, double* out, const RaTail& t
   return TEA_HIP_OK;
 }
 
+bool dev_alloc_bytes(tea_hip_chunk* c, void** p, size_t bytes) {
+  *p = nullptr;
+  if (bytes > c->extra_limit - c->extra_bytes) return false;
+  if (hipMalloc(p, bytes) != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+    return false;
+  }
+  c->extra_sizes[*p] = bytes;
+  c->extra_bytes += bytes;
+  return true;
+}
+
+double* host_slots(int n, double** dev) {
+  double* host = nullptr;
+  if (hipHostMalloc(&host, n * sizeof(double), hipHostMallocMapped | hipHostMallocCoherent) ==
+      hipSuccess) {
+    if (hipHostGetDevicePointer((void**)dev, host, 0) == hipSuccess) return host;
+    (void)hipHostFree(host);
+  }
+  (void)hipGetLastError();
+  return nullptr;
+}
+
+void dev_free_bytes(tea_hip_chunk* c, void* p) {
+  if (!p) return;
+  const auto it = c->extra_sizes.find(p);
+  if (it != c->extra_sizes.end()) {
+    c->extra_bytes -= it->second;
+    c->extra_sizes.erase(it);
+  }
+  (void)hipFree(p);
+}
+
 // dst = src in 16-byte pieces, one per thread, nontemporal both ways: the
 // streaming ceiling for tea_hip_copy_bandwidth.
 __global__ __launch_bounds__(kBlock) void stream_copy_kernel(const double* __restrict__ src,
@@ -429,6 +463,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   }
   if (const char* pv = getenv("TEA_HIP_POLL")) c->poll = atoi(pv) != 0;
   if (const char* rv = getenv("TEA_HIP_RUN_AHEAD")) c->ra_enabled = atoi(rv) != 0;
+  if (const char* ev = getenv("TEA_HIP_EXTRA_BYTES")) c->extra_limit = strtoull(ev, nullptr, 10);
   if (const char* sv = getenv("TEA_HIP_STACK")) c->stack = atoi(sv);
   if (const char* sp = getenv("TEA_HIP_SPIN"))
     if (atoi(sp) != 0) (void)hipSetDeviceFlags(hipDeviceScheduleSpin);

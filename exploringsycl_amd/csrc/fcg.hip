@@ -1415,15 +1415,12 @@ __global__ __launch_bounds__(kGammaThreads) void joint_gamma_kernel(
 int ensure_fcg_buffers(tea_hip_chunk* c) {
   if (c->fcg_z) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
-  if (hipMalloc(&c->fcg_z, bytes) != hipSuccess) {
-    c->fcg_z = nullptr;
+  if (!dev_alloc(c, &c->fcg_z, bytes)) {
     set_error("hipMalloc of the FCG z buffer failed");
     return TEA_HIP_ENOMEM;
   }
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_z, 0, bytes, c->stream));
-  if (hipMalloc(&c->fcg_z_alt, bytes) != hipSuccess) {
-    c->fcg_z_alt = nullptr;
-    (void)hipGetLastError();
+  if (!dev_alloc(c, &c->fcg_z_alt, bytes)) {
     c->mra_off = true;  // no run-ahead without it
     return TEA_HIP_OK;
   }
@@ -1663,11 +1660,10 @@ int launch_precondition(tea_hip_chunk* c, int use_net, int slot, int* len) {
 
 }  // namespace tea
 
-static void free_level(FcgLevel& L) {
-  for (float* b : {L.feat, L.rbar, L.kc, L.dis, L.sig, L.y})
-    if (b) (void)hipFree(b);
-  if (L.rms) (void)hipFree(L.rms);
-  if (L.tpart) (void)hipFree(L.tpart);
+static void free_level(tea_hip_chunk* c, FcgLevel& L) {
+  for (float* b : {L.feat, L.rbar, L.kc, L.dis, L.sig, L.y}) dev_free(c, b);
+  dev_free(c, L.rms);
+  dev_free(c, L.tpart);
   if (L.net) tea_nn_destroy(L.net);
   L = FcgLevel();
 }
@@ -1687,11 +1683,9 @@ static int ensure_net_lds(int device) {
 
 // Frees every coarse level and the buffers shared between them.
 static void release_levels(tea_hip_chunk* c) {
-  for (FcgLevel& L : c->fcg_lv) free_level(L);
-  if (c->fcg_xsum) (void)hipFree(c->fcg_xsum);
-  c->fcg_xsum = nullptr;
-  if (c->fcg_g) (void)hipFree(c->fcg_g);
-  c->fcg_g = nullptr;
+  for (FcgLevel& L : c->fcg_lv) free_level(c, L);
+  dev_free(c, c->fcg_xsum);
+  dev_free(c, c->fcg_g);
   c->fcg_levels = 0;
   c->fcg_sweeps = 0;
 }
@@ -1724,18 +1718,17 @@ int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int lev
     L.wc = nx / cl;
     L.ntiles = ((L.wc + kSweepTile - 1) / kSweepTile) * ((L.hc + kSweepTile - 1) / kSweepTile);
     const size_t cn = (size_t)L.hc * L.wc;
-    if (hipMalloc(&L.kc, 2 * cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.rbar, cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.y, cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.tpart, 2 * (size_t)L.ntiles * sizeof(double)) != hipSuccess)
+    if (!dev_alloc(c, &L.kc, 2 * cn * sizeof(float)) ||
+        !dev_alloc(c, &L.rbar, cn * sizeof(float)) || !dev_alloc(c, &L.y, cn * sizeof(float)) ||
+        !dev_alloc(c, &L.tpart, 2 * (size_t)L.ntiles * sizeof(double)))
       return fail();
     c->fcg_levels = l + 1;
   }
-  if (hipMalloc(&c->fcg_g, 2 * sizeof(float)) != hipSuccess) return fail();
+  if (!dev_alloc(c, &c->fcg_g, 2 * sizeof(float))) return fail();
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_g, 0, 2 * sizeof(float), c->stream));
   if (c->fcg_levels == 2) {
     const size_t n1 = (size_t)c->fcg_lv[1].hc * c->fcg_lv[1].wc;
-    if (hipMalloc(&c->fcg_xsum, n1 * sizeof(double)) != hipSuccess) return fail();
+    if (!dev_alloc(c, &c->fcg_xsum, n1 * sizeof(double))) return fail();
   }
   c->fcg_sweeps = sweeps;
   return TEA_HIP_OK;
@@ -1782,22 +1775,20 @@ int tea_hip_fcg_attach(tea_hip_chunk* c, const float* params, size_t count,
     const FcgLevel& L0 = c->fcg_lv[0];
     L.nrms = ((L0.wc + 31) / 32) * ((L0.hc + 3) / 4);
     L.ntiles = ((L.wc + fused::kT - 1) / fused::kT) * ((L.hc + fused::kT - 1) / fused::kT);
-    if (hipMalloc(&L.feat, 2 * cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.kc, 2 * cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.dis, cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.sig, cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.rbar, cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.y, cn * sizeof(float)) != hipSuccess ||
-        hipMalloc(&L.rms, (size_t)L.nrms * sizeof(double)) != hipSuccess ||
-        hipMalloc(&L.tpart, 2 * (size_t)L.ntiles * sizeof(double)) != hipSuccess)
+    if (!dev_alloc(c, &L.feat, 2 * cn * sizeof(float)) ||
+        !dev_alloc(c, &L.kc, 2 * cn * sizeof(float)) ||
+        !dev_alloc(c, &L.dis, cn * sizeof(float)) || !dev_alloc(c, &L.sig, cn * sizeof(float)) ||
+        !dev_alloc(c, &L.rbar, cn * sizeof(float)) || !dev_alloc(c, &L.y, cn * sizeof(float)) ||
+        !dev_alloc(c, &L.rms, (size_t)L.nrms * sizeof(double)) ||
+        !dev_alloc(c, &L.tpart, 2 * (size_t)L.ntiles * sizeof(double)))
       return fail();
     c->fcg_levels = l + 1;
   }
-  if (hipMalloc(&c->fcg_g, 2 * sizeof(float)) != hipSuccess) return fail();
+  if (!dev_alloc(c, &c->fcg_g, 2 * sizeof(float))) return fail();
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_g, 0, 2 * sizeof(float), c->stream));
   if (c->fcg_levels == 2) {
     const size_t n1 = (size_t)c->fcg_lv[1].hc * c->fcg_lv[1].wc;
-    if (hipMalloc(&c->fcg_xsum, n1 * sizeof(double)) != hipSuccess) return fail();
+    if (!dev_alloc(c, &c->fcg_xsum, n1 * sizeof(double))) return fail();
   }
   TEA_RETURN_IF(ensure_net_lds(c->device));
   return TEA_HIP_OK;

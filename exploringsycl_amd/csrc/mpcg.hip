@@ -790,9 +790,7 @@ int ensure_mp_buffers(tea_hip_chunk* c) {
                     &c->mp_r, &c->mp_p[3], &c->mp_r_alt, &c->mp_w_alt};
   for (float** b : bufs) {
     if (*b) continue;
-    if (hipMalloc(b, bytes) != hipSuccess) {
-      *b = nullptr;
-      (void)hipGetLastError();
+    if (!dev_alloc(c, b, bytes)) {
       if (c->mp_r) {
         c->mra_off = true;
         break;
@@ -866,21 +864,11 @@ void swap_buf(T*& a, T*& b) {
 // Whether the run-ahead's buffers are there (else there is no run-ahead).
 bool ensure_mra(tea_hip_chunk* c) {
   if (c->mra_host) return true;
-  if (!c->u_alt && hipMalloc(&c->u_alt, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess)
-    c->u_alt = nullptr;
-  if (!c->mra_dev && hipMalloc(&c->mra_dev, 3 * sizeof(double)) != hipSuccess)
-    c->mra_dev = nullptr;
-  double* host = nullptr;
-  if (c->u_alt && c->mra_dev &&
-      hipHostMalloc(&host, 16 * sizeof(double),
-                    hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
-    if (hipHostGetDevicePointer((void**)&c->mra_host_dev, host, 0) == hipSuccess) {
-      c->mra_host = host;
-      return true;
-    }
-    (void)hipHostFree(host);
-  }
-  (void)hipGetLastError();
+  if ((c->u_alt || dev_alloc(c, &c->u_alt, pair_bytes(c->geo.n, sizeof(double)))) &&
+      (c->mra_dev || dev_alloc(c, &c->mra_dev, 3 * sizeof(double))))
+    c->mra_host = host_slots(16, &c->mra_host_dev);
+  if (c->mra_host) return true;
+  if (!c->ra_host) dev_free(c, c->u_alt);
   c->mra_off = true;
   return false;
 }

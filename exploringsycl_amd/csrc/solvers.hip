@@ -391,9 +391,7 @@ int launch_each_cell(tea_hip_chunk* c, int kid, const Body& body) {
 // The fused Chebyshev and PPCG passes need the x*y spare buffer.
 int ensure_spare(tea_hip_chunk* c) {
   if (c->spare) return TEA_HIP_OK;
-  if (hipMalloc(&c->spare, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
-    c->spare = nullptr;
-    (void)hipGetLastError();
+  if (!dev_alloc(c, &c->spare, pair_bytes(c->geo.n, sizeof(double)))) {
     set_error("hipMalloc of the spare field buffer failed");
     return TEA_HIP_ENOMEM;
   }
@@ -403,9 +401,7 @@ int ensure_spare(tea_hip_chunk* c) {
 // The second spare buffer, allocated on first use.
 int ensure_spare2(tea_hip_chunk* c) {
   if (c->spare2) return TEA_HIP_OK;
-  if (hipMalloc(&c->spare2, pair_bytes(c->geo.n, sizeof(double))) != hipSuccess) {
-    c->spare2 = nullptr;
-    (void)hipGetLastError();
+  if (!dev_alloc(c, &c->spare2, pair_bytes(c->geo.n, sizeof(double)))) {
     set_error("hipMalloc of the second spare field buffer failed");
     return TEA_HIP_ENOMEM;
   }
@@ -895,17 +891,11 @@ bool jacobi_ahead_possible(const tea_hip_chunk* c) {
 // Whether the buffers of sweeps ahead are there (else there are none).
 bool ensure_jacobi_ahead(tea_hip_chunk* c) {
   if (c->j_host) return true;
-  double* host = nullptr;
-  if (ensure_spare(c) == TEA_HIP_OK && ensure_spare2(c) == TEA_HIP_OK &&
-      hipHostMalloc(&host, 2 * sizeof(double),
-                    hipHostMallocMapped | hipHostMallocCoherent) == hipSuccess) {
-    if (hipHostGetDevicePointer((void**)&c->j_host_dev, host, 0) == hipSuccess) {
-      c->j_host = host;
-      return true;
-    }
-    (void)hipHostFree(host);
-  }
-  (void)hipGetLastError();
+  const bool had = c->spare != nullptr;
+  if (ensure_spare(c) == TEA_HIP_OK && ensure_spare2(c) == TEA_HIP_OK)
+    c->j_host = host_slots(2, &c->j_host_dev);
+  if (c->j_host) return true;
+  if (!had) dev_free(c, c->spare);
   c->j_off = true;
   return false;
 }

@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "tea_hip.h"
@@ -1000,6 +1001,12 @@ struct tea_hip_chunk {
   // halo slot, or -1).
   int pre_halo = -1;
 
+  // Device memory of the solvers' buffers (dev_alloc), their sizes, and the
+  // most that they may take (TEA_HIP_EXTRA_BYTES; a refusal is that of a full
+  // device).
+  std::unordered_map<const void*, size_t> extra_sizes;
+  size_t extra_bytes = 0, extra_limit = SIZE_MAX;
+
   // Deferred CG work (fused mode).
   int fused = 1;
   int batch = 0;   // load batch of the fused stencil kernel (0: default)
@@ -1057,6 +1064,8 @@ struct tea_hip_chunk {
   bool ra_r = false, ra_w = false;
   CgStep ra_step;             // the w-step in flight
   bool ra_enabled = true;     // TEA_HIP_RUN_AHEAD=0 turns it off
+  bool ra_off = false;        // a buffer it needs could not be allocated
+  bool p_ring_off = false;    // the same of the held updates' p buffers
   // Blocks one row apart per workgroup of the stencil passes mp_w4_kernel,
   // fused_w1_kernel and jacobi_pair_kernel: 1, 2 (the default) or 4
   // (TEA_HIP_STACK).  (fcg_z4_kernel, whose only row above is ky's, took
@@ -1298,6 +1307,23 @@ int launch_halo_of(tea_hip_chunk* c, double* field);
 // One reflective-halo launch (all flagged fields and external faces).
 int launch_halos(tea_hip_chunk* c, int depth, const int neighbours[4],
                  const int fields[6]);
+
+// Device memory for one of the solvers' buffers, within the chunk's limit:
+// false (and *p null) where there is none.
+bool dev_alloc_bytes(tea_hip_chunk* c, void** p, size_t bytes);
+void dev_free_bytes(tea_hip_chunk* c, void* p);
+template <class T>
+bool dev_alloc(tea_hip_chunk* c, T** p, size_t bytes) {
+  return dev_alloc_bytes(c, (void**)p, bytes);
+}
+// `n` doubles of pinned, coherent host memory for values that the device
+// leaves (null: there is none), and the device's view of them.
+double* host_slots(int n, double** dev);
+template <class T>
+void dev_free(tea_hip_chunk* c, T*& p) {
+  dev_free_bytes(c, p);
+  p = nullptr;
+}
 
 // Drops a run-ahead of the fused CG iteration (cg.hip): it wrote only
 // spare buffers and device scalars, so nothing is undone.
