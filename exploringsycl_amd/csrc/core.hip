@@ -345,15 +345,35 @@ int launch_span_finish_ra(tea_hip_chunk* c, int nr, double* out, const RaTail& t
 
 bool dev_alloc_bytes(tea_hip_chunk* c, void** p, size_t bytes) {
   *p = nullptr;
-  if (bytes > c->extra_limit - c->extra_bytes) return false;
+  if (bytes > c->dev_limit - c->dev_bytes) return false;
   if (hipMalloc(p, bytes) != hipSuccess) {
     *p = nullptr;
     (void)hipGetLastError();
     return false;
   }
-  c->extra_sizes[*p] = bytes;
-  c->extra_bytes += bytes;
+  c->dev_sizes[*p] = bytes;
+  c->dev_bytes += bytes;
   return true;
+}
+
+int release_spares(tea_hip_chunk* c, bool keep_pair) {
+  TEA_RETURN_IF(drop_ahead(c, kAheadNone));
+  if (c->hold) TEA_RETURN_IF(apply_mp_hold(c));
+  TEA_RETURN_IF(apply_held_u(c));
+  TEA_RETURN_IF(sync_chunk(c));
+  for (double** b : {&c->p_alt[1], &c->p_alt[2], &c->r_alt, &c->w_alt, &c->u_alt})
+    dev_free(c, *b);
+  if (c->mp_cur == 3) {
+    std::swap(c->mp_p[0], c->mp_p[3]);
+    c->mp_cur = 0;
+  }
+  for (float** b : {&c->mp_p[3], &c->mp_r_alt, &c->mp_w_alt, &c->fcg_z_alt}) dev_free(c, *b);
+  c->p_ring_off = c->ra_off = c->mra_off = true;
+  if (keep_pair) return TEA_HIP_OK;
+  dev_free(c, c->spare);
+  dev_free(c, c->spare2);
+  c->j_off = true;
+  return TEA_HIP_OK;
 }
 
 double* host_slots(int n, double** dev) {
@@ -369,11 +389,9 @@ double* host_slots(int n, double** dev) {
 
 void dev_free_bytes(tea_hip_chunk* c, void* p) {
   if (!p) return;
-  const auto it = c->extra_sizes.find(p);
-  if (it != c->extra_sizes.end()) {
-    c->extra_bytes -= it->second;
-    c->extra_sizes.erase(it);
-  }
+  const auto it = c->dev_sizes.find(p);
+  c->dev_bytes -= it->second;
+  c->dev_sizes.erase(it);
   (void)hipFree(p);
 }
 
@@ -463,7 +481,6 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   }
   if (const char* pv = getenv("TEA_HIP_POLL")) c->poll = atoi(pv) != 0;
   if (const char* rv = getenv("TEA_HIP_RUN_AHEAD")) c->ra_enabled = atoi(rv) != 0;
-  if (const char* ev = getenv("TEA_HIP_EXTRA_BYTES")) c->extra_limit = strtoull(ev, nullptr, 10);
   if (const char* sv = getenv("TEA_HIP_STACK")) c->stack = atoi(sv);
   if (const char* sp = getenv("TEA_HIP_SPIN"))
     if (atoi(sp) != 0) (void)hipSetDeviceFlags(hipDeviceScheduleSpin);
@@ -495,8 +512,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
 
   for (int f = 0; f < TEA_NUM_FIELDS; ++f) {
     const size_t bytes = pair_bytes((long)c->field_len[f], sizeof(double));
-    if (hipMalloc(&c->field[f], bytes) != hipSuccess) {
-      c->field[f] = nullptr;
+    if (!dev_alloc(c, &c->field[f], bytes)) {
       set_error("hipMalloc of a field failed");
       return fail(TEA_HIP_ENOMEM);
     }
@@ -505,8 +521,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
       return fail(TEA_HIP_EHIP);
     }
   }
-  if (hipMalloc(&c->p_alt[0], pair_bytes(n, sizeof(double))) != hipSuccess) {
-    c->p_alt[0] = nullptr;
+  if (!dev_alloc(c, &c->p_alt[0], pair_bytes(n, sizeof(double)))) {
     set_error("hipMalloc of the second p buffer failed");
     return fail(TEA_HIP_ENOMEM);
   }
@@ -514,8 +529,7 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   // finisher's counter.
   const size_t ns = (size_t)kSubMaxNr * sub_stride(c->nblk), ng = ns / kGroupBlocks;
   const size_t rbytes = (2 * ns + ng + 1) * sizeof(double);
-  if (hipMalloc(&c->sub, rbytes) != hipSuccess) {
-    c->sub = nullptr;
+  if (!dev_alloc(c, &c->sub, rbytes)) {
     set_error("hipMalloc of the reduction workspace failed");
     return fail(TEA_HIP_ENOMEM);
   }
@@ -542,6 +556,10 @@ int tea_hip_chunk_create(int device, int x, int y, int halo_depth,
   if (hipStreamSynchronize(c->stream) != hipSuccess) {
     set_error("hipStreamSynchronize failed");
     return fail(TEA_HIP_EHIP);
+  }
+  if (const char* ev = getenv("TEA_HIP_EXTRA_BYTES")) {
+    const size_t extra = strtoull(ev, nullptr, 10);
+    if (extra < SIZE_MAX - c->dev_bytes) c->dev_limit = c->dev_bytes + extra;
   }
   *out = c;
   return TEA_HIP_OK;

@@ -1415,12 +1415,9 @@ __global__ __launch_bounds__(kGammaThreads) void joint_gamma_kernel(
 int ensure_fcg_buffers(tea_hip_chunk* c) {
   if (c->fcg_z) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
-  if (!dev_alloc(c, &c->fcg_z, bytes)) {
-    set_error("hipMalloc of the FCG z buffer failed");
-    return TEA_HIP_ENOMEM;
-  }
+  TEA_RETURN_IF(need_alloc(c, &c->fcg_z, bytes, "the FCG z buffer"));
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_z, 0, bytes, c->stream));
-  if (!dev_alloc(c, &c->fcg_z_alt, bytes)) {
+  if (c->mra_off || !dev_alloc(c, &c->fcg_z_alt, bytes)) {
     c->mra_off = true;  // no run-ahead without it
     return TEA_HIP_OK;
   }
@@ -1704,9 +1701,8 @@ int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int lev
   const int nx = c->geo.x - 2 * c->geo.h, ny = c->geo.y - 2 * c->geo.h;
   TEA_CHECK_ARG(nx % coarsen == 0 && ny % coarsen == 0,
                 "the interior must be a multiple of the coarsening factor");
-  auto fail = [] {
-    set_error("hipMalloc of the preconditioner's coarse buffers failed");
-    return TEA_HIP_ENOMEM;
+  auto get = [c](auto** p, size_t bytes) {
+    return need_alloc(c, p, bytes, "the preconditioner's coarse buffers");
   };
   // Level l coarsens by 8 * 4^l while the interior divides.
   for (int l = 0; l < levels; ++l) {
@@ -1718,17 +1714,16 @@ int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int lev
     L.wc = nx / cl;
     L.ntiles = ((L.wc + kSweepTile - 1) / kSweepTile) * ((L.hc + kSweepTile - 1) / kSweepTile);
     const size_t cn = (size_t)L.hc * L.wc;
-    if (!dev_alloc(c, &L.kc, 2 * cn * sizeof(float)) ||
-        !dev_alloc(c, &L.rbar, cn * sizeof(float)) || !dev_alloc(c, &L.y, cn * sizeof(float)) ||
-        !dev_alloc(c, &L.tpart, 2 * (size_t)L.ntiles * sizeof(double)))
-      return fail();
+    TEA_RETURN_IF(get(&L.kc, 2 * cn * sizeof(float)));
+    for (float** b : {&L.rbar, &L.y}) TEA_RETURN_IF(get(b, cn * sizeof(float)));
+    TEA_RETURN_IF(get(&L.tpart, 2 * (size_t)L.ntiles * sizeof(double)));
     c->fcg_levels = l + 1;
   }
-  if (!dev_alloc(c, &c->fcg_g, 2 * sizeof(float))) return fail();
+  TEA_RETURN_IF(get(&c->fcg_g, 2 * sizeof(float)));
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_g, 0, 2 * sizeof(float), c->stream));
   if (c->fcg_levels == 2) {
     const size_t n1 = (size_t)c->fcg_lv[1].hc * c->fcg_lv[1].wc;
-    if (!dev_alloc(c, &c->fcg_xsum, n1 * sizeof(double))) return fail();
+    TEA_RETURN_IF(get(&c->fcg_xsum, n1 * sizeof(double)));
   }
   c->fcg_sweeps = sweeps;
   return TEA_HIP_OK;
@@ -1755,9 +1750,8 @@ int tea_hip_fcg_attach(tea_hip_chunk* c, const float* params, size_t count,
   TEA_CHECK_ARG((nx / coarsen) % 32 == 0, "coarse width must be a multiple of 32");
   // Level l coarsens by coarsen * 4^l; a level is added while the grid
   // divides and its width stays a multiple of 32.
-  auto fail = [] {
-    set_error("hipMalloc of the preconditioner's coarse buffers failed");
-    return TEA_HIP_ENOMEM;
+  auto get = [c](auto** p, size_t bytes) {
+    return need_alloc(c, p, bytes, "the preconditioner's coarse buffers");
   };
   TEA_CHECK_ARG(coarsen == 8, "the network's restriction needs a coarsening factor of 8");
   for (int l = 0; l < levels; ++l) {
@@ -1768,27 +1762,29 @@ int tea_hip_fcg_attach(tea_hip_chunk* c, const float* params, size_t count,
     L.hc = ny / cl;
     L.wc = nx / cl;
     const size_t cn = (size_t)L.hc * L.wc;
-    TEA_RETURN_IF(tea_nn_create(c->device, 1, L.hc, L.wc, &L.net));
+    int st = tea_nn_create(c->device, 1, L.hc, L.wc, &L.net);
+    if (st == TEA_HIP_ENOMEM) {
+      TEA_RETURN_IF(release_spares(c, false));
+      st = tea_nn_create(c->device, 1, L.hc, L.wc, &L.net);
+    }
+    TEA_RETURN_IF(st);
     TEA_RETURN_IF(tea_nn_set_params(L.net, params, count));
     // One RMS partial per block of the restriction (restrict8_kernel's grid
     // over level 0), for either level.
     const FcgLevel& L0 = c->fcg_lv[0];
     L.nrms = ((L0.wc + 31) / 32) * ((L0.hc + 3) / 4);
     L.ntiles = ((L.wc + fused::kT - 1) / fused::kT) * ((L.hc + fused::kT - 1) / fused::kT);
-    if (!dev_alloc(c, &L.feat, 2 * cn * sizeof(float)) ||
-        !dev_alloc(c, &L.kc, 2 * cn * sizeof(float)) ||
-        !dev_alloc(c, &L.dis, cn * sizeof(float)) || !dev_alloc(c, &L.sig, cn * sizeof(float)) ||
-        !dev_alloc(c, &L.rbar, cn * sizeof(float)) || !dev_alloc(c, &L.y, cn * sizeof(float)) ||
-        !dev_alloc(c, &L.rms, (size_t)L.nrms * sizeof(double)) ||
-        !dev_alloc(c, &L.tpart, 2 * (size_t)L.ntiles * sizeof(double)))
-      return fail();
+    for (float** b : {&L.feat, &L.kc}) TEA_RETURN_IF(get(b, 2 * cn * sizeof(float)));
+    for (float** b : {&L.dis, &L.sig, &L.rbar, &L.y}) TEA_RETURN_IF(get(b, cn * sizeof(float)));
+    TEA_RETURN_IF(get(&L.rms, (size_t)L.nrms * sizeof(double)));
+    TEA_RETURN_IF(get(&L.tpart, 2 * (size_t)L.ntiles * sizeof(double)));
     c->fcg_levels = l + 1;
   }
-  if (!dev_alloc(c, &c->fcg_g, 2 * sizeof(float))) return fail();
+  TEA_RETURN_IF(get(&c->fcg_g, 2 * sizeof(float)));
   TEA_HIP_TRY(hipMemsetAsync(c->fcg_g, 0, 2 * sizeof(float), c->stream));
   if (c->fcg_levels == 2) {
     const size_t n1 = (size_t)c->fcg_lv[1].hc * c->fcg_lv[1].wc;
-    if (!dev_alloc(c, &c->fcg_xsum, n1 * sizeof(double))) return fail();
+    TEA_RETURN_IF(get(&c->fcg_xsum, n1 * sizeof(double)));
   }
   TEA_RETURN_IF(ensure_net_lds(c->device));
   return TEA_HIP_OK;

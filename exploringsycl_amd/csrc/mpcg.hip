@@ -785,18 +785,20 @@ struct MpTrueResidualBody {
 int ensure_mp_buffers(tea_hip_chunk* c) {
   if (c->mp_r) return TEA_HIP_OK;
   const size_t bytes = pair_bytes(c->geo.n, sizeof(float));
-  // The last three, for the run-ahead alone, may be missing.
-  float** bufs[] = {&c->mp_p[0], &c->mp_p[1], &c->mp_p[2], &c->mp_w, &c->mp_kx, &c->mp_ky,
-                    &c->mp_r, &c->mp_p[3], &c->mp_r_alt, &c->mp_w_alt};
-  for (float** b : bufs) {
+  for (float** b : {&c->mp_p[0], &c->mp_p[1], &c->mp_p[2], &c->mp_w, &c->mp_kx, &c->mp_ky,
+                    &c->mp_r}) {
     if (*b) continue;
+    TEA_RETURN_IF(need_alloc(c, b, bytes, "an FP32 CG buffer"));
+    TEA_HIP_TRY(hipMemsetAsync(*b, 0, bytes, c->stream));
+  }
+  // For the run-ahead alone.
+  for (float** b : {&c->mp_p[3], &c->mp_r_alt, &c->mp_w_alt}) {
+    if (c->mra_off) break;
     if (!dev_alloc(c, b, bytes)) {
-      if (c->mp_r) {
-        c->mra_off = true;
-        break;
-      }
-      set_error("hipMalloc of an FP32 CG buffer failed");
-      return TEA_HIP_ENOMEM;
+      dev_free(c, c->mp_p[3]);
+      dev_free(c, c->mp_r_alt);
+      c->mra_off = true;
+      break;
     }
     TEA_HIP_TRY(hipMemsetAsync(*b, 0, bytes, c->stream));
   }

@@ -811,6 +811,7 @@ size_t act_elems(const tea_nn* n, int c) {
 int nn_alloc(void** p, size_t bytes, hipStream_t st) {
   if (hipMalloc(p, bytes) != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();
     set_error("hipMalloc failed in the network workspace");
     return TEA_HIP_ENOMEM;
   }

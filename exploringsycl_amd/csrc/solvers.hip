@@ -391,21 +391,15 @@ int launch_each_cell(tea_hip_chunk* c, int kid, const Body& body) {
 // The fused Chebyshev and PPCG passes need the x*y spare buffer.
 int ensure_spare(tea_hip_chunk* c) {
   if (c->spare) return TEA_HIP_OK;
-  if (!dev_alloc(c, &c->spare, pair_bytes(c->geo.n, sizeof(double)))) {
-    set_error("hipMalloc of the spare field buffer failed");
-    return TEA_HIP_ENOMEM;
-  }
-  return TEA_HIP_OK;
+  return need_alloc(c, &c->spare, pair_bytes(c->geo.n, sizeof(double)), "the spare field buffer",
+                    true);
 }
 
 // The second spare buffer, allocated on first use.
 int ensure_spare2(tea_hip_chunk* c) {
   if (c->spare2) return TEA_HIP_OK;
-  if (!dev_alloc(c, &c->spare2, pair_bytes(c->geo.n, sizeof(double)))) {
-    set_error("hipMalloc of the second spare field buffer failed");
-    return TEA_HIP_ENOMEM;
-  }
-  return TEA_HIP_OK;
+  return need_alloc(c, &c->spare2, pair_bytes(c->geo.n, sizeof(double)),
+                    "the second spare field buffer", true);
 }
 
 // Fused passes run in the default mode.
@@ -892,7 +886,8 @@ bool jacobi_ahead_possible(const tea_hip_chunk* c) {
 bool ensure_jacobi_ahead(tea_hip_chunk* c) {
   if (c->j_host) return true;
   const bool had = c->spare != nullptr;
-  if (ensure_spare(c) == TEA_HIP_OK && ensure_spare2(c) == TEA_HIP_OK)
+  const size_t bytes = pair_bytes(c->geo.n, sizeof(double));
+  if ((c->spare || dev_alloc(c, &c->spare, bytes)) && (c->spare2 || dev_alloc(c, &c->spare2, bytes)))
     c->j_host = host_slots(2, &c->j_host_dev);
   if (c->j_host) return true;
   if (!had) dev_free(c, c->spare);

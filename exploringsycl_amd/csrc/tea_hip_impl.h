@@ -1001,11 +1001,11 @@ struct tea_hip_chunk {
   // halo slot, or -1).
   int pre_halo = -1;
 
-  // Device memory of the solvers' buffers (dev_alloc), their sizes, and the
-  // most that they may take (TEA_HIP_EXTRA_BYTES; a refusal is that of a full
-  // device).
-  std::unordered_map<const void*, size_t> extra_sizes;
-  size_t extra_bytes = 0, extra_limit = SIZE_MAX;
+  // Device memory of the chunk (dev_alloc), its buffers' sizes, and the most
+  // that it may take (TEA_HIP_EXTRA_BYTES beyond what creation took; a refusal
+  // is that of a full device).
+  std::unordered_map<const void*, size_t> dev_sizes;
+  size_t dev_bytes = 0, dev_limit = SIZE_MAX;
 
   // Deferred CG work (fused mode).
   int fused = 1;
@@ -1308,13 +1308,26 @@ int launch_halo_of(tea_hip_chunk* c, double* field);
 int launch_halos(tea_hip_chunk* c, int depth, const int neighbours[4],
                  const int fields[6]);
 
-// Device memory for one of the solvers' buffers, within the chunk's limit:
-// false (and *p null) where there is none.
+// Device memory within the chunk's limit: false (and *p null) where there is
+// none.  Buffers of one size may have changed places with a field's.
 bool dev_alloc_bytes(tea_hip_chunk* c, void** p, size_t bytes);
 void dev_free_bytes(tea_hip_chunk* c, void* p);
 template <class T>
 bool dev_alloc(tea_hip_chunk* c, T** p, size_t bytes) {
   return dev_alloc_bytes(c, (void**)p, bytes);
+}
+// Gives back the buffers that solvers only run faster with (those of passes in
+// flight and held updates, which end first; the spare field pair unless
+// keep_pair) and leaves them out from then on.
+int release_spares(tea_hip_chunk* c, bool keep_pair);
+// A buffer that a solver cannot do without.
+template <class T>
+int need_alloc(tea_hip_chunk* c, T** p, size_t bytes, const char* what, bool keep_pair = false) {
+  if (dev_alloc(c, p, bytes)) return TEA_HIP_OK;
+  TEA_RETURN_IF(release_spares(c, keep_pair));
+  if (dev_alloc(c, p, bytes)) return TEA_HIP_OK;
+  set_error(std::string("hipMalloc of ") + what + " failed");
+  return TEA_HIP_ENOMEM;
 }
 // `n` doubles of pinned, coherent host memory for values that the device
 // leaves (null: there is none), and the device's view of them.

@@ -1,6 +1,7 @@
 """Solves where the spare buffers do not fit (TEA_HIP_EXTRA_BYTES limits what a
-chunk may take beyond its fields): the solvers run in the memory they cannot do
-without, with the scalars and fields of the unlimited one bit for bit."""
+chunk may take beyond its fields): every solver runs in the memory it cannot do
+without, after any other on the same chunk, with the scalars and fields of the
+unlimited one bit for bit."""
 
 import os
 
@@ -122,13 +123,29 @@ SIZES = [(132, 68), (134, 68), (1028, 1028)]
 
 
 @pytest.mark.parametrize("x,y", SIZES + [(133, 69)])
-@pytest.mark.parametrize("name", ["cg", "jacobi", "mixed"])
+@pytest.mark.parametrize("name", [n for n in SOLVERS if n != "fcg"])
 def test_solves_in_what_it_cannot_do_without(name, x, y):
     """From the least memory, in steps of half a field (one FP32 buffer), until
     every spare buffer fits: each buffer in turn is the first refused."""
     need = SOLVERS[name][1]
     for halves in range(15):
         _check(x, y, [name], (need + halves / 2) * _field(x, y) + SMALL // 2)
+
+
+@pytest.mark.parametrize("x,y", [(132, 68), (1028, 1028)])
+def test_fcg_solves_in_what_it_cannot_do_without(x, y):
+    for halves in range(12):
+        _check(x, y, ["fcg"], (4 + halves / 2) * _field(x, y) + (x * y) // 2 + SMALL)
+
+
+@pytest.mark.parametrize("order", [
+    ("cg", "mixed", "fcg", "cheby", "cg"), ("jacobi", "fcg", "ppcg", "mixed"),
+    ("mixed", "cg", "jacobi", "fcg"), ("fcg", "jacobi", "cheby", "mixed", "jacobi")])
+@pytest.mark.parametrize("x,y", [(132, 68), (1028, 1028)])
+def test_spare_buffers_of_one_solver_make_room_for_another(x, y, order):
+    need = 4 + (2 if "cheby" in order or "ppcg" in order else 0)
+    for halves in (0, 1, 3, 6, 9):
+        _check(x, y, order, (need + halves / 2) * _field(x, y) + (x * y) // 2 + SMALL)
 
 
 def test_what_does_not_fit_is_refused_and_the_chunk_goes_on():
