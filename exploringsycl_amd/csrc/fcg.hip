@@ -1687,6 +1687,15 @@ static void release_levels(tea_hip_chunk* c) {
   c->fcg_sweeps = 0;
 }
 
+// Frees them when an attach ends half way: levels without the buffers shared
+// between them (null in the kernels) are no preconditioner.
+struct LevelsGuard {
+  tea_hip_chunk* c;
+  ~LevelsGuard() {
+    if (c) release_levels(c);
+  }
+};
+
 extern "C" {
 
 int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int levels) {
@@ -1698,6 +1707,7 @@ int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int lev
   TEA_FLUSH_HELD(c);
   TEA_RETURN_IF(ensure_fcg_buffers(c));
   release_levels(c);
+  LevelsGuard guard{c};
   const int nx = c->geo.x - 2 * c->geo.h, ny = c->geo.y - 2 * c->geo.h;
   TEA_CHECK_ARG(nx % coarsen == 0 && ny % coarsen == 0,
                 "the interior must be a multiple of the coarsening factor");
@@ -1726,6 +1736,7 @@ int tea_hip_fcg_attach_sweeps(tea_hip_chunk* c, int sweeps, int coarsen, int lev
     TEA_RETURN_IF(get(&c->fcg_xsum, n1 * sizeof(double)));
   }
   c->fcg_sweeps = sweeps;
+  guard.c = nullptr;
   return TEA_HIP_OK;
 }
 
@@ -1737,6 +1748,7 @@ int tea_hip_fcg_attach(tea_hip_chunk* c, const float* params, size_t count,
   TEA_RETURN_IF(ensure_fcg_buffers(c));
   release_levels(c);
   if (!params) return TEA_HIP_OK;  // Jacobi only
+  LevelsGuard guard{c};
   TEA_CHECK_ARG(feature_norm != nullptr, "null feature normalisation");
   TEA_CHECK_ARG(coarsen >= 1 && (coarsen & (coarsen - 1)) == 0,
                 "coarsening factor must be a power of two");
@@ -1787,6 +1799,7 @@ int tea_hip_fcg_attach(tea_hip_chunk* c, const float* params, size_t count,
     TEA_RETURN_IF(get(&c->fcg_xsum, n1 * sizeof(double)));
   }
   TEA_RETURN_IF(ensure_net_lds(c->device));
+  guard.c = nullptr;
   return TEA_HIP_OK;
 }
 

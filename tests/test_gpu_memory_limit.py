@@ -162,3 +162,31 @@ def test_what_does_not_fit_is_refused_and_the_chunk_goes_on():
         got = _cg(c)
     for a, b in zip(want, got):
         assert np.array_equal(np.atleast_1d(a).view(np.uint8), np.atleast_1d(b).view(np.uint8))
+
+
+@pytest.mark.parametrize("room", [0.1, 0.6, 0.97])
+@pytest.mark.parametrize("net", [False, True])
+def test_an_attach_that_fails_half_way_leaves_no_level(net, room):
+    """The coarse levels take less than a field: with `room` of what they need
+    some of their buffers are there (with 0.97 the first level's) and the attach
+    fails; the Jacobi preconditioner goes on."""
+    from exploringsycl_amd import learned
+    from exploringsycl_amd.native import TeaHipError, check
+    x, y = 1028, 516   # two levels, of 128 x 64 and 32 x 16 cells
+    coarse = 4 * (128 * 64 + 32 * 16) * (8 if net else 4)
+    rng = np.random.default_rng(x)
+    with _chunk(x, y, 4 * _field(x, y) + 64 + room * coarse) as c:
+        c.write("density", rng.uniform(0.1, 100.0, x * y))
+        c.write("energy", rng.uniform(0.1, 25.0, x * y))
+        c.mpcg_init(2, 0.8, 1.3)
+        with pytest.raises(TeaHipError, match=r"\(-3\)"):
+            if net:
+                params, norm, coarsen = learned.read_weights()
+                c.fcg_attach(params, norm, coarsen=coarsen, levels=2)
+            else:
+                check(c.lib.tea_hip_fcg_attach_sweeps(c.handle, 6, 8, 2), "attach")
+        assert c.fcg_levels() == 0
+        c.fcg_init(2, 0.8, 1.3)
+        with pytest.raises(TeaHipError, match="no coarse correction"):
+            c.fcg_precondition(1)
+        assert np.isfinite(c.fcg_precondition(0))
