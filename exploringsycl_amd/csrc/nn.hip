@@ -800,6 +800,7 @@ struct tea_nn {
   float *ds_in = nullptr, *ds_tgt = nullptr;
   int ds_n = 0;
   int* ds_order = nullptr;
+  int order_len = 0;         // samples that ds_order holds
 };
 
 namespace {
@@ -1210,10 +1211,12 @@ int tea_nn_load_dataset(tea_nn* n, int count, const float* inputs, const float* 
   if (n->ds_order) (void)hipFree(n->ds_order);
   n->ds_in = n->ds_tgt = nullptr;
   n->ds_order = nullptr;
+  n->ds_n = 0;
   const size_t px = (size_t)n->H * n->W;
   TEA_RETURN_IF(nn_alloc((void**)&n->ds_in, (size_t)count * px * kIn * sizeof(float), n->stream));
   TEA_RETURN_IF(nn_alloc((void**)&n->ds_tgt, (size_t)count * px * sizeof(float), n->stream));
   TEA_RETURN_IF(nn_alloc((void**)&n->ds_order, (size_t)count * sizeof(int), n->stream));
+  n->order_len = count;
   TEA_HIP_TRY(hipMemcpyAsync(n->ds_in, inputs, (size_t)count * px * kIn * sizeof(float),
                              hipMemcpyHostToDevice, n->stream));
   TEA_HIP_TRY(hipMemcpyAsync(n->ds_tgt, targets, (size_t)count * px * sizeof(float),
@@ -1228,12 +1231,20 @@ int tea_nn_load_dataset(tea_nn* n, int count, const float* inputs, const float* 
 int tea_nn_train_epoch(tea_nn* n, const int* order, int count, int batch, float lr,
                        float* mean_loss) {
   NN_CHECK(n);
-  TEA_CHECK_ARG(n->ds_in != nullptr, "no dataset loaded");
+  TEA_CHECK_ARG(n->ds_n > 0, "no dataset loaded");
   TEA_CHECK_ARG(n->del[0] != nullptr, "training needs width <= 128");
   TEA_CHECK_ARG(batch >= 1 && batch <= n->max_batch && count >= batch, "bad batch");
   TEA_HIP_TRY(hipSetDevice(n->device));
   for (int i = 0; i < count; ++i)
     TEA_CHECK_ARG(order[i] >= 0 && order[i] < n->ds_n, "sample index out of range");
+  // An epoch may be longer than the set (samples drawn with repetition).
+  if (count > n->order_len) {
+    int* more = nullptr;
+    TEA_RETURN_IF(nn_alloc((void**)&more, (size_t)count * sizeof(int), n->stream));
+    (void)hipFree(n->ds_order);
+    n->ds_order = more;
+    n->order_len = count;
+  }
   TEA_HIP_TRY(hipMemcpyAsync(n->ds_order, order, (size_t)count * sizeof(int),
                              hipMemcpyHostToDevice, n->stream));
   // The batches' loss partials stay on the device until the epoch's end: a

@@ -66,3 +66,20 @@ def test_forward_of_more_tiles_than_waves_is_the_samples_one_by_one():
     y = net.forward(x)
     for i in (0, 31, 51, 63):
         assert np.array_equal(y[i], net.forward(x[i:i + 1])[0])
+
+
+def test_epoch_longer_than_the_set():
+    """Samples drawn with repetition: ten batches from a set of five."""
+    b, h, w = 4, 8, 32
+    x, t = _data(11, 5, h, w)
+    order = np.random.default_rng(2).integers(0, 5, 10 * b).astype(np.int32)
+    p = O.init_params(4)
+    one, many = _net(b, h, w), _net(b, h, w)
+    one.set_params(p)
+    many.set_params(p)
+    losses = [one.train_step(x[order[k:k + b]], t[order[k:k + b]], 1e-3)
+              for k in range(0, 10 * b, b)]
+    many.load_dataset(x, t)
+    mean = many.train_epoch(order, b, 1e-3)
+    assert mean == np.float32(sum(float(v) for v in losses) / 10)
+    assert np.array_equal(one.get_params().view(np.int32), many.get_params().view(np.int32))
