@@ -284,6 +284,12 @@ class DeviceChunk:
     def timing(self, on=True):
         check(self.lib.tea_hip_timing_enable(self.handle, 1 if on else 0), "timing")
 
+    def ahead_taken(self):
+        """Passes queued ahead that calls took over: (CG, mixed/FCG, Jacobi)."""
+        v = (ctypes.c_long * 3)()
+        check(self.lib.tea_hip_ahead_taken(self.handle, v), "ahead_taken")
+        return tuple(v)
+
     def kernel_stats(self):
         out = {}
         for k, name in enumerate(native.kernel_names()):

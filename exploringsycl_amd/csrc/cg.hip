@@ -1088,6 +1088,7 @@ int tea_hip_cg_calc_w(tea_hip_chunk* c, double* pw) {
     if (c->ra_w && c->pend_u && c->pend_p && c->pend_halo && !c->held && c->pre_halo < 0 &&
         c->pend_alpha == c->ra_alpha && c->pend_beta == c->ra_beta) {
       commit_cg_step(c, c->ra_step, c->pend_alpha);
+      c->taken[0] += 1;
       c->ra_w = false;
       c->ra_fail = 0;
       const int slot = c->ra_wi;
@@ -1171,6 +1172,7 @@ int tea_hip_cg_calc_ur(tea_hip_chunk* c, double alpha, double* rrn) {
     if (c->ra_r && c->ra_w && alpha == c->ra_alpha && !c->pend_u && !c->pend_p &&
         !c->pend_halo && !c->held && c->pre_halo < 0) {
       swap_ptr(f[TEA_FIELD_R], c->r_alt);
+      c->taken[0] += 1;
       c->pend_u = true;
       c->pend_alpha = alpha;
       c->ra_r = false;

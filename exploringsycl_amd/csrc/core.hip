@@ -682,6 +682,13 @@ int tea_hip_kernel_stats(tea_hip_chunk* c, int kernel_id, long* launches,
   return TEA_HIP_OK;
 }
 
+int tea_hip_ahead_taken(tea_hip_chunk* c, long taken[3]) {
+  TEA_CHECK_CHUNK(c);
+  TEA_CHECK_ARG(taken != nullptr, "null output");
+  for (int k = 0; k < 3; ++k) taken[k] = c->taken[k];
+  return TEA_HIP_OK;
+}
+
 int tea_hip_timing_reset(tea_hip_chunk* c) {
   TEA_CHECK_CHUNK(c);
   TEA_RETURN_IF(sync_chunk(c));

@@ -1058,6 +1058,7 @@ int mp_calc_w(tea_hip_chunk* c, bool fcg, double alpha, int apply_u, double beta
   int len = c->nspan;
   if (taken) {
     commit_mp_step(c, c->mra_step, alpha);
+    c->taken[1] += 1;
     c->mra_w = false;
     c->mra_fail = 0;
   } else if (use_pair_blocks(c, 1)) {
@@ -1133,6 +1134,7 @@ int mp_calc_r(tea_hip_chunk* c, bool fcg, double alpha, int use_net, double* rr,
   if (c->mra_r && c->mra_turn == kMraSlotR && c->mra_fcg == fcg && alpha == c->mra_alpha &&
       (!fcg || use_net == c->mra_coarse)) {
     swap_buf(c->mp_r, c->mp_r_alt);
+    c->taken[1] += 1;
     if (fcg) swap_buf(c->fcg_z, c->fcg_z_alt);
     c->mra_r = false;
     c->mra_turn = kMraSlotW;

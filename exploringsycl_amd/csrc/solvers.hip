@@ -1123,6 +1123,7 @@ int tea_hip_jacobi_iterate(tea_hip_chunk* c, double* error) {
     f[TEA_FIELD_U] = t;
     c->j_buf[0] = c->j_buf[1];
     c->jra -= 1;
+    c->taken[2] += 1;
     c->j_ring = true;
     c->j_since += 1;
     c->j_slot ^= 1;

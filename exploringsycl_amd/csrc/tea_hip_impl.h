@@ -1056,6 +1056,10 @@ struct tea_hip_chunk {
   double* fcg_xsum = nullptr;
   float* fcg_g = nullptr;
 
+  // Passes in flight that calls have taken over: FP64 CG, mixed-precision CG and
+  // FCG, Jacobi (tea_hip_ahead_taken).
+  long taken[3] = {};
+
   // Run-ahead of the fused CG iteration (cg.hip): the device forms alpha and
   // beta from its own sums and runs the next passes of the iteration, the
   // r-step (ra_r) and the w-step behind it (ra_w), into spare buffers before

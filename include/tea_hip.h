@@ -460,10 +460,17 @@ int tea_hip_flush(tea_hip_chunk* chunk);
 /* Kernel timing with HIP events on the handle's stream (off by default). */
 int tea_hip_timing_enable(tea_hip_chunk* chunk, int enable);
 /* Launch count and summed device time of kernel `kernel_id`
- * (0 <= kernel_id < tea_hip_num_kernels()). */
+ * (0 <= kernel_id < tea_hip_num_kernels()).  "cg_ra_finish" counts the sums
+ * that the device finished for the CG run-ahead: on grids of up to 2048 blocks
+ * of 512 cells the pass behind forms them and nothing of that name is launched
+ * (its time is then 0). */
 int tea_hip_kernel_stats(tea_hip_chunk* chunk, int kernel_id,
                          long* launches, double* total_ms);
 int tea_hip_timing_reset(tea_hip_chunk* chunk);
+/* Passes queued ahead of the host that calls have taken over since the chunk
+ * was created: taken[0] FP64 CG's w- and r-steps, taken[1] those of
+ * mixed-precision CG and FCG, taken[2] Jacobi sweeps. */
+int tea_hip_ahead_taken(tea_hip_chunk* chunk, long taken[3]);
 int tea_hip_num_kernels(void);
 const char* tea_hip_kernel_name(int kernel_id);
 

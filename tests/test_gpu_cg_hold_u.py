@@ -97,12 +97,17 @@ def _run(x, y, h, on, iters, between=(), where="end"):
             scalars += [pw, rrn]
             rro = rrn
         fields = [c.read(n) for n in FIELDS]
-    return np.array(scalars), seen + fields
+        taken = c.ahead_taken()[0]
+    return np.array(scalars), seen + fields, taken
 
 
 def _check(x, y, h, iters, **kw):
-    s0, f0 = _run(x, y, h, False, iters, **kw)
-    s1, f1 = _run(x, y, h, True, iters, **kw)
+    s0, f0, n0 = _run(x, y, h, False, iters, **kw)
+    s1, f1, n1 = _run(x, y, h, True, iters, **kw)
+    # Every step but the first and, with three interruptions, those they drop;
+    # none at odd x.
+    assert n0 == 0
+    assert n1 == 0 if x % 2 else n1 >= (2 * iters - 1 if not kw else iters)
     assert np.isfinite(s0).all()
     assert np.array_equal(s0.view(np.uint64), s1.view(np.uint64))
     assert len(f0) == len(f1)

@@ -1,10 +1,12 @@
 """The CG run-ahead on grids whose passes form alpha and beta from the block
 sums of the pass before them (up to 2048 blocks of 512 cells) and on the
 first size past that, where a finisher forms them: bit for bit the iteration
-without the run-ahead, at the edges of the tree's groups of 512 blocks."""
+without the run-ahead, every pass but the first taken over, at the edges of the
+tree's groups of 512 blocks."""
 
 import pytest
 
+from tests.test_gpu_cg_hold_u import _check
 from tests.test_gpu_run_ahead import H, _cg, _same
 
 pytestmark = pytest.mark.gpu
@@ -23,3 +25,4 @@ def test_consuming_passes_match_the_plain_iteration(x, y):
     assert _same(s0, s1)
     for n in f0:
         assert _same(f0[n], f1[n]), n
+    _check(x, y, H, 12)

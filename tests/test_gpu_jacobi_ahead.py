@@ -92,7 +92,8 @@ def _run(x, y, h, sweeps, between, env):
                 _between(c, between[it // 5], seen)
         seen.extend(c.read(n) for n in ("u", "r"))
         seen.append(np.array(c.field_summary()))
-    return np.array(errors), seen
+        taken = c.ahead_taken()[2]
+    return np.array(errors), seen, taken
 
 
 MIXED = ("mixed w", "mixed r", "mixed iteration", "precondition", "fcg")
@@ -128,6 +129,14 @@ def _check(x, y, h, between):
     want = _run(x, y, h, sweeps, between, {"TEA_HIP_PAIRS": "0"})
     for env in ({"TEA_HIP_RUN_AHEAD": "0"}, {"TEA_HIP_RUN_AHEAD": "1"}):
         got = _run(x, y, h, sweeps, between, env)
+        if env["TEA_HIP_RUN_AHEAD"] == "0" or -(-x * y // 512) > 128 * 512:
+            assert got[2] == 0   # or more block sums than one block adds
+        elif between:
+            # of each five sweeps between two interruptions the first is not
+            # taken over, nor the one after a guess of the sequence's end
+            assert got[2] >= 3 * (sweeps // 5)
+        else:
+            assert got[2] == sweeps - 1
         assert np.array_equal(want[0], got[0])
         assert len(want[1]) == len(got[1])
         for a, b in zip(want[1], got[1]):

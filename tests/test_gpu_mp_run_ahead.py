@@ -84,16 +84,19 @@ def _solve(cells, coarse, ahead, iters, refresh, stray=None):
         if fcg:
             fields.append(c.read_z())
         fields.append(c.read("u"))
-    return np.array(scalars), fields
+        taken = c.ahead_taken()[1]
+    return np.array(scalars), fields, taken
 
 
 def _same(a, b):
     return np.array_equal(np.asarray(a).view(np.uint8), np.asarray(b).view(np.uint8))
 
 
-def _check(cells, coarse, **kw):
-    s0, f0 = _solve(cells, coarse, False, **kw)
-    s1, f1 = _solve(cells, coarse, True, **kw)
+def _check(cells, coarse, least, **kw):
+    """`least`: passes that the run-ahead has to have been taken over for."""
+    s0, f0, n0 = _solve(cells, coarse, False, **kw)
+    s1, f1, n1 = _solve(cells, coarse, True, **kw)
+    assert n0 == 0 and n1 >= least, (n0, n1)
     assert np.isfinite(s0).all()
     assert _same(s0, s1)
     for a, b in zip(f0, f1):
@@ -108,8 +111,9 @@ def _check(cells, coarse, **kw):
     ((128, 64), "sweeps"), ((1024, 1024), "sweeps"), ((256, 64), "net"), ((1024, 96), "net")])
 def test_run_ahead_is_the_plain_iteration(cells, coarse):
     """22 iterations, a refresh after every 7: the second refresh falls where
-    the first taught the library not to queue a w-step."""
-    _check(cells, coarse, iters=22, refresh=7)
+    the first taught the library not to queue a w-step.  Every step but the
+    first w-step and those after a refresh is taken over."""
+    _check(cells, coarse, 2 * 22 - 4, iters=22, refresh=7)
 
 
 @pytest.mark.parametrize("coarse", [None, "sweeps"])
@@ -134,7 +138,7 @@ def test_run_ahead_is_dropped_when_the_host_strays(coarse):
             c.cg_calc_ur(1e-3)
         return alpha, use
 
-    _check((128, 64), coarse, iters=18, refresh=50, stray=stray)
+    _check((128, 64), coarse, 18, iters=18, refresh=50, stray=stray)
 
 
 @pytest.mark.parametrize("cells,coarse", [((128, 64), None), ((121, 50), None),
@@ -152,7 +156,7 @@ def test_a_pass_in_flight_is_taken_over_only_in_its_turn(cells, coarse):
             alpha = pr / pw
         return alpha, use
 
-    _check(cells, coarse, iters=9, refresh=50, stray=stray)
+    _check(cells, coarse, 9, iters=9, refresh=50, stray=stray)
 
 
 def test_init_of_a_second_solve_drops_a_pass_in_flight():
