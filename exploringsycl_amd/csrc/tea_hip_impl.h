@@ -133,11 +133,17 @@ __device__ inline int band_index(bool bands = true) {
   return seg + xcd_span((int)blockIdx.x - seg, left < seg_len ? left : seg_len);
 }
 // FP64 passes keep the launch order where rows are 8 blocks (or a multiple)
-// and up to 48 cells long: the rows above and below then lie on the same XCD
-// anyway, and the plain front is 1% faster (4096^2 249.6 against 251.5 us,
-// x = 4124 185.9 against 188.2; even at x = 4156, where a fifth of the cells
-// above is on another XCD; x = 4060 193.2 against 182.1).
-inline int bands_for(int x) { return x < kNumXcd * 512 || x % (kNumXcd * 512) > 48; }
+// and up to an eighth of a block long: all but that share of the cells above
+// and below a block then lie on its own XCD anyway, and the plain front is
+// faster.  CG per iteration, launch order against bands: x = 4100 239.1, 240.8
+// us, 4156 242.4, 243.4, 8196 476.5, 483.2, 8252 478.9, 486.4; past the line 4176
+// 240.1, 240.3, 4200 243.6, 242.6, 8300 481.3, 485.3, 8400 486.5, 480.0, 4352
+// 251.1, 240.6; below whole rows 4080 250.7, 236.4.  (The crossing lies at 80 to
+// 150 cells, later with longer rows.)
+inline int bands_for(int x) {
+  const int row = kNumXcd * 512;
+  return x < row || x % row > 512 / 8;
+}
 
 // Cross-lane moves on the VALU's data-parallel-primitive (DPP) path instead
 // of LDS permutes.  CTRL is a DPP control: 0x130 wave_shl:1 (lane l takes
