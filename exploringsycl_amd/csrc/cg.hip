@@ -654,7 +654,8 @@ struct NormBody {
   }
 };
 
-// The 2-norm over cell pairs, one pair per lane (more than one group): 8 bytes per cell, the sum tree's first level in-lane.
+// The 2-norm over cell pairs, one pair per lane (more than one group): 8 bytes
+// per cell, the sum tree's first level in-lane.
 __global__ __launch_bounds__(kBlock) void norm_pair_kernel(
     Geo g, const double* __restrict__ b, double* sub, int nblk) {
   const int blk = band_index(g.bands);
@@ -758,13 +759,11 @@ void ensure_p_ring(tea_hip_chunk* c) {
 // (TeaLeaf/drivers/cg_driver.c:87-113): two host round trips per iteration,
 // each costing the wait for the finisher's values, the host's arithmetic and
 // a launch (about 13.5 us of a 272 us iteration at 4096^2).  The device
-// forms the same scalars itself: the last block of each finisher runs the
-// host's final tree passes over the grid's partials and divides
-// (span_finish_kernel's run-ahead tail, core.hip), and the next pass of the
-// iteration is already queued behind it, writing only spare buffers (on grids
-// of at most kConsumeBlocks blocks there is no finisher: the next pass itself
-// sums and divides, see RaScalar, and its first block hands the host the
-// values):
+// forms the same scalars itself, and the next passes of the iteration are
+// already queued, writing only spare buffers.  On grids of at most
+// kConsumeBlocks blocks the next pass sums and divides (RaScalar), and its
+// first block hands the host the values; beyond, a finisher does both
+// (finish_out, core.hip):
 //   the r-step: r - alpha w into r_alt, and r.r;
 //   the w-step: u + alpha p into u_alt (or held), p = beta p + r into a spare
 //     p with the U/P halo ring, w = A p into w_alt, p.w.
@@ -782,6 +781,8 @@ void ensure_p_ring(tea_hip_chunk* c) {
 
 constexpr int kRaW = 0, kRaRStep = 1;  // slot kinds
 
+// x even: the passes take odd x too, and mixed precision runs ahead there, but
+// FP64 CG's run-ahead has been measured and tested at even x only.
 bool ra_possible(const tea_hip_chunk* c) {
   return c->ra_enabled && !c->ra_off && c->fused && c->poll && c->pairs && c->geo.x % 2 == 0 &&
          c->ra_rro_known && c->ra_fail < 3 && use_pair_blocks(c, 1) && use_pair_blocks(c, 2);

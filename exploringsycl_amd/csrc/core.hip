@@ -250,7 +250,10 @@ __global__ __launch_bounds__(kFinishWaves * kWave) void span_finish_kernel(
 // one to count itself done runs the remaining passes over the group sums in
 // part.  Those are stored and read at device scope (past the XCDs' own L2s),
 // and the count follows its sum's store, so no fence is needed: a release
-// fence writes back a whole L2.
+// fence writes back a whole L2.  That order rests on the hardware, not on the
+// language's memory model (all these accesses are relaxed): s_waitcnt vmcnt(0)
+// ends once the device-scope store is out, and the last block's loads are issued
+// only after the branch on the count it read.
 __device__ inline void st_agent(double* p, double v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

@@ -1307,7 +1307,7 @@ __global__ __launch_bounds__(256) void out_tile_kernel(OutLevel lv0, OutLevel lv
 // The factors g of the coarse directions, into g[0] and g[1].  One level:
 // g = (y.rbar) / (y.T y), 0 unless y.T y > 0 and the ratio is finite.  Two
 // levels: the joint minimiser of the energy norm of e - g0 P0 y0 - g1 P1 y1
-// (the system of gamma2_kernel), whose cross entry c0^2 y0.T0 (Q y1) is the
+// (a 2 x 2 system), whose cross entry c0^2 y0.T0 (Q y1) is the
 // sum over level-1 cells of xsum * y1 (T0 is symmetric).  Each sum in the
 // order of one kGammaThreads-thread block: thread t adds elements t,
 // t + kGammaThreads, ... in turn, then the LDS tree.

@@ -429,6 +429,9 @@ __global__ __launch_bounds__(kQuadThreads * KS) void mp_w4_kernel(Geo g, MpArgs 
     UB = ld2_nt(a.u, inB0 || inB1 ? ub : x + 2, g.nt_half);
   }
   if (UM == 3) {
+    // With a ring of three (no room for the run-ahead's fourth p) p_h is the
+    // p_new buffer: each of its cells is read here by the wave that overwrites
+    // it below, and by no other.
     HA = ld2(a.p_h, inA0 || inA1 ? ua : x + 2);
     HB = ld2(a.p_h, inB0 || inB1 ? ub : x + 2);
     GA = ld2(a.p_h2, inA0 || inA1 ? ua : x + 2);
@@ -653,9 +656,11 @@ __global__ __launch_bounds__(kQuadThreads) void mp_r4_kernel(
   block_sums_quads<RW ? 2 : 1>(v, sub, nblk, blk, threadIdx.x);
 }
 
-// MpTrueResidualBody's arithmetic (below) with one cell pair per thread: r = u0 - A u in FP64 with the FP64 coefficients, r rounded to FP32
-// into r32, and the three sums (r32.r32, r.r, r32.w) as block sums.  u's left and right neighbours come from the adjacent
-// lanes by DPP; lane 0 loads u at e - 1, lane 63 u and kx at e + 2.
+// MpTrueResidualBody's arithmetic (below) with one cell pair per thread: r =
+// u0 - A u in FP64 with the FP64 coefficients, r rounded to FP32 into r32, and
+// the three sums (r32.r32, r.r, r32.w) as block sums.  u's left and right
+// neighbours come from the adjacent lanes by DPP; lane 0 loads u at e - 1, lane
+// 63 u and kx at e + 2.
 __global__ __launch_bounds__(kBlock) void mp_residual1_kernel(
     Geo g, const double* __restrict__ u, const double* __restrict__ u0,
     const double* __restrict__ kx, const double* __restrict__ ky, float* __restrict__ r32,

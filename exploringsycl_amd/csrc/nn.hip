@@ -283,11 +283,11 @@ __device__ inline void conv_fwd_lds_block(
   store_out_row(out + pix * kC, acc, bco, hf);
 }
 
-// conv_fwd_lds_kernel over R output rows per block: the block stages R + 2
+// conv_fwd_lds_block over R output rows per block: the block stages R + 2
 // input rows once (instead of 3 per output row) and each wave keeps its
 // weight fragments in registers across the R rows (instead of reloading
 // them per 32-pixel tile).  Each tile's MFMA sequence, bias and ReLU are
-// those of conv_fwd_lds_kernel, so the output is bitwise the same.
+// those of conv_fwd_lds_block, so the output is bitwise the same.
 // W / 128 x H / R x B blocks.
 template <int CIN, int R>
 __device__ inline void conv_fwd_rows_block(
@@ -305,7 +305,7 @@ __device__ inline void conv_fwd_rows_block(
   const size_t plane = (size_t)(H + 2) * Wp;
   const bf16* inb = in + (size_t)b * plane * CIN;
   const int x0 = seg * 128;
-  // Weights and biases first (as conv_fwd_lds_kernel).
+  // Weights and biases first (as conv_fwd_lds_block).
   bf16x8 A[NS];
 #pragma unroll
   for (int t = 0; t < NS; ++t) A[t] = weight_frag(wt, t, lane);

@@ -281,8 +281,8 @@ __device__ inline double block_total(const double* __restrict__ sub, int nblk) {
 // in the last-level cache) 12.4 us in launch order, 8.8 in bands and kept in that
 // cache.  A sweep was 24.9 us there with the halo update (3.5), the finisher
 // (3.4) and the host's round trip between sweeps.
-// With HALO the depth-1 U halo update that precedes it is folded in: a neighbour on the ring is the cell's own mirror image, and the ring of
-// the new u gets what that update leaves (the old values); the ring of the
+// With HALO the depth-1 U halo update that precedes it is folded in: a neighbour
+// on the ring is the cell's own mirror image, and the ring of the new u gets what that update leaves (the old values); the ring of the
 // old u is left to jacobi_settle.  With prev the first block also finishes
 // the sum of the sweep before (its block sums in prev) into out.
 template <int KS, bool HALO>
@@ -989,7 +989,8 @@ int cheby_two_steps(tea_hip_chunk* c, double a0, double b0, double a1,
   return TEA_HIP_OK;
 }
 
-// One inner step: the single pass or one launch per reference kernel; the new sd goes to the second buffer in the single pass.
+// One inner step: the single pass or one launch per reference kernel; the new sd
+// goes to the second buffer in the single pass.
 int ppcg_step(tea_hip_chunk* c, double alpha, double beta) {
   double** f = c->field;
   const Geo g = c->geo;

@@ -1191,11 +1191,6 @@ int resolve_ready(tea_hip_chunk* c);
 // partials; results go to out[0..nr).
 int finish_reduction(tea_hip_chunk* c, int nr, double* out);
 
-// Finishes nr sums from their block sums (the first nr arrays of sub, c->sub
-// unless given), sum q into the first value of array slot + q of c->partials
-// (*len = 1).  With poll (slot 0), the next finish waits for the values
-// themselves instead of the stream; only for a finish that follows with no
-// other kernel writing the partials in between.
 // The run-ahead's scalar, formed by the finisher: mode 0 (after a w-step)
 // alpha = rro / sum into ra[0]; mode 1 (after an r-step) beta = sum / rro into
 // ra[1] and sum into ra[2].  rro is ra[2] when from_dev, else the value.  The
@@ -1212,6 +1207,11 @@ struct RaTail {
 // The finisher of nr sums (1 or 2) of c->sub with the run-ahead's scalar, into
 // out; not waited for.
 int launch_span_finish_ra(tea_hip_chunk* c, int nr, double* out, const RaTail& tail);
+// Finishes nr sums from their block sums (the first nr arrays of sub, c->sub
+// unless given), sum q into the first value of array slot + q of c->partials
+// (*len = 1).  With poll (slot 0), the next finish waits for the values
+// themselves instead of the stream; only for a finish that follows with no
+// other kernel writing the partials in between.
 int launch_span_finish(tea_hip_chunk* c, int nr, int* len, int slot = 0,
                        bool poll = false, const double* sub = nullptr);
 

@@ -1,8 +1,7 @@
 """The run-ahead of the fused CG iteration: after cg_calc_w and cg_calc_ur
-the library queues the next pass with alpha or beta formed on the device
-(the finisher's last block runs the host's final tree passes and divides),
-into spare buffers, and the host's next call takes it over when
-its scalar is bitwise the device's.  These tests run the CG driver's call
+the library queues the next passes with alpha or beta formed on the device
+(by the pass behind, or by a finisher on larger grids), into spare buffers,
+and the host's next call takes it over when its scalar is bitwise the device's.  These tests run the CG driver's call
 sequence (TeaLeaf/drivers/cg_driver.c:69-124) with the run-ahead on and off
 (TEA_HIP_RUN_AHEAD=0) and require the same scalars and fields bit for bit,
 also when the host strays from the sequence (another alpha, reads and
@@ -45,7 +44,8 @@ def _fields(x, y, seed):
 def _cg(x, y, seed, run_ahead, iters, stray=None):
     """cg_init, then `iters` iterations of the driver's sequence; `stray(c,
     it, alpha)` may act between the calls and return the alpha to pass.
-    Returns the scalars, the final fields and the run-ahead finisher launches."""
+    Returns the scalars, the final fields and the number of sums that the
+    device finished for the run-ahead (cg_ra_finish)."""
     density, energy = _fields(x, y, seed)
     with _chunk(x, y, run_ahead) as c:
         c.timing(True)
@@ -82,7 +82,7 @@ def test_run_ahead_is_the_plain_iteration_bit_for_bit(cells):
     s0, f0, r0 = _cg(x, y, 3, False, 40)
     s1, f1, r1 = _cg(x, y, 3, True, 40)
     assert r0 == 0
-    # Two run-ahead finishers per iteration.
+    # Two sums per iteration.
     assert r1 >= 2 * 36, r1
     assert _same(s0, s1)
     for n in f0:
@@ -90,7 +90,7 @@ def test_run_ahead_is_the_plain_iteration_bit_for_bit(cells):
 
 
 def test_run_ahead_with_odd_width_stays_off():
-    """x odd: the pair-per-thread kernels (and the run-ahead) do not apply."""
+    """x odd: the pair-per-thread kernels apply, the FP64 run-ahead does not."""
     x, y = 121 + 2 * H, 50 + 2 * H
     s0, f0, r0 = _cg(x, y, 5, False, 10)
     s1, f1, r1 = _cg(x, y, 5, True, 10)
@@ -129,7 +129,8 @@ def test_run_ahead_is_dropped_when_the_host_strays():
 def test_run_ahead_whole_solves_match(tmp_path):
     """Three timesteps of a rectangle deck through the host program with
     the run-ahead on and off: the same iterations, summaries and final
-    field, bit for bit, and the run-ahead taken over most passes."""
+    field, bit for bit, and a sum finished for the run-ahead in every
+    iteration."""
     deck = Deck.with_random_rectangles(
         512, 512, 16, problem_seed(2, 7), density="uniform", end_step=3,
         coefficient="inverse", extent=10.0)
